@@ -934,41 +934,7 @@ int run_small_m(const GemmArgs &a)
 
 }  // namespace
 
-// 33 <= M <= 64 with few channels: see run_gemm.
-static bool takes_slabs(int M, int N)
-{
-    const int tile_wgs = ((M + 31) / 32) * ((N + 127) / 128);
-    return M <= 64 && tile_wgs < 150;
-}
-
-static int run_gemm(const GemmArgs &a)
-{
-    if (a.M <= 32)
-        return run_small_m(a);
-    // 33 <= M <= 64 with few channels and no workspace to split the k range with: the 32 x 128
-    // MFMA tiles would number under ~150 and each would walk the whole k range alone (19 us at
-    // N = 4096, K = 4096 whatever M is), so the small-M kernel runs over 32-row slabs instead
-    // (12-15 us; the weights are re-read per slab, from L2 / Infinity Cache).  With the workspace
-    // the split MFMA launch is faster still (10-11 us; 16 against 24-34 us at K = 11008).
-    const size_t split_bytes = eet::large_m_workspace(a.M, a.N, a.K, a.epi);
-    const bool can_split = split_bytes > 0 && a.ws != nullptr && a.ws_bytes >= split_bytes &&
-                           reinterpret_cast<uintptr_t>(a.ws) % 16 == 0;
-    if (takes_slabs(a.M, a.N) && !can_split && !eet::tuning().has_large_m) {
-        const int n_out = (a.epi == kEpiSwiglu) ? a.N / 2 : a.N;
-        for (int m0 = 0; m0 < a.M; m0 += 32) {
-            GemmArgs s = a;
-            s.M = (a.M - m0 < 32) ? a.M - m0 : 32;
-            s.A = a.A + (size_t)m0 * a.K;
-            s.C = a.C + (size_t)m0 * n_out;
-            if (a.residual)
-                s.residual = a.residual + (size_t)m0 * a.N;
-            if (int rc = run_small_m(s))
-                return rc;
-        }
-        return EET_OK;
-    }
-    return eet::run_large_m(a);
-}
+static int run_gemm(const GemmArgs &a) { return a.M <= 32 ? run_small_m(a) : eet::run_large_m(a); }
 
 static int check_gemm_args(const char *fn, const void *A, const void *W, const void *scale, const void *C, int M,
                            int N, int K)

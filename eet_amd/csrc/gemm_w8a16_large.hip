@@ -1,80 +1,78 @@
-// Large-M fused dequant-GEMM (M > 32 apart from the 32-row-slab case; prefill;
-// fp16-MFMA bound).
+// Large-M fused dequant-GEMM (M > 32: prompts, and decode steps of more than 32 sequences).
 //
 // Replaces the tensor-core side of fastertransformer::gemm_fp16_int_bias_act<uint8_t>
 // (3rdparty/cutlass_kernels/fpA_intB_gemm/fpA_intB_gemm_template.h:48-177).
 //
-// A workgroup of WNW wavefronts side by side owns a block tile of TM*16 rows x
-// WNW*TN*16 channels; each wavefront owns TM x TN tiles of
-// v_mfma_f32_16x16x32_f16 (TM*TN*4 fp32 accumulator registers).  What bounds
-// such a kernel on a CU is the LDS port (256 B/clk at best) against the matrix cores
-// (4 x 1024 flop/clk): a wavefront tile of WM x WN outputs needs (WM + WN) * 2 B
-// of operands per k for 2 * WM * WN flop, so wavefront tiles are made large
-// (128 x 64 where M allows) and only one operand goes through LDS:
-//   weights      every wavefront reads its own TN packed tiles straight from
-//                global memory into registers, two k-tiles ahead -- the packed
-//                layout is already the MFMA operand layout -- and widens them
-//                once per k-tile;
-//   activations  the block's rows x 64 slab is copied global -> LDS by the
-//                memory pipeline itself (buffer_load_dwordx4 ... lds: no
-//                staging registers, no ds_write) into a ring of four k-tile
-//                stages, three tiles ahead of the one being multiplied, and
-//                read from there by every wavefront.
-// One wavefront row per workgroup, so that two (or more) workgroups share a CU
-// with independent barriers; a 256 x 256 block of eight wavefronts with one
-// barrier measured 5-10 % slower than two 128 x 256 blocks.  Workgroups are
-// numbered so that the ones resident on an XCD at one time (workgroup i lands on
-// XCD i % 8) cover a compact block of rows x columns and share both operands in its L2.
+// A workgroup of WM x WN wavefronts owns a block of WM*TM*16 rows x WN*TN*16 channels; each wavefront owns
+// TM x TN tiles of v_mfma_f32_16x16x32_f16 (TM*TN*4 fp32 accumulator registers).  Both operands of a 64-wide
+// k-tile are copied global -> LDS by the memory pipeline itself (buffer_load_dwordx4 ... lds: no staging
+// registers, no ds_write) into a ring of D stages:
+//   weights      the packed 1 KiB tiles as they are: lane l of a wavefront reads its 16 bytes back with one
+//                conflict-free ds_read_b128, already in operand order, and widens them (one vector
+//                instruction per weight) while the matrix cores work on the step before;
+//   activations  16 "super-rows" of 256 B per pair of m-tiles (2u, 2u + 1), super-row j holding row j of both:
+//                the 16-byte piece 2g + h of row j of m-tile 2u + e sits at slot (4 * (2e + h) + g) ^ j, which
+//                lets a ds_read_b128 of the whole wavefront run at the full 256 B/clk of the LDS (128-byte rows
+//                with any XOR of the row index reach 150 B/clk); the lanes of one copy fetch whole 128-byte lines.
 //
-// A stage holds TM / 2 blocks of 4 KiB, one per pair of m-tiles (2u, 2u + 1):
-// 16 "super-rows" of 256 B, super-row j holding row j of both m-tiles.  The MFMA
-// operand of lane (g, j) for m-tile 2u + e, k half h -- the 16-byte piece 2g + h
-// of row j -- sits at slot (4 * (2e + h) + g) ^ j of super-row j.  With that
-// placement a ds_read_b128 of the whole wavefront runs at the full 256 B/clk of
-// the LDS (measured: 128-byte rows with any XOR of the row index reach 150 B/clk).
-// One DMA instruction fills 1 KiB = four super-rows; its lanes fetch whole
-// 128-byte lines of eight activation rows (the XOR only permutes the lanes
-// within a line).
+// What bounds it.  At thousands of rows the power the matrix cores draw (1.25-1.35 PFLOP/s at the clock that is
+// left), below that the way the k-loop is fed: an XCD's L2 hands a CU 118 KB/us when everything hits, but with
+// misses among the requests the two times add (60 KB/us at one miss in five), so what counts is few bytes per
+// flop, i.e. large blocks, on all 256 CUs at once.  The earlier form of this kernel kept the weights in registers,
+// two k-tiles ahead, and had to wait for all but the copies of the current step before each barrier (a copy whose
+// rows are all past M completes at once, ahead of older ones, and makes a deeper counted wait unsafe); a workgroup
+// alone on its CU then took 0.26-0.33 us per k-tile whatever its size.  Here
+//   * every copy touches memory (rows past M re-read row M - 1, a k-tile past the end re-reads the last one), so
+//     completion is in order, the wait before the hand-over counts the copies of D - 2 whole k-tiles, and the ring
+//     is really D deep;
+//   * the hand-over (wait, s_barrier) sits inside the stream of matrix instructions of the second-to-last of the
+//     TN steps of a k-tile, the operands of the next k-tile are read under those of the last step, and the widening
+//     is interleaved with them one vector instruction per matrix instruction: neither the barrier nor the LDS
+//     latency is exposed even with one wavefront per SIMD;
+//   * the block shape follows the problem (kTiles below): 20 shapes from 32 x 64 to 256 x 256.
+// Measured against that earlier kernel (us, QKV / O / gate-up / down of a 4096-wide layer, weights from HBM):
+//   M = 64    12288 <- 4096  21.7 -> 18.7   4096 <- 4096  13.9 -> 11.7   22016 <- 4096  32.5 -> 28.1   4096 <- 11008  22.9 -> 20.0
+//   M = 406                  49.8 -> 52.1                 26.5 -> 25.7                  87.6 -> 83.4                  51.2 -> 50.5
+//   M = 1024                100.0 -> 88.3                 38.2 -> 40.0                   157 -> 156                   92.5 -> 88.7
+//   M = 2048                  174 -> 169                  69.5 -> 65.1                   303 -> 308                    180 -> 159
+//   M = 8192                  629 -> 615                   232 -> 227                   1098 -> 1102                   562 -> 541
+// (geometric mean over 20 weight matrices of decoders 1024 .. 5120 wide, 40 .. 8192 rows: 1.10 x).
+// 32x32x16 matrix instructions (operands free by addressing, the weights being in LDS) were 8-12 % slower, wavefront
+// tiles of 128 x 128 with one wavefront per SIMD 20-30 %.
 #include "gemm_common.h"
 #include "tuning.h"
+
+#include <type_traits>
 
 using namespace eet;
 
 namespace {
 
-constexpr int kDmaStages = 4, kDmaAhead = 3;
-
-__device__ __forceinline__ constexpr int vmcnt_imm(int n)
-{
-    return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14);  // expcnt, lgkmcnt: no wait
-}
-
-template <int WNW, int TM, int TN>
-struct DmaShape {
-    static constexpr int kThreads = 64 * WNW;
-    static constexpr int kBM = TM * 16, kBN = WNW * TN * 16;
-    static constexpr int kStageVec = TM * 128;          // u32x4 per stage
-    static constexpr int kRowGroups = TM * 2;           // DMA instructions per k-tile (8 rows each)
-    static constexpr int kPerWave = kRowGroups / WNW;   // ... per wavefront
-    static_assert(kRowGroups % WNW == 0, "row groups must divide over the wavefronts");
+template <int TM, int TN, int WM, int WN, int D>
+struct TileShape {
+    static constexpr int kWaves = WM * WN;
+    static constexpr int kBM = WM * TM * 16, kBN = WN * TN * 16;
+    static constexpr int kAUnits = WM * TM * 2, kWUnits = WN * TN;      // 1 KiB copies per k-tile
+    static constexpr int kAVec = kAUnits * 64, kWVec = kWUnits * 64;    // u32x4 per stage
+    static constexpr int kA = (kAUnits + kWaves - 1) / kWaves, kW = (kWUnits + kWaves - 1) / kWaves;   // ... per wavefront
     static_assert(TM % 2 == 0, "a stage block holds a pair of m-tiles");
-    static_assert(kDmaStages * kStageVec * 16 <= 65536, "the stage ring must fit 64 KiB");
+    static_assert(D >= 2 && D <= 5 && D * (kAVec + kWVec) * 16 <= 163840, "the stage ring must fit the LDS");
+    static_assert((D - 1) * (kA + kW) <= 63, "the copies in flight must fit the wait counter");
 };
 
-template <int WNW, int TM, int TN>
-__global__ __launch_bounds__(64 * WNW) __attribute__((amdgpu_waves_per_eu(2))) void w8a16_large_m_kernel(
+template <int TM, int TN, int WM, int WN, int D>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2))) void w8a16_large_m_kernel(
     const _Float16 *__restrict__ A, const u32x4 *__restrict__ Wp, const _Float16 *__restrict__ scale,
     _Float16 *__restrict__ C, int M, int N, int K, int m_blocks, int n_blocks,
     const _Float16 *__restrict__ residual, int epi, int ksplit, float *__restrict__ partial)
 {
 #if defined(__HIP_DEVICE_COMPILE__)  // buffer-resource builtins exist in the device pass only
-    using S = DmaShape<WNW, TM, TN>;
-    // one array per stage: the compiler tells them apart when it places waits
-    // between the DMA writes and the LDS reads
-    __shared__ u32x4 st0[S::kStageVec], st1[S::kStageVec], st2[S::kStageVec], st3[S::kStageVec];
+    using S = TileShape<TM, TN, WM, WN, D>;
+    __shared__ u32x4 lds[D][S::kAVec + S::kWVec];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: feeds scalar offsets and M0
+    const int wm = wave / WN, wn = wave % WN;
     const int g = lane >> 4, j = lane & 15;
     const int ktiles = K >> 6, ntiles = N >> 4;
     // With ksplit > 1 (grid.y) the workgroup covers k-tiles [kbeg, kbeg + nk) only and
@@ -83,56 +81,53 @@ __global__ __launch_bounds__(64 * WNW) __attribute__((amdgpu_waves_per_eu(2))) v
     const int kbeg = (int)((long)split * ktiles / ksplit);
     const int nk = (int)((long)(split + 1) * ktiles / ksplit) - kbeg;
 
+    // Workgroups are numbered so that the ones resident on an XCD at one time (workgroup i lands on XCD i % 8)
+    // cover a compact block of rows x columns and share both operands in its L2: bands of kBand column blocks
+    // across all row blocks, the column block running fastest inside a band, a contiguous range of that order per
+    // XCD (with one column block after the other, 64 row blocks shared one weight block and each fetched activation
+    // rows of its own from the fabric: M = 8192, 4096 -> 12288 went from 1.18 to 1.28 PFLOP/s with the bands).
     const int total = m_blocks * n_blocks;
     const int per_xcd = (total + 7) / 8;
     const int tile = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (tile >= total)
         return;
-    // Tile order: bands of kBand column blocks across all row blocks, the column block running fastest inside a
-    // band.  An XCD works through a contiguous range of that order, so the ~64 workgroups resident on it at one
-    // time cover about 8 row blocks x 8 column blocks and every activation and weight line they fetch is shared
-    // by eight of them in its L2 (with one column block after the other, 64 row blocks shared one weight block
-    // and each fetched activation rows of its own from the fabric: M = 8192, 4096 -> 12288 went from 1.18 to
-    // 1.28 PFLOP/s with the bands, the M = 2048 shapes gained 0-3 %).
     constexpr int kBand = 8;
     const int band = tile / (kBand * m_blocks), r = tile % (kBand * m_blocks);
     const int bw = min(kBand, n_blocks - band * kBand);   // column blocks of this band (the last one may be narrower)
     const int n_blk = band * kBand + r % bw, m_blk = r / bw;
     const int m0 = m_blk * S::kBM;
-    const int nt0 = n_blk * (WNW * TN) + wave * TN;
+    const int ntb = n_blk * (WN * TN), nt0 = ntb + wn * TN;
+    const int rows = min(M - m0, S::kBM);
 
-    // Both operands are addressed through buffer resources: a 32-bit lane offset
-    // plus a scalar offset per tile.  The range check of a buffer load covers the
-    // lane offset only, not the scalar one: activation rows >= M are out of range
-    // by their lane offset and read as zeros; the weight tile index lives in the
-    // scalar offset, so an n-tile >= N/16 of a block that overhangs N is clamped
-    // to the last real tile (its products are never stored).
-    const size_t a_bytes = (size_t)(M - m0) * K * 2;
+    // Both operands are addressed through buffer resources: a 32-bit lane offset plus a scalar offset per tile.
+    // Rows past M re-read row M - 1 and an n-tile past N / 16 the last one: their products are never stored, and no
+    // copy is out of range (see above).  A wavefront whose share of a k-tile's copies is smaller repeats its last.
     const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<_Float16 *>(A + (size_t)m0 * K), 0, a_bytes > 0xffffffffull ? 0xffffffffu : (unsigned)a_bytes,
-        0x00020000);
+        const_cast<_Float16 *>(A + (size_t)m0 * K), 0, (unsigned)rows * (unsigned)K * 2u, 0x00020000);
     const __amdgpu_buffer_rsrc_t wrsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4 *>(Wp), 0, (unsigned)((size_t)K * N), 0x00020000);
+    auto aunit = [&](int i) { return min(wave * S::kA + i, S::kAUnits - 1); };
+    auto wunit = [&](int i) { return min(wave * S::kW + i, S::kWUnits - 1); };
     const int woff = lane * 16;
-    unsigned wtile[TN];  // byte offset of the n-tile's first k-tile
+    unsigned wtile[S::kW];  // byte offset of the n-tile's first k-tile
 #pragma unroll
-    for (int t = 0; t < TN; ++t)
-        wtile[t] = (unsigned)min(nt0 + t, ntiles - 1) * (unsigned)ktiles * 1024u;
-
-    // DMA instruction rg = wave * kPerWave + i fills slots [64 rg, 64 rg + 64): block u = rg / 4,
-    // super-rows 4 (rg % 4) .. + 3.  Lane l writes slot s = l % 16 of super-row sj = 4 (rg % 4) + l / 16,
-    // which holds piece 2 pg + h of row sj of m-tile 2u + e, where 4 (2e + h) + pg = s ^ sj.
-    int aoff[S::kPerWave];
+    for (int i = 0; i < S::kW; ++i)
+        wtile[i] = (unsigned)min(ntb + wunit(i), ntiles - 1) * (unsigned)ktiles * 1024u;
+    // Copy rg of the activations fills slots [64 rg, 64 rg + 64): block u = rg / 4, super-rows 4 (rg % 4) .. + 3.
+    // Lane l writes slot s = l % 16 of super-row sj = 4 (rg % 4) + l / 16, which holds piece 2 pg + h of row sj of
+    // m-tile 2u + e, where 4 (2e + h) + pg = s ^ sj.
+    int aoff[S::kA];
 #pragma unroll
-    for (int i = 0; i < S::kPerWave; ++i) {
-        const int rg = wave * S::kPerWave + i, u = rg >> 2, sj = 4 * (rg & 3) + (lane >> 4);
+    for (int i = 0; i < S::kA; ++i) {
+        const int rg = aunit(i), u = rg >> 2, sj = 4 * (rg & 3) + (lane >> 4);
         const int p = (lane & 15) ^ sj, pg = p & 3, h = (p >> 2) & 1, e = p >> 3;
-        aoff[i] = ((2 * u + e) * 16 + sj) * K * 2 + (2 * pg + h) * 16;
+        aoff[i] = min((2 * u + e) * 16 + sj, rows - 1) * K * 2 + (2 * pg + h) * 16;
     }
     int rs[4];  // operand slot of this lane within a block, by 2e + h
 #pragma unroll
     for (int c = 0; c < 4; ++c)
-        rs[c] = j * 16 + ((4 * c + g) ^ j);
+        rs[c] = wm * TM * 128 + j * 16 + ((4 * c + g) ^ j);
+    const int wr0 = S::kAVec + wn * TN * 64 + lane;
 
     floatx4 acc[TN][TM];
 #pragma unroll
@@ -141,96 +136,126 @@ __global__ __launch_bounds__(64 * WNW) __attribute__((amdgpu_waves_per_eu(2))) v
         for (int mt = 0; mt < TM; ++mt)
             acc[t][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    u32x4 wraw[2][TN];
-
-    auto dma_tile = [&](u32x4 *stage, int kt) {
+    constexpr int L = S::kA + S::kW;   // copies of one k-tile per wavefront
+    auto dma_tile = [&](int s, int kt) {
 #pragma unroll
-        for (int i = 0; i < S::kPerWave; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(arsrc, stage + (wave * S::kPerWave + i) * 64, 16, aoff[i], kt * 128,
-                                                     0, 0);
-    };
-    auto load_w = [&](u32x4 (&dst)[TN], int kt) {
+        for (int i = 0; i < S::kW; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wrsrc, &lds[s][S::kAVec + wunit(i) * 64], 16, woff,
+                                                     wtile[i] + (unsigned)(kbeg + kt) * 1024u, 0, 0);
 #pragma unroll
-        for (int t = 0; t < TN; ++t)
-            dst[t] = __builtin_bit_cast(
-                u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, woff, wtile[t] + (unsigned)kt * 1024u, 0));
+        for (int i = 0; i < S::kA; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(arsrc, &lds[s][aunit(i) * 64], 16, aoff[i], (kbeg + kt) * 128, 0, 0);
+    };
+    auto read_op = [&](half8 (&op)[2], const u32x4 *cur, int mt) {
+        op[0] = __builtin_bit_cast(half8, cur[(mt >> 1) * 256 + rs[2 * (mt & 1)]]);
+        op[1] = __builtin_bit_cast(half8, cur[(mt >> 1) * 256 + rs[2 * (mt & 1) + 1]]);
     };
 
-    // One k-tile: A from `cur`, raw weights from wb; the DMA for tile kt + 3 goes
-    // to `ahead`, the weights of tile kt + 2 replace wb once it is widened.
-    auto step = [&](const u32x4 *cur, u32x4 *ahead, u32x4 (&wb)[TN], int kt) {
-        dma_tile(ahead, kbeg + min(kt + kDmaAhead, nk - 1));
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+        dma_tile(i, min(i, nk - 1));
         __builtin_amdgcn_sched_barrier(0);
-        half8 w0[TN], w1[TN];
+    }
+    half8 op[TM][2], w0, w1;   // operands of the current k-tile, weights of the current step
+    u32x4 raw;                 // the packed weights of the step after
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((D - 1) * L) : "memory");
+#pragma unroll
+    for (int mt = 0; mt < TM; ++mt)
+        read_op(op[mt], lds[0], mt);
+    {
+        const u32x4 r0 = lds[0][wr0];
+        if (TN > 1)
+            raw = lds[0][wr0 + 64];
+        w0 = widen8(r0.x, r0.y);
+        w1 = widen8(r0.z, r0.w);
+    }
+
+    // One k-tile, in stage s of the ring: TN steps of one n-tile against all m-tiles.  kReq: k-tile `nx` is copied
+    // into the stage once every wavefront has read it.
+    constexpr int TB = TN >= 2 ? TN - 2 : 0;   // the step that starts with the hand-over
+    auto tile_step = [&](auto s_c, auto req_c, int nx) {
+        constexpr int s = decltype(s_c)::value, sn = (s + 1) % D;
+        constexpr bool kReq = decltype(req_c)::value;
 #pragma unroll
         for (int t = 0; t < TN; ++t) {
-            w0[t] = widen8(wb[t].x, wb[t].y);
-            w1[t] = widen8(wb[t].z, wb[t].w);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        load_w(wb, kbeg + min(kt + 2, nk - 1));
-        half8 aop[2][2];
-        aop[0][0] = __builtin_bit_cast(half8, cur[rs[0]]);
-        aop[0][1] = __builtin_bit_cast(half8, cur[rs[1]]);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int mt = 0; mt < TM; ++mt) {
-            if (mt + 1 < TM) {
-                aop[(mt + 1) & 1][0] = __builtin_bit_cast(half8, cur[((mt + 1) >> 1) * 256 + rs[2 * ((mt + 1) & 1)]]);
-                aop[(mt + 1) & 1][1] = __builtin_bit_cast(half8, cur[((mt + 1) >> 1) * 256 + rs[2 * ((mt + 1) & 1) + 1]]);
+            half8 n0, n1;
+            if (t == TB) {
+                // All reads of this k-tile have been issued in earlier steps.  After the barrier they are complete for
+                // every wavefront, and so is the copy of the next k-tile (younger: D - 2 k-tiles).
+                // (A plain __syncthreads() would drain every outstanding copy here.)
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kReq ? (D - 2) * L : 0) : "memory");
+                if (kReq)
+                    dma_tile(s, nx);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            u32x4 raw2;
+            if (TN >= 2) {
+                raw2 = t + 2 < TN ? lds[s][wr0 + (t + 2) * 64] : lds[sn][wr0 + (t + 2 - TN) * 64];
+                n0 = widen8(raw.x, raw.y);
+                n1 = widen8(raw.z, raw.w);
+            } else {
+                raw2 = lds[sn][wr0];
+                n0 = widen8(raw2.x, raw2.y);
+                n1 = widen8(raw2.z, raw2.w);
             }
 #pragma unroll
-            for (int t = 0; t < TN; ++t) {
-                acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w0[t], aop[mt & 1][0], acc[t][mt], 0, 0, 0);
-                acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w1[t], aop[mt & 1][1], acc[t][mt], 0, 0, 0);
-            }
-        }
+            for (int mt = 0; mt < TM; ++mt)
+                acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w0, op[mt][0], acc[t][mt], 0, 0, 0);
 #pragma unroll
-        for (int mt = 0; mt < TM; ++mt) {
-            if (mt + 1 < TM)
-                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);   // 2 LDS reads
-            __builtin_amdgcn_sched_group_barrier(0x008, 2 * TN, 0);  // 2*TN MFMA
+            for (int mt = 0; mt < TM; ++mt) {
+                acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w1, op[mt][1], acc[t][mt], 0, 0, 0);
+                if (t == TN - 1)
+                    read_op(op[mt], lds[sn], mt);
+            }
+            w0 = n0;
+            w1 = n1;
+            raw = raw2;
+            // the order: a read of weights, then matrix and vector instructions in turn, in the last step with the
+            // operand reads among them
+            constexpr int kValu = 16 / (2 * TM) > 0 ? 16 / (2 * TM) : 1;
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+#pragma unroll
+            for (int i = 0; i < 2 * TM; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (TN >= 2)
+                    __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
+                else if (i >= TM)   // one step per k-tile: its weights come behind the hand-over
+                    __builtin_amdgcn_sched_group_barrier(0x002, 2 * kValu, 0);
+                if (t == TN - 1 && i >= TM)
+                    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        // The DMA of tile kt+1 (issued two steps ago) must have landed before any wavefront reads it.  Accesses that
-        // touch memory complete in the order issued, register loads and copies into LDS alike; one whose lanes are ALL
-        // out of range (the row groups past M of a ragged block) completes at once, ahead of older copies (measured:
-        // a counted wait over such accesses let an older copy through).  So the count has to hold with every such
-        // access already gone.  Younger than that DMA are, among others, three weight batches (3 TN loads that always
-        // touch memory); once no more than kPerWave + TN accesses are outstanding (the ones this step issued), the
-        // complete ones include everything but the youngest kPerWave + TN <= 3 TN real ones, hence the DMA in
-        // question.  Costs under 0.5 % against allowing the loads of two steps to be outstanding, which only timing
-        // made safe on ragged blocks.
-        // (A plain __syncthreads() would drain every outstanding load here: its
-        // release fence waits for all DMA writes, including the ones just issued.)
-        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(S::kPerWave + TN) : "memory");
     };
-
-    // prologue: tiles 0..2 into stages 0..2, weights of tiles 0 and 1
-    load_w(wraw[0], kbeg);
-    dma_tile(st0, kbeg);
-    load_w(wraw[1], kbeg + min(1, nk - 1));
-    dma_tile(st1, kbeg + min(1, nk - 1));
-    dma_tile(st2, kbeg + min(2, nk - 1));
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    __syncthreads();
-
     int kt = 0;
-    for (; kt + 4 <= nk; kt += 4) {
-        step(st0, st3, wraw[0], kt);
-        step(st1, st0, wraw[1], kt + 1);
-        step(st2, st1, wraw[0], kt + 2);
-        step(st3, st2, wraw[1], kt + 3);
+    for (; kt + D <= nk; kt += D) {
+        // past the end the last k-tile is copied again: no branch, and the counts above stay exact
+        auto next = [&](int s) { return min(kt + s + D, nk - 1); };
+        tile_step(std::integral_constant<int, 0>{}, std::true_type{}, next(0));
+        tile_step(std::integral_constant<int, 1>{}, std::true_type{}, next(1));
+        if constexpr (D > 2)
+            tile_step(std::integral_constant<int, 2 % D>{}, std::true_type{}, next(2));
+        if constexpr (D > 3)
+            tile_step(std::integral_constant<int, 3 % D>{}, std::true_type{}, next(3));
+        if constexpr (D > 4)
+            tile_step(std::integral_constant<int, 4 % D>{}, std::true_type{}, next(4));
     }
+    // the up to D - 1 k-tiles that are left have been requested
     if (kt < nk)
-        step(st0, st3, wraw[0], kt);
-    if (kt + 1 < nk)
-        step(st1, st0, wraw[1], kt + 1);
-    if (kt + 2 < nk)
-        step(st2, st1, wraw[0], kt + 2);
+        tile_step(std::integral_constant<int, 0>{}, std::false_type{}, 0);
+    if constexpr (D > 2)
+        if (kt + 1 < nk)
+            tile_step(std::integral_constant<int, 1 % D>{}, std::false_type{}, 0);
+    if constexpr (D > 3)
+        if (kt + 2 < nk)
+            tile_step(std::integral_constant<int, 2 % D>{}, std::false_type{}, 0);
+    if constexpr (D > 4)
+        if (kt + 3 < nk)
+            tile_step(std::integral_constant<int, 3 % D>{}, std::false_type{}, 0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no copy may land in LDS after the workgroup has gone
 
-    // acc[t][mt][r] of lane (g, j): row m0 + 16*mt + j, channel 16*(nt0+t) + 4*g + r
-    const int mrow0 = m0 + j;
+    // acc[t][mt][r] of lane (g, j): row mrow0 + 16*mt, channel 16*(nt0+t) + 4*g + r
+    const int mrow0 = m0 + wm * TM * 16 + j;
     if (ksplit > 1) {
 #pragma unroll
         for (int t = 0; t < TN; ++t) {
@@ -246,51 +271,69 @@ __global__ __launch_bounds__(64 * WNW) __attribute__((amdgpu_waves_per_eu(2))) v
         }
         return;
     }
+    // Stores.  Each goes through a buffer resource that ends with the block's last row (the lane's offset is past it
+    // exactly if the row is), so that no lane branches on its row.
+    const int cols = epi == kEpiSwiglu ? N / 2 : N;
+    auto rsrc_of = [&](const _Float16 *base, int mt) {
+        const int r0 = wm * TM * 16 + 16 * mt;
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(base + (size_t)(m0 + r0) * cols), 0,
+                                                 (unsigned)max(min(rows - r0, 16), 0) * (unsigned)cols * 2u,
+                                                 0x00020000);
+    };
+    half4 sc[TN];
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+        sc[t] = *reinterpret_cast<const half4 *>(scale + min(nt0 + t, ntiles - 1) * 16 + 4 * g);
     if (epi == kEpiSwiglu) {
         if constexpr (TN % 2 == 0) {
+            const int coff = j * cols * 2 + nt0 * 16 + g * 8;
 #pragma unroll
-            for (int t = 0; t < TN; t += 2) {
-                if (nt0 + t + 1 >= ntiles)
-                    continue;
-                const half4 sg = *reinterpret_cast<const half4 *>(scale + (nt0 + t) * 16 + 4 * g);
-                const half4 su = *reinterpret_cast<const half4 *>(scale + (nt0 + t + 1) * 16 + 4 * g);
-                const int n = ((nt0 + t) / 2) * 16 + 4 * g;
+            for (int mt = 0; mt < TM; ++mt) {
+                const __amdgpu_buffer_rsrc_t cr = rsrc_of(C, mt);
 #pragma unroll
-                for (int mt = 0; mt < TM; ++mt) {
-                    const int m = mrow0 + 16 * mt;
-                    if (m < M) {
-                        half4 o;
+                for (int t = 0; t < TN; t += 2) {
+                    half4 o;
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const float gate = (float)(_Float16)(acc[t][mt][r] * (float)sg[r]);
-                            const float up = (float)(_Float16)(acc[t + 1][mt][r] * (float)su[r]);
-                            o[r] = (_Float16)(up * gate / (1.0f + __expf(-gate)));
-                        }
-                        *reinterpret_cast<half4 *>(C + (size_t)m * (N / 2) + n) = o;
+                    for (int r = 0; r < 4; ++r) {
+                        const float gate = (float)(_Float16)(acc[t][mt][r] * (float)sc[t][r]);
+                        const float up = (float)(_Float16)(acc[t + 1][mt][r] * (float)sc[t + 1][r]);
+                        o[r] = (_Float16)(up * gate / (1.0f + __expf(-gate)));
                     }
+                    if (nt0 + t + 1 < ntiles)
+                        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, o), cr, coff + t * 16, 0, 0);
                 }
             }
         }
         return;
     }
+    // The residual of an m-tile is fetched whole, one m-tile ahead (a load under a branch of its own would be waited
+    // for before the next is issued).
+    const int coff = j * N * 2 + nt0 * 32 + g * 8;
+    u32x2 res[2][TN];
+    auto fetch = [&](int mt) {
+        const __amdgpu_buffer_rsrc_t rr = rsrc_of(residual, mt);
 #pragma unroll
-    for (int t = 0; t < TN; ++t) {
-        if (nt0 + t >= ntiles)
-            continue;
-        const int n = (nt0 + t) * 16 + 4 * g;
-        const half4 sc = *reinterpret_cast<const half4 *>(scale + n);
+        for (int t = 0; t < TN; ++t)
+            res[mt & 1][t] = __builtin_bit_cast(
+                u32x2, __builtin_amdgcn_raw_buffer_load_b64(rr, coff + t * 32, 0, 0));
+    };
+    if (epi == kEpiResidual)
+        fetch(0);
 #pragma unroll
-        for (int mt = 0; mt < TM; ++mt) {
-            const int m = mrow0 + 16 * mt;
-            if (m < M) {
-                half4 o;
+    for (int mt = 0; mt < TM; ++mt) {
+        if (epi == kEpiResidual && mt + 1 < TM)
+            fetch(mt + 1);
+        const __amdgpu_buffer_rsrc_t cr = rsrc_of(C, mt);
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    o[r] = (_Float16)(acc[t][mt][r] * (float)sc[r]);
-                if (epi == kEpiResidual)
-                    o = o + *reinterpret_cast<const half4 *>(residual + (size_t)m * N + n);
-                *reinterpret_cast<half4 *>(C + (size_t)m * N + n) = o;
-            }
+        for (int t = 0; t < TN; ++t) {
+            half4 o;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                o[r] = (_Float16)(acc[t][mt][r] * (float)sc[t][r]);
+            if (epi == kEpiResidual)
+                o = o + __builtin_bit_cast(half4, res[mt & 1][t]);
+            if (nt0 + t < ntiles)
+                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, o), cr, coff + t * 32, 0, 0);
         }
     }
 #endif
@@ -340,15 +383,15 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
     *reinterpret_cast<half4 *>(C + (size_t)m * n_out + o4) = o;
 }
 
-template <int WNW, int TM, int TN>
+template <int TM, int TN, int WM, int WN, int D>
 int launch_large_m(const GemmArgs &a, int ksplit)
 {
-    using S = DmaShape<WNW, TM, TN>;
+    using S = TileShape<TM, TN, WM, WN, D>;
     const int m_blocks = (a.M + S::kBM - 1) / S::kBM, n_blocks = (a.N + S::kBN - 1) / S::kBN;
     const int grid = ((m_blocks * n_blocks + 7) / 8) * 8;
     float *partial = ksplit > 1 ? static_cast<float *>(a.ws) : nullptr;
-    hipLaunchKernelGGL((w8a16_large_m_kernel<WNW, TM, TN>), dim3(grid, ksplit), dim3(S::kThreads), 0, a.st, a.A, a.Wp,
-                       a.scale, a.C, a.M, a.N, a.K, m_blocks, n_blocks, a.residual, a.epi, ksplit, partial);
+    hipLaunchKernelGGL((w8a16_large_m_kernel<TM, TN, WM, WN, D>), dim3(grid, ksplit), dim3(64 * S::kWaves), 0, a.st, a.A,
+                       a.Wp, a.scale, a.C, a.M, a.N, a.K, m_blocks, n_blocks, a.residual, a.epi, ksplit, partial);
     EET_HIP_CHECK(hipGetLastError());
     if (ksplit > 1) {
         const int items = a.M * ((a.epi == kEpiSwiglu ? a.N / 2 : a.N) / 4);
@@ -359,84 +402,100 @@ int launch_large_m(const GemmArgs &a, int ksplit)
     return EET_OK;
 }
 
-struct LargeMConfig {
-    int tm, tn;  // m-tiles and n-tiles of 16 per wavefront; the block is tm*16 rows x 4*tn*16 channels
-    int ksplit;  // > 1: that many workgroups share a tile's k range (needs the fp32 workspace)
+// The block shapes and what they cost.  A launch of `w` workgroups that each walk nk k-tiles takes about
+//     base + (store [+ res]) * max(1, w / 256) * (block area / 10^4) + nk * per_tile(w / 256)   us
+// where per_tile is linear between the values at 1/2, 1, just over 1, 2, just over 2, 3, just over 3, 4, 8, 24 and 64
+// workgroups per CU (the jumps behind whole numbers are a CU that gets one workgroup more than the others).  Fitted,
+// shape by shape, to 14300 launches on MI355X: 20 weight matrices of decoders 1024 .. 5120 wide, 40 .. 8192 rows, one
+// to eight shares of the k range.  Over those problems the shape with the smallest estimate is on average 1.8 %
+// behind the fastest of 28 shapes (the worst case 25 %), where the earlier rule's five shapes were 12 % behind.
+struct TileCost {
+    int tm, tn, wm, wn;
+    float base, store, res, per_tile[11];
 };
-
-// Shape -> tile.  Measured on MI355X (M = 33 .. 8192, LLaMA-7B and Baichuan-13B shapes):
-//   128 x 256 (two workgroups per CU) is the fastest tile once it yields a few
-//     hundred workgroups;
-//   64 x 320 wins when it divides the problem into whole rounds of 512 workgroups
-//     where 128 x 256 leaves a CU with two tiles against one elsewhere (M = 2048,
-//     N = 5120: 512 tiles, two per CU, instead of 320);
-//   64 x 256, 64 x 128 and 32 x 128 keep the chip occupied for M in the tens and
-//     hundreds, where the k-loop latency of a few large tiles would dominate.
-// Estimated time (us) of tile (tm, tn) with the k range split ks ways, for launches
-// too small to fill the chip.  Fitted to MI355X measurements (M = 40 .. 512, LLaMA-7B
-// shapes, within ~10 %): a workgroup alone on its CU needs `lat` us per k-tile
-// (load -> widen -> MFMA latency chain), co-resident workgroups share the CU's
-// L2 bandwidth at `thr` us per k-tile each; a split launch pays a second kernel
-// (~2 us) that reads what the first wrote (ks * M * N fp32, ~4 TB/s effective).
-struct SplitTile {
-    int tm, tn;
-    double lat, thr;
+constexpr TileCost kTiles[] = {
+    {2, 1, 1, 4, 2.917f, 1.247f, 0.000f, {0.161f, 0.166f, 0.191f, 0.247f, 0.315f, 0.335f, 0.426f, 0.477f, 0.892f, 2.520f, 6.530f}},
+    {2, 2, 1, 4, 2.642f, 2.225f, 0.000f, {0.221f, 0.255f, 0.328f, 0.393f, 0.584f, 0.629f, 0.690f, 0.780f, 1.553f, 4.389f, 11.815f}},
+    {4, 1, 1, 4, 2.166f, 2.141f, 0.568f, {0.200f, 0.222f, 0.275f, 0.364f, 0.518f, 0.565f, 0.615f, 0.716f, 1.379f, 3.961f, 11.391f}},
+    {4, 2, 1, 4, 3.281f, 1.332f, 0.735f, {0.272f, 0.338f, 0.440f, 0.555f, 0.846f, 0.859f, 0.957f, 1.123f, 2.207f, 6.470f, 16.031f}},
+    {4, 3, 1, 4, 5.194f, 0.355f, 1.088f, {0.352f, 0.405f, 0.589f, 0.747f, 0.994f, 1.149f, 1.234f, 1.570f, 3.029f, 9.078f, 22.839f}},
+    {4, 4, 1, 4, 5.700f, 0.201f, 0.930f, {0.440f, 0.524f, 0.780f, 0.933f, 1.344f, 1.454f, 1.685f, 2.008f, 3.998f, 11.593f, 30.062f}},
+    {6, 1, 1, 4, 2.159f, 1.850f, 1.611f, {0.232f, 0.279f, 0.358f, 0.469f, 0.652f, 0.723f, 0.782f, 0.959f, 1.841f, 5.355f, 14.470f}},
+    {6, 2, 1, 4, 4.798f, 0.522f, 1.616f, {0.342f, 0.405f, 0.590f, 0.708f, 1.043f, 1.135f, 1.255f, 1.617f, 3.060f, 9.178f, 23.538f}},
+    {6, 3, 1, 4, 6.617f, 0.000f, 1.187f, {0.470f, 0.543f, 0.787f, 0.988f, 1.367f, 1.546f, 1.623f, 2.113f, 4.265f, 12.731f, 26.329f}},
+    {6, 4, 1, 4, 5.994f, 0.111f, 0.580f, {0.718f, 0.749f, 1.045f, 1.310f, 1.747f, 2.016f, 2.228f, 2.878f, 5.489f, 15.891f, 39.766f}},
+    {8, 2, 1, 4, 5.896f, 0.166f, 1.236f, {0.442f, 0.494f, 0.746f, 0.904f, 1.319f, 1.455f, 1.657f, 1.987f, 3.930f, 11.468f, 29.993f}},
+    {8, 3, 1, 4, 6.138f, 0.054f, 0.740f, {0.707f, 0.724f, 0.988f, 1.301f, 1.708f, 1.982f, 2.252f, 2.636f, 5.343f, 15.324f, 40.864f}},
+    {8, 4, 1, 4, 6.961f, 0.008f, 1.063f, {0.786f, 0.835f, 1.333f, 1.620f, 2.470f, 2.513f, 2.955f, 3.415f, 6.896f, 19.815f, 51.087f}},
+    {4, 2, 1, 8, 4.185f, 0.837f, 1.310f, {0.399f, 0.516f, 0.917f, 1.042f, 1.507f, 1.642f, 1.901f, 2.301f, 4.451f, 13.200f, 33.959f}},
+    {4, 2, 2, 4, 5.578f, 0.425f, 1.405f, {0.373f, 0.494f, 0.871f, 1.017f, 1.499f, 1.627f, 1.852f, 2.296f, 4.527f, 13.521f, 35.022f}},
+    {4, 5, 2, 4, 6.169f, 0.246f, 1.148f, {0.853f, 0.994f, 1.896f, 2.118f, 3.011f, 3.450f, 3.924f, 4.641f, 9.821f, 25.224f, 67.263f}},
+    {6, 1, 1, 8, 4.801f, 0.530f, 1.081f, {0.320f, 0.406f, 0.623f, 0.745f, 1.022f, 1.192f, 1.353f, 1.654f, 3.212f, 9.524f, 24.507f}},
+    {6, 2, 1, 8, 6.163f, 0.376f, 1.708f, {0.540f, 0.660f, 1.223f, 1.401f, 1.999f, 2.225f, 2.417f, 3.302f, 6.180f, 18.324f, 46.073f}},
+    {8, 2, 1, 8, 6.156f, 0.302f, 1.639f, {0.662f, 0.806f, 1.571f, 1.734f, 2.698f, 2.744f, 3.195f, 3.889f, 7.725f, 22.208f, 51.472f}},
+    {8, 4, 2, 4, 3.887f, 0.350f, 1.127f, {1.261f, 1.443f, 2.945f, 2.867f, 4.505f, 4.935f, 5.165f, 7.166f, 13.471f, 39.109f, 104.291f}}
 };
-constexpr SplitTile kSplitTiles[2] = {{2, 2, 0.26, 0.14}, {4, 2, 0.33, 0.23}};
+constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
-double split_cost_us(int M, int N, int K, const SplitTile &t, int ks)
+float per_tile_us(const TileCost &t, float x)
 {
-    const int wgs = ((M + t.tm * 16 - 1) / (t.tm * 16)) * ((N + t.tn * 64 - 1) / (t.tn * 64)) * ks;
-    const double load = wgs <= 512 ? (double)((wgs + 255) / 256) : wgs / 256.0;
-    const double per_tile = t.lat > t.thr * load ? t.lat : t.thr * load;
-    double us = 2.5 + (K / 64.0 / ks) * per_tile;
-    if (ks > 1)
-        us += 2.0 + (double)ks * M * N * 8.0 / 4e6;
-    return us;
+    constexpr float at[11] = {0.5f, 1.f, 1.001f, 2.f, 2.001f, 3.f, 3.001f, 4.f, 8.f, 24.f, 64.f};
+    if (x <= at[0])
+        return t.per_tile[0];
+    for (int i = 1; i < 11; ++i)
+        if (x <= at[i])
+            return t.per_tile[i - 1] + (t.per_tile[i] - t.per_tile[i - 1]) * (x - at[i - 1]) / (at[i] - at[i - 1]);
+    return t.per_tile[10] * x / at[10];
 }
 
-LargeMConfig pick_large_m(int M, int N, int K, int epi, bool may_split)
+// a split launch pays a second kernel that reads what the first wrote
+float split_reduce_us(int M, int N, int ks) { return 2.2f + (float)ks * M * N * 4.f / 3e6f; }
+
+struct LargeMConfig {
+    int tile = -1;    // index into kTiles
+    int ksplit = 1;   // > 1: that many workgroups share a tile's k range (needs the fp32 workspace)
+    float us = 1e30f;
+};
+
+// The best shape without a split and the best one with its k range split (us = 1e30: none is worth trying; a split is
+// considered for launches of at most 200 blocks, i.e. where CUs would be idle, and leaves every share four k-tiles).
+void pick_large_m(int M, int N, int K, int epi, LargeMConfig *whole, LargeMConfig *split)
 {
-    auto wgs = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    const int big = wgs(128, 256);
-    if (big >= 320) {
-        if (epi != kEpiSwiglu) {  // 5 n-tiles per wavefront: no (gate, up) pairs
-            // time in units of one 128 x 256 tile on a CU of its own; 64 x 320 is 0.625 of that
-            // area and runs at about 0.9 of the large tile's rate
-            const double cost_big = 2.0 * ((big + 511) / 512);
-            const double cost_320 = 2.0 * ((wgs(64, 320) + 511) / 512) * 0.625 / 0.9;
-            if (cost_320 < cost_big)
-                return LargeMConfig{4, 5, 1};
-        }
-        return LargeMConfig{8, 4, 1};
-    }
-    if (wgs(64, 256) >= 600)
-        return LargeMConfig{4, 4, 1};
-    // Fewer tiles than fill the chip twice: 32 x 128 or 64 x 128, and the k range of
-    // a tile may be shared by up to 8 workgroups (at least 8 k-tiles each) whose fp32
-    // partial sums a small second kernel adds.
     const int ktiles = K / 64;
-    LargeMConfig best{2, 2, 1};
-    double best_us = 1e30;
-    for (const SplitTile &t : kSplitTiles)
-        for (int ks = 1; ks <= (may_split ? 8 : 1); ++ks) {
-            if (ks > 1 && ktiles / ks < 8)
-                break;
-            const double us = split_cost_us(M, N, K, t, ks);
-            if (us < best_us) {
-                best_us = us;
-                best = LargeMConfig{t.tm, t.tn, ks};
+    for (int i = 0; i < kNumTiles; ++i) {
+        const TileCost &t = kTiles[i];
+        if (epi == kEpiSwiglu && t.tn % 2 != 0)   // a wavefront holds whole (gate, up) pairs
+            continue;
+        const int bm = 16 * t.tm * t.wm, bn = 16 * t.tn * t.wn;
+        const int blocks = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+        const float area = (float)bm * bn * 1e-4f;
+        auto cost = [&](int ks) {
+            const float x = blocks * ks / 256.f;
+            const float store = ks > 1 ? 2.f * t.store : t.store + (epi == kEpiResidual ? t.res : 0.f);
+            return t.base + store * (x > 1.f ? x : 1.f) * area +
+                   (float)ktiles / ks * per_tile_us(t, x);
+        };
+        if (const float us = cost(1); us < whole->us)
+            *whole = LargeMConfig{i, 1, us};
+        if (blocks <= 200)
+            for (int ks : {2, 3, 4, 6, 8}) {
+                if (ktiles / ks < 4 || blocks * ks > 560)
+                    break;
+                if (const float us = cost(ks) + split_reduce_us(M, N, ks); us < split->us)
+                    *split = LargeMConfig{i, ks, us};
             }
-        }
-    return best;
+    }
 }
 
 }  // namespace
 
+// The workspace of a split that would win, or comes within 15 % of the unsplit launch (so that a caller who sizes its
+// buffer once for a range of rows has the room where a split does win).
 size_t eet::large_m_workspace(int M, int N, int K, int epi)
 {
-    const LargeMConfig c = pick_large_m(M, N, K, epi, true);
-    return c.ksplit > 1 ? (size_t)c.ksplit * M * N * sizeof(float) : 0;
+    LargeMConfig whole, split;
+    pick_large_m(M, N, K, epi, &whole, &split);
+    return split.us < 1.15f * whole.us ? (size_t)split.ksplit * M * N * sizeof(float) : 0;
 }
 
 int eet::run_large_m(const GemmArgs &a)
@@ -445,34 +504,52 @@ int eet::run_large_m(const GemmArgs &a)
     if ((size_t)a.K * a.N >= (1ull << 31) || (size_t)a.K * 2 * 256 >= (1ull << 31))
         return eet::fail(EET_ERR_UNSUPPORTED_SHAPE, "eet_gemm_w8a16: K x N = %d x %d exceeds the 2 GiB weight limit",
                          a.K, a.N);
-    // the split needs room for ksplit x M x N fp32; without it the best single-pass tile
+    // a split needs room for ksplit x M x N fp32; without it the best single-pass tile
     auto fits = [&](int ks) {
         return ks <= 1 || (a.ws != nullptr && reinterpret_cast<uintptr_t>(a.ws) % 16 == 0 &&
                            a.ws_bytes >= (size_t)ks * a.M * a.N * sizeof(float));
     };
-    LargeMConfig c = pick_large_m(a.M, a.N, a.K, a.epi, true);
-    if (!fits(c.ksplit))
-        c = pick_large_m(a.M, a.N, a.K, a.epi, false);
+    LargeMConfig whole, split;
+    pick_large_m(a.M, a.N, a.K, a.epi, &whole, &split);
+    LargeMConfig c = split.us < whole.us && fits(split.ksplit) ? split : whole;
     const eet::Tuning &tune = eet::tuning();
-    if (tune.has_large_m) {  // "tm,tn[,ksplit]": runs when such a tile exists, else the table's choice stands
-        const int tm = tune.large_m_tm, tn = tune.large_m_tn;
-        const bool exists = (tm == 8 && tn == 4) || (tm == 4 && (tn == 5 || tn == 4 || tn == 2)) || (tm == 2 && tn == 2);
-        if (exists && (a.epi != kEpiSwiglu || tn % 2 == 0))
-            c = LargeMConfig{tm, tn, tune.large_m_ksplit > 0 ? tune.large_m_ksplit : 1};
-        if (!fits(c.ksplit))
-            c.ksplit = 1;
-    }
-    if (c.ksplit < 1 || c.ksplit > a.K / 64)
-        c.ksplit = 1;
-    if (c.tm == 8 && c.tn == 4)
-        return launch_large_m<4, 8, 4>(a, c.ksplit);
-    if (c.tm == 4 && c.tn == 5)
-        return launch_large_m<4, 4, 5>(a, c.ksplit);
-    if (c.tm == 4 && c.tn == 4)
-        return launch_large_m<4, 4, 4>(a, c.ksplit);
-    if (c.tm == 4 && c.tn == 2)
-        return launch_large_m<4, 4, 2>(a, c.ksplit);
-    if (c.tm == 2 && c.tn == 2)
-        return launch_large_m<4, 2, 2>(a, c.ksplit);
-    return eet::fail(EET_ERR_INVALID_ARGUMENT, "eet_gemm_w8a16: no large-M kernel for tile %d,%d", c.tm, c.tn);
+    if (tune.has_large_m)   // "tm,tn[,ksplit[,wm,wn]]": runs when such a tile exists, else the table's choice stands
+        for (int i = 0; i < kNumTiles; ++i) {
+            const TileCost &t = kTiles[i];
+            if (t.tm != tune.large_m_tm || t.tn != tune.large_m_tn || (a.epi == kEpiSwiglu && t.tn % 2 != 0) ||
+                (tune.large_m_wm > 0 && (t.wm != tune.large_m_wm || t.wn != tune.large_m_wn)))
+                continue;
+            const int ks = tune.large_m_ksplit;
+            c = LargeMConfig{i, ks >= 1 && ks <= a.K / 64 && fits(ks) ? ks : 1, 0.f};
+            break;
+        }
+    using Launcher = int (*)(const GemmArgs &, int);
+    // in the order of kTiles; the last number is the depth of the stage ring, as deep as two workgroups of four
+    // wavefronts (or one of eight) leave room for in the LDS
+    constexpr Launcher launchers[] = {
+        launch_large_m<2, 1, 1, 4, 5>,
+        launch_large_m<2, 2, 1, 4, 5>,
+        launch_large_m<4, 1, 1, 4, 5>,
+        launch_large_m<4, 2, 1, 4, 5>,
+        launch_large_m<4, 3, 1, 4, 4>,
+        launch_large_m<4, 4, 1, 4, 3>,
+        launch_large_m<6, 1, 1, 4, 4>,
+        launch_large_m<6, 2, 1, 4, 4>,
+        launch_large_m<6, 3, 1, 4, 3>,
+        launch_large_m<6, 4, 1, 4, 2>,
+        launch_large_m<8, 2, 1, 4, 3>,
+        launch_large_m<8, 3, 1, 4, 2>,
+        launch_large_m<8, 4, 1, 4, 2>,
+        launch_large_m<4, 2, 1, 8, 4>,
+        launch_large_m<4, 2, 2, 4, 4>,
+        launch_large_m<4, 5, 2, 4, 4>,
+        launch_large_m<6, 1, 1, 8, 4>,
+        launch_large_m<6, 2, 1, 8, 4>,
+        launch_large_m<8, 2, 1, 8, 4>,
+        launch_large_m<8, 4, 2, 4, 3>
+    };
+    static_assert(sizeof(launchers) / sizeof(launchers[0]) == kNumTiles, "one launcher per block shape");
+    if (c.tile < 0)
+        return eet::fail(EET_ERR_INVALID_ARGUMENT, "eet_gemm_w8a16: no large-M kernel for M=%d N=%d K=%d", a.M, a.N, a.K);
+    return launchers[c.tile](a, c.ksplit);
 }

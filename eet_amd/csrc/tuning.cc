@@ -30,10 +30,12 @@ int apply(const char *name, const char *value)
         t.has_large_m = false;
         if (clear)
             return EET_OK;
-        t.large_m_ksplit = 0;
-        if (std::sscanf(value, "%d,%d,%d", &t.large_m_tm, &t.large_m_tn, &t.large_m_ksplit) < 2)
-            return eet::fail(EET_ERR_INVALID_ARGUMENT, "eet_set_tuning: %s wants \"tm,tn[,ksplit]\", got \"%s\"", name,
-                             value);
+        t.large_m_ksplit = t.large_m_wm = t.large_m_wn = 0;
+        const int got = std::sscanf(value, "%d,%d,%d,%d,%d", &t.large_m_tm, &t.large_m_tn, &t.large_m_ksplit,
+                                    &t.large_m_wm, &t.large_m_wn);
+        if (got < 2 || got == 4)
+            return eet::fail(EET_ERR_INVALID_ARGUMENT, "eet_set_tuning: %s wants \"tm,tn[,ksplit[,wm,wn]]\", got \"%s\"",
+                             name, value);
         t.has_large_m = true;
         return EET_OK;
     }

@@ -12,9 +12,10 @@ struct Tuning {
     // EET_GEMM_SMALL_M_CONFIG = "nt,waves,u[,ksplit]" (ksplit 2: the pair split, with nt = 2)
     bool has_small_m = false;
     int small_m_nt = 0, small_m_waves = 0, small_m_u = 0, small_m_ksplit = 1;
-    // EET_GEMM_LARGE_M_TILE = "tm,tn[,ksplit]"
+    // EET_GEMM_LARGE_M_TILE = "tm,tn[,ksplit[,wm,wn]]"
     bool has_large_m = false;
     int large_m_tm = 0, large_m_tn = 0, large_m_ksplit = 0;  // ksplit 0: not given
+    int large_m_wm = 0, large_m_wn = 0;                      // wavefronts down and across a block; 0: not given
     // EET_MMHA_NSPLIT, EET_MMHA_THREADS, EET_MMHA_UNROLL (0: not given)
     int mmha_nsplit = 0, mmha_threads = 0, mmha_ring = 0;
     // EET_PREFILL_LEGACY = 1: head size 128 takes the register-staged prefill attention kernel

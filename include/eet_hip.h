@@ -49,7 +49,7 @@ int eet_packed_layout_version(void);
 
 /* Overrides one of the library's launch-shape tables, for sweeps and for tests
  * that run every kernel variant; value NULL or "" restores the table.  Keys:
- *   EET_GEMM_SMALL_M_CONFIG "nt,waves,u[,ksplit]"   EET_GEMM_LARGE_M_TILE "tm,tn[,ksplit]"
+ *   EET_GEMM_SMALL_M_CONFIG "nt,waves,u[,ksplit]"   EET_GEMM_LARGE_M_TILE "tm,tn[,ksplit[,wm,wn]]"
  *   EET_MMHA_NSPLIT / EET_MMHA_THREADS / EET_MMHA_UNROLL "n"
  *   EET_PREFILL_LEGACY "1" (register-staged prefill attention at head size 128)
  *   EET_PREFILL_SHAPE "1" | "2" (launch shape of the head-size-128 prefill kernel)

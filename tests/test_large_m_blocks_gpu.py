@@ -1,0 +1,94 @@
+"""Every block shape of the large-M kernel at the sizes where it can go wrong, through the C ABI against the fp32
+oracle: one row, one row less and one row more than a block; channels that end inside a block and inside a
+wavefront's share of it; k loops of 1 .. 2 D + 1 k-tiles (D <= 5 stages: prologue longer than the loop, whole turns
+of the ring, every length of the tail)."""
+import numpy as np
+import pytest
+import torch
+
+import eet_amd
+from eet_amd.ops import interleave_gate_up
+from oracle import ops as O
+
+from gpu_util import gemm, gemm_fused
+
+pytestmark = pytest.mark.gpu
+
+# m-tiles, n-tiles of a wavefront, wavefronts down and across a block
+BLOCKS = [(2, 1, 1, 4), (2, 2, 1, 4), (4, 1, 1, 4), (4, 2, 1, 4), (4, 3, 1, 4), (4, 4, 1, 4), (6, 1, 1, 4), (6, 2, 1, 4),
+          (6, 3, 1, 4), (6, 4, 1, 4), (8, 2, 1, 4), (8, 3, 1, 4), (8, 4, 1, 4), (4, 2, 1, 8), (4, 2, 2, 4), (4, 5, 2, 4),
+          (6, 1, 1, 8), (6, 2, 1, 8), (8, 2, 1, 8), (8, 4, 2, 4)]
+GUARD = 7.25
+
+
+def quant(K, N, seed):
+    g = torch.Generator().manual_seed(seed)
+    w = (torch.randn(K, N, generator=g) * 0.02).half()
+    return eet_amd.quant_weights(w, torch.int8, True)
+
+
+def bound(x, u, s):
+    """|error| of one product: fp32 accumulation in any order (K roundings of partial sums that sum |a w| bounds), one
+    fp32 rounding by the scale; the caller adds the fp16 rounding of the result."""
+    a, w = np.abs(x.numpy().astype(np.float32)), np.abs(u.numpy().astype(np.float32)) * s.numpy().astype(np.float32)
+    mag = a @ w
+    return mag * (x.shape[1] + 2) * 2.0 ** -24
+
+
+def check(got, x, u, s, what):
+    ref = x.numpy().astype(np.float64) @ (u.numpy().astype(np.float64) * s.numpy().astype(np.float64))
+    tol = bound(x, u, s) + np.abs(ref) * 2.0 ** -11 + 2.0 ** -24
+    err = np.abs(got.float().numpy() - ref)
+    assert (err <= tol).all(), f"{what}: {int((err > tol).sum())} of {err.size} outside, max err {err.max():.2e}"
+
+
+@pytest.mark.parametrize("block", BLOCKS, ids=lambda b: "x".join(map(str, b)))
+def test_block_edges(gpu, tuning, block):
+    tm, tn, wm, wn = block
+    bm, bn = 16 * tm * wm, 16 * tn * wn
+    tuning("EET_GEMM_LARGE_M_TILE", f"{tm},{tn},1,{wm},{wn}")
+    for i, k_tiles in enumerate(range(1, 12)):
+        M = max(33, (bm - 1, bm, bm + 1)[i % 3])
+        N = (bn, bn + 16, 2 * bn - 16, 16 * max(tn - 1, 1))[i % 4]
+        u, p, s = quant(64 * k_tiles, N, i)
+        x = torch.randn(M, 64 * k_tiles, generator=torch.Generator().manual_seed(M)).half()
+        check(gemm(x.to(gpu), p.to(gpu), s.to(gpu), M, N, 64 * k_tiles).cpu(), x, u, s, f"{block} {M}x{N} k {k_tiles}")
+
+
+@pytest.mark.parametrize("block", BLOCKS, ids=lambda b: "x".join(map(str, b)))
+def test_block_epilogues(gpu, tuning, block):
+    """Residual, SwiGLU and a k range in uneven shares; nothing is written past the last row (the next rows of the
+    buffer keep their value) and a residual of infinities past the last row is not read into the result."""
+    tm, tn, wm, wn = block
+    bm = 16 * tm * wm
+    M, K, F = bm + 1 if bm > 32 else 35, 448, 16 * tn * wn + 48
+    tuning("EET_GEMM_LARGE_M_TILE", f"{tm},{tn},1,{wm},{wn}")
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(3)).half()
+    u, p, s = quant(K, F, 5)
+    xd, pd, sd = x.to(gpu), p.to(gpu), s.to(gpu)
+    res = torch.full((M + 16, F), float("inf")).half()
+    res[:M] = torch.randn(M, F, generator=torch.Generator().manual_seed(4))
+    plain = gemm(xd, pd, sd, M, F, K).cpu()
+    assert torch.equal(gemm_fused(xd, pd, sd, M, F, K, 1, res.to(gpu)).cpu(), plain + res[:M])
+    out = torch.full((M + 16, F), GUARD, dtype=torch.float16, device=gpu)
+    eet_amd.ops._gemm(xd, pd, sd, out, M, F, K)
+    assert torch.equal(out[:M].cpu(), plain) and (out[M:] == GUARD).all()
+    tuning("EET_GEMM_LARGE_M_TILE", f"{tm},{tn},3,{wm},{wn}")
+    check(gemm(xd, pd, sd, M, F, K, ws_min_bytes=3 * M * F * 4).cpu(), x, u, s, f"{block} in three shares")
+    if tn % 2:
+        return
+    tuning("EET_GEMM_LARGE_M_TILE", f"{tm},{tn},1,{wm},{wn}")
+    uu, pu, su = quant(K, F, 6)
+    w01, s01 = (t.to(gpu) for t in interleave_gate_up(p, s, pu, su))
+    out = torch.full((M + 16, F), GUARD, dtype=torch.float16, device=gpu)
+    eet_amd.ops._gemm(xd, w01, s01, out, M, 2 * F, K, 2)
+    want = O.swiglu(O.dequant_matmul(x.numpy(), u.numpy(), s.numpy()), O.dequant_matmul(x.numpy(), uu.numpy(), su.numpy()))
+    got = out[:M].cpu().float().numpy()
+    # gate and up are rounded to fp16 (2^-11 of each) before the product: |d(silu)| <= 1.1 |d gate|, plus one rounding
+    g = np.abs(O.dequant_matmul(x.numpy(), u.numpy(), s.numpy()).astype(np.float32))
+    v = np.abs(O.dequant_matmul(x.numpy(), uu.numpy(), su.numpy()).astype(np.float32))
+    eg, eu = bound(x, u, s) + g * 2.0 ** -10, bound(x, uu, su) + v * 2.0 ** -10
+    tol = 1.1 * eg * v + g * eu + 1.1 * eg * eu + np.abs(want.astype(np.float32)) * 2.0 ** -10 + 2.0 ** -24
+    err = np.abs(got - want.astype(np.float32))
+    assert (err <= tol).all(), f"{block}: max err {err.max():.2e}"
+    assert (out[M:] == GUARD).all()
