@@ -32,6 +32,7 @@ SIGNATURES = {
     "eet_chain_status": (_i, [_vp, _i, _vp]),
     "eet_mmha_decode_workspace": (_sz, [_i, _i, _i, _i]),
     "eet_mmha_decode": (_i, [_vp, _vp, _vp, _l, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _sz, _vp]),
+    "eet_mmha_decode_beams": (_i, [_vp, _vp, _vp, _l, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i] + [_vp] * 5 + [_sz, _vp]),
     "eet_mmha_decode_static_capacity": (_sz, []),
     "eet_mmha_decode_static": (_i, [_vp, _vp, _vp, _l, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp]),
     "eet_step_advance": (_i, [_vp, _i, _vp]),
@@ -42,6 +43,7 @@ SIGNATURES = {
                                                                                                  _sz, _vp, _sz, _vp]),
     "eet_mmha_int8_decode_workspace": (_sz, [_i, _i, _i, _i]),
     "eet_mmha_int8_decode": (_i, [_vp, _vp, _f] + [_vp] * 12 + [_i] * 6 + [_vp, _sz, _vp, _sz, _vp]),
+    "eet_mmha_int8_decode_beams": (_i, [_vp, _vp, _f] + [_vp] * 12 + [_i] * 6 + [_vp] * 4 + [_sz, _vp, _sz, _vp]),
     "eet_gated_ffn_int8_decode": (_i, [_vp, _vp, _f] + [_vp] * 6 + [_i] * 4 + [_vp, _sz, _vp]),
     "eet_rope_table": (_i, [_vp, _i, _i, _vp]),
     "eet_rmsnorm": (_i, [_vp, _vp, _vp, _i, _i, _f, _vp]),
@@ -52,6 +54,7 @@ SIGNATURES = {
     "eet_swiglu": (_i, [_vp, _vp, _i, _i, _vp]),
     "eet_residual_add": (_i, [_vp, _vp, _i, _i, _vp]),
     "eet_kv_cache_reorder": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
+    "eet_kv_cache_gather_rows": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "eet_prefill_attention": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
 }
 

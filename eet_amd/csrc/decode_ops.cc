@@ -28,18 +28,18 @@ extern "C" size_t eet_mmha_int8_decode_workspace(int B, int H, int dh, int step)
     return eet_mmha_decode_workspace(B, H, dh, step);
 }
 
-extern "C" int eet_mmha_int8_decode(const void *x, const void *rms_gamma, float rms_eps, const void *qkv_w,
+static int mmha_int8_decode(const char *fn, const void *x, const void *rms_gamma, float rms_eps, const void *qkv_w,
                                     const void *qkv_scale, const void *o_w, const void *o_scale, void *k_cache,
                                     void *v_cache, const void *alibi, const int64_t *pad, const float *rope_cos_sin,
                                     void *qkv_buf, void *ctx_buf, void *out, int B, int H, int dh, int hidden,
                                     int step, int T_cap, void *workspace, size_t workspace_bytes, void *gemm_workspace,
-                                    size_t gemm_workspace_bytes, void *stream)
+                                    size_t gemm_workspace_bytes, const int32_t *beam_rows_in, int32_t *beam_rows_out,
+                            const int64_t *reorder_index, void *stream)
 {
     EET_REQUIRE(x && rms_gamma && qkv_buf && ctx_buf && out, EET_ERR_INVALID_ARGUMENT,
-                "eet_mmha_int8_decode: null pointer");
+                "%s: null pointer", fn);
     EET_REQUIRE(B > 0 && B <= 32 && H > 0 && dh > 0 && hidden > 0, EET_ERR_UNSUPPORTED_SHAPE,
-                "eet_mmha_int8_decode: B=%d must be 1..32 (one token per sequence), H=%d dh=%d hidden=%d", B, H, dh,
-                hidden);
+                "%s: B=%d must be 1..32 (one token per sequence), H=%d dh=%d hidden=%d", fn, B, H, dh, hidden);
     const int inner = H * dh;
     {
         // x is read by the first launch and again, as the residual, by the last; every
@@ -48,10 +48,9 @@ extern "C" int eet_mmha_int8_decode(const void *x, const void *rms_gamma, float 
         const size_t xb = (size_t)B * hidden * 2, qb = (size_t)B * 3 * inner * 2, cb = (size_t)B * inner * 2;
         EET_REQUIRE(!overlaps(out, xb, x, xb) && !overlaps(qkv_buf, qb, x, xb) && !overlaps(ctx_buf, cb, x, xb),
                     EET_ERR_INVALID_ARGUMENT,
-                    "eet_mmha_int8_decode: out, qkv_buf and ctx_buf must not overlap x (x is the residual of the "
-                    "last launch)");
+                    "%s: out, qkv_buf and ctx_buf must not overlap x (x is the residual of the last launch)", fn);
         EET_REQUIRE(!overlaps(ctx_buf, cb, qkv_buf, qb) && !overlaps(out, xb, ctx_buf, cb), EET_ERR_INVALID_ARGUMENT,
-                    "eet_mmha_int8_decode: ctx_buf must not overlap qkv_buf, nor out ctx_buf");
+                    "%s: ctx_buf must not overlap qkv_buf, nor out ctx_buf", fn);
     }
     // RMSnorm + QKV projection (llama_mmha.cpp:222-227)
     if (int rc = eet_gemm_w8a16_fused(x, qkv_w, qkv_scale, qkv_buf, B, 3 * inner, hidden, EET_EPILOGUE_NONE, nullptr,
@@ -59,12 +58,47 @@ extern "C" int eet_mmha_int8_decode(const void *x, const void *rms_gamma, float 
         return rc;
     // rotary (when a table row is given) + cache append + attention (:229-258): q, k, v are rows of qkv_buf
     const _Float16 *base = static_cast<const _Float16 *>(qkv_buf);
-    if (int rc = eet_mmha_decode(base, base + inner, base + 2 * inner, 3L * inner, k_cache, v_cache, ctx_buf, alibi,
-                                 pad, B, H, dh, step, T_cap, rope_cos_sin, workspace, workspace_bytes, stream))
+    const int rc = beam_rows_out != nullptr
+                       ? eet_mmha_decode_beams(base, base + inner, base + 2 * inner, 3L * inner, k_cache, v_cache, ctx_buf,
+                                               alibi, pad, B, H, dh, step, T_cap, rope_cos_sin, beam_rows_in,
+                                               beam_rows_out, reorder_index, workspace, workspace_bytes, stream)
+                       : eet_mmha_decode(base, base + inner, base + 2 * inner, 3L * inner, k_cache, v_cache, ctx_buf,
+                                         alibi, pad, B, H, dh, step, T_cap, rope_cos_sin, workspace, workspace_bytes,
+                                         stream);
+    if (rc != EET_OK)
         return rc;
     // output projection + residual (:260-262, 428-462)
     return eet_gemm_w8a16_fused(ctx_buf, o_w, o_scale, out, B, hidden, inner, EET_EPILOGUE_RESIDUAL, x, nullptr, 0.f,
                                 gemm_workspace, gemm_workspace_bytes, stream);
+}
+
+extern "C" int eet_mmha_int8_decode(const void *x, const void *rms_gamma, float rms_eps, const void *qkv_w,
+                                    const void *qkv_scale, const void *o_w, const void *o_scale, void *k_cache,
+                                    void *v_cache, const void *alibi, const int64_t *pad, const float *rope_cos_sin,
+                                    void *qkv_buf, void *ctx_buf, void *out, int B, int H, int dh, int hidden,
+                                    int step, int T_cap, void *workspace, size_t workspace_bytes, void *gemm_workspace,
+                                    size_t gemm_workspace_bytes, void *stream)
+{
+    return mmha_int8_decode("eet_mmha_int8_decode", x, rms_gamma, rms_eps, qkv_w, qkv_scale, o_w, o_scale, k_cache,
+                            v_cache, alibi, pad, rope_cos_sin, qkv_buf, ctx_buf, out, B, H, dh, hidden, step, T_cap,
+                            workspace, workspace_bytes, gemm_workspace, gemm_workspace_bytes, nullptr, nullptr, nullptr,
+                            stream);
+}
+
+extern "C" int eet_mmha_int8_decode_beams(const void *x, const void *rms_gamma, float rms_eps, const void *qkv_w,
+                                          const void *qkv_scale, const void *o_w, const void *o_scale, void *k_cache,
+                                          void *v_cache, const void *alibi, const int64_t *pad,
+                                          const float *rope_cos_sin, void *qkv_buf, void *ctx_buf, void *out, int B,
+                                          int H, int dh, int hidden, int step, int T_cap, const int32_t *beam_rows_in,
+                                          int32_t *beam_rows_out, const int64_t *reorder_index, void *workspace,
+                                          size_t workspace_bytes, void *gemm_workspace, size_t gemm_workspace_bytes,
+                                          void *stream)
+{
+    EET_REQUIRE(beam_rows_out != nullptr, EET_ERR_INVALID_ARGUMENT, "eet_mmha_int8_decode_beams: null pointer");
+    return mmha_int8_decode("eet_mmha_int8_decode_beams", x, rms_gamma, rms_eps, qkv_w, qkv_scale, o_w, o_scale, k_cache,
+                            v_cache, alibi, pad, rope_cos_sin, qkv_buf, ctx_buf, out, B, H, dh, hidden, step, T_cap,
+                            workspace, workspace_bytes, gemm_workspace, gemm_workspace_bytes, beam_rows_in,
+                            beam_rows_out, reorder_index, stream);
 }
 
 extern "C" int eet_gated_ffn_int8_decode(const void *x, const void *rms_gamma, float rms_eps, const void *w01,

@@ -305,6 +305,24 @@ __global__ __launch_bounds__(256) void kv_reorder_kernel(const _Float16 *__restr
     }
 }
 
+// Puts every row of every sequence into the sequence's own slab: dst[b][h][t] = src[rows[b][t]][h][t] (a name
+// outside [0, B) stands for b).  grid = (chunks of rows, H, B); dh/8 lanes copy a row.
+__global__ __launch_bounds__(256) void kv_gather_rows_kernel(const uint4 *__restrict__ k_src,
+                                                             const uint4 *__restrict__ v_src, uint4 *__restrict__ k_dst,
+                                                             uint4 *__restrict__ v_dst, const int *__restrict__ names,
+                                                             int B, int H, int T_cap, int row_vec, int nvec)
+{
+    const int b = blockIdx.z, h = blockIdx.y;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < nvec; i += gridDim.x * 256) {
+        const int name = names[(size_t)b * T_cap + i / row_vec];
+        const int from = name >= 0 && name < B ? name : b;
+        const size_t so = ((size_t)from * H + h) * T_cap * row_vec + i, dst_o = ((size_t)b * H + h) * T_cap * row_vec + i;
+        const uint4 a = k_src[so], c = v_src[so];
+        k_dst[dst_o] = a;
+        v_dst[dst_o] = c;
+    }
+}
+
 }  // namespace
 
 extern "C" int eet_rmsnorm(const void *x, const void *gamma, void *out, int M, int N, float eps, void *stream)
@@ -429,18 +447,15 @@ extern "C" int eet_residual_add(void *out, const void *residual, int M, int N, v
     return EET_OK;
 }
 
-extern "C" int eet_kv_cache_reorder(const void *k_src, const void *v_src, void *k_dst, void *v_dst,
-                                    const int64_t *reorder_index, int B, int H, int dh, int rows, int T_cap,
-                                    void *stream)
+// Argument checks shared by the two cache gathers; returns EET_OK when there is something to launch or nothing to do.
+static int check_gather(const char *fn, const void *k_src, const void *v_src, const void *k_dst, const void *v_dst,
+                        const void *index, int B, int H, int dh, int rows, int T_cap)
 {
-    EET_REQUIRE(k_src && v_src && k_dst && v_dst && reorder_index, EET_ERR_INVALID_ARGUMENT,
-                "eet_kv_cache_reorder: null pointer");
+    EET_REQUIRE(k_src && v_src && k_dst && v_dst && index, EET_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
     EET_REQUIRE(B >= 0 && H > 0 && dh > 0 && rows >= 0 && rows <= T_cap, EET_ERR_INVALID_ARGUMENT,
-                "eet_kv_cache_reorder: bad sizes B=%d H=%d dh=%d rows=%d T_cap=%d", B, H, dh, rows, T_cap);
-    EET_REQUIRE(dh % 8 == 0, EET_ERR_UNSUPPORTED_SHAPE, "eet_kv_cache_reorder: head size %d must be a multiple of 8",
-                dh);
-    EET_REQUIRE(B <= 65535 && H <= 65535, EET_ERR_UNSUPPORTED_SHAPE, "eet_kv_cache_reorder: B=%d / H=%d too large", B,
-                H);
+                "%s: bad sizes B=%d H=%d dh=%d rows=%d T_cap=%d", fn, B, H, dh, rows, T_cap);
+    EET_REQUIRE(dh % 8 == 0, EET_ERR_UNSUPPORTED_SHAPE, "%s: head size %d must be a multiple of 8", fn, dh);
+    EET_REQUIRE(B <= 65535 && H <= 65535, EET_ERR_UNSUPPORTED_SHAPE, "%s: B=%d / H=%d too large", fn, B, H);
     // The gather reads beams that other workgroups write: in place it would race.
     const size_t bytes = (size_t)B * H * T_cap * dh * sizeof(_Float16);
     auto overlap = [bytes](const void *a, const void *b) {
@@ -448,7 +463,16 @@ extern "C" int eet_kv_cache_reorder(const void *k_src, const void *v_src, void *
         return x < y + bytes && y < x + bytes;
     };
     EET_REQUIRE(!overlap(k_src, k_dst) && !overlap(v_src, v_dst) && !overlap(k_src, v_dst) && !overlap(v_src, k_dst),
-                EET_ERR_INVALID_ARGUMENT, "eet_kv_cache_reorder: source and destination caches overlap");
+                EET_ERR_INVALID_ARGUMENT, "%s: source and destination caches overlap", fn);
+    return EET_OK;
+}
+
+extern "C" int eet_kv_cache_reorder(const void *k_src, const void *v_src, void *k_dst, void *v_dst,
+                                    const int64_t *reorder_index, int B, int H, int dh, int rows, int T_cap,
+                                    void *stream)
+{
+    if (int rc = check_gather("eet_kv_cache_reorder", k_src, v_src, k_dst, v_dst, reorder_index, B, H, dh, rows, T_cap))
+        return rc;
     if (B == 0 || rows == 0)
         return EET_OK;
     const int nvec = rows * (dh / 8);
@@ -459,6 +483,23 @@ extern "C" int eet_kv_cache_reorder(const void *k_src, const void *v_src, void *
                        static_cast<const _Float16 *>(k_src), static_cast<const _Float16 *>(v_src),
                        static_cast<_Float16 *>(k_dst), static_cast<_Float16 *>(v_dst),
                        reinterpret_cast<const long long *>(reorder_index), B, H, (size_t)T_cap * (dh / 8), nvec);
+    EET_HIP_CHECK(hipGetLastError());
+    return EET_OK;
+}
+
+extern "C" int eet_kv_cache_gather_rows(const void *k_src, const void *v_src, void *k_dst, void *v_dst,
+                                        const int32_t *beam_rows, int B, int H, int dh, int rows, int T_cap,
+                                        void *stream)
+{
+    if (int rc = check_gather("eet_kv_cache_gather_rows", k_src, v_src, k_dst, v_dst, beam_rows, B, H, dh, rows, T_cap))
+        return rc;
+    if (B == 0 || rows == 0)
+        return EET_OK;
+    const int nvec = rows * (dh / 8);
+    hipLaunchKernelGGL(kv_gather_rows_kernel, dim3((nvec + 1023) / 1024, H, B), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), static_cast<const uint4 *>(k_src),
+                       static_cast<const uint4 *>(v_src), static_cast<uint4 *>(k_dst), static_cast<uint4 *>(v_dst),
+                       beam_rows, B, H, T_cap, dh / 8, nvec);
     EET_HIP_CHECK(hipGetLastError());
     return EET_OK;
 }

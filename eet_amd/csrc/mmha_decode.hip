@@ -23,6 +23,7 @@
 #define eet_rope_table eet_timeline_rope_table
 #define eet_mmha_decode_workspace eet_timeline_mmha_decode_workspace
 #define eet_mmha_decode eet_timeline_mmha_decode
+#define eet_mmha_decode_beams eet_timeline_mmha_decode_beams
 #define eet_step_advance eet_timeline_step_advance
 #define eet_mmha_decode_replayable_workspace eet_timeline_mmha_decode_replayable_workspace
 #define eet_mmha_decode_replayable eet_timeline_mmha_decode_replayable
@@ -118,13 +119,27 @@ __device__ __forceinline__ u32x4 rotate8(const u32x4 &x, const u32x4 &y, int sub
 
 // DH: head size.  The DH/8 slices of a row are covered by one 16-byte load per lane.
 // One query per (b, h) attends rows [0, step); grid = (B*H, nsplit).
-template <int DH, int UN, int THREADS>
+//
+// BEAMS: a row of a sequence may lie in another sequence's slab of the cache.  beam_rows_in[b][t] names the
+// sequence whose slab holds row t of sequence b (NULL: every row in its own).  With `reorder` given, sequence b
+// goes on from the rows of sequence reorder[b] (an index outside [0, B) keeps its own): the launch reads row
+// reorder[b] of beam_rows_in and writes the composed names of the step - 1 older rows to beam_rows_out, the
+// H * nsplit workgroups of a sequence sharing that copy; the new token's row is always the sequence's own.
+// Beam search so moves 4 bytes per row and step instead of the 4 * H * DH bytes of its K and V (a copy before the
+// attention, which is bound by HBM as well): 16 beams of 32 heads x 128 at
+// 400 rows, copy + attention 31 + 19 us per layer before; six steps of four whole layers 2707 -> 1882 us.
+// A row's name is requested when the request for the row one ring length before it goes out, so it is as old as
+// the ring is deep when it is needed and adds no wait.  Rows come through the caches here (not non-temporal):
+// beams that share an ancestor read the same row, and the workgroups of one head, B apart by a multiple of
+// H workgroups, sit on the same XCD whenever H is a multiple of eight.
+template <int DH, int UN, int THREADS, bool BEAMS>
 __global__ __launch_bounds__(THREADS) void mmha_decode_split_kernel(
     const _Float16 *__restrict__ q, const _Float16 *__restrict__ k_new, const _Float16 *__restrict__ v_new,
     long qkv_stride, _Float16 *__restrict__ k_cache, _Float16 *__restrict__ v_cache, _Float16 *__restrict__ ctx,
     const _Float16 *__restrict__ alibi, const int64_t *__restrict__ pad, float *__restrict__ partial, int H,
     int step, int T_cap, int nsplit, float scale, const float *__restrict__ rope_row,
-    const int *__restrict__ step_dev, int alibi_ld_arg EET_ATL_PARAM)
+    const int *__restrict__ step_dev, int alibi_ld_arg, const int *beam_rows_in, int *beam_rows_out,
+    const int64_t *__restrict__ reorder, int B EET_ATL_PARAM)
 {
 #if defined(EET_TIMELINE)
     unsigned long long tl_t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -185,6 +200,19 @@ __global__ __launch_bounds__(THREADS) void mmha_decode_split_kernel(
     // They go through buffer resources of size zero when there is nothing to read
     // (no append, no rotary row): zeros come back and no branch surrounds the loads.
     const int r_last = own_last ? step - 1 - t0 : -1;
+    // BEAMS: whose rows this sequence goes on from, their names, and this workgroup's share of the name copy
+    int from = b, copied = 0, copy0 = 0, copy1 = 0;
+    const int *names = nullptr;
+    if (BEAMS) {
+        if (reorder != nullptr) {
+            const int64_t r = reorder[b];
+            from = r >= 0 && r < B ? (int)r : b;
+            const int share = (step - 1 + H * nsplit - 1) / (H * nsplit);
+            copy0 = (split * H + h) * share;
+            copy1 = min(step - 1, copy0 + share);
+        }
+        names = beam_rows_in ? beam_rows_in + (size_t)from * T_cap : nullptr;
+    }
     u32x4 knew, kpair, vnew, qv;
     float rcs[8], rsn[8];
 #if defined(__HIP_DEVICE_COMPILE__)  // buffer-resource builtins exist in the device pass only
@@ -200,6 +228,12 @@ __global__ __launch_bounds__(THREADS) void mmha_decode_split_kernel(
         const __amdgpu_buffer_rsrc_t qr = __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(q + qoff), 0,
                                                                             (unsigned)(DH * 2), 0x00020000);
         const unsigned i0 = (unsigned)(sub % (NS / 2)) * 8u;
+        if (BEAMS) {
+            const __amdgpu_buffer_rsrc_t crs = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<int *>(names ? names + copy0 : reinterpret_cast<const int *>(q)), 0,
+                names && copy1 > copy0 ? (unsigned)(copy1 - copy0) * 4u : 0u, 0x00020000);
+            copied = (int)__builtin_amdgcn_raw_buffer_load_b32(crs, (unsigned)tid * 4u, 0, 0);
+        }
         knew = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(knr, (unsigned)sub * 16u | idle, 0, 0));
         kpair = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(knr, (unsigned)pair * 16u | idle, 0, 0));
         vnew = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(vnr, (unsigned)sub * 16u | idle, 0, 0));
@@ -230,16 +264,34 @@ __global__ __launch_bounds__(THREADS) void mmha_decode_split_kernel(
     // whose size is exactly its n rows: requests past the end return zeros
     // without touching memory, which keeps the loop free of branches around loads.
 #if defined(__HIP_DEVICE_COMPILE__)  // buffer-resource builtins exist in the device pass only
-    const unsigned range_bytes = (unsigned)n * (unsigned)(DH * 2);
-    const __amdgpu_buffer_rsrc_t krs =
-        __builtin_amdgcn_make_buffer_rsrc(kc + (size_t)t0 * DH, 0, range_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t vrs =
-        __builtin_amdgcn_make_buffer_rsrc(vc + (size_t)t0 * DH, 0, range_bytes, 0x00020000);
+    // BEAMS: the resources begin at head h's row t0 of sequence 0 and end with the cache, which the host has
+    // checked to be at most 2^31 bytes; a request past the range has its top offset bit set.
+    const unsigned beam_bytes = BEAMS ? (unsigned)H * (unsigned)T_cap * (unsigned)(DH * 2) : 0u;
+    const size_t range_at = BEAMS ? ((size_t)h * T_cap + t0) * DH : 0;   // in halves, from the cache's start
+    const unsigned range_bytes =
+        BEAMS ? (n > 0 ? (unsigned)B * beam_bytes - (unsigned)(range_at * 2) : 0u) : (unsigned)n * (unsigned)(DH * 2);
+    const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
+        BEAMS ? k_cache + range_at : kc + (size_t)t0 * DH, 0, range_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
+        BEAMS ? v_cache + range_at : vc + (size_t)t0 * DH, 0, range_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<_Float16 *>(alibi ? alibi + (size_t)h * alibi_ld + t0 : q), 0, alibi ? (unsigned)n * 2u : 0u,
         0x00020000);
-    constexpr int kStream = 2;  // aux bits of a buffer load: non-temporal (every row is read exactly once)
-    auto row_off = [&](int i) { return (unsigned)((rs + i * RPB) * (DH * 2) + sub * 16) | idle; };
+    constexpr int kStream = BEAMS ? 0 : 2;  // aux bits of a buffer load: non-temporal (every row is read exactly once)
+    const __amdgpu_buffer_rsrc_t irs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<int *>(names ? names + t0 : reinterpret_cast<const int *>(q)), 0, names ? (unsigned)n * 4u : 0u,
+        0x00020000);
+    int name[UN];   // BEAMS: the sequence that holds the row which slot u requests next
+    auto request_name = [&](int u, int i) {
+        if (BEAMS)
+            name[u] = (int)__builtin_amdgcn_raw_buffer_load_b32(irs, (unsigned)((rs + i * RPB) * 4), 0, 0);
+    };
+    auto row_off = [&](int u, int i) {
+        const unsigned off = (unsigned)((rs + i * RPB) * (DH * 2) + sub * 16) | idle;
+        if (!BEAMS)
+            return off;
+        return rs + i * RPB < n ? (unsigned)(names ? name[u] : from) * beam_bytes + off : 0x80000000u;
+    };
     // Slot u is consumed first and refilled afterwards, so a slot's registers are
     // never live twice and the compiler keeps every slot in place: with the refill
     // ahead of the use it moved freshly requested registers at the end of each pass,
@@ -249,10 +301,14 @@ __global__ __launch_bounds__(THREADS) void mmha_decode_split_kernel(
     u32x4 kv[UN], vv[UN];
     int ab[UN];
     auto request = [&](int u, int i) {
-        kv[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(krs, row_off(i), 0, kStream));
-        vv[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(vrs, row_off(i), 0, kStream));
+        kv[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(krs, row_off(u, i), 0, kStream));
+        vv[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(vrs, row_off(u, i), 0, kStream));
         ab[u] = (int)(short)__builtin_amdgcn_raw_buffer_load_b16(ars, (unsigned)((rs + i * RPB) * 2), 0, 0);
+        request_name(u, i + UN);
     };
+#pragma unroll
+    for (int u = 0; u < UN; ++u)
+        request_name(u, u);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
@@ -278,6 +334,17 @@ __global__ __launch_bounds__(THREADS) void mmha_decode_split_kernel(
             *reinterpret_cast<u32x4 *>(kc + (size_t)(step - 1) * DH + sub * 8) = knew;
             *reinterpret_cast<u32x4 *>(vc + (size_t)(step - 1) * DH + sub * 8) = vnew;
         }
+    }
+    if (BEAMS) {
+        int *out = beam_rows_out + (size_t)b * T_cap;
+        if (reorder != nullptr) {
+            if (copy0 + tid < copy1)
+                out[copy0 + tid] = names ? copied : from;
+            for (int t = copy0 + tid + THREADS; t < copy1; t += THREADS)   // steps beyond H * nsplit * THREADS
+                out[t] = names ? names[t] : from;
+        }
+        if (append && h == 0 && tid == 0)
+            out[step - 1] = b;
     }
     __builtin_amdgcn_sched_barrier(0);
     EET_ATL_STAMP(1);   // new token rotated and appended, the ring requested
@@ -434,23 +501,34 @@ Plan pick_plan(int BH, int dh, int step)
     return p;
 }
 
+// Row names of a call whose sequences share cache rows (rows_out == nullptr: none, every row in its own slab).
+struct Beams {
+    const int *rows_in = nullptr;
+    int *rows_out = nullptr;
+    const int64_t *reorder = nullptr;
+};
+
 template <int DH, int THREADS>
 int launch_split(const void *q, const void *k, const void *v, long qkv_stride, void *kc, void *vc, void *ctx,
                  const void *alibi, const int64_t *pad, int B, int H, int step, int T_cap, void *ws, Plan plan,
-                 const float *rope_row, hipStream_t st, const int *step_dev = nullptr, int alibi_ld = 0)
+                 const float *rope_row, hipStream_t st, const int *step_dev = nullptr, int alibi_ld = 0,
+                 Beams beams = {})
 {
     const float scale = (float)(_Float16)(1.0f / sqrtf((float)DH));
     const int nsplit = plan.nsplit;
     dim3 grid(B * H, nsplit);
-    auto kern = (plan.ring == 8)   ? mmha_decode_split_kernel<DH, 8, THREADS>
-                : (plan.ring == 2) ? mmha_decode_split_kernel<DH, 2, THREADS>
-                                   : mmha_decode_split_kernel<DH, 4, THREADS>;
+    auto kern = (plan.ring == 8)   ? mmha_decode_split_kernel<DH, 8, THREADS, false>
+                : (plan.ring == 2) ? mmha_decode_split_kernel<DH, 2, THREADS, false>
+                                   : mmha_decode_split_kernel<DH, 4, THREADS, false>;
+    if (beams.rows_out != nullptr)
+        kern = (plan.ring == 2) ? mmha_decode_split_kernel<DH, 2, THREADS, true>
+                                : mmha_decode_split_kernel<DH, 4, THREADS, true>;
     hipLaunchKernelGGL(kern, grid, dim3(THREADS), 0, st,
                        static_cast<const _Float16 *>(q), static_cast<const _Float16 *>(k),
                        static_cast<const _Float16 *>(v), qkv_stride, static_cast<_Float16 *>(kc),
                        static_cast<_Float16 *>(vc), static_cast<_Float16 *>(ctx),
                        static_cast<const _Float16 *>(alibi), pad, static_cast<float *>(ws), H, step, T_cap, nsplit,
-                       scale, rope_row, step_dev, alibi_ld EET_ATL_ARG);
+                       scale, rope_row, step_dev, alibi_ld, beams.rows_in, beams.rows_out, beams.reorder, B EET_ATL_ARG);
     EET_HIP_CHECK(hipGetLastError());
     if (nsplit > 1) {
         hipLaunchKernelGGL((mmha_decode_merge_kernel<DH>), dim3(B * H), dim3(DH), 0, st,
@@ -463,16 +541,16 @@ int launch_split(const void *q, const void *k, const void *v, long qkv_stride, v
 template <int DH>
 int launch(const void *q, const void *k, const void *v, long qkv_stride, void *kc, void *vc, void *ctx,
            const void *alibi, const int64_t *pad, int B, int H, int step, int T_cap, void *ws, Plan plan,
-           const float *rope_row, hipStream_t st, const int *step_dev = nullptr, int alibi_ld = 0)
+           const float *rope_row, hipStream_t st, const int *step_dev = nullptr, int alibi_ld = 0, Beams beams = {})
 {
     if (plan.threads == 1024)
         return launch_split<DH, 1024>(q, k, v, qkv_stride, kc, vc, ctx, alibi, pad, B, H, step, T_cap, ws, plan,
-                                      rope_row, st, step_dev, alibi_ld);
+                                      rope_row, st, step_dev, alibi_ld, beams);
     if (plan.threads == 512)
         return launch_split<DH, 512>(q, k, v, qkv_stride, kc, vc, ctx, alibi, pad, B, H, step, T_cap, ws, plan,
-                                     rope_row, st, step_dev, alibi_ld);
+                                     rope_row, st, step_dev, alibi_ld, beams);
     return launch_split<DH, 256>(q, k, v, qkv_stride, kc, vc, ctx, alibi, pad, B, H, step, T_cap, ws, plan, rope_row,
-                                 st, step_dev, alibi_ld);
+                                 st, step_dev, alibi_ld, beams);
 }
 
 }  // namespace
@@ -535,21 +613,21 @@ static int check_mmha_args(const char *fn, const void *q, const void *k, const v
 static int run_mmha(const void *q, const void *k, const void *v, long qkv_stride, void *k_cache, void *v_cache,
                     void *ctx, const void *alibi, const int64_t *pad, int B, int H, int dh, int step, int T_cap,
                     const float *rope_cos_sin, void *partials, Plan plan, hipStream_t st,
-                    const int *step_dev = nullptr, int alibi_ld = 0)
+                    const int *step_dev = nullptr, int alibi_ld = 0, Beams beams = {})
 {
     switch (dh) {
         case 32:
             return launch<32>(q, k, v, qkv_stride, k_cache, v_cache, ctx, alibi, pad, B, H, step, T_cap, partials,
-                              plan, rope_cos_sin, st, step_dev, alibi_ld);
+                              plan, rope_cos_sin, st, step_dev, alibi_ld, beams);
         case 64:
             return launch<64>(q, k, v, qkv_stride, k_cache, v_cache, ctx, alibi, pad, B, H, step, T_cap, partials,
-                              plan, rope_cos_sin, st, step_dev, alibi_ld);
+                              plan, rope_cos_sin, st, step_dev, alibi_ld, beams);
         case 96:
             return launch<96>(q, k, v, qkv_stride, k_cache, v_cache, ctx, alibi, pad, B, H, step, T_cap, partials,
-                              plan, rope_cos_sin, st, step_dev, alibi_ld);
+                              plan, rope_cos_sin, st, step_dev, alibi_ld, beams);
         default:
             return launch<128>(q, k, v, qkv_stride, k_cache, v_cache, ctx, alibi, pad, B, H, step, T_cap, partials,
-                               plan, rope_cos_sin, st, step_dev, alibi_ld);
+                               plan, rope_cos_sin, st, step_dev, alibi_ld, beams);
     }
 }
 
@@ -567,6 +645,33 @@ extern "C" int eet_mmha_decode(const void *q, const void *k, const void *v, long
                 "eet_mmha_decode: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
     return run_mmha(q, k, v, qkv_stride, k_cache, v_cache, ctx, alibi, pad, B, H, dh, step, T_cap, rope_cos_sin,
                     workspace, plan, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int eet_mmha_decode_beams(const void *q, const void *k, const void *v, long qkv_stride, void *k_cache,
+                                     void *v_cache, void *ctx, const void *alibi, const int64_t *pad, int B, int H,
+                                     int dh, int step, int T_cap, const float *rope_cos_sin,
+                                     const int32_t *beam_rows_in, int32_t *beam_rows_out, const int64_t *reorder_index,
+                                     void *workspace, size_t workspace_bytes, void *stream)
+{
+    Plan plan;
+    if (int rc = check_mmha_args("eet_mmha_decode_beams", q, k, v, qkv_stride, k_cache, v_cache, ctx, B, H, dh, step,
+                                 T_cap, rope_cos_sin, &plan))
+        return rc;
+    EET_REQUIRE(k != nullptr && beam_rows_out != nullptr, EET_ERR_INVALID_ARGUMENT,
+                "eet_mmha_decode_beams: k, v and beam_rows_out must be given");
+    EET_REQUIRE(reorder_index != nullptr ? beam_rows_in != beam_rows_out : beam_rows_in == beam_rows_out,
+                EET_ERR_INVALID_ARGUMENT,
+                "eet_mmha_decode_beams: a reorder writes another table than it reads; without one the table is updated "
+                "in place (beam_rows_in == beam_rows_out)");
+    // row offsets are 32 bits wide, the top bit marks a request that must not touch memory
+    EET_REQUIRE((size_t)B * H * T_cap * dh * 2 <= ((size_t)1 << 31), EET_ERR_UNSUPPORTED_SHAPE,
+                "eet_mmha_decode_beams: the K cache of %d sequences is larger than 2 GiB", B);
+    const size_t need = plan.nsplit > 1 ? (size_t)B * H * plan.nsplit * (dh + 2) * sizeof(float) : 0;
+    EET_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), EET_ERR_WORKSPACE,
+                "eet_mmha_decode_beams: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
+    return run_mmha(q, k, v, qkv_stride, k_cache, v_cache, ctx, alibi, pad, B, H, dh, step, T_cap, rope_cos_sin,
+                    workspace, plan, static_cast<hipStream_t>(stream), nullptr, 0,
+                    Beams{beam_rows_in, beam_rows_out, reorder_index});
 }
 
 // ---------------------------------------------------------------------------

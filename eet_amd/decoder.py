@@ -289,6 +289,8 @@ class Int8Decoder:
         if self.reorder_state is not None and self.reorder_state.numel() != 0:
             raise RuntimeError("[EET][ERROR] capture_decode_step: a decoder that reorders its KV cache (beam search) "
                                "cannot replay a recorded step: the reorder swaps the cache buffers the graph points to")
+        for attn, _ in self.layers:
+            attn.settle_cache()     # rows named by an earlier beam search move before anything is recorded
         B = next_ids.shape[0]
         lib = ops.lib()
         step_dev = torch.tensor([self.layers[0][0].step], dtype=torch.int32, device=dev)

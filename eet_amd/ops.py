@@ -96,10 +96,10 @@ workspaces = _Workspaces()
 
 
 class _SpareKV:
-    """The second KV buffer of the beam-search reorder, shared by every attention op with the
-    same cache shape on a device: an op gathers into the spare pair, takes it as its cache and
-    leaves its old pair as the new spare.  The ops of a decoder run one after another on one
-    stream, so a single spare serves all layers."""
+    """The second KV buffer of a cache gather (a beam reorder that cannot go through row names, or an op
+    settling its cache), shared by every attention op with the same cache shape on a device: an op
+    gathers into the spare pair, takes it as its cache and leaves its old pair as the new spare.  The
+    ops of a decoder run one after another on one stream, so a single spare serves all layers."""
 
     def __init__(self):
         self._pairs = {}
@@ -338,8 +338,11 @@ class _MmhaInt8:
         dev = QKV_weights.device
         self.t_cap = desc.max_full_seq_len
         # KV cache, private to the op (csrc/op/llama_mmha.cpp:47-48); layout [B][H][T][dh]
-        self.k_cache = torch.zeros(desc.batch_size, H, self.t_cap, self.dh, dtype=torch.float16, device=dev)
-        self.v_cache = torch.zeros_like(self.k_cache)
+        self._k = torch.zeros(desc.batch_size, H, self.t_cap, self.dh, dtype=torch.float16, device=dev)
+        self._v = torch.zeros_like(self._k)
+        # Beam search: which sequence's slab holds row t of sequence b (eet_mmha_decode_beams), None while every
+        # row is in its own slab; two tables in turn, [batch_size][t_cap] int32
+        self._rows, self._row_tables = None, []
         self.step = 1
         self.first_batch = 0
         self.rope_table = _rope_table(self.t_cap, self.dh, dev) if self._rope else None
@@ -354,6 +357,80 @@ class _MmhaInt8:
             _check_vec("Output_bias", Output_bias, hidden)
             self.o_bias = Output_bias
         self.biased = self.with_bias or self.o_bias is not None
+
+    @property
+    def k_cache(self):
+        """[batch_size, H, max_full_seq_len, dh]; every sequence's rows in its own slab."""
+        self.settle_cache()
+        return self._k
+
+    @k_cache.setter
+    def k_cache(self, cache):
+        self.settle_cache()
+        self._k = cache
+
+    @property
+    def v_cache(self):
+        self.settle_cache()
+        return self._v
+
+    @v_cache.setter
+    def v_cache(self, cache):
+        self.settle_cache()
+        self._v = cache
+
+    def settle_cache(self):
+        """After a beam reorder the rows stay where they are and the attention reads them through a table of
+        row names; this moves every row into its own sequence's slab and drops the table."""
+        if self._rows is None:
+            return
+        rows, L = min(self.step, self.t_cap), lib()
+
+        def gather(k_dst, v_dst):
+            check(L.eet_kv_cache_gather_rows(self._k.data_ptr(), self._v.data_ptr(), k_dst.data_ptr(), v_dst.data_ptr(),
+                                             self._rows.data_ptr(), self.first_batch, self.desc.head_num, self.dh, rows,
+                                             self.t_cap, _stream()), "eet_kv_cache_gather_rows")
+        self._k, self._v = spare_kv.swap(self._k, self._v, gather)
+        self._rows = None
+
+    def _beam_rows(self, B, reorder, device):
+        """(beam_rows_in, beam_rows_out) of an incremental call, (None, None) for one without shared rows.
+        Row names need every beam in the call and 32-bit row offsets; what does not fit moves its rows."""
+        if self._rows is None and reorder is None:
+            return None, None
+        if (B != self.first_batch or replay_state is not None
+                or B * self.desc.head_num * self.t_cap * self.dh * 2 > 2 ** 31):
+            self.settle_cache()
+            if reorder is not None:
+                # beam b continues from the rows of beam reorder[b]: gather into the spare cache pair
+                # (one per cache shape, shared by all layers), then take that pair as this op's cache
+                def gather(k_dst, v_dst):
+                    check(lib().eet_kv_cache_reorder(self._k.data_ptr(), self._v.data_ptr(), k_dst.data_ptr(),
+                                                     v_dst.data_ptr(), reorder.data_ptr(), self.first_batch,
+                                                     self.desc.head_num, self.dh, self.step - 1, self.t_cap, _stream()),
+                          "eet_kv_cache_reorder")
+                self._k, self._v = spare_kv.swap(self._k, self._v, gather)
+            return None, None
+        if reorder is None:
+            return self._rows, self._rows
+        if not self._row_tables:
+            self._row_tables = [torch.zeros(self.desc.batch_size, self.t_cap, dtype=torch.int32, device=device)
+                                for _ in range(2)]
+        return self._rows, self._row_tables[1 if self._rows is self._row_tables[0] else 0]
+
+    def _attend(self, qkv, ctx, alibi, pad, B, rope, ws, rows_in, rows_out, reorder):
+        """q, k, v straight from the fused QKV rows; the kernel rotates q and k (rotary op only) and appends
+        k, v at row step-1."""
+        L, hd, base = lib(), self.inner, qkv.data_ptr()
+        args = (base, base + 2 * hd, base + 4 * hd, 3 * hd, self._k.data_ptr(), self._v.data_ptr(), ctx.data_ptr(),
+                _ptr(alibi), _ptr(pad), B, self.desc.head_num, self.dh, self.step, self.t_cap, rope)
+        tail = (ws.data_ptr(), ws.numel() * 4, _stream())
+        if rows_out is None:
+            check(L.eet_mmha_decode(*args, *tail), "eet_mmha_decode")
+        else:
+            check(L.eet_mmha_decode_beams(*args, _ptr(rows_in), rows_out.data_ptr(), _ptr(reorder), *tail),
+                  "eet_mmha_decode_beams")
+            self._rows = rows_out
 
     def forward(self, input, pre_padding_len, reorder_state, pre_layernorm, add_residual, first_pass,
                 relative_attention_bias=_EMPTY):
@@ -408,15 +485,13 @@ class _MmhaInt8:
             t0, time_step = self.step - 1, self.step - 1
         M = B * S
         L = lib()
-        if reorder is not None and not first_pass:
-            # beam b continues from the rows of beam reorder[b] (csrc/op/llama_mmha.cpp:248-252):
-            # gather into the spare cache pair (one per cache shape, shared by all layers), then
-            # take that pair as this op's cache
-            def gather(k_dst, v_dst):
-                check(L.eet_kv_cache_reorder(self.k_cache.data_ptr(), self.v_cache.data_ptr(), k_dst.data_ptr(),
-                                             v_dst.data_ptr(), reorder.data_ptr(), self.first_batch, H, dh,
-                                             self.step - 1, self.t_cap, _stream()), "eet_kv_cache_reorder")
-            self.k_cache, self.v_cache = spare_kv.swap(self.k_cache, self.v_cache, gather)
+        rows_in = rows_out = None
+        if first_pass:
+            self._rows = None       # a new prompt: its rows go to their own slabs
+            reorder = None
+        else:
+            # beam b continues from the rows of beam reorder[b] (csrc/op/llama_mmha.cpp:248-252)
+            rows_in, rows_out = self._beam_rows(B, reorder, dev)
         f16 = torch.float16
         xn = workspaces.get("layernorm", desc.batch_size * max(desc.max_seq_len, 1) * hidden, f16, dev)
         qkv = workspaces.get("qkv", desc.batch_size * max(desc.max_seq_len, 1) * 3 * self.inner, f16, dev)
@@ -450,8 +525,8 @@ class _MmhaInt8:
                 ws = workspaces.get("mmha_ws", max(need // 4, 1), torch.float32, dev)
                 check(L.eet_mmha_int8_decode_replayable(
                     x.data_ptr(), self.gamma.data_ptr(), desc.layernorm_eps, self.qkv_w.data_ptr(),
-                    self.qkv_s.data_ptr(), self.o_w.data_ptr(), self.o_s.data_ptr(), self.k_cache.data_ptr(),
-                    self.v_cache.data_ptr(), _ptr(alibi), ld, _ptr(pad),
+                    self.qkv_s.data_ptr(), self.o_w.data_ptr(), self.o_s.data_ptr(), self._k.data_ptr(),
+                    self._v.data_ptr(), _ptr(alibi), ld, _ptr(pad),
                     self.rope_table.data_ptr() if self._rope else None, qkv.data_ptr(), cbuf.data_ptr(), out.data_ptr(),
                     B, H, dh, hidden, rs.step_dev.data_ptr(), rs.step_max, self.t_cap, ws.data_ptr(), ws.numel() * 4,
                     *_k_split_ws(B, hidden, self.inner, EPI_RESIDUAL, dev), _stream()), "eet_mmha_int8_decode_replayable")
@@ -459,25 +534,27 @@ class _MmhaInt8:
                 return out[: M * hidden].view(B, S, hidden)
             rope = self.rope_table.data_ptr() + (self.step - 1) * dh * 4 if self._rope else None
             if launch_timer is not None:
-                inner, base = self.inner, qkv.data_ptr()
+                inner = self.inner
                 _timed("qkv_gemm+rmsnorm", linear_bytes(B, hidden, 3 * inner), lambda: _gemm(
                     x, self.qkv_w, self.qkv_s, qkv, B, 3 * inner, hidden, EPI_NONE, None, self.gamma, desc.layernorm_eps))
                 attn_bytes = 2 * self.step * B * inner * 2 + 6 * B * inner * 2 + (2 * H * self.step if alibi is not None else 0)
-                _timed("decode_attention", attn_bytes, lambda: check(L.eet_mmha_decode(
-                    base, base + 2 * inner, base + 4 * inner, 3 * inner, self.k_cache.data_ptr(), self.v_cache.data_ptr(),
-                    cbuf.data_ptr(), _ptr(alibi), _ptr(pad), B, H, dh, self.step, self.t_cap, rope, ws.data_ptr(),
-                    ws.numel() * 4, _stream()), "eet_mmha_decode"))
+                _timed("decode_attention", attn_bytes,
+                       lambda: self._attend(qkv, cbuf, alibi, pad, B, rope, ws, rows_in, rows_out, reorder))
                 _timed("o_gemm+residual", linear_bytes(B, inner, hidden, EPI_RESIDUAL), lambda: _gemm(
                     cbuf, self.o_w, self.o_s, out, B, hidden, inner, EPI_RESIDUAL, x))
                 self._keep = (x, pad, alibi, reorder)
                 return out[: M * hidden].view(B, S, hidden)
-            check(L.eet_mmha_int8_decode(x.data_ptr(), self.gamma.data_ptr(), desc.layernorm_eps,
-                                         self.qkv_w.data_ptr(), self.qkv_s.data_ptr(), self.o_w.data_ptr(),
-                                         self.o_s.data_ptr(), self.k_cache.data_ptr(), self.v_cache.data_ptr(),
-                                         _ptr(alibi), _ptr(pad), rope, qkv.data_ptr(), cbuf.data_ptr(),
-                                         out.data_ptr(), B, H, dh, hidden, self.step, self.t_cap, ws.data_ptr(),
-                                         ws.numel() * 4, *_k_split_ws(B, hidden, self.inner, EPI_RESIDUAL, dev),
-                                         _stream()), "eet_mmha_int8_decode")
+            args = (x.data_ptr(), self.gamma.data_ptr(), desc.layernorm_eps, self.qkv_w.data_ptr(),
+                    self.qkv_s.data_ptr(), self.o_w.data_ptr(), self.o_s.data_ptr(), self._k.data_ptr(),
+                    self._v.data_ptr(), _ptr(alibi), _ptr(pad), rope, qkv.data_ptr(), cbuf.data_ptr(), out.data_ptr(),
+                    B, H, dh, hidden, self.step, self.t_cap)
+            tail = (ws.data_ptr(), ws.numel() * 4, *_k_split_ws(B, hidden, self.inner, EPI_RESIDUAL, dev), _stream())
+            if rows_out is None:
+                check(L.eet_mmha_int8_decode(*args, *tail), "eet_mmha_int8_decode")
+            else:
+                check(L.eet_mmha_int8_decode_beams(*args, _ptr(rows_in), rows_out.data_ptr(), _ptr(reorder), *tail),
+                      "eet_mmha_int8_decode_beams")
+                self._rows = rows_out
             self._keep = (x, pad, alibi, reorder)  # inputs of kernels still in flight
             return out[: M * hidden].view(B, S, hidden)
         if self.with_bias:
@@ -496,8 +573,8 @@ class _MmhaInt8:
             _gemm(xn, self.qkv_w, self.qkv_s, qkv, M, 3 * self.inner, hidden)
         if first_pass:
             # split (+ rotary at position s) and write K, V rows [0, S) of the cache
-            check(L.eet_qkv_split(qkv.data_ptr(), qbuf.data_ptr(), self.k_cache.data_ptr(),
-                                  self.v_cache.data_ptr(), B, S, H, dh, 1 if self._rope else 0, -1, 0, self.t_cap,
+            check(L.eet_qkv_split(qkv.data_ptr(), qbuf.data_ptr(), self._k.data_ptr(),
+                                  self._v.data_ptr(), B, S, H, dh, 1 if self._rope else 0, -1, 0, self.t_cap,
                                   _stream()), "eet_qkv_split")
             alibi = None
             if bias is not None:
@@ -505,7 +582,7 @@ class _MmhaInt8:
                 if bias.dim() != 3 or bias.shape[0] != H or bias.shape[2] != S:
                     raise RuntimeError(f"[EET][ERROR] {self._name}: relative_attention_bias must be [H, S, S]")
                 alibi = bias[:, -1, :].to(f16).contiguous()
-            check(L.eet_prefill_attention(qbuf.data_ptr(), self.k_cache.data_ptr(), self.v_cache.data_ptr(),
+            check(L.eet_prefill_attention(qbuf.data_ptr(), self._k.data_ptr(), self._v.data_ptr(),
                                           cbuf.data_ptr(), _ptr(alibi), _ptr(pad), B, H, S, dh, self.t_cap,
                                           _stream()), "eet_prefill_attention")
         else:
@@ -517,14 +594,8 @@ class _MmhaInt8:
                 alibi = bias.to(f16).contiguous()
             need = L.eet_mmha_decode_workspace(B, H, dh, self.step)
             ws = workspaces.get("mmha_ws", max(need // 4, 1), torch.float32, dev)
-            # q, k, v are read straight from the fused GEMM output; the kernel rotates q and k
-            # (rotary op only) and appends k, v at row step-1
-            base, hd = qkv.data_ptr(), self.inner
             rope = self.rope_table.data_ptr() + (self.step - 1) * dh * 4 if self._rope else None
-            check(L.eet_mmha_decode(base, base + 2 * hd, base + 4 * hd, 3 * hd, self.k_cache.data_ptr(),
-                                    self.v_cache.data_ptr(), cbuf.data_ptr(), _ptr(alibi), _ptr(pad), B, H, dh,
-                                    self.step, self.t_cap, rope, ws.data_ptr(), ws.numel() * 4, _stream()),
-                  "eet_mmha_decode")
+            self._attend(qkv, cbuf, alibi, pad, B, rope, ws, rows_in, rows_out, reorder)
         # output projection with the residual add (csrc/op/llama_mmha.cpp:428-462) in its epilogue
         _gemm(cbuf, self.o_w, self.o_s, out, M, hidden, self.inner, EPI_RESIDUAL, x)
         if self.o_bias is not None:     # (out + input) + bias, csrc/core/add_bias.cu:13-20

@@ -237,6 +237,26 @@ int eet_mmha_decode(const void *q, const void *k, const void *v, long qkv_stride
                     const float *rope_cos_sin, void *workspace, size_t workspace_bytes,
                     void *stream);
 
+/* eet_mmha_decode for sequences that share cache rows (beam search): row t of
+ * sequence b lies in the slab of sequence beam_rows_in[b][t] (int32 [B][T_cap] in
+ * device memory; NULL: every row in its own slab).
+ *   reorder_index  NULL, or int64[B] in device memory: sequence b goes on from
+ *                  the rows of sequence reorder_index[b] (an entry outside [0, B)
+ *                  keeps its own), as eet_kv_cache_reorder ahead of the call would
+ *                  have it, without moving the rows
+ *   beam_rows_out  the names of the step rows after the call, entry step-1 (the
+ *                  appended row) being b: another table than beam_rows_in with a
+ *                  reorder, the same table (updated in place) without
+ * Entries of beam_rows_in at t >= step-1 are not used; the others must be in
+ * [0, B).  k, v must be given; B*H*T_cap*dh*2 must not exceed 2^31.  The results
+ * are those of eet_kv_cache_reorder followed by eet_mmha_decode, bit for bit. */
+int eet_mmha_decode_beams(const void *q, const void *k, const void *v, long qkv_stride,
+                          void *k_cache, void *v_cache, void *ctx, const void *alibi,
+                          const int64_t *pad, int B, int H, int dh, int step, int T_cap,
+                          const float *rope_cos_sin, const int32_t *beam_rows_in,
+                          int32_t *beam_rows_out, const int64_t *reorder_index, void *workspace,
+                          size_t workspace_bytes, void *stream);
+
 /* eet_mmha_decode for callers that cannot allocate device memory or carry a
  * workspace around: code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc.  It has no counterpart in the reference.  Same
@@ -317,6 +337,13 @@ int eet_kv_cache_reorder(const void *k_src, const void *v_src, void *k_dst, void
                          const int64_t *reorder_index, int B, int H, int dh, int rows, int T_cap,
                          void *stream);
 
+/* dst[b][h][t][:] = src[beam_rows[b][t]][h][t][:] for t < rows: the caches behind
+ * a table of eet_mmha_decode_beams with every row in its own sequence's slab (a
+ * name outside [0, B) stands for b).  Other arguments as in eet_kv_cache_reorder. */
+int eet_kv_cache_gather_rows(const void *k_src, const void *v_src, void *k_dst, void *v_dst,
+                             const int32_t *beam_rows, int B, int H, int dh, int rows, int T_cap,
+                             void *stream);
+
 /* One incremental call (one new token per sequence, B <= 32) of the attention
  * sub-layer, all launches from one call: RMSnorm + QKV projection, rotary (when
  * rope_cos_sin is given) + cache append + masked attention, output projection +
@@ -338,6 +365,16 @@ int eet_mmha_int8_decode(const void *x, const void *rms_gamma, float rms_eps, co
                          int B, int H, int dh, int hidden, int step, int T_cap, void *workspace,
                          size_t workspace_bytes, void *gemm_workspace, size_t gemm_workspace_bytes,
                          void *stream);
+
+/* eet_mmha_int8_decode over caches with shared rows: see eet_mmha_decode_beams. */
+int eet_mmha_int8_decode_beams(const void *x, const void *rms_gamma, float rms_eps,
+                               const void *qkv_w, const void *qkv_scale, const void *o_w,
+                               const void *o_scale, void *k_cache, void *v_cache, const void *alibi,
+                               const int64_t *pad, const float *rope_cos_sin, void *qkv_buf,
+                               void *ctx_buf, void *out, int B, int H, int dh, int hidden, int step,
+                               int T_cap, const int32_t *beam_rows_in, int32_t *beam_rows_out,
+                               const int64_t *reorder_index, void *workspace, size_t workspace_bytes,
+                               void *gemm_workspace, size_t gemm_workspace_bytes, void *stream);
 
 /* The gated FFN sub-layer for B <= 32 rows, both launches from one call:
  * RMSnorm + gate and up projections + SwiGLU (w01 / scale01: gate and up

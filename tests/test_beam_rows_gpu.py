@@ -1,0 +1,108 @@
+"""Beam search over shared cache rows (eet_mmha_decode_beams): against the cache reorder followed by the ordinary
+call, which moves the same rows -- the same sums in the same order, so the outputs are equal bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+from eet_amd import decoder as D
+from eet_amd._lib import check, lib
+from gpu_util import mmha, stream
+
+
+def test_argument_errors():
+    L = lib()
+    buf = np.zeros(4096, np.uint8)
+    p, q = buf.ctypes.data, buf.ctypes.data + 1024
+
+    def call(k=p, rows_in=p, rows_out=q, reorder=p, B=1, H=1, dh=64, step=4, cap=8):
+        return L.eet_mmha_decode_beams(p, k, k, 0, p, p, p, None, None, B, H, dh, step, cap, None, rows_in, rows_out,
+                                       reorder, None, 0, None)
+    assert call(k=None) == -1
+    assert call(rows_out=None) == -1
+    assert call(rows_in=q) == -1                     # a reorder may not read the table it writes
+    assert call(reorder=None) == -1                  # without one the table is updated in place
+    assert call(reorder=None, rows_in=None) == -1
+    assert call(B=65, H=32, dh=128, cap=4096) == -2  # 2 GiB of K cache is the largest
+    assert call(step=9) == -1
+    assert call(dh=40) == -2
+    assert L.eet_kv_cache_gather_rows(p, p, p, p, p, 1, 1, 64, 4, 8, None) == -1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,dh,first,cap,padded,alibi", [
+    (2, 1, 32, 1, 8, False, False),          # from a one-row prompt on
+    (5, 3, 96, 30, 40, True, True),          # idle lanes, padding, bias
+    (16, 8, 64, 255, 262, True, False),      # around one split of the time axis
+    (3, 8, 128, 1021, 1030, False, True),    # several splits
+    (260, 1, 32, 700, 704, False, False),    # more names per workgroup than lanes
+])
+def test_rows_by_name_equal_moved_rows(gpu, B, H, dh, first, cap, padded, alibi):
+    g = torch.Generator().manual_seed(B * 1000 + dh)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).half().to(gpu)
+    L = lib()
+    kc, vc = rnd(B, H, cap, dh), rnd(B, H, cap, dh)              # rows by name: never moved
+    km, vm = kc.clone(), vc.clone()                              # moved before every call
+    tables = [torch.zeros(B, cap, dtype=torch.int32, device=gpu) for _ in range(2)]
+    names = None
+    pad = torch.tensor([(7 * b) % max(first, 1) for b in range(B)], device=gpu) if padded else None
+    rope = torch.empty(cap, dh, device=gpu)
+    check(L.eet_rope_table(rope.data_ptr(), cap, dh, stream()))
+    for step, reordered in zip(range(first + 1, cap + 1), [True, True, False, True, True, False, True, True, True]):
+        q, k, v = rnd(B, H * dh), rnd(B, H * dh), rnd(B, H * dh)
+        bias = rnd(H, step) if alibi else None
+        order = None
+        if reordered:
+            order = torch.randint(0, B, (B,), generator=g)
+            order[B // 2] = B if step % 2 else -1                # out of range: the beam keeps its own rows
+            order = order.to(gpu)
+            k2, v2 = torch.zeros_like(km), torch.zeros_like(vm)
+            check(L.eet_kv_cache_reorder(km.data_ptr(), vm.data_ptr(), k2.data_ptr(), v2.data_ptr(), order.data_ptr(),
+                                         B, H, dh, step - 1, cap, stream()))
+            km, vm = k2, v2
+        row = rope[step - 1]
+        want = mmha(q, k, v, km, vm, step, pad, bias, rope_row=row)
+        if names is None and order is None:
+            got = mmha(q, k, v, kc, vc, step, pad, bias, rope_row=row)
+        else:
+            out = names if order is None else tables[1 if names is tables[0] else 0]
+            got = torch.empty_like(want)
+            need = L.eet_mmha_decode_workspace(B, H, dh, step)
+            ws = torch.empty(max(need // 4, 1), device=gpu)
+            check(L.eet_mmha_decode_beams(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), 0, kc.data_ptr(), vc.data_ptr(), got.data_ptr(),
+                bias.data_ptr() if alibi else None, pad.data_ptr() if padded else None, B, H, dh, step, cap,
+                row.data_ptr(), names.data_ptr() if names is not None else None, out.data_ptr(),
+                order.data_ptr() if order is not None else None, ws.data_ptr(), ws.numel() * 4, stream()))
+            names = out
+        assert torch.equal(got, want), f"step {step}"
+        if names is not None:
+            ks, vs = torch.zeros_like(kc), torch.zeros_like(vc)
+            check(L.eet_kv_cache_gather_rows(kc.data_ptr(), vc.data_ptr(), ks.data_ptr(), vs.data_ptr(),
+                                             names.data_ptr(), B, H, dh, step, cap, stream()))
+            assert torch.equal(ks[:, :, :step], km[:, :, :step]) and torch.equal(vs[:, :, :step], vm[:, :, :step])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [3, 40])          # one library call per op, separate launches
+def test_op_settles_its_cache(gpu, rows):
+    """A call that cannot name rows (fewer sequences than the prompt had) and a read of the cache in between give
+    what rows that moved on every reorder give."""
+    cfg = D.DecoderConfig(num_layers=1, hidden=256, heads=4, d_ff=704, vocab=64, max_batch=rows, max_prompt=8,
+                          max_full_seq=32)
+    sd, _ = D.random_state_dict(cfg, seed=3)
+    a, b = (D.Int8Decoder(cfg, sd, device="cuda:0") for _ in range(2))
+    g = torch.Generator().manual_seed(1)
+    ids = torch.randint(0, 64, (rows, 6), generator=g).to(gpu)
+    assert torch.equal(a.logits(ids, True), b.logits(ids, True))
+    for t, n in enumerate([rows, rows, rows - 1, rows - 1, rows]):
+        order = torch.randint(0, rows, (rows,), generator=g).to(gpu) if t != 3 else torch.empty(0, dtype=torch.long)
+        ids = torch.randint(0, 64, (n, 1), generator=g).to(gpu)
+        a.reorder_state = b.reorder_state = order
+        la, lb = a.logits(ids, False), b.logits(ids, False)
+        assert torch.equal(la, lb)
+        ka = b.layers[0][0].k_cache                # b settles after every step, a only when it must
+        assert b.layers[0][0]._rows is None and ka.shape[0] == rows
+    step = a.layers[0][0].step
+    assert torch.equal(a.layers[0][0].k_cache[: rows - 1, :, :step], b.layers[0][0].k_cache[: rows - 1, :, :step])
