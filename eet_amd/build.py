@@ -18,7 +18,8 @@ LIB = os.path.join(HERE, "libeet_hip.so")
 BENCH_LIB = os.path.join(HERE, "libeet_bench.so")
 
 SOURCES = ["packer.cc", "tuning.cc", "decode_ops.cc", "chain.hip", "packer_device.hip", "gemm_w8a16.hip",
-           "gemm_w8a16_large.hip", "mmha_decode.hip", "prefill_attention.hip", "glue.hip"]
+           "gemm_w8a16_large.hip", "mmha_decode.hip", "prefill_attention.hip", "glue.hip",
+           "head.hip"]
 BENCH_SOURCES = ["probe.hip"]
 # compiled again with -DEET_TIMELINE for libeet_bench.so
 TIMELINE_SOURCES = {"gemm_w8a16.hip": "gemm_w8a16.timeline.o", "mmha_decode.hip": "mmha_decode.timeline.o"}

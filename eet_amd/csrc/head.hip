@@ -1,0 +1,124 @@
+// The output head of a decode step: out[M][N] = x[M][K] * w[N][K]^T in fp16 with fp32 sums, M <= 16 rows (one per
+// sequence), w the row-major fp16 matrix of the checkpoint.
+//
+// HBM-bound: 2*N*K weight bytes, each read once.  A workgroup owns NT tiles of 16 output columns over the whole k
+// range; its wavefronts take blocks of 64 k (one 128-byte line per row) in turn, so that together they stream NT * 16
+// adjacent rows.  Weights and activations are loaded as the operands of v_mfma_f32_16x16x32_f16 (lane (g, i): row i,
+// 16 bytes at 16 g) into a ring of U register slots, a slot being refilled as soon as it is consumed; nothing goes
+// through LDS before the wavefronts' fp32 sums meet there.  Requests past the last k block have the top offset bit
+// set: they return zeros and touch no memory, which keeps the loop free of branches around loads.  The two halves of
+// a line are two requests: with the non-temporal bit the second one missed again (M = 1, 64000 <- 5120: 138 us
+// against 108).
+// What the activations cost sets NT: every workgroup reads all M*K of them.  Measured on MI355X with the weights
+// from HBM, us, M = 1 / 16, NT = 1, 2, 4 (library GEMM): 32000 <- 4096 48.6 / 64.5, 53.4 / 60.2, 49.4 / 50.0 (55.8 / 56.1);
+// 32000 <- 2048 27.6 / 35.2, 25.2 / 30.6, 26.4 / 28.1 (31.1 / 31.5); 8000 <- 1024 4.9 / 6.2, 4.6 / 5.2, 6.1 / 6.8 (19.1: its
+// own launch cost on the host).  64000 <- 5120 at M = 16 is 127 against the library's 110: matrices that large
+// are refused here and left to it.
+#include <hip/hip_runtime.h>
+
+#include "common.h"
+
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// NT: tiles of 16 columns per workgroup.
+template <int NT, int WAVES, int U>
+__global__ __launch_bounds__(64 * WAVES) void head_kernel(const _Float16 *__restrict__ x, long x_stride,
+                                                          const _Float16 *__restrict__ w, _Float16 *__restrict__ out,
+                                                          int M, int N, int K)
+{
+    __shared__ float part[WAVES][NT][4][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * (NT * 16);
+    const int blocks = K / 64;
+    f32x4 acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+        acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#if defined(__HIP_DEVICE_COMPILE__)  // buffer-resource builtins exist in the device pass only
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<_Float16 *>(w + (size_t)n0 * K), 0, (unsigned)min(NT * 16, N - n0) * (unsigned)K * 2u, 0x00020000);
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<_Float16 *>(x), 0, ((unsigned)(M - 1) * (unsigned)x_stride + (unsigned)K) * 2u, 0x00020000);
+    const unsigned wlane = (unsigned)i * (unsigned)K * 2u + (unsigned)g * 16u;
+    const unsigned xlane = i < M ? (unsigned)i * (unsigned)x_stride * 2u + (unsigned)g * 16u : 0x80000000u;
+    u32x4 wv[U][NT][2], xv[U][2];
+    auto request = [&](int u, int kb) {
+        const unsigned off = kb < blocks ? (unsigned)kb * 128u : 0x80000000u;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                wv[u][t][h] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                    wr, (wlane + (unsigned)t * 16u * (unsigned)K * 2u + h * 64u + off) | (off & 0x80000000u), 0, 0));
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            xv[u][h] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                xr, (xlane + h * 64u + off) | ((off | xlane) & 0x80000000u), 0, 0));
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        request(u, wave + u * WAVES);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    for (int kb = wave; kb < blocks; kb += U * WAVES) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, xv[u][h]),
+                                                                    __builtin_bit_cast(half8, wv[u][t][h]), acc[t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            request(u, kb + (u + U) * WAVES);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#endif
+    // lane (g, i) of a tile holds rows 4 g + r of column i
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            part[wave][t][r][lane] = acc[t][r];
+    __syncthreads();
+    for (int e = threadIdx.x; e < NT * 256; e += 64 * WAVES) {
+        const int l = e & 63, r = (e >> 6) & 3, t = e >> 8;
+        const int row = (l >> 4) * 4 + r, col = n0 + t * 16 + (l & 15);
+        if (row >= M || col >= N)
+            continue;
+        float s = 0.f;
+#pragma unroll
+        for (int v = 0; v < WAVES; ++v)
+            s += part[v][t][r][l];
+        out[(size_t)row * N + col] = (_Float16)s;
+    }
+}
+
+}  // namespace
+
+extern "C" int eet_head_f16(const void *x, long x_stride, const void *w, void *out, int M, int N, int K, void *stream)
+{
+    EET_REQUIRE(x && w && out, EET_ERR_INVALID_ARGUMENT, "eet_head_f16: null pointer");
+    EET_REQUIRE(M > 0 && M <= 16 && N > 0 && K > 0 && K % 64 == 0 && N % 16 == 0, EET_ERR_UNSUPPORTED_SHAPE,
+                "eet_head_f16: need 1 <= M <= 16, K %% 64 == 0 and N %% 16 == 0, got M=%d N=%d K=%d", M, N, K);
+    EET_REQUIRE((size_t)N * K <= ((size_t)1 << 28), EET_ERR_UNSUPPORTED_SHAPE,
+                "eet_head_f16: a matrix of %d x %d is larger than 2^28 elements", N, K);
+    EET_REQUIRE(x_stride >= K && x_stride % 8 == 0 && ((size_t)(M - 1) * x_stride + K) * 2 <= ((size_t)1 << 31),
+                EET_ERR_INVALID_ARGUMENT, "eet_head_f16: x_stride %ld must be a multiple of 8, at least K", x_stride);
+    EET_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) % 16 == 0, EET_ERR_INVALID_ARGUMENT,
+                "eet_head_f16: x and w need 16-byte alignment");
+    // four tiles per workgroup once that leaves two workgroups per CU, two where it leaves about one (figures above)
+    const int tiles = N / 16, nt = tiles >= 1792 ? 4 : tiles >= 256 ? 2 : 1;
+    auto kern = nt == 4 ? head_kernel<4, 8, 1> : nt == 2 ? head_kernel<2, 8, 2> : head_kernel<1, 8, 2>;
+    hipLaunchKernelGGL(kern, dim3((tiles + nt - 1) / nt), dim3(512), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const _Float16 *>(x), x_stride, static_cast<const _Float16 *>(w),
+                       static_cast<_Float16 *>(out), M, N, K);
+    EET_HIP_CHECK(hipGetLastError());
+    return EET_OK;
+}

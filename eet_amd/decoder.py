@@ -5,8 +5,7 @@ the greedy loop that drives it.
 Counterpart of python/eet/transformers/modeling_llama.py:51-297, 452-471
 (EETLlamaSelfMaskedAttention ... EETLlamaForCausalLM), modeling_baichuan.py:
 51-80, 270-317 (ALiBi mask) and pipelines/generation.py:1144-1218 (greedy
-search).  Embedding and lm_head stay fp16 torch ops, as in the reference
-(modeling_llama.py:370-372, 471).
+search).  Embedding and lm_head stay fp16, as in the reference (modeling_llama.py:370-372, 471).
 """
 import math
 from dataclasses import dataclass
@@ -173,8 +172,8 @@ class Int8Decoder:
     def logits(self, input_ids, first_pass=True, attention_mask=None):
         h = self(input_ids, first_pass, attention_mask)
         B = h.shape[0]
-        return ops._timed("lm_head fp16 (torch)", self.lm_head.numel() * 2 + B * (self.cfg.hidden + self.cfg.vocab) * 2,
-                          lambda: torch.nn.functional.linear(h[:, -1:, :], self.lm_head))
+        return ops._timed("lm_head fp16", self.lm_head.numel() * 2 + B * (self.cfg.hidden + self.cfg.vocab) * 2,
+                          lambda: ops.head(h, self.lm_head))
 
     @torch.no_grad()
     def greedy(self, input_ids, max_new_tokens, attention_mask=None):

@@ -744,6 +744,23 @@ class GatedFeedForwardNetworkInt8:
         return out[: M * hidden].view(B, S, hidden)
 
 
+def head(h, weight):
+    """Logits [B, 1, V] of the last position of h [B, S, K] under the fp16 output matrix [V, K].  Up to 16 sequences
+    and 2^28 weights run on eet_head_f16; the rest, and whatever torch does beyond the product (autograd on the
+    matrix, autocast), on torch's linear."""
+    B, S, K = h.shape
+    V = weight.shape[0]
+    if (B > 16 or K % 64 or V % 16 or V * K > 2 ** 28 or weight.dtype != torch.float16 or h.dtype != torch.float16
+            or not weight.is_contiguous() or not h.is_contiguous() or weight.device != h.device or not h.is_cuda
+            or weight.shape != (V, K) or weight.data_ptr() % 16 or h.data_ptr() % 16
+            or (weight.requires_grad and torch.is_grad_enabled()) or torch.is_autocast_enabled()):
+        return torch.nn.functional.linear(h[:, -1:, :], weight)
+    out = torch.empty(B, 1, V, dtype=torch.float16, device=h.device)
+    check(lib().eet_head_f16(h.data_ptr() + 2 * (S - 1) * K, S * K, weight.data_ptr(), out.data_ptr(), B, V, K, _stream()),
+          "eet_head_f16")
+    return out
+
+
 class LayerNorm:
     """csrc/op/layer_norm.cpp:8-33: LayerNorm(gamma, beta), RMSnorm when beta is empty."""
 

@@ -390,6 +390,14 @@ int eet_gated_ffn_int8_decode(const void *x, const void *rms_gamma, float rms_ep
                               int add_residual, void *gemm_workspace, size_t gemm_workspace_bytes,
                               void *stream);
 
+/* The output head of a decode step: out[M][N] = x[M][K] * w[N][K]^T, fp16 with fp32
+ * sums.  Row m of x begins at x + m*x_stride halves (x_stride >= K, a multiple of 8);
+ * w row-major, out contiguous.  M <= 16, K % 64 == 0, N % 16 == 0, N*K <= 2^28, x and w
+ * 16-byte aligned.  Stands in for the fp16 linear of the reference's caller
+ * (python/eet/transformers/modeling_llama.py:471) at decode sizes. */
+int eet_head_f16(const void *x, long x_stride, const void *w, void *out, int M, int N, int K,
+                 void *stream);
+
 /* Causal prefill attention over the prompt, reading K and V from the caches
  * filled by eet_qkv_split.  q [B][H][S][dh]; ctx [B][S][H*dh]; alibi NULL or
  * [H][S] half (slope * j, the diagonal row of the reference's mask); pad as in

@@ -1,0 +1,52 @@
+"""The fp16 output head (eet_head_f16, ops.head) against an fp32 product."""
+import numpy as np
+import pytest
+import torch
+
+from eet_amd import ops
+from eet_amd._lib import lib
+
+
+def test_argument_errors():
+    buf = np.zeros(8192, np.uint8)
+    p = buf.ctypes.data + (-buf.ctypes.data) % 16
+
+    def call(x=p, stride=64, M=1, N=16, K=64):
+        return lib().eet_head_f16(x, stride, p, p, M, N, K, None)
+    assert call(x=None) == -1
+    assert call(M=17) == -2 and call(M=0) == -2
+    assert call(K=96) == -2 and call(N=24) == -2
+    assert call(N=65536, K=8192, stride=8192) == -2          # more than 2^28 weights
+    assert call(stride=56) == -1 and call(stride=68) == -1
+    assert call(x=p + 2) == -1
+    assert call(M=16, stride=1 << 27) == -1                  # rows beyond 32-bit offsets
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,S,N,K", [(1, 1, 16, 64), (16, 3, 48, 128), (3, 1, 4096, 1024), (15, 2, 4080, 576),
+                                     (8, 1, 8000, 1024), (9, 5, 28704, 448), (16, 1, 32000, 4096)])
+def test_head(gpu, M, S, N, K):
+    """One and several tiles per workgroup, a last workgroup with fewer, fewer k blocks than wavefronts, whole and
+    broken rounds of them, the last position of several.  fp32 sums of at most 2^12 products and one rounding to fp16:
+    2^-11 of the result plus 2^-12 (K * 2^-24) of the sum of magnitudes."""
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    h = torch.randn(M, S, K, generator=g, device=gpu).half()
+    w = (torch.randn(N, K, generator=g, device=gpu) * 0.02).half()
+    got = ops.head(h, w)
+    assert got.shape == (M, 1, N) and got.dtype == torch.float16
+    x = h[:, -1].double()
+    want, size = x @ w.double().t(), x.abs() @ w.double().abs().t()
+    assert ((got[:, 0].double() - want).abs() <= 2 ** -11 * want.abs() + 2 ** -12 * size * K / 2 ** 12 + 2 ** -25).all()
+
+
+@pytest.mark.gpu
+def test_what_stays_with_torch(gpu):
+    h = torch.randn(2, 1, 64, device=gpu).half()
+    w = torch.randn(32, 64, device=gpu).half()
+    wide = torch.randn(17, 1, 64, device=gpu).half()
+    assert torch.equal(ops.head(wide, w), torch.nn.functional.linear(wide, w))
+    assert ops.head(h, w.clone().requires_grad_()).requires_grad
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert ops.head(h, w).dtype == torch.bfloat16
+    odd = torch.randn(33, 64, device=gpu).half()
+    assert torch.equal(ops.head(h, odd), torch.nn.functional.linear(h, odd))
