@@ -61,7 +61,7 @@ class _Workspaces:
         self._recorders = []
 
     def get(self, name, numel, dtype, device, zero=False):
-        key = (name, str(device), dtype)
+        key = (name, device, dtype)
         buf = self._bufs.get(key)
         if buf is None or buf.numel() < numel:
             alloc = torch.zeros if zero else torch.empty      # zero: a buffer whose first use needs zeros
@@ -434,9 +434,55 @@ class _MmhaInt8:
 
     def forward(self, input, pre_padding_len, reorder_state, pre_layernorm, add_residual, first_pass,
                 relative_attention_bias=_EMPTY):
+        if not first_pass and launch_timer is None and replay_state is None:
+            y = self._decode(input, pre_padding_len, reorder_state, relative_attention_bias)
+            if y is not None:
+                return y
         with _StreamScope():
             return self._forward(input, pre_padding_len, reorder_state, pre_layernorm, add_residual, first_pass,
                                  relative_attention_bias)
+
+    def _decode(self, x, pad, reorder, bias):
+        """The incremental call as a server makes it -- whole fp16 rows, every cache row in its own slab -- with no
+        host work beside the library call; None for any other call, valid or not, before anything has changed.
+        (A token step of a small decoder is bound by the host: of the 9 us that an attention call spent outside
+        the library, whose three launches take 10, 6 are left.)"""
+        desc = self.desc
+        if (x.dtype != torch.float16 or x.dim() != 3 or not x.is_cuda or not x.is_contiguous() or self.biased
+                or self._rows is not None or (reorder is not None and reorder.numel() != 0)):
+            return None
+        (B, S, hidden), H, step = x.shape, desc.head_num, self.step + 1
+        if S != 1 or hidden != desc.hidden_units or B > desc.batch_size or B > RMS_FUSE_MAX_M or step > self.t_cap:
+            return None
+        pad_ptr = alibi_ptr = rope = ws_ptr = None
+        if pad is not None and pad.numel() != 0:
+            if pad.dtype != torch.int64 or pad.numel() < B or not pad.is_cuda or not pad.is_contiguous():
+                return None
+            pad_ptr = pad.data_ptr()
+        if bias is not None and bias.numel() != 0:
+            if (self._rope or bias.numel() != H * step or bias.dtype != torch.float16 or not bias.is_cuda
+                    or not bias.is_contiguous()):
+                return None
+            alibi_ptr = bias.data_ptr()
+        if self._rope:
+            rope = self.rope_table.data_ptr() + (step - 1) * self.dh * 4
+        L, f16, dev, st = lib(), torch.float16, x.device, _current_stream()
+        rows = desc.batch_size * max(desc.max_seq_len, 1)
+        qkv = workspaces.get("qkv", rows * 3 * self.inner, f16, dev)
+        cbuf = workspaces.get("context_buf", rows * self.inner, f16, dev)
+        out = workspaces.get("self_mask_attn_cache", rows * hidden, f16, dev)
+        need = L.eet_mmha_int8_decode_workspace(B, H, self.dh, step)
+        if need:
+            ws_ptr = workspaces.get("mmha_ws", need // 4, torch.float32, dev).data_ptr()
+        gemm_ws, gemm_ws_bytes = _k_split_ws(B, hidden, self.inner, EPI_RESIDUAL, dev)
+        self.step = step
+        check(L.eet_mmha_int8_decode(x.data_ptr(), self.gamma.data_ptr(), desc.layernorm_eps, self.qkv_w.data_ptr(),
+                                     self.qkv_s.data_ptr(), self.o_w.data_ptr(), self.o_s.data_ptr(), self._k.data_ptr(),
+                                     self._v.data_ptr(), alibi_ptr, pad_ptr, rope, qkv.data_ptr(), cbuf.data_ptr(),
+                                     out.data_ptr(), B, H, self.dh, hidden, step, self.t_cap, ws_ptr, need, gemm_ws,
+                                     gemm_ws_bytes, st), "eet_mmha_int8_decode")
+        self._keep = (x, pad, bias, reorder)  # inputs of kernels still in flight
+        return out.as_strided((B, 1, hidden), (hidden, hidden, 1))
 
     def _forward(self, input, pre_padding_len, reorder_state, pre_layernorm, add_residual, first_pass,
                  relative_attention_bias):
@@ -661,8 +707,33 @@ class GatedFeedForwardNetworkInt8:
                                                 Intermediate_1_weights, Intermediate_1_scale)
 
     def forward(self, input, pre_layernorm, add_residual):
+        if launch_timer is None and (pre_layernorm or not add_residual):
+            y = self._decode(input, add_residual)
+            if y is not None:
+                return y
         with _StreamScope():
             return self._forward(input, pre_layernorm, add_residual)
+
+    def _decode(self, x, add_residual):
+        """_MmhaInt8._decode for the feed-forward call: RMSnorm in front, no output bias, at most 32 whole rows."""
+        desc = self.desc
+        if (x.dtype != torch.float16 or x.dim() != 3 or not x.is_cuda or not x.is_contiguous()
+                or self.beta is not None or self.o_bias is not None):
+            return None
+        B, S, hidden = x.shape
+        M, seq = B * S, max(desc.max_seq_len, 1)
+        if hidden != desc.hidden_units or B > desc.batch_size or S > seq or M > RMS_FUSE_MAX_M:
+            return None
+        L, f16, dev, st, cap = lib(), torch.float16, x.device, _current_stream(), desc.batch_size * seq
+        act = workspaces.get("ffn_inner_act", cap * self.d_ff, f16, dev)
+        out = workspaces.get(self.cache_name, cap * hidden, f16, dev)
+        gemm_ws, gemm_ws_bytes = _k_split_ws(M, hidden, self.d_ff, EPI_RESIDUAL if add_residual else EPI_NONE, dev)
+        check(L.eet_gated_ffn_int8_decode(x.data_ptr(), self.gamma.data_ptr(), desc.layernorm_eps, self.w01.data_ptr(),
+                                          self.s01.data_ptr(), self.w2.data_ptr(), self.s2.data_ptr(), act.data_ptr(),
+                                          out.data_ptr(), M, hidden, self.d_ff, 1 if add_residual else 0, gemm_ws,
+                                          gemm_ws_bytes, st), "eet_gated_ffn_int8_decode")
+        self._keep = x
+        return out.as_strided((B, S, hidden), (S * hidden, hidden, 1))
 
     def _forward(self, input, pre_layernorm, add_residual):
         desc = self.desc
@@ -696,16 +767,7 @@ class GatedFeedForwardNetworkInt8:
             self._keep = x
             return out[: M * hidden].view(B, S, hidden)
         if M <= RMS_FUSE_MAX_M:
-            check(lib().eet_gated_ffn_int8_decode(x.data_ptr(), self.gamma.data_ptr(), desc.layernorm_eps,
-                                                  self.w01.data_ptr(), self.s01.data_ptr(), self.w2.data_ptr(),
-                                                  self.s2.data_ptr(), act.data_ptr(), out.data_ptr(), M, hidden,
-                                                  self.d_ff, 1 if add_residual else 0,
-                                                  *_k_split_ws(M, hidden, self.d_ff,
-                                                               EPI_RESIDUAL if add_residual else EPI_NONE, dev),
-                                                  _stream()),
-                  "eet_gated_ffn_int8_decode")
-            self._keep = x
-            return out[: M * hidden].view(B, S, hidden)
+            return self._decode(x, add_residual)      # a strided input, now whole
         _rmsnorm(x, self.gamma, xn, M, hidden, desc.layernorm_eps)
         _gemm(xn, self.w01, self.s01, act, M, 2 * self.d_ff, hidden, EPI_SWIGLU)
         # fc3 with add_input_bias_layernorm's residual add (:303-357) in its epilogue
@@ -782,7 +844,7 @@ class LayerNorm:
             raise RuntimeError("[EET][ERROR] LayerNorm: input must be fp16 [B, S, hidden]")
         x = input.contiguous()
         B, S, hidden = x.shape
-        if B * S > self.output.shape[0] * self.output.shape[1]:
+        if B * S * hidden > self.output.numel():
             raise RuntimeError("[EET][ERROR] LayerNorm: input larger than batch_size * max_seq_len")
         if self.beta is not None:
             check(lib().eet_layernorm(x.data_ptr(), self.gamma.data_ptr(), self.beta.data_ptr(), self.output.data_ptr(),
@@ -790,7 +852,7 @@ class LayerNorm:
         else:
             _rmsnorm(x, self.gamma, self.output, B * S, hidden, desc.layernorm_eps)
         self._keep = x
-        return self.output.view(-1)[: B * S * hidden].view(B, S, hidden)
+        return self.output.as_strided((B, S, hidden), (S * hidden, hidden, 1))
 
 
 # ----------------------------------------------------------------------------

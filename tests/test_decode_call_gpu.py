@@ -1,0 +1,51 @@
+"""The ops' short incremental call and the general one give the same rows, the same step and the same errors."""
+import pytest
+import torch
+
+from eet_amd import decoder as D
+
+
+def decoders(alibi, rows):
+    cfg = D.DecoderConfig(num_layers=1, hidden=256, heads=2, d_ff=704, vocab=64, alibi=alibi, max_batch=rows,
+                          max_prompt=8, max_full_seq=12)
+    sd, _ = D.random_state_dict(cfg, seed=5)
+    return cfg, [D.Int8Decoder(cfg, sd, device="cuda:0").layers[0] for _ in range(2)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("alibi", [False, True])
+@pytest.mark.parametrize("rows", [1, 5, 32, 33])
+def test_forms_of_one_call(gpu, alibi, rows):
+    cfg, ((a, fa), (b, fb)) = decoders(alibi, rows)
+    g = torch.Generator().manual_seed(rows)
+    none = torch.empty(0)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).half().to(gpu)
+    pad = torch.randint(0, 4, (rows, 1), generator=g).to(gpu)
+    wide = torch.stack([pad, pad], 1)[:, 0]                            # the same values, strided
+    x = rnd(rows, 6, 256)
+    mask = D.alibi_mask(2, 6).to(gpu) if alibi else none
+    for op in (a, b):
+        op.forward(x, pad, none, True, True, True, mask)
+    for t in range(3):
+        x = rnd(rows, 1, 512)[:, :, ::2]                               # strided rows: the general call
+        bias = D.alibi_mask(2, 7 + t)[:, -1:].contiguous().to(gpu) if alibi else none
+        ya = a.forward(x.contiguous(), pad, none, True, True, False, bias).clone()
+        yb = b.forward(x, wide, none, True, True, False, bias.float()).clone()
+        assert torch.equal(ya, yb) and ya.shape == (rows, 1, 256) and a.step == b.step == 7 + t
+        za = fa.forward(ya, True, True).clone()
+        assert torch.equal(za, fb.forward(torch.stack([yb, yb], 2)[:, :, 0], True, True))
+        assert torch.equal(fa.forward(ya, False, False), fb.forward(yb, True, False))
+    x = x.contiguous()
+    for bad in (dict(input=x.float()), dict(input=x[:, :, :128]), dict(input=x.expand(rows, 2, 256)), dict(input=x.cpu()),
+                dict(pre_padding_len=pad.int()), dict(relative_attention_bias=rnd(2, 1, 3))):
+        call = dict(dict(input=x, pre_padding_len=pad, reorder_state=none, pre_layernorm=True, add_residual=True,
+                         first_pass=False, relative_attention_bias=bias), **bad)
+        step = a.step
+        with pytest.raises(RuntimeError, match="EET"):
+            a.forward(**call)
+        a.step = step
+    a.step = cfg.max_full_seq
+    with pytest.raises(RuntimeError, match="max_full_seq_len"):
+        a.forward(x, pad, none, True, True, False, none)
