@@ -354,47 +354,67 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 
 
 // ---------------------------------------------------------------------------
-// Head size 128 (LLaMA-7B, Baichuan-13B): the same transposed formulation with
-// the K and V chunks brought into LDS by the memory pipeline itself.
+// Head sizes 64, 96 and 128: the same transposed formulation with the K and V chunks brought into LDS by the memory pipeline itself.
 //
 // A workgroup of 8 wavefronts takes 256 queries of one (b, h); wavefront w owns
 // the 16-query tiles w and w + 8 of the block (one early, one late, so that the
 // causal triangle is split evenly) and skips a tile once the chunks have passed
-// its diagonal.  K and V rows stay row-major in LDS, 256 B per row, copied
+// its diagonal.  K and V rows stay row-major in LDS as they lie in the cache, copied
 // global -> LDS with buffer_load_dwordx4 ... lds (no staging registers, no
 // ds_write) into a ring of four 64-key stages, one pair of chunks ahead of the
-// pair being multiplied; one s_barrier per pair.  Piece p (16 B) of row r sits at
-// position p ^ swz(r), with one swizzle for K and another for V, so that the K
-// operand reads (lane = row) and the V reads hit distinct banks.  V^T operands come out of the row-major rows through
+// pair being multiplied; one s_barrier per pair.  The 16-byte pieces of a chunk, numbered
+// through (DH / 8 per row), form lines of 256 B; piece p of line r sits at position p ^ swz(r), with one swizzle for K
+// and another for V, so that the K operand reads (lane = row) and the V reads hit distinct banks.  V^T operands come out of the row-major rows through
 // ds_read_b64_tr_b16, which hands lane i column i of a 4 x 16 block of halves.
+//
+// The register-staged kernel above spends its time between barriers: load, transpose, store, wait, with one chunk in
+// flight.  Against it, us, 32 heads, no bias: head size 64 4 x 500 tokens 20.9 -> 12.2, 1 x 2048 54.3 -> 31.9, 8 x 1000
+// 94.4 -> 61.8; 96 25.6 -> 17.9, 79.5 -> 44.8, 118 -> 86.6; 128 28.0 -> 20.5, 75.8 -> 51.0, 136 -> 100.  It is left with
+// head size 32 and with bias rows that are not whole 4-byte units.
 // ---------------------------------------------------------------------------
-constexpr int kD = 128;
-
 constexpr int kKAhead = 6, kVAhead = 4;    // K operand reads / V operands (two reads each) in flight ahead of their MFMAs
-constexpr int kStageVec = 2 * 1024 + 16;   // u32x4 per stage: K rows, V rows, bias row (+ padding)
 
 // Measured on MI355X with 8 wavefronts reading back to back: a 16-byte operand read (lane = row) runs at
 // full rate when the piece index is XORed with the row number itself, and at half rate with the V
 // swizzle or with rows padded to 272 B; the transposing 8-byte reads of V run at full rate with the
 // swizzle below (4 consecutive rows must land on 4 different pairs of positions) and not with padding.
-__device__ __forceinline__ int k_swz(int r) { return r & 15; }
-__device__ __forceinline__ int row_swz(int r) { return ((r & 7) << 1) | ((r >> 3) & 1); }
+// A line holds one row of 128, two of 64 or four thirds of one of 96 halves.  Sixteen lanes that read one piece
+// each of sixteen rows must land on sixteen positions: the row number itself does it at 128; at 64 the row's
+// parity is the top bit of the position and the line number has to move the other three; at 96 the rows four
+// apart, three lines on, meet in one position, so the line number moves the low two bits.  The V reads need eight
+// consecutive rows on eight different pairs of positions, rows eight apart on the other half of a pair.
+template <int DH>
+__device__ __forceinline__ int k_swz(int r)
+{
+    return DH == 128 ? r & 15 : DH == 64 ? r & 7 : r & 3;
+}
+template <int DH>
+__device__ __forceinline__ int row_swz(int r)
+{
+    return DH == 128 ? ((r & 7) << 1) | ((r >> 3) & 1)
+           : DH == 64 ? ((r & 3) << 1) | ((r >> 2) & 1)
+                      : ((r & 1) << 1) | ((r >> 1) & 1);
+}
 
 typedef short short4v __attribute__((ext_vector_type(4)));
 
 // NQT 16-query tiles per wavefront, WAVES wavefronts, STAGES chunk buffers: 16 NQT WAVES queries per workgroup.
 // <2, 8, 4>: two wavefronts per SIMD with 256 registers each, every K and V operand read feeds two tiles;
 // <1, 8, 2>: half the queries and half the ring, so that two workgroups fit a CU, four wavefronts per SIMD, twice
-// the operand reads per query (the LDS has the room).  launch_dh128 says which runs when.
-template <bool ALIBI, int NQT, int WAVES, int STAGES>
+// the operand reads per query (the LDS has the room).  launch_dma says which runs when.
+template <int DH, bool ALIBI, int NQT, int WAVES, int STAGES>
 __global__ __launch_bounds__(64 * WAVES)
-    __attribute__((amdgpu_waves_per_eu(STAGES == 2 ? 2 * WAVES / 4 : WAVES / 4, STAGES == 2 ? 2 * WAVES / 4 : WAVES / 4))) void prefill_attention_dh128_kernel(
+    __attribute__((amdgpu_waves_per_eu(STAGES == 2 ? 2 * WAVES / 4 : WAVES / 4, STAGES == 2 ? 2 * WAVES / 4 : WAVES / 4))) void prefill_attention_dma_kernel(
     const _Float16 *__restrict__ q, const _Float16 *__restrict__ k_cache, const _Float16 *__restrict__ v_cache,
     _Float16 *__restrict__ ctx, const _Float16 *__restrict__ alibi, const int64_t *__restrict__ pad, int H, int S,
     int T_cap, float scale, int group)
 {
 #if defined(__HIP_DEVICE_COMPILE__)  // buffer-resource builtins exist in the device pass only
-    constexpr int DC = kD / 32, DT = kD / 16;
+    constexpr int DC = DH / 32, DT = DH / 16, PPR = DH / 8;   // PPR: 16-byte pieces per row
+    constexpr int kRowsVec = kBK * PPR;                       // u32x4 of a chunk's K (or V) rows
+    constexpr int kStageVec = 2 * kRowsVec + 16;              // ... of a stage: K rows, V rows, bias row (+ padding)
+    // Head size 128 takes the denominators through the matrix cores (below); the others add the fp32 weights up.
+    constexpr bool kMfmaSum = DH == 128;
     constexpr int kBQ2 = 16 * NQT * WAVES;   // queries per workgroup
     constexpr int kGroup = STAGES / 2;       // chunks per barrier
     __shared__ u32x4 lds[STAGES * kStageVec];
@@ -410,19 +430,20 @@ __global__ __launch_bounds__(64 * WAVES)
     const int q0 = qblock * kBQ2;
     const int padb = pad ? (int)min((int64_t)S, max((int64_t)0, pad[b])) : 0;
 
-    const _Float16 *kbase = k_cache + (size_t)bh * T_cap * kD;
-    const _Float16 *vbase = v_cache + (size_t)bh * T_cap * kD;
-    const _Float16 *qbase = q + (size_t)bh * S * kD;
+    const _Float16 *kbase = k_cache + (size_t)bh * T_cap * DH;
+    const _Float16 *vbase = v_cache + (size_t)bh * T_cap * DH;
+    const _Float16 *qbase = q + (size_t)bh * S * DH;
     // rows >= S are out of range: they read as zeros (and are masked: such a key follows every query)
     const __amdgpu_buffer_rsrc_t krs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(kbase), 0, (unsigned)S * (kD * 2), 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(kbase), 0, (unsigned)S * (DH * 2), 0x00020000);
     const __amdgpu_buffer_rsrc_t vrs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(vbase), 0, (unsigned)S * (kD * 2), 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(vbase), 0, (unsigned)S * (DH * 2), 0x00020000);
     const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<_Float16 *>(ALIBI ? alibi + (size_t)h * S : q), 0, ALIBI ? (unsigned)S * 2u : 0u, 0x00020000);
 
     static_assert((NQT == 1 || NQT == 2) && 16 % WAVES == 0 && (STAGES == 2 || STAGES == 4), "launch shape");
-    constexpr int KI = 16 / WAVES;   // DMA instructions per wavefront for the K rows of a chunk (and for the V rows)
+    constexpr int kDma = kRowsVec / 64;               // DMA instructions for the K rows of a chunk (and for the V rows)
+    constexpr int KI = (kDma + WAVES - 1) / WAVES;    // ... per wavefront
     // the query tiles of this wavefront: one early, one late (the causal triangle is split evenly)
     int tq0[NQT];
 #pragma unroll
@@ -434,7 +455,7 @@ __global__ __launch_bounds__(64 * WAVES)
         const int qi = min(tq0[qt] + j, S - 1);
 #pragma unroll
         for (int c = 0; c < DC; ++c)
-            qop[qt][c] = *reinterpret_cast<const half8 *>(qbase + (size_t)qi * kD + 32 * c + 8 * g);
+            qop[qt][c] = *reinterpret_cast<const half8 *>(qbase + (size_t)qi * DH + 32 * c + 8 * g);
     }
     floatx4 oacc[NQT][DT];
     // The softmax denominators ride along as one more accumulator tile per query tile: P^T times a V^T operand of
@@ -442,37 +463,40 @@ __global__ __launch_bounds__(64 * WAVES)
     // fp16, like the numerator) -- two matrix instructions per chunk and tile instead of sixteen vector adds per
     // lane, and no cross-lane sum at the end.
     floatx4 lacc[NQT];
-    float m_run[NQT];
+    float m_run[NQT], l_run[NQT];
     const half8 ones8 = {(_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f,
                          (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f};
 #pragma unroll
     for (int qt = 0; qt < NQT; ++qt) {
         m_run[qt] = -INFINITY;
+        l_run[qt] = 0.f;
         lacc[qt] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
             oacc[qt][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
 
-    // DMA: instruction t of a chunk fills rows 4t .. 4t+3 (1 KiB); lane l carries position l % 16 of row
-    // 4t + l / 16, i.e. piece (l % 16) ^ swz(row).  Wavefront w issues instructions KI w .. KI w + KI - 1 of K and of V.
+    // DMA: instruction t of a chunk fills lines 4t .. 4t+3 (1 KiB); lane l carries position l % 16 of line
+    // 4t + l / 16, i.e. piece (l % 16) ^ swz(line).  Wavefront w issues instructions KI w .. KI w + KI - 1 of K and of V.
     int dma_off_k[KI], dma_off_v[KI];   // byte offset of this lane's piece within a chunk, per instruction
 #pragma unroll
     for (int i = 0; i < KI; ++i) {
-        const int row = 4 * (KI * wave + i) + (lane >> 4);
-        dma_off_k[i] = row * (kD * 2) + (((lane & 15) ^ k_swz(row)) << 4);
-        dma_off_v[i] = row * (kD * 2) + (((lane & 15) ^ row_swz(row)) << 4);
+        const int line = 4 * (KI * wave + i) + (lane >> 4);
+        dma_off_k[i] = line * 256 + (((lane & 15) ^ k_swz<DH>(line)) << 4);
+        dma_off_v[i] = line * 256 + (((lane & 15) ^ row_swz<DH>(line)) << 4);
     }
     auto dma_chunk = [&](int stage, int kc0) {
         u32x4 *st = lds + stage * kStageVec;
-        const int base = kc0 * (kD * 2);   // in the lane offset: the range check of a buffer load covers it
+        const int base = kc0 * (DH * 2);   // in the lane offset: the range check of a buffer load covers it
 #pragma unroll
         for (int i = 0; i < KI; ++i) {
+            if (kDma % WAVES != 0 && KI * wave + i >= kDma)   // fewer instructions than the wavefronts have room for
+                continue;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, st + (KI * wave + i) * 64, 16, base + dma_off_k[i], 0, 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(vrs, st + 1024 + (KI * wave + i) * 64, 16, base + dma_off_v[i], 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(vrs, st + kRowsVec + (KI * wave + i) * 64, 16, base + dma_off_v[i], 0, 0, 0);
         }
         if (ALIBI)   // the chunk's 64 bias terms (128 B): every wavefront writes the same bytes
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, st + 2048, 4, kc0 * 2 + (lane & 31) * 4, 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, st + 2 * kRowsVec, 4, kc0 * 2 + (lane & 31) * 4, 0, 0, 0);
     };
 
     constexpr float kLog2e = 1.4426950408889634f;
@@ -482,11 +506,26 @@ __global__ __launch_bounds__(64 * WAVES)
     const int k_end = min(S, q0 + kBQ2);
     const int nchunks = (k_end - k_begin + kBK - 1) / kBK;
 
+    // Operand addresses within a stage.  Sixteen rows on are PPR whole lines on, which leaves the swizzles as they
+    // are: a key tile is a constant offset.  V: lane j of a 16-lane group supplies 8 bytes (d = 16*dt + 4*(j%4) .. +3)
+    // of key row 4g + j/4.
+    int k_at[DC], v_at[DT];   // in u32x4 / in bytes
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+        const int piece = j * PPR + 4 * c + g;
+        k_at[c] = (piece & ~15) + ((piece & 15) ^ k_swz<DH>(piece >> 4));
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+        const int piece = (4 * g + (j >> 2)) * PPR + 2 * dt + ((j & 3) >> 1);
+        v_at[dt] = ((piece & ~15) + ((piece & 15) ^ row_swz<DH>(piece >> 4))) * 16 + (j & 1) * 8;
+    }
+
     // the work on one chunk for the query tiles named in MASK (bit qt)
     auto compute = [&](auto mask_c, const u32x4 *st, int kc0) {
         constexpr int MASK = decltype(mask_c)::value;
         const u32x4 *kst = st;
-        const unsigned char *vst = reinterpret_cast<const unsigned char *>(st + 1024);
+        const unsigned char *vst = reinterpret_cast<const unsigned char *>(st + kRowsVec);
         floatx4 sacc[NQT][4];
 #pragma unroll
         for (int qt = 0; qt < NQT; ++qt)
@@ -495,10 +534,9 @@ __global__ __launch_bounds__(64 * WAVES)
                 sacc[qt][kt] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
-            const int row = 16 * kt + j;
 #pragma unroll
             for (int c = 0; c < DC; ++c) {
-                const half8 kop = __builtin_bit_cast(half8, kst[row * 16 + ((4 * c + g) ^ k_swz(row))]);
+                const half8 kop = __builtin_bit_cast(half8, kst[k_at[c] + kt * 16 * PPR]);
 #pragma unroll
                 for (int qt = 0; qt < NQT; ++qt)
                     if (MASK & (1 << qt))
@@ -511,7 +549,7 @@ __global__ __launch_bounds__(64 * WAVES)
             constexpr int kPer = (MASK == 3) ? 2 : 1;   // query tiles taking part
             __builtin_amdgcn_sched_group_barrier(0x100, kKAhead, 0);
 #pragma unroll
-            for (int n = 0; n < 16 - kKAhead; ++n) {
+            for (int n = 0; n < 4 * DC - kKAhead; ++n) {
                 __builtin_amdgcn_sched_group_barrier(0x008, kPer, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
@@ -519,7 +557,7 @@ __global__ __launch_bounds__(64 * WAVES)
         }
         half4 bias4[4];
         if (ALIBI) {
-            const _Float16 *bst = reinterpret_cast<const _Float16 *>(st + 2048);
+            const _Float16 *bst = reinterpret_cast<const _Float16 *>(st + 2 * kRowsVec);
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt)
                 bias4[kt] = *reinterpret_cast<const half4 *>(bst + 16 * kt + 4 * g);
@@ -571,7 +609,10 @@ __global__ __launch_bounds__(64 * WAVES)
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt)
                     oacc[qt][dt] *= corr;
-                lacc[qt] *= corr;
+                if (kMfmaSum)
+                    lacc[qt] *= corr;
+                else
+                    l_run[qt] *= corr;
                 m_run[qt] = raise ? cmax : m_ref;
             }
             const float m_safe = (m_run[qt] == -INFINITY) ? 0.f : m_run[qt];
@@ -582,6 +623,15 @@ __global__ __launch_bounds__(64 * WAVES)
                 for (int r = 0; r < 4; ++r)
                     p[kt][r] = ALIBI ? __builtin_amdgcn_exp2f(sacc[qt][kt][r] - m_safe)
                                      : __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[qt][kt][r], scale2, -m_safe));
+            if (!kMfmaSum) {   // this lane's share of the keys; the lanes of a query meet at the end
+                float psum = 0.f;
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        psum += p[kt][r];
+                l_run[qt] += psum;
+            }
 #pragma unroll
             for (int hf = 0; hf < 2; ++hf) {
                 half8 o;
@@ -594,9 +644,7 @@ __global__ __launch_bounds__(64 * WAVES)
             }
         }
         // O^T += V^T . P^T.  Lane (g, j) needs d = 16*dt + j and keys 4g .. 4g+3 of tiles 2*hf and 2*hf + 1.
-        // One transposing read covers the 4 keys of one tile: lane j of a 16-lane group supplies 8 bytes
-        // (d = 16*dt + 4*(j%4) .. +3) of key row 4g + j/4 and receives the column d = 16*dt + j.
-        const int vr = j >> 2, vc4 = j & 3;
+        // One transposing read covers the 4 keys of one tile: lane j of a 16-lane group receives column d = 16*dt + j.
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
 #pragma unroll
@@ -604,9 +652,7 @@ __global__ __launch_bounds__(64 * WAVES)
                 short4v part[2];
 #pragma unroll
                 for (int a = 0; a < 2; ++a) {
-                    const int key = 32 * hf + 16 * a + 4 * g + vr;
-                    const int pos = (2 * dt + (vc4 >> 1)) ^ row_swz(key);
-                    const unsigned char *addr = vst + key * (kD * 2) + pos * 16 + (vc4 & 1) * 8;
+                    const unsigned char *addr = vst + v_at[dt] + (2 * hf + a) * 256 * PPR;
                     part[a] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                         (short4v __attribute__((address_space(3))) *)(addr));
                 }
@@ -619,7 +665,7 @@ __global__ __launch_bounds__(64 * WAVES)
             }
         }
 #pragma unroll
-        for (int hf = 0; hf < 2; ++hf)
+        for (int hf = 0; hf < 2 * kMfmaSum; ++hf)
 #pragma unroll
             for (int qt = 0; qt < NQT; ++qt)
                 if (MASK & (1 << qt))
@@ -633,7 +679,7 @@ __global__ __launch_bounds__(64 * WAVES)
                 __builtin_amdgcn_sched_group_barrier(0x008, kPer, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, (kVAhead + 2) * kPer, 0);   // + the two of the denominators
+            __builtin_amdgcn_sched_group_barrier(0x008, (kVAhead + 2 * kMfmaSum) * kPer, 0);   // + the two of the denominators
         }
     };
 
@@ -670,12 +716,17 @@ __global__ __launch_bounds__(64 * WAVES)
 
 #pragma unroll
     for (int qt = 0; qt < NQT; ++qt) {
-        const float l = lacc[qt][0];   // every row of the tile holds the sum for query j
+        float l = lacc[qt][0];   // every row of the tile holds the sum for query j
+        if (!kMfmaSum) {
+            l = l_run[qt];
+            l += __shfl_xor(l, 16, 64);
+            l += __shfl_xor(l, 32, 64);
+        }
         const int qi = tq0[qt] + j;
         if (qi >= S)
             continue;
         const float inv = (qi < padb) ? 0.f : 1.0f / (l + 1e-6f);
-        _Float16 *dst = ctx + ((size_t)(b * S + qi) * H + h) * kD;
+        _Float16 *dst = ctx + ((size_t)(b * S + qi) * H + h) * DH;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
             half4 o;
@@ -705,22 +756,32 @@ int pairs_per_group(int slots_per_xcd, int q_blocks, int pairs)
     return g < 4 ? 4 : g;
 }
 
-int launch_dh128(const void *q, const void *kc, const void *vc, void *ctx, const void *alibi, const int64_t *pad, int B,
+bool prefers_wide_blocks(long long blocks, int S)
+{
+    const long long rounds = (blocks + 255) / 256;
+    return S > 1536 && rounds >= 2 && blocks * 10 >= rounds * 256 * 9;
+}
+
+template <int DH>
+int launch_dma(const void *q, const void *kc, const void *vc, void *ctx, const void *alibi, const int64_t *pad, int B,
                  int H, int S, int T_cap, hipStream_t st)
 {
-    const float scale = (float)(_Float16)(1.0f / sqrtf(128.0f));
-    // Launch shape by prompt length (measured at B*H = 256 .. 320):
+    const float scale = (float)(_Float16)(1.0f / sqrtf((float)DH));
+    // Two launch shapes:
     //   1  128 queries per workgroup, eight one-tile wavefronts, two stages: two workgroups share a CU, so the
-    //      start-up, the diagonal chunks and the drain of one overlap the other's work -- up to 1536 tokens
-    //      (+13 % at 256, +20 % at 512, +6-9 % at 1024, +2-3 % at 1536; 3-6 % behind from 2048 on);
-    //   2  256 queries, eight two-tile wavefronts, four stages (every operand read feeds two tiles) -- beyond.
-    // (256 queries as sixteen one-tile wavefronts was within 2 % of shape 2 everywhere and is not kept.)
-    // A tuning override picks either.
+    //      start-up, the diagonal chunks and the drain of one overlap the other's work;
+    //   2  256 queries, eight two-tile wavefronts, four stages (every operand read feeds two tiles).
+    // Shape 2 wins once its workgroups last (over 1536 tokens) and fill the CUs in at least two nearly whole rounds;
+    // with one round, or a part of one left over, the longest blocks decide and half the block is better.  Measured,
+    // us, shape 1 / 2, one prompt of 2048 tokens (32 heads): head size 64 31.9 / 41.5, 96 44.8 / 54.7, 128 51.0 / 61.9;
+    // 40 heads of 128 with bias 72.5 / 79.8; two prompts: 56.4 / 52.4, 78.8 / 69.6, 89.2 / 85.1, but 40 heads (2.5
+    // rounds) 124 / 138; eight prompts of 1000: 61.8 / 66.1, 86.6 / 89.1, 100 / 105.  (256 queries as sixteen one-tile
+    // wavefronts was within 2 % of shape 2 everywhere and is not kept.)  A tuning override picks either.
     int shape = eet::tuning().prefill_shape;
     if (shape < 1 || shape > 2)
-        shape = S <= 1536 ? 1 : 2;
+        shape = prefers_wide_blocks((long long)B * H * ((S + 255) / 256), S) ? 2 : 1;
 #define EET_PF_LAUNCH(A_, N_, W_, S_)                                                                              \
-    hipLaunchKernelGGL((prefill_attention_dh128_kernel<A_, N_, W_, S_>),                                          \
+    hipLaunchKernelGGL((prefill_attention_dma_kernel<DH, A_, N_, W_, S_>),                                          \
                        dim3(B * H, (S + 16 * N_ * W_ - 1) / (16 * N_ * W_)), dim3(64 * W_), 0, st,                \
                        static_cast<const _Float16 *>(q), static_cast<const _Float16 *>(kc),                       \
                        static_cast<const _Float16 *>(vc), static_cast<_Float16 *>(ctx),                           \
@@ -771,16 +832,19 @@ extern "C" int eet_prefill_attention(const void *q, const void *k_cache, const v
     EET_REQUIRE((long long)B * H < (1ll << 31) && (S + kBQ - 1) / kBQ <= 65535, EET_ERR_UNSUPPORTED_SHAPE,
                 "eet_prefill_attention: B*H = %lld or S = %d too large", (long long)B * H, S);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    switch (dh) {
-        case 32: return launch<32>(q, k_cache, v_cache, ctx, alibi, pad, B, H, S, T_cap, st);
-        case 64: return launch<64>(q, k_cache, v_cache, ctx, alibi, pad, B, H, S, T_cap, st);
-        case 96: return launch<96>(q, k_cache, v_cache, ctx, alibi, pad, B, H, S, T_cap, st);
-        default: break;
-    }
-    // head size 128: the DMA kernel; it addresses a (b, h) cache range with 32-bit byte offsets and reads the
-    // bias row in 4-byte units
+    // The DMA kernel addresses a (b, h) cache range with 32-bit byte offsets and reads the bias row in 4-byte units;
+    // head size 32 has the other one.
     const bool alibi_ok = alibi == nullptr || (S % 2 == 0 && reinterpret_cast<uintptr_t>(alibi) % 4 == 0);
-    if ((long long)S * 256 < (1ll << 31) && alibi_ok && eet::tuning().prefill_legacy == 0)
-        return launch_dh128(q, k_cache, v_cache, ctx, alibi, pad, B, H, S, T_cap, st);
-    return launch<128>(q, k_cache, v_cache, ctx, alibi, pad, B, H, S, T_cap, st);
+    const bool dma = (long long)S * 256 < (1ll << 31) && alibi_ok && eet::tuning().prefill_legacy == 0;
+#define EET_PF_CASE(DH_)                                                                                \
+    case DH_:                                                                                           \
+        return dma ? launch_dma<DH_>(q, k_cache, v_cache, ctx, alibi, pad, B, H, S, T_cap, st)          \
+                   : launch<DH_>(q, k_cache, v_cache, ctx, alibi, pad, B, H, S, T_cap, st)
+    switch (dh) {
+        EET_PF_CASE(64);
+        EET_PF_CASE(96);
+        EET_PF_CASE(128);
+        default: return launch<32>(q, k_cache, v_cache, ctx, alibi, pad, B, H, S, T_cap, st);
+    }
+#undef EET_PF_CASE
 }

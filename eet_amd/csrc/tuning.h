@@ -18,9 +18,9 @@ struct Tuning {
     int large_m_wm = 0, large_m_wn = 0;                      // wavefronts down and across a block; 0: not given
     // EET_MMHA_NSPLIT, EET_MMHA_THREADS, EET_MMHA_UNROLL (0: not given)
     int mmha_nsplit = 0, mmha_threads = 0, mmha_ring = 0;
-    // EET_PREFILL_LEGACY = 1: head size 128 takes the register-staged prefill attention kernel
+    // EET_PREFILL_LEGACY = 1: every head size takes the register-staged prefill attention kernel
     int prefill_legacy = 0;
-    int prefill_shape = 0;   // 1, 2: launch shape of the head-size-128 prefill attention kernel; 0 = by prompt length
+    int prefill_shape = 0;   // 1, 2: launch shape of the prefill attention's DMA kernel; 0 = by rule
     int prefill_group = 0;   // EET_PREFILL_GROUP: (batch, head) pairs per XCD group of the prefill attention order; -1: ungrouped
     // EET_CHAIN_SPIN_LIMIT: polls before a chained wait gives up (-1: the default, 65536; 0 gives up at once);
     // EET_CHAIN_SLEEP: s_sleep(8) repetitions between two polls (0: the default, 1)
