@@ -368,8 +368,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 // ds_read_b64_tr_b16, which hands lane i column i of a 4 x 16 block of halves.
 //
 // The register-staged kernel above spends its time between barriers: load, transpose, store, wait, with one chunk in
-// flight.  Against it, us, 32 heads, no bias: head size 64 4 x 500 tokens 20.9 -> 12.2, 1 x 2048 54.3 -> 31.9, 8 x 1000
-// 94.4 -> 61.8; 96 25.6 -> 17.9, 79.5 -> 44.8, 118 -> 86.6; 128 28.0 -> 20.5, 75.8 -> 51.0, 136 -> 100.  It is left with
+// flight.  Against it, us, 32 heads, no bias: head size 64 4 x 500 tokens 21.3 -> 12.8, 1 x 2048 54.6 -> 32.9, 8 x 1000
+// 92.3 -> 61.8; 96 25.2 -> 17.0, 79.7 -> 45.6, 111 -> 86.7; 128 28.0 -> 20.5, 75.8 -> 51.0, 136 -> 100.  It is left with
 // head size 32 and with bias rows that are not whole 4-byte units.
 // ---------------------------------------------------------------------------
 constexpr int kKAhead = 6, kVAhead = 4;    // K operand reads / V operands (two reads each) in flight ahead of their MFMAs
@@ -500,7 +500,11 @@ __global__ __launch_bounds__(64 * WAVES)
     };
 
     constexpr float kLog2e = 1.4426950408889634f;
-    constexpr float kLazy = 8.0f;   // in powers of two
+    // How far (in powers of two) a query's maximum may pass its reference exponent before the accumulators are
+    // rescaled.  With fp32 denominators the reference is the maximum itself: the largest weight is then exactly 1 and
+    // not rounded for the second product (error of a 2048-token prompt against 64 bits, head size 64, scores of
+    // deviation 9: 2.1e-4; with a lag of 8 and a denominator that does not share the rounding 2.4e-4).
+    constexpr float kLazy = kMfmaSum ? 8.0f : 0.0f;
     const float scale2 = scale * kLog2e;
     const int k_begin = (padb / kBK) * kBK;
     const int k_end = min(S, q0 + kBQ2);
@@ -773,9 +777,9 @@ int launch_dma(const void *q, const void *kc, const void *vc, void *ctx, const v
     //   2  256 queries, eight two-tile wavefronts, four stages (every operand read feeds two tiles).
     // Shape 2 wins once its workgroups last (over 1536 tokens) and fill the CUs in at least two nearly whole rounds;
     // with one round, or a part of one left over, the longest blocks decide and half the block is better.  Measured,
-    // us, shape 1 / 2, one prompt of 2048 tokens (32 heads): head size 64 31.9 / 41.5, 96 44.8 / 54.7, 128 51.0 / 61.9;
-    // 40 heads of 128 with bias 72.5 / 79.8; two prompts: 56.4 / 52.4, 78.8 / 69.6, 89.2 / 85.1, but 40 heads (2.5
-    // rounds) 124 / 138; eight prompts of 1000: 61.8 / 66.1, 86.6 / 89.1, 100 / 105.  (256 queries as sixteen one-tile
+    // us, shape 1 / 2, one prompt of 2048 tokens (32 heads): head size 64 32.9 / 43.9, 96 45.6 / 55.1, 128 51.0 / 61.9;
+    // 40 heads of 128 with bias 72.5 / 79.8; two prompts: 57.1 / 54.0, 78.2 / 71.6, 89.2 / 85.1, but 40 heads (2.5
+    // rounds) 124 / 138; eight prompts of 1000: 61.8 / 64.9, 86.7 / 87.8, 100 / 105.  (256 queries as sixteen one-tile
     // wavefronts was within 2 % of shape 2 everywhere and is not kept.)  A tuning override picks either.
     int shape = eet::tuning().prefill_shape;
     if (shape < 1 || shape > 2)
