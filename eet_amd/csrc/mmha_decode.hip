@@ -130,8 +130,8 @@ __device__ __forceinline__ u32x4 rotate8(const u32x4 &x, const u32x4 &y, int sub
 // 400 rows, copy + attention 31 + 19 us per layer before; six steps of four whole layers 2707 -> 1882 us.
 // A row's name is requested when the request for the row one ring length before it goes out, so it is as old as
 // the ring is deep when it is needed and adds no wait.  Rows come through the caches here (not non-temporal):
-// beams that share an ancestor read the same row, and the workgroups of one head, B apart by a multiple of
-// H workgroups, sit on the same XCD whenever H is a multiple of eight.
+// beams that share an ancestor read the same row, and the B workgroups of one head, H apart in the grid, sit on
+// the same XCD whenever H is a multiple of eight.
 template <int DH, int UN, int THREADS, bool BEAMS>
 __global__ __launch_bounds__(THREADS) void mmha_decode_split_kernel(
     const _Float16 *__restrict__ q, const _Float16 *__restrict__ k_new, const _Float16 *__restrict__ v_new,
