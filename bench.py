@@ -544,7 +544,7 @@ def decode_bench(torch, eet, weights, dev, batch, prompt, gen, seed, model=LLAMA
             "breakdown_note": f"{bd_steps} further token steps with every launch issued on its own between two events; "
                               "us_per_call is the bracketed time scaled so that the kernels of a step sum to "
                               "ms_per_token_step (the brackets themselves cost time); bytes are algorithmic",
-            "note": "greedy decode, random-init weights, random token ids; lm_head and embedding are fp16 torch ops"}
+            "note": "greedy decode, random-init weights, random token ids; lm_head and embedding are fp16"}
 
 
 MFMA_FP16_PEAK_TFLOPS = 2500.0   # MI355X published dense fp16 MFMA peak
