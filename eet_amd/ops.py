@@ -740,6 +740,8 @@ class GatedFeedForwardNetworkInt8:
         if input.dtype != torch.float16 or input.dim() != 3 or input.shape[2] != desc.hidden_units:
             raise RuntimeError(f"[EET][ERROR] GatedFeedForwardNetworkInt8: input must be fp16 [B, S, "
                                f"{desc.hidden_units}], got {input.dtype} {tuple(input.shape)}")
+        if input.device.type != "cuda":
+            raise RuntimeError("[EET][ERROR] GatedFeedForwardNetworkInt8: input must be on the GPU")
         post_ln = add_residual and not pre_layernorm
         if post_ln and self.o_bias is not None and self.beta is None:
             raise RuntimeError("[EET][ERROR] GatedFeedForwardNetworkInt8: the post-layernorm tail with an output bias is "

@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from eet_amd import decoder as D
+from eet_amd import ops
 
 
 def decoders(alibi, rows):
@@ -49,3 +50,17 @@ def test_forms_of_one_call(gpu, alibi, rows):
     a.step = cfg.max_full_seq
     with pytest.raises(RuntimeError, match="max_full_seq_len"):
         a.forward(x, pad, none, True, True, False, none)
+
+
+@pytest.mark.parametrize("rows", [1, 32, 33])
+@pytest.mark.parametrize("pre_layernorm", [True, False])
+def test_feed_forward_refuses_a_host_input(monkeypatch, rows, pre_layernorm):
+    """Before any buffer is asked for and any kernel sees the host pointer, at the sizes of both paths."""
+    monkeypatch.setattr(ops, "_current_stream", lambda: 0)
+    monkeypatch.setattr(ops, "check", lambda status, what: pytest.fail(f"{what} was called"))
+    op = object.__new__(ops.GatedFeedForwardNetworkInt8)       # the constructor wants weights on a GPU
+    op.desc = ops.MetaDesc(torch.float16, rows, 2, 64, 1, 1, activation_fn="silu", d_ff=64, is_int8=True)
+    op.d_ff, op.beta, op.o_bias, op.cache_name = 64, None, None, "test_feed_forward_host_input"
+    with pytest.raises(RuntimeError, match="must be on the GPU"):
+        op.forward(torch.zeros(rows, 1, 64, dtype=torch.float16), pre_layernorm, True)
+    assert not any(key[1].type == "cpu" for key in ops.workspaces._bufs)
