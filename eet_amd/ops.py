@@ -808,17 +808,31 @@ class GatedFeedForwardNetworkInt8:
         return out[: M * hidden].view(B, S, hidden)
 
 
+_transformed = torch._C._functorch.is_functorch_wrapped_tensor
+
+
+def _head_kernel_takes(h, weight):
+    """The plain calls of `head`: whole fp16 rows on the current device, row offsets within 32 bits, and nothing that
+    torch would do beyond the product (autograd in either mode, autocast, tensor subclasses and transforms)."""
+    (B, S, K), V = h.shape, weight.shape[0]
+    return (0 < B <= 16 and S > 0 and 0 < K and K % 64 == 0 and 0 < V and V % 16 == 0 and V * K <= 2 ** 28
+            and ((B - 1) * S + 1) * K * 2 <= 2 ** 31 and weight.dim() == 2 and weight.shape[1] == K
+            and h.dtype == torch.float16 and weight.dtype == torch.float16 and h.is_cuda and weight.device == h.device
+            and h.is_contiguous() and weight.is_contiguous() and type(h) is torch.Tensor
+            and type(weight) in (torch.Tensor, torch.nn.Parameter)
+            and not _transformed(h) and not _transformed(weight)
+            and not (torch.is_grad_enabled() and (h.requires_grad or weight.requires_grad))
+            and torch.autograd.forward_ad._current_level < 0 and not torch.is_autocast_enabled()
+            and h.device.index == torch.cuda.current_device()
+            and weight.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0)
+
+
 def head(h, weight):
-    """Logits [B, 1, V] of the last position of h [B, S, K] under the fp16 output matrix [V, K].  Up to 16 sequences
-    and 2^28 weights run on eet_head_f16; the rest, and whatever torch does beyond the product (autograd on the
-    matrix, autocast), on torch's linear."""
-    B, S, K = h.shape
-    V = weight.shape[0]
-    if (B > 16 or K % 64 or V % 16 or V * K > 2 ** 28 or weight.dtype != torch.float16 or h.dtype != torch.float16
-            or not weight.is_contiguous() or not h.is_contiguous() or weight.device != h.device or not h.is_cuda
-            or weight.shape != (V, K) or weight.data_ptr() % 16 or h.data_ptr() % 16
-            or (weight.requires_grad and torch.is_grad_enabled()) or torch.is_autocast_enabled()):
+    """Logits [B, 1, V] of the last position of h [B, S, K] under the fp16 output matrix [V, K].  Plain calls of up to
+    16 sequences and 2^28 weights run on eet_head_f16, all others on torch's linear."""
+    if not _head_kernel_takes(h, weight):
         return torch.nn.functional.linear(h[:, -1:, :], weight)
+    (B, S, K), V = h.shape, weight.shape[0]
     out = torch.empty(B, 1, V, dtype=torch.float16, device=h.device)
     check(lib().eet_head_f16(h.data_ptr() + 2 * (S - 1) * K, S * K, weight.data_ptr(), out.data_ptr(), B, V, K, _stream()),
           "eet_head_f16")

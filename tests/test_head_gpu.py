@@ -50,3 +50,37 @@ def test_what_stays_with_torch(gpu):
         assert ops.head(h, w).dtype == torch.bfloat16
     odd = torch.randn(33, 64, device=gpu).half()
     assert torch.equal(ops.head(h, odd), torch.nn.functional.linear(h, odd))
+
+
+@pytest.mark.gpu
+def test_sizes_and_calls_that_the_kernel_does_not_have(gpu, monkeypatch):
+    """Rows beyond 32-bit offsets, nothing to multiply, another current device, forward-mode and backward autograd of
+    the hidden states, a tensor subclass: what torch's linear gives, as it gives it."""
+    linear = torch.nn.functional.linear
+    w = torch.randn(32, 64, device=gpu).half()
+    long = torch.zeros(16, 1 << 21, 64, device=gpu, dtype=torch.float16)      # 16 rows 256 MiB apart
+    long[:, -1] = torch.randn(16, 64, device=gpu).half()
+    got = ops.head(long, w)
+    assert torch.equal(got, linear(long[:, -1:], w)) and got.abs().max() > 0
+    del long
+    h = torch.randn(2, 3, 64, device=gpu).half()
+    want = linear(h[:, -1:], w)
+    for empty, weight in ((h[:0], w), (h[:, :0], w), (h, w[:0])):
+        assert ops.head(empty, weight).shape == linear(empty[:, -1:], weight).shape
+    calls = []
+    monkeypatch.setattr(ops.torch.nn.functional, "linear", lambda *a: calls.append(1) or linear(*a))
+    with monkeypatch.context() as m:
+        m.setattr(ops.torch.cuda, "current_device", lambda: 1)
+        assert torch.equal(ops.head(h, w), want) and calls == [1]
+    assert ops.head(h.clone().requires_grad_(), w).requires_grad and len(calls) == 2
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(w, torch.ones_like(w))
+        tangent = torch.autograd.forward_ad.unpack_dual(ops.head(h, dual)).tangent
+        assert torch.equal(tangent, linear(h[:, -1:], torch.ones_like(w))) and len(calls) >= 3
+
+    class Sub(torch.Tensor):
+        pass
+    assert type(ops.head(h, w.as_subclass(Sub))) is Sub
+    calls.clear()
+    ops.head(h, torch.nn.Parameter(w, requires_grad=False))
+    assert not calls                                                        # a plain call: the kernel
