@@ -17,6 +17,8 @@ Differences that a caller can observe, all deliberate:
   * outputs are views of per-process named torch buffers that own their
     storage (the reference returns from_blob views, llama_mmha.cpp:197-198).
 """
+import threading
+
 import torch
 
 from ._lib import check, lib
@@ -97,15 +99,16 @@ workspaces = _Workspaces()
 
 class _SpareKV:
     """The second KV buffer of a cache gather (a beam reorder that cannot go through row names, or an op
-    settling its cache), shared by every attention op with the same cache shape on a device: an op
-    gathers into the spare pair, takes it as its cache and leaves its old pair as the new spare.  The
-    ops of a decoder run one after another on one stream, so a single spare serves all layers."""
+    settling its cache), shared by every attention op with the same cache shape on a device and stream: an
+    op gathers into the spare pair, takes it as its cache and leaves its old pair as the new spare.  The
+    ops of a decoder run one after another on one stream, so a single spare serves all layers; what
+    another stream left behind may still be read there."""
 
     def __init__(self):
         self._pairs = {}
 
     def swap(self, k_cache, v_cache, gather):
-        key = (tuple(k_cache.shape), k_cache.dtype, str(k_cache.device))
+        key = (tuple(k_cache.shape), k_cache.dtype, str(k_cache.device), _current_stream())
         pair = self._pairs.get(key)
         if pair is None:
             pair = (torch.zeros_like(k_cache), torch.zeros_like(v_cache))
@@ -118,6 +121,11 @@ class _SpareKV:
 
 
 spare_kv = _SpareKV()
+
+# Held by whoever settles a cache and by the calls that read or write row names (beam search): a thread that looks at a
+# cache between two steps must not move rows under a call that is being issued.  Reentrant; one for all ops, since
+# ops are copied and share the spare pair.
+_rows_lock = threading.RLock()
 
 
 # ----------------------------------------------------------------------------
@@ -343,6 +351,7 @@ class _MmhaInt8:
         # Beam search: which sequence's slab holds row t of sequence b (eet_mmha_decode_beams), None while every
         # row is in its own slab; two tables in turn, [batch_size][t_cap] int32
         self._rows, self._row_tables = None, []
+        self._rows_stream = 0       # the stream of the last call over named rows
         self.step = 1
         self.first_batch = 0
         self.rope_table = _rope_table(self.t_cap, self.dh, dev) if self._rope else None
@@ -360,7 +369,8 @@ class _MmhaInt8:
 
     @property
     def k_cache(self):
-        """[batch_size, H, max_full_seq_len, dh]; every sequence's rows in its own slab."""
+        """[batch_size, H, max_full_seq_len, dh]; every sequence's rows in its own slab.  During a beam search this
+        moves rows (settle_cache) and takes the spare cache pair for it."""
         self.settle_cache()
         return self._k
 
@@ -381,7 +391,24 @@ class _MmhaInt8:
 
     def settle_cache(self):
         """After a beam reorder the rows stay where they are and the attention reads them through a table of
-        row names; this moves every row into its own sequence's slab and drops the table."""
+        row names; this moves every row into its own sequence's slab and drops the table.  May be called from any
+        thread and stream: the rows move on the stream of the op's own calls, between two of them, and the current
+        stream waits for that."""
+        if self._rows is None:
+            return
+        with _rows_lock:
+            if self._rows is None:
+                return
+            dev, handle = self._k.device, self._rows_stream
+            mine = torch.cuda.current_stream(dev)
+            theirs = torch.cuda.ExternalStream(handle, device=dev) if handle else torch.cuda.default_stream(dev)
+            with torch.cuda.stream(theirs):
+                self._settle()
+            if mine.cuda_stream != handle:
+                mine.wait_stream(theirs)
+
+    def _settle(self):
+        """settle_cache on the current stream."""
         if self._rows is None:
             return
         rows, L = min(self.step, self.t_cap), lib()
@@ -389,9 +416,13 @@ class _MmhaInt8:
         def gather(k_dst, v_dst):
             check(L.eet_kv_cache_gather_rows(self._k.data_ptr(), self._v.data_ptr(), k_dst.data_ptr(), v_dst.data_ptr(),
                                              self._rows.data_ptr(), self.first_batch, self.desc.head_num, self.dh, rows,
-                                             self.t_cap, _stream()), "eet_kv_cache_gather_rows")
+                                             self.t_cap, _current_stream()), "eet_kv_cache_gather_rows")
         self._k, self._v = spare_kv.swap(self._k, self._v, gather)
         self._rows = None
+
+    def _name_rows(self, rows):
+        """The table of names that a call has left behind."""
+        self._rows, self._rows_stream = rows, _stream()
 
     def _beam_rows(self, B, reorder, device):
         """(beam_rows_in, beam_rows_out) of an incremental call, (None, None) for one without shared rows.
@@ -400,7 +431,7 @@ class _MmhaInt8:
             return None, None
         if (B != self.first_batch or replay_state is not None
                 or B * self.desc.head_num * self.t_cap * self.dh * 2 > 2 ** 31):
-            self.settle_cache()
+            self._settle()
             if reorder is not None:
                 # beam b continues from the rows of beam reorder[b]: gather into the spare cache pair
                 # (one per cache shape, shared by all layers), then take that pair as this op's cache
@@ -430,7 +461,7 @@ class _MmhaInt8:
         else:
             check(L.eet_mmha_decode_beams(*args, _ptr(rows_in), rows_out.data_ptr(), _ptr(reorder), *tail),
                   "eet_mmha_decode_beams")
-            self._rows = rows_out
+            self._name_rows(rows_out)
 
     def forward(self, input, pre_padding_len, reorder_state, pre_layernorm, add_residual, first_pass,
                 relative_attention_bias=_EMPTY):
@@ -438,6 +469,10 @@ class _MmhaInt8:
             y = self._decode(input, pre_padding_len, reorder_state, relative_attention_bias)
             if y is not None:
                 return y
+        if self._rows is not None or (reorder_state is not None and reorder_state.numel() != 0):
+            with _rows_lock, _StreamScope():
+                return self._forward(input, pre_padding_len, reorder_state, pre_layernorm, add_residual, first_pass,
+                                     relative_attention_bias)
         with _StreamScope():
             return self._forward(input, pre_padding_len, reorder_state, pre_layernorm, add_residual, first_pass,
                                  relative_attention_bias)
@@ -600,7 +635,7 @@ class _MmhaInt8:
             else:
                 check(L.eet_mmha_int8_decode_beams(*args, _ptr(rows_in), rows_out.data_ptr(), _ptr(reorder), *tail),
                       "eet_mmha_int8_decode_beams")
-                self._rows = rows_out
+                self._name_rows(rows_out)
             self._keep = (x, pad, alibi, reorder)  # inputs of kernels still in flight
             return out[: M * hidden].view(B, S, hidden)
         if self.with_bias:

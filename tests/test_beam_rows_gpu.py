@@ -1,5 +1,8 @@
 """Beam search over shared cache rows (eet_mmha_decode_beams): against the cache reorder followed by the ordinary
 call, which moves the same rows -- the same sums in the same order, so the outputs are equal bit for bit."""
+import copy
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -106,3 +109,75 @@ def test_op_settles_its_cache(gpu, rows):
         assert b.layers[0][0]._rows is None and ka.shape[0] == rows
     step = a.layers[0][0].step
     assert torch.equal(a.layers[0][0].k_cache[: rows - 1, :, :step], b.layers[0][0].k_cache[: rows - 1, :, :step])
+
+
+def beam_decoders(rows, steps):
+    cfg = D.DecoderConfig(num_layers=2, hidden=256, heads=4, d_ff=704, vocab=64, max_batch=rows, max_prompt=8,
+                          max_full_seq=8 + steps)
+    sd, _ = D.random_state_dict(cfg, seed=3)
+    a, b = (D.Int8Decoder(cfg, sd, device="cuda:0") for _ in range(2))
+    g = torch.Generator().manual_seed(rows)
+    ids = torch.randint(0, 64, (rows, 8), generator=g).cuda()
+    assert torch.equal(a.logits(ids, True), b.logits(ids, True))
+    calls = [(torch.randint(0, 64, (rows, 1), generator=g).cuda(), torch.randint(0, rows, (rows,), generator=g).cuda())
+             for _ in range(steps)]
+
+    def step(model, t):
+        ids, model.reorder_state = calls[t]
+        return model.logits(ids, False)
+    return a, b, step
+
+
+@pytest.mark.gpu
+def test_cache_read_on_another_stream(gpu):
+    """While the ops' stream is far behind: the rows that the reader gets are those of the finished step, and the
+    steps after it go on from them."""
+    a, b, step = beam_decoders(5, 6)
+    side = torch.cuda.Stream()
+    for t in range(6):
+        torch.cuda._sleep(20_000_000)
+        la = step(a, t).clone()
+        if t % 2 == 0:
+            with torch.cuda.stream(side):
+                k = a.layers[1][0].k_cache.clone()
+                v = a.layers[0][0].v_cache.clone()
+            side.synchronize()
+        assert torch.equal(la, step(b, t))
+        if t % 2 == 0:
+            n = b.layers[0][0].step
+            assert torch.equal(k[:, :, :n], b.layers[1][0].k_cache[:, :, :n])
+            assert torch.equal(v[:, :, :n], b.layers[0][0].v_cache[:, :, :n])
+
+
+@pytest.mark.gpu
+def test_cache_read_from_another_thread(gpu):
+    """A thread that looks at the caches all the time, on a stream of its own, changes no step."""
+    steps = 60
+    a, b, step = beam_decoders(4, steps)
+    want = [step(b, t).clone() for t in range(steps)]
+    done, seen = threading.Event(), []
+
+    def watch():
+        with torch.cuda.stream(torch.cuda.Stream()):
+            while not done.is_set():
+                seen.append(tuple(a.layers[len(seen) % 2][0].k_cache.shape))
+    reader = threading.Thread(target=watch)
+    reader.start()
+    try:
+        got = [step(a, t).clone() for t in range(steps)]
+    finally:
+        done.set()
+        reader.join()
+    assert seen and all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+@pytest.mark.gpu
+def test_copied_op(gpu):
+    """A deep copy taken in mid-search goes on by itself."""
+    a, b, step = beam_decoders(3, 4)
+    for t in range(2):
+        step(a, t), step(b, t)
+    c = copy.deepcopy(a)
+    for t in (2, 3):
+        want = step(b, t).clone()
+        assert torch.equal(step(a, t), want) and torch.equal(step(c, t), want)
