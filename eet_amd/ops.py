@@ -352,6 +352,7 @@ class _MmhaInt8:
         # row is in its own slab; two tables in turn, [batch_size][t_cap] int32
         self._rows, self._row_tables = None, []
         self._rows_stream = 0       # the stream of the last call over named rows
+        self._rows_named = 0        # how many rows the table names: more than `step` once a caller has set that back
         self.step = 1
         self.first_batch = 0
         self.rope_table = _rope_table(self.t_cap, self.dh, dev) if self._rope else None
@@ -411,17 +412,19 @@ class _MmhaInt8:
         """settle_cache on the current stream."""
         if self._rows is None:
             return
-        rows, L = min(self.step, self.t_cap), lib()
+        L = lib()
 
         def gather(k_dst, v_dst):
             check(L.eet_kv_cache_gather_rows(self._k.data_ptr(), self._v.data_ptr(), k_dst.data_ptr(), v_dst.data_ptr(),
-                                             self._rows.data_ptr(), self.first_batch, self.desc.head_num, self.dh, rows,
-                                             self.t_cap, _current_stream()), "eet_kv_cache_gather_rows")
+                                             self._rows.data_ptr(), self.first_batch, self.desc.head_num, self.dh,
+                                             self._rows_named, self.t_cap, _current_stream()), "eet_kv_cache_gather_rows")
         self._k, self._v = spare_kv.swap(self._k, self._v, gather)
         self._rows = None
 
-    def _name_rows(self, rows):
-        """The table of names that a call has left behind."""
+    def _name_rows(self, rows, reorder):
+        """The table of names that a call has left behind: of the rows up to the new one after a reorder, with the new
+        one among those it had without."""
+        self._rows_named = self.step if reorder is not None else max(self._rows_named, self.step)
         self._rows, self._rows_stream = rows, _stream()
 
     def _beam_rows(self, B, reorder, device):
@@ -461,7 +464,7 @@ class _MmhaInt8:
         else:
             check(L.eet_mmha_decode_beams(*args, _ptr(rows_in), rows_out.data_ptr(), _ptr(reorder), *tail),
                   "eet_mmha_decode_beams")
-            self._name_rows(rows_out)
+            self._name_rows(rows_out, reorder)
 
     def forward(self, input, pre_padding_len, reorder_state, pre_layernorm, add_residual, first_pass,
                 relative_attention_bias=_EMPTY):
@@ -635,7 +638,7 @@ class _MmhaInt8:
             else:
                 check(L.eet_mmha_int8_decode_beams(*args, _ptr(rows_in), rows_out.data_ptr(), _ptr(reorder), *tail),
                       "eet_mmha_int8_decode_beams")
-                self._name_rows(rows_out)
+                self._name_rows(rows_out, reorder)
             self._keep = (x, pad, alibi, reorder)  # inputs of kernels still in flight
             return out[: M * hidden].view(B, S, hidden)
         if self.with_bias:

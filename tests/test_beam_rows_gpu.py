@@ -181,3 +181,23 @@ def test_copied_op(gpu):
     for t in (2, 3):
         want = step(b, t).clone()
         assert torch.equal(step(a, t), want) and torch.equal(step(c, t), want)
+
+
+@pytest.mark.gpu
+def test_cache_of_a_sequence_set_back(gpu):
+    """Setting `step` back loses no row: what a reader finds behind it are the rows that moved on every reorder."""
+    a, b, step = beam_decoders(4, 6)
+    for t in range(5):
+        step(a, t), step(b, t)
+        b.layers[0][0].k_cache, b.layers[1][0].k_cache        # settles after every step
+    for model in (a, b):
+        for attn, _ in model.layers:
+            attn.step = 9
+    ids = torch.arange(4).view(4, 1).cuda()                   # a call over named rows, without a reorder, in between
+    for model in (a, b):
+        model.reorder_state = torch.empty(0, dtype=torch.long)
+        model.logits(ids, False)
+    for (x, _), (y, _) in zip(a.layers, b.layers):
+        assert x.step == y.step == 10
+        assert torch.equal(x.k_cache[:, :, :13], y.k_cache[:, :, :13])
+        assert torch.equal(x.v_cache[:, :, :13], y.v_cache[:, :, :13])
