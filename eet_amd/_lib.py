@@ -27,6 +27,7 @@ SIGNATURES = {
     "eet_gemm_w8a16": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _vp, _sz, _vp]),
     "eet_gemm_w8a16_workspace": (_sz, [_i, _i, _i, _i]),
     "eet_gemm_w8a16_fused": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _f, _vp, _sz, _vp]),
+    "eet_gemm_w8a16_large_m_shape": (_i, [_i, _i, _i, _i, _sz, _vp, _vp, _vp, _vp, _vp]),
     "eet_gemm_w8a16_small_m_shape": (_i, [_i, _i, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "eet_gemm_w8a16_chained": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _f, _i, _vp]),
     "eet_chain_status": (_i, [_vp, _i, _vp]),

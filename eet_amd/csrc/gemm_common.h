@@ -57,7 +57,9 @@ struct GemmArgs {
     int chain = 0;  // kChainOff / kChainFirst / kChainNext (chain.h; small-M kernel only)
 };
 
-// gemm_w8a16_large.hip: the MFMA-tile kernel for M > 32, and the workspace it can use.
+// gemm_w8a16_large.hip: the MFMA-tile kernel for M > 32, and the workspace it can use.  kTakesSlabs, with nothing
+// launched, for a call that 32-row slabs of the small-M kernel run faster.
+constexpr int kTakesSlabs = 1;
 int run_large_m(const GemmArgs &a);
 size_t large_m_workspace(int M, int N, int K, int epi);
 

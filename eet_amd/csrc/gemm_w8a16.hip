@@ -934,7 +934,26 @@ int run_small_m(const GemmArgs &a)
 
 }  // namespace
 
-static int run_gemm(const GemmArgs &a) { return a.M <= 32 ? run_small_m(a) : eet::run_large_m(a); }
+static int run_gemm(const GemmArgs &a)
+{
+    if (a.M <= 32)
+        return run_small_m(a);
+    if (const int rc = eet::run_large_m(a); rc != eet::kTakesSlabs)
+        return rc;
+    const int n_out = (a.epi == kEpiSwiglu) ? a.N / 2 : a.N;
+    for (int m0 = 0; m0 < a.M; m0 += 32) {
+        GemmArgs s = a;
+        s.M = (a.M - m0 < 32) ? a.M - m0 : 32;
+        s.A = a.A + (size_t)m0 * a.K;
+        s.C = a.C + (size_t)m0 * n_out;
+        if (a.residual)
+            s.residual = a.residual + (size_t)m0 * a.N;
+        s.ws = nullptr, s.ws_bytes = 0;   // too small for the split of an M > 32 call, and its counters need not be zero
+        if (int rc = run_small_m(s))
+            return rc;
+    }
+    return EET_OK;
+}
 
 static int check_gemm_args(const char *fn, const void *A, const void *W, const void *scale, const void *C, int M,
                            int N, int K)

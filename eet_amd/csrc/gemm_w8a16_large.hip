@@ -1,4 +1,5 @@
-// Large-M fused dequant-GEMM (M > 32: prompts, and decode steps of more than 32 sequences).
+// Large-M fused dequant-GEMM (M > 32: prompts, and decode steps of more than 32 sequences; see slabs_win for the calls
+// of up to 64 rows that stay with the small-M kernel).
 //
 // Replaces the tensor-core side of fastertransformer::gemm_fp16_int_bias_act<uint8_t>
 // (3rdparty/cutlass_kernels/fpA_intB_gemm/fpA_intB_gemm_template.h:48-177).
@@ -487,6 +488,50 @@ void pick_large_m(int M, int N, int K, int epi, LargeMConfig *whole, LargeMConfi
     }
 }
 
+// 33 to 64 rows and no workspace for a split: with few channels the blocks leave most of the chip idle and each walks
+// the whole k range alone, so its time is that of the k loop whatever M and N are.  The small-M kernel over 32-row
+// slabs shares a block's k range among its wavefronts and has eight times the blocks; its weights are read twice, from
+// the Infinity Cache the second time, its second slab costs by its rows, and below 3072 k (2048 with SwiGLU) two short
+// launches cost the host more than one.  Measured, us, slabs / blocks, at 33, 48
+// and 64 rows: 1024 <- 1024 6.2 / 5.4, 6.3 / 5.5, 6.1 / 5.5; 1024 <- 8192 14 / 23, 17 / 23, 21 / 23; 2048 <- 4096
+// 10.1 / 13.0, 11.6 / 12.7, 13.4 / 12.7; 3072 <- 2048 9.0 / 8.2, 10.0 / 8.1, 9.7 / 8.1; 4096 <- 11008 24 / 31, 28 / 31,
+// 32 / 31; 5120 <- 4096 13.7 / 13.6, 15.4 / 13.3, 16.6 / 13.8.  SwiGLU blocks hold whole (gate, up) pairs and are
+// wider: 4096 <- 4096 13.0 / 17.4, 14.6 / 17.6, 16.3 / 17.7; 7168 <- 4096 15.6 / 17.7, 16.6 / 17.8, 18.4 / 18.5;
+// 9216 <- 4096 22 / 18, 23 / 18, 25 / 19.
+bool slabs_win(int M, int N, int K, int epi)
+{
+    if (M > 64 || K < 2048)
+        return false;
+    if (epi == kEpiSwiglu)
+        return N <= 4096 || (N <= 8192 && M <= 48 && 8 * (long)K >= 3 * (long)N);
+    return K >= 3072 && N <= 4096 && (M <= 48 || (N <= 2048 && K >= 6144));
+}
+
+// What a call runs as (some block shape always does: the unsplit estimates are finite); tile < 0: 32-row slabs of the
+// small-M kernel.
+LargeMConfig plan_large_m(int M, int N, int K, int epi, size_t ws_bytes)
+{
+    // a split needs room for ksplit x M x N fp32; without it the best single-pass tile
+    auto fits = [&](int ks) { return ks <= 1 || ws_bytes >= (size_t)ks * M * N * sizeof(float); };
+    const eet::Tuning &tune = eet::tuning();
+    LargeMConfig whole, split;
+    pick_large_m(M, N, K, epi, &whole, &split);
+    LargeMConfig c = split.us < whole.us && fits(split.ksplit) ? split : whole;
+    if (tune.has_large_m) {   // "tm,tn[,ksplit[,wm,wn]]": runs when such a tile exists, else the table's choice stands
+        for (int i = 0; i < kNumTiles; ++i) {
+            const TileCost &t = kTiles[i];
+            if (t.tm != tune.large_m_tm || t.tn != tune.large_m_tn || (epi == kEpiSwiglu && t.tn % 2 != 0) ||
+                (tune.large_m_wm > 0 && (t.wm != tune.large_m_wm || t.wn != tune.large_m_wn)))
+                continue;
+            const int ks = tune.large_m_ksplit;
+            return LargeMConfig{i, ks >= 1 && ks <= K / 64 && fits(ks) ? ks : 1, 0.f};
+        }
+    } else if (c.ksplit == 1 && slabs_win(M, N, K, epi)) {
+        c = LargeMConfig{};
+    }
+    return c;
+}
+
 }  // namespace
 
 // The workspace of a split that would win, or comes within 15 % of the unsplit launch (so that a caller who sizes its
@@ -498,31 +543,31 @@ size_t eet::large_m_workspace(int M, int N, int K, int epi)
     return split.us < 1.15f * whole.us ? (size_t)split.ksplit * M * N * sizeof(float) : 0;
 }
 
+extern "C" int eet_gemm_w8a16_large_m_shape(int M, int N, int K, int epilogue, size_t workspace_bytes, int *tm, int *tn,
+                                            int *wm, int *wn, int *k_split)
+{
+    EET_REQUIRE(tm && tn && wm && wn && k_split, EET_ERR_INVALID_ARGUMENT, "eet_gemm_w8a16_large_m_shape: null pointer");
+    EET_REQUIRE(M > 32 && N > 0 && K > 0 && K % 64 == 0 && N % 16 == 0 &&
+                    (epilogue == kEpiNone || epilogue == kEpiResidual || (epilogue == kEpiSwiglu && N % 32 == 0)),
+                EET_ERR_UNSUPPORTED_SHAPE,
+                "eet_gemm_w8a16_large_m_shape: not a shape the large-M kernel takes (M=%d N=%d K=%d epilogue %d)", M, N, K,
+                epilogue);
+    const LargeMConfig c = plan_large_m(M, N, K, epilogue, workspace_bytes);
+    const TileCost none{}, &t = c.tile < 0 ? none : kTiles[c.tile];
+    *tm = t.tm, *tn = t.tn, *wm = t.wm, *wn = t.wn, *k_split = c.ksplit;
+    return EET_OK;
+}
+
 int eet::run_large_m(const GemmArgs &a)
 {
     // the kernel addresses A rows and the packed weights with 32-bit byte offsets
     if ((size_t)a.K * a.N >= (1ull << 31) || (size_t)a.K * 2 * 256 >= (1ull << 31))
         return eet::fail(EET_ERR_UNSUPPORTED_SHAPE, "eet_gemm_w8a16: K x N = %d x %d exceeds the 2 GiB weight limit",
                          a.K, a.N);
-    // a split needs room for ksplit x M x N fp32; without it the best single-pass tile
-    auto fits = [&](int ks) {
-        return ks <= 1 || (a.ws != nullptr && reinterpret_cast<uintptr_t>(a.ws) % 16 == 0 &&
-                           a.ws_bytes >= (size_t)ks * a.M * a.N * sizeof(float));
-    };
-    LargeMConfig whole, split;
-    pick_large_m(a.M, a.N, a.K, a.epi, &whole, &split);
-    LargeMConfig c = split.us < whole.us && fits(split.ksplit) ? split : whole;
-    const eet::Tuning &tune = eet::tuning();
-    if (tune.has_large_m)   // "tm,tn[,ksplit[,wm,wn]]": runs when such a tile exists, else the table's choice stands
-        for (int i = 0; i < kNumTiles; ++i) {
-            const TileCost &t = kTiles[i];
-            if (t.tm != tune.large_m_tm || t.tn != tune.large_m_tn || (a.epi == kEpiSwiglu && t.tn % 2 != 0) ||
-                (tune.large_m_wm > 0 && (t.wm != tune.large_m_wm || t.wn != tune.large_m_wn)))
-                continue;
-            const int ks = tune.large_m_ksplit;
-            c = LargeMConfig{i, ks >= 1 && ks <= a.K / 64 && fits(ks) ? ks : 1, 0.f};
-            break;
-        }
+    const size_t ws_bytes = a.ws != nullptr && reinterpret_cast<uintptr_t>(a.ws) % 16 == 0 ? a.ws_bytes : 0;
+    const LargeMConfig c = plan_large_m(a.M, a.N, a.K, a.epi, ws_bytes);
+    if (c.tile < 0)
+        return kTakesSlabs;
     using Launcher = int (*)(const GemmArgs &, int);
     // in the order of kTiles; the last number is the depth of the stage ring, as deep as two workgroups of four
     // wavefronts (or one of eight) leave room for in the LDS
@@ -549,7 +594,5 @@ int eet::run_large_m(const GemmArgs &a)
         launch_large_m<8, 4, 2, 4, 3>
     };
     static_assert(sizeof(launchers) / sizeof(launchers[0]) == kNumTiles, "one launcher per block shape");
-    if (c.tile < 0)
-        return eet::fail(EET_ERR_INVALID_ARGUMENT, "eet_gemm_w8a16: no large-M kernel for M=%d N=%d K=%d", a.M, a.N, a.K);
     return launchers[c.tile](a, c.ksplit);
 }

@@ -113,8 +113,8 @@ int eet_quantize_pack_device(const void *w, int w_dtype, size_t K, size_t N, int
 
 /* C[M][N] (half) = A[M][K] (half) . (int8 W[K][N] * scale[N] (half)), fp32
  * accumulation, one rounding to half.  Wpacked comes from eet_pack_gfx950.
- * M <= 32 takes the HBM-streaming small-M kernel, larger M the LDS-staged MFMA
- * kernel.  The workspace is optional (NULL / 0 accepted): with
+ * M <= 32 takes the HBM-streaming small-M kernel (up to 64 rows do in slabs of 32,
+ * with few channels and no workspace), larger M the LDS-staged MFMA kernel.  The workspace is optional (NULL / 0 accepted): with
  * eet_gemm_w8a16_workspace(M, N, K, epilogue) bytes of 16-byte aligned device
  * memory the library may split the k range of a launch -- the reference's
  * split-k workspace, which its callers never pass
@@ -178,6 +178,14 @@ int eet_gemm_w8a16_fused(const void *A, const void *Wpacked, const void *scale, 
  * heuristic returns (cutlass_heuristic.cc:106-207). */
 int eet_gemm_w8a16_small_m_shape(int M, int N, int K, int epilogue, int rms_prologue, int *nt,
                                  int *waves, int *k_tiles_per_batch, int *k_split);
+
+/* The same for M > 32: the block shape (m-tiles of 16 rows and n-tiles of 16 channels
+ * per wavefront, wavefronts down and across a block) and the shares of the k range
+ * that a call handing over workspace_bytes of workspace runs with.  tm = 0: 32-row
+ * slabs of the small-M kernel (up to 64 rows and few channels, without the workspace
+ * of a split).  Decided on the host; nothing is launched. */
+int eet_gemm_w8a16_large_m_shape(int M, int N, int K, int epilogue, size_t workspace_bytes,
+                                 int *tm, int *tn, int *wm, int *wn, int *k_split);
 
 /* Chained launches (1 <= M <= 32): eet_gemm_w8a16_fused for a sequence of launches
  * in which each reads what the previous one wrote -- the decode step of

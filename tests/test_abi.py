@@ -181,3 +181,39 @@ def test_every_table_answer_has_a_kernel():
                         continue
                     rc = L.eet_gemm_w8a16_small_m_shape(M, N, K, epi, rms, *[ctypes.byref(x) for x in q])
                     assert rc == 0, L.eet_last_error().decode()
+
+
+def large_m_shape(M, N, K, epi, ws=0):
+    v = [ctypes.c_int() for _ in range(5)]
+    rc = _lib.lib().eet_gemm_w8a16_large_m_shape(M, N, K, epi, ws, *[ctypes.byref(x) for x in v])
+    assert rc == 0, _lib.lib().eet_last_error().decode()
+    return tuple(x.value for x in v)
+
+
+SLABS = (0, 0, 0, 0, 1)
+
+
+@pytest.mark.parametrize("M,N,K,epi,slabs", [
+    (33, 1024, 8192, 0, True), (64, 1024, 8192, 1, True), (48, 4096, 11008, 1, True), (33, 4096, 4096, 0, True),
+    (64, 4096, 11008, 1, False), (56, 3072, 8192, 1, False),          # equal or behind from 56 rows on
+    (33, 1024, 1024, 0, False), (48, 4096, 2048, 1, False),           # short k ranges
+    (33, 5120, 5120, 1, False), (48, 12288, 4096, 0, False),          # blocks enough
+    (64, 4096, 4096, 2, True), (48, 7168, 4096, 2, True), (64, 7168, 4096, 2, False), (33, 9216, 4096, 2, False),
+    (65, 1024, 8192, 0, False)])
+def test_calls_without_a_workspace_keep_their_faster_path(M, N, K, epi, slabs):
+    """33 to 64 rows and few channels: the small-M kernel in slabs of 32 rows, unless the caller hands over the
+    workspace of a split or asks for a block shape."""
+    L = _lib.lib()
+    assert (large_m_shape(M, N, K, epi) == SLABS) == slabs
+    need = L.eet_gemm_w8a16_workspace(M, N, K, epi)
+    if slabs:
+        assert need > 0 and large_m_shape(M, N, K, epi, need)[4] > 1
+        assert large_m_shape(M, N, K, epi, need - 16) == SLABS
+    assert L.eet_set_tuning(b"EET_GEMM_LARGE_M_TILE", b"4,2") == 0
+    try:
+        assert large_m_shape(M, N, K, epi)[:2] == (4, 2)
+    finally:
+        assert L.eet_set_tuning(b"EET_GEMM_LARGE_M_TILE", None) == 0
+    v = [ctypes.byref(ctypes.c_int()) for _ in range(5)]
+    for bad in ((32, N, K, 0, 0), (40, 8, 64, 0, 0), (40, 16, 32, 0, 0), (40, 48, 64, 2, 0), (40, 16, 64, 3, 0)):
+        assert L.eet_gemm_w8a16_large_m_shape(*bad, *v) == -2

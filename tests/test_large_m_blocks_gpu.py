@@ -92,3 +92,41 @@ def test_block_epilogues(gpu, tuning, block):
     err = np.abs(got - want.astype(np.float32))
     assert (err <= tol).all(), f"{block}: max err {err.max():.2e}"
     assert (out[M:] == GUARD).all()
+
+
+@pytest.mark.parametrize("M,K,N", [(33, 3072, 288), (48, 3136, 544), (63, 6144, 1056), (64, 8192, 96)])
+def test_slabs_of_32_rows(gpu, M, K, N):
+    """The calls of up to 64 rows that run on the small-M kernel: every epilogue, an odd last slab, and a workspace too
+    small for a split, whose bytes are not looked at."""
+    import ctypes
+    from eet_amd._lib import check as ok, lib
+    v = [ctypes.c_int() for _ in range(5)]
+    for epi in (0, 1, 2):
+        ok(lib().eet_gemm_w8a16_large_m_shape(M, N, K, epi, 4096, *[ctypes.byref(x) for x in v]))
+        assert v[0].value == 0
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(3)).half()
+    u, p, s = quant(K, N, 5)
+    xd, pd, sd = x.to(gpu), p.to(gpu), s.to(gpu)
+    dirty = torch.full((4096,), 255, dtype=torch.uint8, device=gpu)
+
+    def run(w, scale, n_out, epi, res=None):
+        out = torch.full((M + 16, n_out), GUARD, dtype=torch.float16, device=gpu)
+        ok(lib().eet_gemm_w8a16_fused(xd.data_ptr(), w.data_ptr(), scale.data_ptr(), out.data_ptr(), M, w.shape[1], K, epi,
+                                      res.data_ptr() if res is not None else None, None, 0.0, dirty.data_ptr(), 4096,
+                                      torch.cuda.current_stream().cuda_stream))
+        assert (out[M:] == GUARD).all() and (dirty == 255).all()
+        return out[:M].cpu()
+    plain = run(pd, sd, N, 0)
+    check(plain, x, u, s, f"{M}x{N} k {K}")
+    res = torch.randn(M, N, generator=torch.Generator().manual_seed(4)).half()
+    assert torch.equal(run(pd, sd, N, 1, res.to(gpu)), plain + res)
+    F = N // 2
+    w01, s01 = (t.to(gpu) for t in interleave_gate_up(*quant(K, F, 6)[1:], *quant(K, F, 7)[1:]))
+    got = run(w01, s01, F, 2)
+    halves = run(w01, s01, N, 0).view(M, F // 16, 2, 16).float()             # gate and up tiles in turn
+    gate, up = halves[:, :, 0].reshape(M, F), halves[:, :, 1].reshape(M, F)
+    # the launch of this epilogue has a shape of its own and sums in its own order, so its gate and up may be rounded to
+    # the neighbouring fp16 value (2^-10 of each): |d(silu)| <= 1.1 |d gate|, then one rounding of the product
+    want = up * gate / (1 + torch.exp(-gate))
+    tol = 2.0 ** -10 * (1.1 * gate.abs() * up.abs() + 2 * want.abs()) + 2.0 ** -23
+    assert ((got.float() - want).abs() <= tol).all()
