@@ -9,11 +9,16 @@
 // set: they return zeros and touch no memory, which keeps the loop free of branches around loads.  The two halves of
 // a line are two requests: with the non-temporal bit the second one missed again (M = 1, 64000 <- 5120: 138 us
 // against 108).
-// What the activations cost sets NT: every workgroup reads all M*K of them.  Measured on MI355X with the weights
-// from HBM, us, M = 1 / 16, NT = 1, 2, 4 (library GEMM): 32000 <- 4096 48.6 / 64.5, 53.4 / 60.2, 49.4 / 50.0 (55.8 / 56.1);
-// 32000 <- 2048 27.6 / 35.2, 25.2 / 30.6, 26.4 / 28.1 (31.1 / 31.5); 8000 <- 1024 4.9 / 6.2, 4.6 / 5.2, 6.1 / 6.8 (19.1: its
-// own launch cost on the host).  64000 <- 5120 at M = 16 is 127 against the library's 110: matrices that large
-// are refused here and left to it.
+// Three things set NT: the tiles of the CU with the most workgroups (whole rounds of 256, 16 K weights each), the
+// activations that every workgroup reads whole from L2 (at 16 rows as many bytes as a tile, at 0.4 of the cost), and
+// the start and the meeting of its wavefronts (as long as 1024 k of a tile).  head_tiles takes the smallest sum; over
+// 832 sizes (K 512 .. 8192, N 1024 .. 256000, M 1 .. 16; graph replays, weights from HBM) it is 0.6 % behind the best of
+// the three NT on average, 18 % at most.  us, NT = 1 / 2 / 4, M = 1 and 16: 4096 <- 4096 8.3 / 11.2 / 17.7, 10.2 / 13.5 /
+// 21.0; 8000 <- 1024 5.9 / 5.5 / 6.7, 7.0 / 5.9 / 7.5; 10240 <- 4096 19.5 / 23.6 / 19.4, 25.5 / 26.6 / 22.6; 20480 <- 4096
+// 31.2 / 36.5 / 42.5, 42.5 / 41.4 / 45.6; 32000 <- 2048 26.3 / 25.0 / 26.9, 35.1 / 30.6 / 28.5; 32000 <- 4096 46.1 / 48.0 /
+// 48.4, 65.1 / 55.1 / 51.3.  (Thresholds on the number of tiles, from four matrices: 5 % behind on average, 53 % at most.)
+// 64000 <- 5120 at M = 16 took 127 us against the library's 110: matrices that large are refused here (a limit of this
+// kernel's speed, not of its addressing) and left to it.
 #include <hip/hip_runtime.h>
 
 #include "common.h"
@@ -100,6 +105,20 @@ __global__ __launch_bounds__(64 * WAVES) void head_kernel(const _Float16 *__rest
     }
 }
 
+// Tiles per workgroup; see above.
+int head_tiles(int tiles, int M, int K)
+{
+    int best = 1;
+    float least = 0.f;
+    for (int nt : {1, 2, 4}) {
+        const int workgroups = (tiles + nt - 1) / nt, rounds = (workgroups + 255) / 256;
+        const float cost = (float)rounds * ((float)nt + 0.4f * (float)M / 16.f + 1024.f / (float)K);
+        if (nt == 1 || cost < least)
+            best = nt, least = cost;
+    }
+    return best;
+}
+
 }  // namespace
 
 extern "C" int eet_head_f16(const void *x, long x_stride, const void *w, void *out, int M, int N, int K, void *stream)
@@ -113,8 +132,7 @@ extern "C" int eet_head_f16(const void *x, long x_stride, const void *w, void *o
                 EET_ERR_INVALID_ARGUMENT, "eet_head_f16: x_stride %ld must be a multiple of 8, at least K", x_stride);
     EET_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) % 16 == 0, EET_ERR_INVALID_ARGUMENT,
                 "eet_head_f16: x and w need 16-byte alignment");
-    // four tiles per workgroup once that leaves two workgroups per CU, two where it leaves about one (figures above)
-    const int tiles = N / 16, nt = tiles >= 1792 ? 4 : tiles >= 256 ? 2 : 1;
+    const int tiles = N / 16, nt = head_tiles(tiles, M, K);
     auto kern = nt == 4 ? head_kernel<4, 8, 1> : nt == 2 ? head_kernel<2, 8, 2> : head_kernel<1, 8, 2>;
     hipLaunchKernelGGL(kern, dim3((tiles + nt - 1) / nt), dim3(512), 0, static_cast<hipStream_t>(stream),
                        static_cast<const _Float16 *>(x), x_stride, static_cast<const _Float16 *>(w),

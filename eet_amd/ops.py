@@ -846,6 +846,22 @@ class GatedFeedForwardNetworkInt8:
         return out[: M * hidden].view(B, S, hidden)
 
 
+def _head_kernel_wins(B, V, K):
+    """Where eet_head_f16 is ahead of the library product, which streams anything from 2.3 to 5.7 TB/s of weights.
+    Measured over graph replays at K 512 .. 8192, V 1024 .. 256000, B 1 / 4 / 8 / 16, weights from HBM (832 sizes): 0.80
+    of the library's time on the whole, behind it by more than 3 % at 27 sizes and at most 14 %; with the kernel
+    everywhere and thresholds from four matrices it was 0.84, 177 sizes and 51 %.  K = 4096, us, kernel / library, B = 1
+    and 16: V 4096 8.3 / 12.8 and 10.2 / 13.0, 10240 19.5 / 19.5 and 22.6 / 20.1, 20480 31.2 / 54.5 and 41.4 / 55.2, 32000
+    48.4 / 56.4 and 51.3 / 57.6, 50272 78.0 / 85.2 and 89.7 / 86.7."""
+    if K > 6144:                    # its workgroups each read every activation
+        return False
+    if 8192 < V < 16000:            # one to four tiles per CU, in broken rounds: the library splits K
+        return K <= 2048
+    if 45000 < V < 60000:           # the library's best range, but not with rows a multiple of 4 KiB apart
+        return K <= 512 or K % 2048 == 0
+    return B <= 8 or V > 8192 or K <= 4096
+
+
 _transformed = torch._C._functorch.is_functorch_wrapped_tensor
 
 
@@ -854,6 +870,7 @@ def _head_kernel_takes(h, weight):
     torch would do beyond the product (autograd in either mode, autocast, tensor subclasses and transforms)."""
     (B, S, K), V = h.shape, weight.shape[0]
     return (0 < B <= 16 and S > 0 and 0 < K and K % 64 == 0 and 0 < V and V % 16 == 0 and V * K <= 2 ** 28
+            and _head_kernel_wins(B, V, K)
             and ((B - 1) * S + 1) * K * 2 <= 2 ** 31 and weight.dim() == 2 and weight.shape[1] == K
             and h.dtype == torch.float16 and weight.dtype == torch.float16 and h.is_cuda and weight.device == h.device
             and h.is_contiguous() and weight.is_contiguous() and type(h) is torch.Tensor
@@ -867,7 +884,7 @@ def _head_kernel_takes(h, weight):
 
 def head(h, weight):
     """Logits [B, 1, V] of the last position of h [B, S, K] under the fp16 output matrix [V, K].  Plain calls of up to
-    16 sequences and 2^28 weights run on eet_head_f16, all others on torch's linear."""
+    16 sequences and 2^28 weights run on eet_head_f16 where it is the faster one, all others on torch's linear."""
     if not _head_kernel_takes(h, weight):
         return torch.nn.functional.linear(h[:, -1:, :], weight)
     (B, S, K), V = h.shape, weight.shape[0]

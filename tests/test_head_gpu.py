@@ -84,3 +84,24 @@ def test_sizes_and_calls_that_the_kernel_does_not_have(gpu, monkeypatch):
     calls.clear()
     ops.head(h, torch.nn.Parameter(w, requires_grad=False))
     assert not calls                                                        # a plain call: the kernel
+
+
+def test_rule_of_the_kernel():
+    """Where the product stays with the library: very long rows, the ranges of V in which it measured faster."""
+    wins = ops._head_kernel_wins
+    assert all(wins(B, V, K) for B in (1, 16) for V, K in ((8000, 1024), (32000, 2048), (32000, 3072), (32000, 4096),
+                                                           (10240, 2048), (20480, 4096), (50272, 4096), (100352, 1536)))
+    assert not any(wins(B, V, K) for B in (1, 16) for V, K in ((32000, 8192), (10240, 4096), (12288, 3072), (50272, 3072)))
+    assert wins(8, 8000, 5120) and not wins(16, 8000, 5120) and wins(16, 32000, 5120)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,S,N,K", [(1, 1, 8016, 448),      # two tiles per workgroup, the last workgroup with one
+                                     (16, 2, 6144, 1088),    # two, a broken round of k blocks
+                                     (5, 1, 10256, 2048),    # four, the last with one
+                                     (16, 1, 20480, 3072),   # two, several rounds of workgroups
+                                     (2, 1, 18432, 4096)])   # one, several rounds
+def test_tiles_per_workgroup(gpu, M, S, N, K):
+    assert ops._head_kernel_takes(torch.empty(M, S, K, device=gpu, dtype=torch.float16),
+                                  torch.empty(N, K, device=gpu, dtype=torch.float16))
+    test_head(gpu, M, S, N, K)
