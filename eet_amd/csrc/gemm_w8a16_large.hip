@@ -32,12 +32,15 @@
 //     latency is exposed even with one wavefront per SIMD;
 //   * the block shape follows the problem (kTiles below): 20 shapes from 32 x 64 to 256 x 256.
 // Measured against that earlier kernel (us, QKV / O / gate-up / down of a 4096-wide layer, weights from HBM):
-//   M = 64    12288 <- 4096  21.7 -> 18.7   4096 <- 4096  13.9 -> 11.7   22016 <- 4096  32.5 -> 28.1   4096 <- 11008  22.9 -> 20.0
-//   M = 406                  49.8 -> 52.1                 26.5 -> 25.7                  87.6 -> 83.4                  51.2 -> 50.5
-//   M = 1024                100.0 -> 88.3                 38.2 -> 40.0                   157 -> 156                   92.5 -> 88.7
-//   M = 2048                  174 -> 169                  69.5 -> 65.1                   303 -> 308                    180 -> 159
-//   M = 8192                  629 -> 615                   232 -> 227                   1098 -> 1102                   562 -> 541
-// (geometric mean over 20 weight matrices of decoders 1024 .. 5120 wide, 40 .. 8192 rows: 1.10 x).
+//   M = 64    12288 <- 4096  20.7 -> 17.8   4096 <- 4096  12.9 -> 10.8   22016 <- 4096  31.6 -> 25.7   4096 <- 11008  22.1 -> 17.7
+//   M = 406                  50.0 -> 54.2                 25.7 -> 24.7                  91.6 -> 80.8                  50.1 -> 50.9
+//   M = 1024                103.3 -> 88.3                 37.9 -> 40.2                   156 -> 155                   91.8 -> 88.7
+//   M = 2048                  163 -> 164                  69.1 -> 70.2                   293 -> 298                    174 -> 154
+//   M = 8192                  631 -> 624                   217 -> 220                   1097 -> 1106                   544 -> 547
+// Over 649 problems (26 matrices of decoders 1024 .. 8192 wide, 33 .. 8192 rows) the time is 0.92 of what it was in the
+// geometric mean: 0.85 up to 200 rows, 0.91 up to 800, 0.96 to 0.97 beyond.  32 of them are more than 5 % slower, 13 % at
+// most: matrices with 1024 or 2048 columns at 900 rows and more (2048 <- 2048 at 2048 rows 22.2 -> 24.4: its blocks fit
+// the CUs once, and those of the earlier kernel shared a CU in twos), and launches a little over one round.
 // 32x32x16 matrix instructions (operands free by addressing, the weights being in LDS) were 8-12 % slower, wavefront
 // tiles of 128 x 128 with one wavefront per SIMD 20-30 %.
 #include "gemm_common.h"
@@ -403,13 +406,19 @@ int launch_large_m(const GemmArgs &a, int ksplit)
     return EET_OK;
 }
 
-// The block shapes and what they cost.  A launch of `w` workgroups that each walk nk k-tiles takes about
-//     base + (store [+ res]) * max(1, w / 256) * (block area / 10^4) + nk * per_tile(w / 256)   us
+// The block shapes and what they cost.  A launch with x workgroups per CU of the fullest XCD that walk nk k-tiles each
+// takes about
+//     base + (store [+ res]) * max(1, x) * (block area / 10^4) + nk * per_tile(x)   us
 // where per_tile is linear between the values at 1/2, 1, just over 1, 2, just over 2, 3, just over 3, 4, 8, 24 and 64
-// workgroups per CU (the jumps behind whole numbers are a CU that gets one workgroup more than the others).  Fitted,
-// shape by shape, to 14300 launches on MI355X: 20 weight matrices of decoders 1024 .. 5120 wide, 40 .. 8192 rows, one
-// to eight shares of the k range.  Over those problems the shape with the smallest estimate is on average 1.8 %
-// behind the fastest of 28 shapes (the worst case 25 %), where the earlier rule's five shapes were 12 % behind.
+// workgroups per CU (the jumps behind whole numbers are a CU that gets one workgroup more than the others).  The blocks
+// go to the XCDs in eight equal ranges, so 84 blocks in three shares are 252 workgroups, but 33 on the 32 CUs of seven
+// XCDs: counted over the whole chip such a launch looked 20 % cheaper than it is (406 rows, 3072 <- 8192: 43.8 us
+// against 34.7 for what is taken now).  Fitted, shape by shape, to 14300 launches on MI355X: 20 weight matrices of
+// decoders 1024 .. 5120 wide, 40 .. 8192 rows, one to eight shares of the k range; a fit is a fit: some of its
+// constants (a store or residual of nothing, two workgroups cheaper than one and a bit) mean nothing by themselves.
+// Checked against launches that are not in it (649 problems: those matrices at 25 row counts 33 .. 8192 and six
+// matrices 1536 and 8192 wide): on average 1.5 % behind the fastest of the 20 shapes and their shares, at most 25 %;
+// the same on the widths outside the fit.
 struct TileCost {
     int tm, tn, wm, wn;
     float base, store, res, per_tile[11];
@@ -471,10 +480,9 @@ void pick_large_m(int M, int N, int K, int epi, LargeMConfig *whole, LargeMConfi
         const int blocks = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
         const float area = (float)bm * bn * 1e-4f;
         auto cost = [&](int ks) {
-            const float x = blocks * ks / 256.f;
+            const float x = (blocks + 7) / 8 * ks / 32.f;   // the XCD with the most blocks decides
             const float store = ks > 1 ? 2.f * t.store : t.store + (epi == kEpiResidual ? t.res : 0.f);
-            return t.base + store * (x > 1.f ? x : 1.f) * area +
-                   (float)ktiles / ks * per_tile_us(t, x);
+            return t.base + store * (x > 1.f ? x : 1.f) * area + (float)ktiles / ks * per_tile_us(t, x);
         };
         if (const float us = cost(1); us < whole->us)
             *whole = LargeMConfig{i, 1, us};

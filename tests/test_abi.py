@@ -217,3 +217,13 @@ def test_calls_without_a_workspace_keep_their_faster_path(M, N, K, epi, slabs):
     v = [ctypes.byref(ctypes.c_int()) for _ in range(5)]
     for bad in ((32, N, K, 0, 0), (40, 8, 64, 0, 0), (40, 16, 32, 0, 0), (40, 48, 64, 2, 0), (40, 16, 64, 3, 0)):
         assert L.eet_gemm_w8a16_large_m_shape(*bad, *v) == -2
+
+
+@pytest.mark.parametrize("M,N,K", [(406, 3072, 8192), (406, 1536, 6144), (150, 5120, 13696)])
+def test_shares_are_counted_per_xcd(M, N, K):
+    """A launch whose workgroups fit the 256 CUs has none left over on an XCD: its blocks go to the XCDs in eight equal
+    ranges, 32 CUs each."""
+    ws = _lib.lib().eet_gemm_w8a16_workspace(M, N, K, 1)
+    tm, tn, wm, wn, ks = large_m_shape(M, N, K, 1, ws)
+    blocks = -(-M // (16 * tm * wm)) * -(-N // (16 * tn * wn))
+    assert ks > 1 and blocks * ks <= 256 and -(-blocks // 8) * ks <= 32
