@@ -865,21 +865,26 @@ def _head_kernel_wins(B, V, K):
 _transformed = torch._C._functorch.is_functorch_wrapped_tensor
 
 
+def _current_device():
+    try:
+        return torch._C._cuda_getDevice()
+    except AttributeError:
+        return torch.cuda.current_device()
+
+
 def _head_kernel_takes(h, weight):
     """The plain calls of `head`: whole fp16 rows on the current device, row offsets within 32 bits, and nothing that
     torch would do beyond the product (autograd in either mode, autocast, tensor subclasses and transforms)."""
-    (B, S, K), V = h.shape, weight.shape[0]
-    return (0 < B <= 16 and S > 0 and 0 < K and K % 64 == 0 and 0 < V and V % 16 == 0 and V * K <= 2 ** 28
-            and _head_kernel_wins(B, V, K)
-            and ((B - 1) * S + 1) * K * 2 <= 2 ** 31 and weight.dim() == 2 and weight.shape[1] == K
-            and h.dtype == torch.float16 and weight.dtype == torch.float16 and h.is_cuda and weight.device == h.device
+    (B, S, K), shape, device = h.shape, weight.shape, h.get_device()
+    return (device >= 0 and weight.get_device() == device and len(shape) == 2 and shape[1] == K
+            and 0 < B <= 16 and S > 0 and K > 0 and K % 64 == 0 and 0 < shape[0] <= 2 ** 28 // K and shape[0] % 16 == 0
+            and ((B - 1) * S + 1) * K * 2 <= 2 ** 31 and _head_kernel_wins(B, shape[0], K)
+            and h.dtype is torch.float16 and weight.dtype is torch.float16
             and h.is_contiguous() and weight.is_contiguous() and type(h) is torch.Tensor
-            and type(weight) in (torch.Tensor, torch.nn.Parameter)
-            and not _transformed(h) and not _transformed(weight)
-            and not (torch.is_grad_enabled() and (h.requires_grad or weight.requires_grad))
+            and (type(weight) is torch.Tensor or type(weight) is torch.nn.Parameter)
+            and not ((h.requires_grad or weight.requires_grad) and torch.is_grad_enabled()) and not _transformed(weight)
             and torch.autograd.forward_ad._current_level < 0 and not torch.is_autocast_enabled()
-            and h.device.index == torch.cuda.current_device()
-            and weight.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0)
+            and device == _current_device() and weight.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0)
 
 
 def head(h, weight):
@@ -888,7 +893,7 @@ def head(h, weight):
     if not _head_kernel_takes(h, weight):
         return torch.nn.functional.linear(h[:, -1:, :], weight)
     (B, S, K), V = h.shape, weight.shape[0]
-    out = torch.empty(B, 1, V, dtype=torch.float16, device=h.device)
+    out = h.new_empty((B, 1, V))
     check(lib().eet_head_f16(h.data_ptr() + 2 * (S - 1) * K, S * K, weight.data_ptr(), out.data_ptr(), B, V, K, _stream()),
           "eet_head_f16")
     return out

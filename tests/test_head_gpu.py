@@ -70,7 +70,7 @@ def test_sizes_and_calls_that_the_kernel_does_not_have(gpu, monkeypatch):
     calls = []
     monkeypatch.setattr(ops.torch.nn.functional, "linear", lambda *a: calls.append(1) or linear(*a))
     with monkeypatch.context() as m:
-        m.setattr(ops.torch.cuda, "current_device", lambda: 1)
+        m.setattr(ops, "_current_device", lambda: 1)
         assert torch.equal(ops.head(h, w), want) and calls == [1]
     assert ops.head(h.clone().requires_grad_(), w).requires_grad and len(calls) == 2
     with torch.autograd.forward_ad.dual_level():
@@ -105,3 +105,13 @@ def test_tiles_per_workgroup(gpu, M, S, N, K):
     assert ops._head_kernel_takes(torch.empty(M, S, K, device=gpu, dtype=torch.float16),
                                   torch.empty(N, K, device=gpu, dtype=torch.float16))
     test_head(gpu, M, S, N, K)
+
+
+@pytest.mark.gpu
+def test_parameters_without_gradients(gpu):
+    """A matrix that would take gradients stays with the kernel wherever they are off."""
+    h = torch.randn(2, 3, 64, device=gpu).half()
+    w = torch.nn.Parameter(torch.randn(32, 64, device=gpu).half())
+    with torch.no_grad():
+        assert ops._head_kernel_takes(h, w)
+    assert not ops._head_kernel_takes(h, w) and ops._head_kernel_takes(h, w.detach())
