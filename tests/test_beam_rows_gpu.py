@@ -35,9 +35,10 @@ def test_argument_errors():
 @pytest.mark.parametrize("B,H,dh,first,cap,padded,alibi", [
     (2, 1, 32, 1, 8, False, False),          # from a one-row prompt on
     (5, 3, 96, 30, 40, True, True),          # idle lanes, padding, bias
-    (16, 8, 64, 255, 262, True, False),      # around one split of the time axis
+    (16, 8, 64, 255, 262, True, False),      # one workgroup per (sequence, head), whole turns of the ring and a row
     (3, 8, 128, 1021, 1030, False, True),    # several splits
     (260, 1, 32, 700, 704, False, False),    # more names per workgroup than lanes
+    (8, 32, 128, 2058, 2064, True, False),   # 64 rows to a stream: the ring of four by the plan itself
 ])
 def test_rows_by_name_equal_moved_rows(gpu, B, H, dh, first, cap, padded, alibi):
     g = torch.Generator().manual_seed(B * 1000 + dh)
@@ -109,6 +110,20 @@ def test_op_settles_its_cache(gpu, rows):
         assert b.layers[0][0]._rows is None and ka.shape[0] == rows
     step = a.layers[0][0].step
     assert torch.equal(a.layers[0][0].k_cache[: rows - 1, :, :step], b.layers[0][0].k_cache[: rows - 1, :, :step])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ring", [2, 4])
+@pytest.mark.parametrize("threads,nsplit", [(256, 1), (512, 3), (1024, 2)])
+@pytest.mark.parametrize("B,H,dh,first,cap,padded,alibi", [(4, 3, 128, 700, 706, True, True), (3, 2, 96, 411, 416, False, False),
+                                                           (5, 2, 64, 1500, 1504, False, True), (2, 3, 32, 3001, 3005, True, False)])
+def test_every_form_of_the_kernel(gpu, tuning, ring, threads, nsplit, B, H, dh, first, cap, padded, alibi):
+    """Both depths of the ring, whose slots hold the names requested a turn ahead, at every width of a workgroup and
+    with the time axis split: several turns and a ragged last one."""
+    tuning("EET_MMHA_THREADS", threads)
+    tuning("EET_MMHA_UNROLL", ring)
+    tuning("EET_MMHA_NSPLIT", nsplit)
+    test_rows_by_name_equal_moved_rows(gpu, B, H, dh, first, cap, padded, alibi)
 
 
 def beam_decoders(rows, steps):
