@@ -228,8 +228,9 @@ LARGE_M_TILES = ["8,4", "4,5", "4,4", "4,2", "2,2"]   # m-tiles, n-tiles per wav
 
 @pytest.mark.parametrize("tile", LARGE_M_TILES)
 def test_large_m_tiles(gpu, tuning, tile):
-    """Every large-M kernel variant (selected with the tuning override), on ragged M / N edges and on
-    k-loops of 1..9 tiles (prologue, unrolled body and tail of the software pipeline)."""
+    """Large-M kernel variants (selected with the tuning override; every block shape is walked by the tests of the
+    large-M blocks), on ragged M / N edges and on k-loops of 1..9 tiles (prologue, unrolled body and tail of the
+    software pipeline)."""
     tuning("EET_GEMM_LARGE_M_TILE", tile)
     for (M, K, N) in [(129, 64, 48), (300, 128, 272), (257, 192, 720), (200, 256, 336), (512, 320, 256),
                       (130, 448, 64), (333, 576, 1040)]:
@@ -239,15 +240,51 @@ def test_large_m_tiles(gpu, tuning, tile):
                      what=f"tile {tile} M={M} K={K} N={N}")
 
 
-@pytest.mark.parametrize("M,K,N,tile", [(1024, 256, 12288, "128x256"), (2048, 256, 5120, "64x320"),
-                                        (512, 192, 22016, "64x256"), (512, 256, 8192, "64x128"),
-                                        (256, 256, 1024, "32x128"), (100, 320, 12288, "32x128"),
-                                        (64, 256, 4096, "slabs")])
-def test_large_m_dispatch(gpu, M, K, N, tile):
-    """Shapes on which the dispatcher itself picks each tile (named for the record) -- no override."""
+def large_m_block(M, K, N, ws):
+    """"rows x columns of a block, shares of the k range" of the launch that the dispatcher picks; "slabs"."""
+    import ctypes
+    from eet_amd._lib import check, lib
+    v = [ctypes.c_int() for _ in range(5)]
+    check(lib().eet_gemm_w8a16_large_m_shape(M, N, K, 0, ws, *[ctypes.byref(x) for x in v]))
+    tm, tn, wm, wn, ks = (x.value for x in v)
+    return f"{16 * tm * wm}x{16 * tn * wn}" + (f" / {ks}" if ks > 1 else "") if tm else "slabs"
+
+
+@pytest.mark.parametrize("M,K,N,block", [(1024, 256, 12288, "256x256"), (2048, 256, 5120, "128x320"),
+                                         (512, 192, 22016, "128x192"), (512, 256, 8192, "64x256"),
+                                         (256, 256, 1024, "32x64"), (100, 320, 12288, "64x64"),
+                                         (64, 256, 4096, "32x64")])
+def test_large_m_dispatch(gpu, M, K, N, block):
+    """Shapes on which the dispatcher itself picks a block, without a split -- no override."""
+    from eet_amd._lib import lib
+    assert large_m_block(M, K, N, lib().eet_gemm_w8a16_workspace(M, N, K, 0)) == block
     x, u, p, s = make(M, K, N, 77)
     c = gemm(x.to(gpu), p.to(gpu), s.to(gpu), M, N, K)
-    assert_close(c.cpu().numpy(), O.dequant_matmul(x.numpy(), u.numpy(), s.numpy(), np.float32), what=tile)
+    assert_close(c.cpu().numpy(), O.dequant_matmul(x.numpy(), u.numpy(), s.numpy(), np.float32), what=block)
+
+
+@pytest.mark.parametrize("M,K,N,split,alone", [(40, 4096, 1040, "32x64 / 6", "slabs"),
+                                               (70, 11008, 528, "32x64 / 8", "32x64"),
+                                               (203, 2816, 1024, "64x64 / 4", "32x64"),
+                                               (260, 5632, 528, "96x64 / 8", "32x64")])
+def test_large_m_dispatch_of_a_split(gpu, M, K, N, split, alone):
+    """Shapes on which the dispatcher itself splits the k range: with exactly the bytes that the library asks for, with
+    16 fewer and with none, and the memory behind them untouched."""
+    from eet_amd._lib import check, lib
+    from gpu_util import stream
+    need = lib().eet_gemm_w8a16_workspace(M, N, K, 0)
+    assert large_m_block(M, K, N, need) == split
+    assert large_m_block(M, K, N, need - 16) == large_m_block(M, K, N, 0) == alone
+    x, u, p, s = make(M, K, N, 78)
+    ref = O.dequant_matmul(x.numpy(), u.numpy(), s.numpy())
+    xd, pd, sd = x.to(gpu), p.to(gpu), s.to(gpu)
+    ws = torch.full((need + 256,), 77, dtype=torch.uint8, device=gpu)
+    for bytes_given in (need, need - 16, 0):
+        c = torch.empty(M, N, dtype=torch.float16, device=gpu)
+        check(lib().eet_gemm_w8a16(xd.data_ptr(), pd.data_ptr(), sd.data_ptr(), c.data_ptr(), M, N, K,
+                                   ws.data_ptr() if bytes_given else None, bytes_given, stream()))
+        assert_close(c.cpu().numpy(), ref, rtol=1e-2, atol=1e-3, what=f"{bytes_given} bytes")
+        assert (ws[need:] == 77).all()
 
 
 def test_full_size_linearity(gpu):
