@@ -865,11 +865,8 @@ def _head_kernel_wins(B, V, K):
 _transformed = torch._C._functorch.is_functorch_wrapped_tensor
 
 
-def _current_device():
-    try:
-        return torch._C._cuda_getDevice()
-    except AttributeError:
-        return torch.cuda.current_device()
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+_dual_levels = torch.autograd.forward_ad
 
 
 def _head_kernel_takes(h, weight):
@@ -883,7 +880,7 @@ def _head_kernel_takes(h, weight):
             and h.is_contiguous() and weight.is_contiguous() and type(h) is torch.Tensor
             and (type(weight) is torch.Tensor or type(weight) is torch.nn.Parameter)
             and not ((h.requires_grad or weight.requires_grad) and torch.is_grad_enabled()) and not _transformed(weight)
-            and torch.autograd.forward_ad._current_level < 0 and not torch.is_autocast_enabled()
+            and _dual_levels._current_level < 0 and not torch.is_autocast_enabled()
             and device == _current_device() and weight.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0)
 
 
@@ -894,8 +891,8 @@ def head(h, weight):
         return torch.nn.functional.linear(h[:, -1:, :], weight)
     (B, S, K), V = h.shape, weight.shape[0]
     out = h.new_empty((B, 1, V))
-    check(lib().eet_head_f16(h.data_ptr() + 2 * (S - 1) * K, S * K, weight.data_ptr(), out.data_ptr(), B, V, K, _stream()),
-          "eet_head_f16")
+    check(lib().eet_head_f16(h.data_ptr() + 2 * (S - 1) * K, S * K, weight.data_ptr(), out.data_ptr(), B, V, K,
+                             _current_stream()), "eet_head_f16")
     return out
 
 
