@@ -199,7 +199,8 @@ class Int8Decoder:
         num_beams ranks into finished hypotheses (score = sum of log-probabilities / length ** length_penalty,
         the length counting the prompt) and continues with the first num_beams others.  The beam each
         continuation came from is handed to the attention ops as reorder_state with the next call
-        (generation.py:1577), which gathers their KV caches (csrc/op/llama_mmha.cpp:248-252).
+        (generation.py:1577), which goes on from the rows of those beams (csrc/op/llama_mmha.cpp:248-252): the
+        cache rows stay where they are and the attention finds them by name.
         Returns (tokens [B, <= max_new_tokens] padded with pad_token_id, scores [B])."""
         cfg = self.cfg
         B, S = input_ids.shape
@@ -249,7 +250,7 @@ class Int8Decoder:
                 gen = torch.cat([gen[beam_idx], nxt_t.view(-1, 1).to(dev)], dim=1)
                 if all(done) or step == max_new_tokens - 1:
                     break
-                self.reorder_state = beam_idx                                      # the ops gather their caches
+                self.reorder_state = beam_idx                                      # whose rows each beam goes on from
                 logits = self.logits(nxt_t.view(-1, 1).to(dev), False)
         finally:
             self.reorder_state = torch.empty(0, dtype=torch.long)
@@ -282,12 +283,12 @@ class Int8Decoder:
         The graph holds raw device pointers.  Everything they point to is kept alive with the
         graph (the named workspaces handed out while recording, the KV caches, the static
         input / output buffers); a replay refuses to run when a layer's cache tensors are no
-        longer the recorded ones (a beam reorder swaps them), and brings the device-side step
-        back in line when eager calls or a new prompt moved the host-side step in between."""
+        longer the recorded ones (settling a cache after a beam search swaps them), and brings the
+        device-side step back in line when eager calls or a new prompt moved the host-side step in between."""
         cfg, dev = self.cfg, self.embed.device
         if self.reorder_state is not None and self.reorder_state.numel() != 0:
             raise RuntimeError("[EET][ERROR] capture_decode_step: a decoder that reorders its KV cache (beam search) "
-                               "cannot replay a recorded step: the reorder swaps the cache buffers the graph points to")
+                               "cannot replay a recorded step: it reads every row from its own sequence's slab")
         for attn, _ in self.layers:
             attn.settle_cache()     # rows named by an earlier beam search move before anything is recorded
         B = next_ids.shape[0]

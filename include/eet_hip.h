@@ -51,8 +51,8 @@ int eet_packed_layout_version(void);
  * that run every kernel variant; value NULL or "" restores the table.  Keys:
  *   EET_GEMM_SMALL_M_CONFIG "nt,waves,u[,ksplit]"   EET_GEMM_LARGE_M_TILE "tm,tn[,ksplit[,wm,wn]]"
  *   EET_MMHA_NSPLIT / EET_MMHA_THREADS / EET_MMHA_UNROLL "n"
- *   EET_PREFILL_LEGACY "1" (register-staged prefill attention at head size 128)
- *   EET_PREFILL_SHAPE "1" | "2" (launch shape of the head-size-128 prefill kernel)
+ *   EET_PREFILL_LEGACY "1" (register-staged prefill attention at every head size)
+ *   EET_PREFILL_SHAPE "1" | "2" (launch shape of the prefill kernel of head sizes 64, 96 and 128)
  *   EET_PREFILL_GROUP "n" ((batch, head) pairs whose query blocks an XCD works on together in prefill
  *                         attention; "-1": every pair of a query block before the next block)
  *   EET_CHAIN_SPIN_LIMIT "n" / EET_CHAIN_SLEEP "n" (bounded wait of a chained launch)
@@ -400,8 +400,8 @@ int eet_gated_ffn_int8_decode(const void *x, const void *rms_gamma, float rms_ep
 
 /* The output head of a decode step: out[M][N] = x[M][K] * w[N][K]^T, fp16 with fp32
  * sums.  Row m of x begins at x + m*x_stride halves (x_stride >= K, a multiple of 8);
- * w row-major, out contiguous.  M <= 16, K % 64 == 0, N % 16 == 0, N*K <= 2^28, x and w
- * 16-byte aligned.  Stands in for the fp16 linear of the reference's caller
+ * w row-major, out contiguous.  M <= 16, K % 64 == 0, N % 16 == 0, N*K <= 2^28 (larger
+ * matrices are better off with a library product), x and w 16-byte aligned.  Stands in for the fp16 linear of the reference's caller
  * (python/eet/transformers/modeling_llama.py:471) at decode sizes. */
 int eet_head_f16(const void *x, long x_stride, const void *w, void *out, int M, int N, int K,
                  void *stream);
