@@ -2,7 +2,7 @@
 intermediate 13696), against the fp32 oracle, through the C ABI.
 
 Configuration 3: the prefill GEMMs at M = 2048 (QKV 5120 -> 15360, O 5120 -> 5120, gate / up
-5120 -> 13696, down 13696 -> 5120), i.e. the 128 x 256 and 64 x 320 MFMA tiles the dispatcher
+5120 -> 13696, down 13696 -> 5120), i.e. the 256 x 256 and 128 x 320 blocks the dispatcher
 picks there, every output element compared.
 Configuration 5: the decode linears at M = 32 as the decoder ops launch them (RMSnorm prologue on
 QKV and gate|up, SwiGLU epilogue, residual epilogue on O and down).

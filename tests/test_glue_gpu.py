@@ -145,7 +145,7 @@ def test_prefill_attention_rising_scores(gpu, dh, per_chunk):
                                                  (515, True, True), (1700, False, False)])
 def test_prefill_attention_launch_shapes_dh128(gpu, tuning, shape, S, use_pad, use_alibi):
     """Head size 128 runs in one of two launch shapes (queries per workgroup, tiles per wavefront, ring depth)
-    depending on the prompt length; each is forced here at lengths on either side of the switch and held to
+    depending on prompt length and launch size; each is forced here at lengths on either side of 1536 and held to
     the same oracle."""
     tuning("EET_PREFILL_SHAPE", shape)
     test_prefill_attention(gpu, 2, 2, S, 128, use_pad, use_alibi)

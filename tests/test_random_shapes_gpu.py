@@ -1,5 +1,5 @@
 """Seeded random shapes through the C ABI against the fp32 oracle: the fused dequant-GEMM over every
-dispatch range (small-M, 32-row slabs, every large-M tile) with each epilogue and the RMSnorm prologue,
+dispatch range (small-M, large-M blocks with and without a split) with each epilogue and the RMSnorm prologue,
 and the decode attention over random batch / head / step / padding / ALiBi combinations.
 Tolerance: 1e-2 relative / 1e-3 absolute (2e-3 / 3e-3 absolute with the RMSnorm prologue / + SwiGLU,
 whose reference composition rounds once more), as in the per-kernel tests."""
@@ -20,7 +20,7 @@ def _gemm_cases(n, seed):
     rng = np.random.default_rng(seed)
     cases = []
     for i in range(n):
-        m_hi = [8, 32, 128, 700][i % 4]                       # small-M, small-M with 2-4 row groups, slabs, large-M
+        m_hi = [8, 32, 128, 700][i % 4]                       # small-M, small-M with 2-4 row groups, large-M, larger blocks
         M = int(rng.integers(1, m_hi + 1))
         K = 64 * int(rng.integers(1, 24))
         N = 16 * int(rng.integers(1, 70))
