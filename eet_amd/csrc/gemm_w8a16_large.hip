@@ -499,13 +499,12 @@ void pick_large_m(int M, int N, int K, int epi, LargeMConfig *whole, LargeMConfi
 // 33 to 64 rows and no workspace for a split: with few channels the blocks leave most of the chip idle and each walks
 // the whole k range alone, so its time is that of the k loop whatever M and N are.  The small-M kernel over 32-row
 // slabs shares a block's k range among its wavefronts and has a block per few 16-channel tiles; its weights are read
-// twice, from the Infinity Cache the second time, its second slab costs by its rows, and below 3072 k (2048 with SwiGLU) two short
-// launches cost the host more than one.  Measured, us, slabs / blocks, at 33, 48
-// and 64 rows: 1024 <- 1024 6.2 / 5.4, 6.3 / 5.5, 6.1 / 5.5; 1024 <- 8192 14 / 23, 17 / 23, 21 / 23; 2048 <- 4096
-// 10.1 / 13.0, 11.6 / 12.7, 13.4 / 12.7; 3072 <- 2048 9.0 / 8.2, 10.0 / 8.1, 9.7 / 8.1; 4096 <- 11008 24 / 31, 28 / 31,
-// 32 / 31; 5120 <- 4096 13.7 / 13.6, 15.4 / 13.3, 16.6 / 13.8.  SwiGLU blocks hold whole (gate, up) pairs and are
-// wider: 4096 <- 4096 13.0 / 17.4, 14.6 / 17.6, 16.3 / 17.7; 7168 <- 4096 15.6 / 17.7, 16.6 / 17.8, 18.4 / 18.5;
-// 9216 <- 4096 22 / 18, 23 / 18, 25 / 19.
+// twice, from the Infinity Cache the second time, its second slab costs by its rows, and below 3072 k (2048 with SwiGLU)
+// two short launches cost the host more than one.  Measured, us, slabs / blocks, at 33, 48 and 64 rows: 1024 <- 1024
+// 6.2 / 5.4, 6.3 / 5.5, 6.1 / 5.5; 1024 <- 8192 14 / 23, 17 / 23, 21 / 23; 2048 <- 4096 10.1 / 13.0, 11.6 / 12.7,
+// 13.4 / 12.7; 3072 <- 2048 9.0 / 8.2, 10.0 / 8.1, 9.7 / 8.1; 4096 <- 11008 24 / 31, 28 / 31, 32 / 31; 5120 <- 4096
+// 13.7 / 13.6, 15.4 / 13.3, 16.6 / 13.8.  SwiGLU blocks hold whole (gate, up) pairs and are wider: 4096 <- 4096 13.0 /
+// 17.4, 14.6 / 17.6, 16.3 / 17.7; 7168 <- 4096 15.6 / 17.7, 16.6 / 17.8, 18.4 / 18.5; 9216 <- 4096 22 / 18, 23 / 18, 25 / 19.
 bool slabs_win(int M, int N, int K, int epi)
 {
     if (M > 64 || K < 2048)
