@@ -10,10 +10,13 @@
 // reference has no device quantiser; converting a checkpoint on the host costs
 // seconds per billion weights, here the time of reading it twice from HBM.
 //
-// HBM-bound.  Pass 1 reads the matrix once (column absmax, one 32-bit atomic
-// max per column and 128-row chunk); pass 2 reads it again (from the Infinity
-// Cache when it fits) and writes one byte per weight in the packed layout, plus
-// one more in row-major order when the caller wants the unprocessed matrix.
+// HBM-bound.  Most matrices go in one pass that holds them in the registers of
+// the chip (quant_group_kernel; one_pass_wins has the rule and the times).  The
+// others take two: pass 1 reads the matrix once (column absmax, one 32-bit
+// atomic max per column and 128-row chunk); pass 2 reads it again (from the
+// Infinity Cache when it fits) and writes one byte per weight in the packed
+// layout, plus one more in row-major order when the caller wants the
+// unprocessed matrix.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -27,6 +30,9 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kColsPerThread = 8;   // pass 1: 16 bytes of fp16 per load
 constexpr int kMaxRows = 128;       // rows per workgroup in pass 1 (32 per wavefront)
+constexpr int kMaxPolls = 1 << 14;   // one pass: waiting for the other parts of a column group
+constexpr int kMaxParts = 16;
+constexpr int kCountStride = 32;    // words: a line for every count
 constexpr int kTileCols = 128;      // pass 2: one k-tile x 8 n-tiles per workgroup
 
 template <typename T>
@@ -205,27 +211,391 @@ __global__ __launch_bounds__(256) void quant_pack_kernel(const T *__restrict__ w
     }
 }
 
+
+// ---- one pass: the matrix stays in registers between the maxima and the weights ----
+//
+// A group of columns one cache line wide (64 of fp16, 32 of fp32; half a line doubles what the L1 fetches, and stripes of
+// 16 fp16 columns that need no exchange took 65-77 us for 11008 x 4096) is shared by `parts` workgroups, each with a
+// contiguous range of its k-tiles in registers.  They exchange their column maxima through memory -- a slot per part,
+// then a count of the parts that are through, on a line of its own (counts side by side: 62 us instead of 46 at eight
+// parts) -- and then each quantises and packs what it holds.  The wait is bounded: parts of a group are neighbours in
+// the grid and so run together, but where one is kept off the chip the others read its rows themselves.  A wavefront takes
+// units of 32 rows round-robin; a lane holds 4 consecutive rows of the columns that one 16-byte load brings, so that
+// its bytes of a column are whole words of the packed tile.
+constexpr int kUnit = 32;
+
 template <typename T>
-int run(const void *w, size_t K, size_t N, int mode, int8_t *q, int8_t *packed, void *scale, uint32_t *amax,
+struct GroupShape {
+    static constexpr int kCols = 16 / (int)sizeof(T);   // columns of a lane
+    static constexpr int kGroup = 8 * kCols;            // columns of a group: 128 bytes of a row
+};
+
+// largest of |x| over the register's values as unsigned integers, which order like them (NaN above everything)
+template <typename T>
+__device__ __forceinline__ uint32_t max_abs(uint32_t m, uint32_t x)
+{
+    if constexpr (sizeof(T) == 2) {
+        typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, m),
+                                                                     __builtin_bit_cast(u16x2, x & 0x7fff7fffu)));
+    } else {
+        return m > (x & 0x7fffffffu) ? m : x & 0x7fffffffu;
+    }
+}
+
+// x without the values that are NaN (0 in their place)
+template <typename T>
+__device__ __forceinline__ uint32_t drop_nan(uint32_t x)
+{
+    if constexpr (sizeof(T) == 2)
+        return ((x & 0x7fffu) > 0x7c00u ? 0u : x & 0xffffu) | ((x & 0x7fff0000u) > 0x7c000000u ? 0u : x & 0xffff0000u);
+    else
+        return (x & 0x7fffffffu) > 0x7f800000u ? 0u : x;
+}
+
+template <typename T>
+__device__ __forceinline__ float value_at(const u32x4 &v, int i)
+{
+    if constexpr (sizeof(T) == 2) {
+        typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+        return (float)__builtin_bit_cast(f16x8, v)[i];
+    } else {
+        return __uint_as_float(v[i]);
+    }
+}
+
+template <typename T, int WAVES, int UNITS, bool QOUT>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4))) void quant_group_kernel(const T *__restrict__ w, int K, int N, int parts,
+                                                                 int ref128, uint32_t *maxima, uint32_t *arrived,
+                                                                 int8_t *__restrict__ q_out,
+                                                                 uint8_t *__restrict__ packed, T *__restrict__ scale)
+{
+    using S = GroupShape<T>;
+    __shared__ uint32_t part[WAVES][S::kGroup];
+    __shared__ float s_all[S::kGroup], inv_all[S::kGroup];
+    __shared__ int flags[3];    // NaN among the weights; the exact path for all; the other parts did not arrive
+    __shared__ uint32_t lq[WAVES][S::kGroup][9];   // [column][4-row word] of a unit, one word of padding per column
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int group = blockIdx.x / parts, mine = blockIdx.x % parts;
+    const int ktiles = K / 64, kt0 = (int)((long)mine * ktiles / parts), kt1 = (int)((long)(mine + 1) * ktiles / parts);
+    const int col0 = group * S::kGroup, quad = lane >> 3, c0 = (lane & 7) * S::kCols;
+    const bool cols_in = col0 + c0 < N;    // N % 16 == 0: a lane's columns are in range together
+    const T *base = w + (cols_in ? col0 + c0 : N - S::kCols);
+    const float nan_to = ref128 ? 1000.f : 0.f;
+    const int lo = ref128 ? -128 : -127;
+
+    // The wavefront's units: unit0 + wave, + WAVES, ... below unit1, at most UNITS of them.
+    const int unit0 = 2 * kt0, unit1 = 2 * kt1;
+    u32x4 v[UNITS][4];
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+        const int unit = unit0 + wave + WAVES * u;
+        if (unit < unit1) {
+            const T *p = base + (size_t)(unit * kUnit + 4 * quad) * N;
+#pragma unroll
+            for (int it = 0; it < 4; ++it)
+                v[u][it] = *reinterpret_cast<const u32x4 *>(p + (size_t)it * N);
+        }
+    }
+    if (threadIdx.x < 3)
+        flags[threadIdx.x] = 0;
+
+    // lane maxima to column maxima: thread t < kGroup returns that of column t
+    auto column_max = [&](uint32_t (&m)[4]) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+#pragma unroll
+            for (int x = 8; x < 64; x *= 2)
+                m[d] = max_abs<T>(m[d], (uint32_t)__shfl_xor((int)m[d], x));
+        }
+        if (quad == 0) {
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                if constexpr (sizeof(T) == 2) {
+                    part[wave][c0 + 2 * d] = m[d] & 0xffffu;
+                    part[wave][c0 + 2 * d + 1] = m[d] >> 16;
+                } else {
+                    part[wave][c0 + d] = m[d];
+                }
+            }
+        }
+        __syncthreads();
+        uint32_t a = 0;
+        if (threadIdx.x < S::kGroup) {
+#pragma unroll
+            for (int k = 0; k < WAVES; ++k)
+                a = a > part[k][threadIdx.x] ? a : part[k][threadIdx.x];
+        }
+        return a;
+    };
+    // the same from memory, without the weights that are NaN, for the units [from, to)
+    auto column_max_again = [&](int from, int to) {
+        uint32_t m[4] = {0, 0, 0, 0};
+        for (int unit = from + wave; unit < to; unit += WAVES) {
+            const T *p = base + (size_t)(unit * kUnit + 4 * quad) * N;
+#pragma unroll
+            for (int it = 0; it < 4; ++it) {
+                const u32x4 x = *reinterpret_cast<const u32x4 *>(p + (size_t)it * N);
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    m[d] = max_abs<T>(m[d], drop_nan<T>(x[d]));
+            }
+        }
+        return column_max(m);
+    };
+
+    uint32_t m[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u)
+        if (unit0 + wave + WAVES * u < unit1) {
+#pragma unroll
+            for (int it = 0; it < 4; ++it)
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    m[d] = max_abs<T>(m[d], v[u][it][d]);
+        }
+    constexpr uint32_t kInf = sizeof(T) == 2 ? 0x7c00u : 0x7f800000u;
+    uint32_t a = column_max(m);
+    if (a > kInf)
+        flags[0] = flags[1] = 1;
+    __syncthreads();
+    if (flags[0])   // NaN weights are ignored, as on the host
+        a = column_max_again(unit0, unit1);
+    if (parts > 1) {
+        // the first wavefront holds every column's maximum: exchange, count up, wait for the other parts
+        if (wave == 0) {
+            uint32_t *count = arrived + (size_t)group * kCountStride;
+            uint32_t *slots = maxima + (size_t)group * parts * S::kGroup + lane;
+            if (lane < S::kGroup)
+                __hip_atomic_store(slots + mine * S::kGroup, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the maxima are in memory
+            if (lane == 0)
+                __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            bool all = false;
+            for (int poll = 0; poll < kMaxPolls && !all; ++poll) {
+                all = __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= (uint32_t)parts;
+                if (!all)
+                    __builtin_amdgcn_s_sleep(8);
+            }
+            asm volatile("" ::: "memory");
+            if (!all)
+                flags[2] = 1;
+            else if (lane < S::kGroup) {
+                uint32_t o[kMaxParts];
+#pragma unroll
+                for (int p = 0; p < kMaxParts; ++p)
+                    o[p] = __hip_atomic_load(slots + min(p, parts - 1) * S::kGroup, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                for (int p = 0; p < kMaxParts; ++p)
+                    a = a > o[p] ? a : o[p];
+            }
+        }
+        __syncthreads();
+        if (flags[2])   // a part is kept off the chip: its rows are read here
+            a = column_max_again(0, 2 * ktiles);
+    }
+    if (threadIdx.x < S::kGroup) {
+        float m;
+        if constexpr (sizeof(T) == 2)
+            m = (float)__builtin_bit_cast(_Float16, (uint16_t)a);
+        else
+            m = __uint_as_float(a);
+        const float s = ref128 ? m * (1.f / 128.f) : __fdiv_rn(m, 127.f);
+        s_all[threadIdx.x] = s;
+        inv_all[threadIdx.x] = __fdiv_rn(1.f, s);
+        if (mine == 0 && col0 + (int)threadIdx.x < N)
+            scale[col0 + threadIdx.x] = static_cast<T>(s);
+        if (!(s > 0x1p-100f && s < 0x1p100f))
+            flags[1] = 1;
+    }
+    __syncthreads();
+    const bool odd = flags[1] != 0;
+
+    float inv[S::kCols];
+#pragma unroll
+    for (int i = 0; i < S::kCols; ++i)
+        inv[i] = inv_all[c0 + i];
+
+    // the unit's words -- four rows of a column, q + 128 -- leave
+    auto store = [&](const uint32_t (&word)[S::kCols], int unit) {
+        if constexpr (QOUT) {
+            if (cols_in) {
+                // words of four rows to words of four columns
+                uint32_t o[4][S::kCols / 4];
+#pragma unroll
+                for (int h = 0; h < S::kCols / 4; ++h) {
+                    const uint32_t *c = word + 4 * h;
+                    const uint32_t t0 = __builtin_amdgcn_perm(c[1], c[0], 0x05010400u);
+                    const uint32_t t1 = __builtin_amdgcn_perm(c[1], c[0], 0x07030602u);
+                    const uint32_t t2 = __builtin_amdgcn_perm(c[3], c[2], 0x05010400u);
+                    const uint32_t t3 = __builtin_amdgcn_perm(c[3], c[2], 0x07030602u);
+                    o[0][h] = __builtin_amdgcn_perm(t2, t0, 0x05040100u) ^ 0x80808080u;
+                    o[1][h] = __builtin_amdgcn_perm(t2, t0, 0x07060302u) ^ 0x80808080u;
+                    o[2][h] = __builtin_amdgcn_perm(t3, t1, 0x05040100u) ^ 0x80808080u;
+                    o[3][h] = __builtin_amdgcn_perm(t3, t1, 0x07060302u) ^ 0x80808080u;
+                }
+                int8_t *q = q_out + (size_t)(unit * kUnit + 4 * quad) * N + col0 + c0;
+#pragma unroll
+                for (int it = 0; it < 4; ++it)
+                    __builtin_memcpy(__builtin_assume_aligned(q + (size_t)it * N, S::kCols < 8 ? S::kCols : 8), o[it],
+                                     S::kCols);
+            }
+        }
+        // Into packed order through a slab of the wavefront's own: no barrier.  A unit is the g = 0, 1 or the g = 2, 3
+        // half of a k-tile, 512 bytes of each of the group's n-tiles.
+#pragma unroll
+        for (int i = 0; i < S::kCols; ++i)
+            lq[wave][c0 + i][quad] = word[i];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int p = 0; p < S::kGroup / 32; ++p) {
+            const int piece = p * 64 + lane, n16 = piece >> 5, g = (piece >> 4) & 1, i = piece & 15;
+            const int nt = col0 / 16 + n16;
+            const uint32_t *src = &lq[wave][n16 * 16 + i][4 * g];
+            const u32x4 o = {src[0], src[1], src[2], src[3]};
+            if (nt * 16 < N)
+                *reinterpret_cast<u32x4 *>(packed + ((size_t)nt * ktiles + (unit >> 1)) * 1024 + (unit & 1) * 512 +
+                                           (g * 16 + i) * 16) = o;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+
+    // v = x / s + 128 to within 2^-16 (x times the rounded reciprocal: 2^-17 at |x / s| <= 128; the sum, below 256:
+    // 2^-17), and the correctly rounded quotient of the host is within 2^-17 of the exact one: unless v lies within
+    // 2^-15 of a half, both round to the same integer.  The conversion rounds to nearest and clamps to 0 .. 255, i.e. +128
+    // to 127.  Units with a weight near a half (one in eight of random weights) are left to the second loop, which reads
+    // them again and divides.
+    constexpr float kNear = 0x1p-15f;
+    unsigned again = 0;
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+        const int unit = unit0 + wave + WAVES * u;
+        if (unit >= unit1)
+            continue;
+        uint32_t word[S::kCols];
+#pragma unroll
+        for (int i = 0; i < S::kCols; ++i)
+            word[i] = 0;
+        float near = 1.f;
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+#pragma unroll
+            for (int i = 0; i < S::kCols; i += 2) {
+                const float f0 = __builtin_fmaf(value_at<T>(v[u][it], i), inv[i], 128.f);
+                const float f1 = __builtin_fmaf(value_at<T>(v[u][it], i + 1), inv[i + 1], 128.f);
+                word[i] = __builtin_amdgcn_cvt_pk_u8_f32(f0, it, word[i]);
+                word[i + 1] = __builtin_amdgcn_cvt_pk_u8_f32(f1, it, word[i + 1]);
+                // (the compiler's minimum of two magnitudes is four instructions)
+                asm("v_min3_f32 %0, %0, abs(%1), abs(%2)"
+                    : "+v"(near)
+                    : "v"(__builtin_amdgcn_fractf(f0) - 0.5f), "v"(__builtin_amdgcn_fractf(f1) - 0.5f));
+            }
+        }
+        if (odd || __any(near < kNear))
+            again |= 1u << u;
+        else
+            store(word, unit);
+    }
+    while (again != 0) {
+        const int u = __builtin_ctz(again), unit = unit0 + wave + WAVES * u;
+        again &= again - 1;
+        uint32_t word[S::kCols];
+#pragma unroll
+        for (int i = 0; i < S::kCols; ++i)
+            word[i] = 0;
+        const T *p = base + (size_t)(unit * kUnit + 4 * quad) * N;
+        u32x4 x[4];
+#pragma unroll
+        for (int it = 0; it < 4; ++it)
+            x[it] = *reinterpret_cast<const u32x4 *>(p + (size_t)it * N);
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+#pragma unroll
+            for (int i = 0; i < S::kCols; ++i) {
+                const float xi = value_at<T>(x[it], i), f = __builtin_fmaf(xi, inv[i], 128.f);
+                word[i] = __builtin_amdgcn_cvt_pk_u8_f32(f, it, word[i]);
+                if (odd || __builtin_fabsf(__builtin_amdgcn_fractf(f) - 0.5f) < kNear) {
+                    const int t = quant_one(xi, s_all[c0 + i], nan_to, lo) + 128;
+                    word[i] = (word[i] & ~(0xffu << (8 * it))) | (uint32_t)t << (8 * it);
+                }
+            }
+        }
+        store(word, unit);
+    }
+}
+
+template <typename T, int WAVES, int UNITS>
+int launch_groups(const void *w, size_t K, size_t N, int parts, int ref128, int8_t *q, int8_t *packed, void *scale,
+                  uint32_t *counts, hipStream_t st)
+{
+    const size_t groups = (N + GroupShape<T>::kGroup - 1) / GroupShape<T>::kGroup, n = groups * kCountStride;
+    if (parts > 1) {
+        hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, counts, n);
+        EET_HIP_CHECK(hipGetLastError());
+    }
+    const auto kernel = q != nullptr ? quant_group_kernel<T, WAVES, UNITS, true> : quant_group_kernel<T, WAVES, UNITS, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(groups * parts)), dim3(64 * WAVES), 0, st, static_cast<const T *>(w), (int)K,
+                       (int)N, parts, ref128, counts + n, counts, q, reinterpret_cast<uint8_t *>(packed),
+                       static_cast<T *>(scale));
+    EET_HIP_CHECK(hipGetLastError());
+    return EET_OK;
+}
+
+// One pass or two.  fp32: always one (us, two passes / one: 4096 x 4096 31 / 23.5, 11008 x 4096 75 / 59, 5120 x 13696 120 /
+// 87, 16384 x 16384 472 / 286).  fp16 has twice the weights to a byte, so that the quantising of a workgroup's share, which
+// nothing overlaps where the grid fits the chip once, weighs more.  Up to 36 M weights one pass wins by its two launches
+// less (1024 x 1024 17.3 / 14.0, 4096 x 4096 24.3 / 20.1, 16384 x 1024 24.5 / 20.2, 6144 x 4096 30.1 / 27.7), from there the
+// registers of the chip no longer hold the matrix in one round, while the second pass of the other way is read from the
+// Infinity Cache (11008 x 4096 44.8 / 51.4, 4096 x 12288 47.1 / 52.4, 16384 x 4096 64.9 / 66.9); with more rounds, and
+// what does not fit that cache, one pass is ahead again (5120 x 13696 69.6 / 66.4, 16384 x 16384 268 / 219).
+bool one_pass_wins(size_t K, size_t N, size_t size)
+{
+    const size_t n = K * N;
+    return size == 4 || n <= 36000000 || n >= 70000000;
+}
+
+// How many workgroups share a column group: as many as its rows need, and as many as the chip still takes in one round.
+int parts_of(size_t units, size_t groups, int waves, int held, size_t slots)
+{
+    const size_t need = (units + waves * held - 1) / (waves * held), most = units / waves;
+    size_t parts = slots / groups < (size_t)kMaxParts ? slots / groups : (size_t)kMaxParts;
+    parts = parts < most ? parts : most;
+    return (int)(parts > need ? parts : need);
+}
+
+template <typename T>
+int run(const void *w, size_t K, size_t N, int mode, int8_t *q, int8_t *packed, void *scale, uint32_t *ws, size_t ws_bytes,
         hipStream_t st)
 {
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, amax, N);
+    const int ref128 = mode == EET_QUANT_REF128 ? 1 : 0;
+    if (ws_bytes >= eet_quantize_pack_device_workspace(N) && one_pass_wins(K, N, sizeof(T))) {
+        const size_t units = K / kUnit, groups = (N + GroupShape<T>::kGroup - 1) / GroupShape<T>::kGroup;
+        const int wide = parts_of(units, groups, 16, 4, 256), narrow = parts_of(units, groups, 8, 5, 512);
+        if (wide <= kMaxParts && groups * wide <= 256)
+            return launch_groups<T, 16, 4>(w, K, N, wide, ref128, q, packed, scale, ws, st);
+        if (narrow <= kMaxParts)
+            return launch_groups<T, 8, 5>(w, K, N, narrow, ref128, q, packed, scale, ws, st);
+    }
+    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, ws, N);
     EET_HIP_CHECK(hipGetLastError());
     const dim3 g1((unsigned)((N + 64 * kColsPerThread - 1) / (64 * kColsPerThread)),
                   (unsigned)((K + kMaxRows - 1) / kMaxRows));
-    hipLaunchKernelGGL(colmax_kernel<T>, g1, dim3(256), 0, st, static_cast<const T *>(w), K, N, amax);
+    hipLaunchKernelGGL(colmax_kernel<T>, g1, dim3(256), 0, st, static_cast<const T *>(w), K, N, ws);
     EET_HIP_CHECK(hipGetLastError());
     const dim3 g2((unsigned)((N + kTileCols - 1) / kTileCols), (unsigned)(K / 64));
-    hipLaunchKernelGGL(quant_pack_kernel<T>, g2, dim3(256), 0, st, static_cast<const T *>(w), K, N,
-                       mode == EET_QUANT_REF128 ? 1 : 0, amax, q, reinterpret_cast<uint8_t *>(packed),
-                       static_cast<T *>(scale));
+    hipLaunchKernelGGL(quant_pack_kernel<T>, g2, dim3(256), 0, st, static_cast<const T *>(w), K, N, ref128, ws, q,
+                       reinterpret_cast<uint8_t *>(packed), static_cast<T *>(scale));
     EET_HIP_CHECK(hipGetLastError());
     return EET_OK;
 }
 
 }  // namespace
 
-extern "C" size_t eet_quantize_pack_device_workspace(size_t N) { return N * sizeof(uint32_t); }
+// A count per group of columns and the column maxima of each part; the two passes use N words of it.
+extern "C" size_t eet_quantize_pack_device_workspace(size_t N) { return (N * kMaxParts + (N + 31) / 32 * (kCountStride + 32 * kMaxParts)) * sizeof(uint32_t); }
 
 extern "C" int eet_quantize_pack_device(const void *w, int w_dtype, size_t K, size_t N, int mode, int8_t *q,
                                         int8_t *packed, void *scale, void *workspace, size_t workspace_bytes,
@@ -249,6 +619,6 @@ extern "C" int eet_quantize_pack_device(const void *w, int w_dtype, size_t K, si
                 N * sizeof(uint32_t), workspace_bytes);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (w_dtype == EET_DTYPE_F32)
-        return run<float>(w, K, N, mode, q, packed, scale, static_cast<uint32_t *>(workspace), st);
-    return run<_Float16>(w, K, N, mode, q, packed, scale, static_cast<uint32_t *>(workspace), st);
+        return run<float>(w, K, N, mode, q, packed, scale, static_cast<uint32_t *>(workspace), workspace_bytes, st);
+    return run<_Float16>(w, K, N, mode, q, packed, scale, static_cast<uint32_t *>(workspace), workspace_bytes, st);
 }

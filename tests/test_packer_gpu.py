@@ -130,3 +130,28 @@ def test_converter_on_device(gpu):
                 assert dev[k].device.type == "cuda", k
         else:
             assert dev[k] == v
+
+
+@pytest.mark.parametrize("K,N", [(64, 16), (128, 80), (2048, 16), (2112, 48), (1280, 1040), (8256, 112), (32832, 32),
+                                 (2624, 16400)])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+def test_one_pass_matches_two_passes(gpu, K, N, dtype):
+    """The one-pass kernel at the edges of its shares (rows a workgroup holds, one to sixteen workgroups per column
+    group, groups cut off by N) and with NaN and infinite weights, against the two-pass kernels, which a call with no
+    more than 4 N bytes of workspace takes, and the host packer.  Exact: every step is one correctly rounded operation."""
+    from eet_amd._lib import check, lib
+    w = tricky(K, N, dtype, K * 3 + N)
+    w[K // 2, 8], w[K - 1, 9], w[:, 10], w[5, 11] = np.nan, np.inf, np.nan, np.nan
+    uh, ph, sh = eet_amd.quant_weights(torch.from_numpy(w), torch.int8, True)
+    wd = torch.from_numpy(w).to(gpu)
+    code = 0 if dtype == np.float32 else 1
+    for nbytes in (lib().eet_quantize_pack_device_workspace(N), 4 * N):
+        ws = torch.full((nbytes // 4,), -1, dtype=torch.int32, device=gpu)
+        for want_q in (True, False):
+            q, p = (torch.zeros(K, N, dtype=torch.int8, device=gpu) for _ in range(2))
+            s = torch.zeros(N, dtype=wd.dtype, device=gpu)
+            check(lib().eet_quantize_pack_device(wd.data_ptr(), code, K, N, 0, q.data_ptr() if want_q else None, p.data_ptr(),
+                                                 s.data_ptr(), ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream))
+            assert torch.equal(p.cpu(), ph)
+            assert not want_q or torch.equal(q.cpu(), uh)
+            assert torch.equal(s.cpu().view(torch.int16 if code else torch.int32), sh.view(torch.int16 if code else torch.int32))
