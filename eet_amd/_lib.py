@@ -52,6 +52,7 @@ SIGNATURES = {
     "eet_add_bias_residual_norm": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _f, _vp]),
     "eet_add_bias": (_i, [_vp, _vp, _i, _i, _vp]),
     "eet_qkv_split": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp]),
+    "eet_gemm_w8a16_qkv": (_i, [_vp] * 8 + [_i] * 6 + [_vp, _sz, _vp]),
     "eet_swiglu": (_i, [_vp, _vp, _i, _i, _vp]),
     "eet_residual_add": (_i, [_vp, _vp, _i, _i, _vp]),
     "eet_kv_cache_reorder": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),

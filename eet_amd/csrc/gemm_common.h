@@ -40,6 +40,16 @@ __device__ __forceinline__ half8 widen8(uint32_t x0, uint32_t x1)
 // Epilogues: plain; + residual[M][N] (fp16 add); SwiGLU over (gate, up) n-tile
 // pairs of an interleaved weight, output [M][N/2].
 constexpr int kEpiNone = 0, kEpiResidual = 1, kEpiSwiglu = 2;
+// The fused Q | K | V rows of a prompt, split on their way out (large-M kernel, its own entry point).
+constexpr int kEpiQkv = 3;
+
+// Row m = b * S + s, channel (part * H + h) * dh + d goes to q[b][h][s][d] of [B][H][S][dh] or to k / v[b][h][s][d] of
+// [B][H][T][dh]; with a table (cos | sin of position s) the pairs (d, d + dh / 2) of q and k are rotated.
+struct QkvOut {
+    _Float16 *q, *k, *v;
+    const float *rope;   // [>= S][dh] or null
+    int S, H, dh, T;
+};
 
 struct GemmArgs {
     const _Float16 *A;
@@ -54,12 +64,15 @@ struct GemmArgs {
     void *ws;  // optional fp32 workspace (split-k partial results)
     size_t ws_bytes;
     hipStream_t st;
+    QkvOut qkv = {};  // kEpiQkv
     int chain = 0;  // kChainOff / kChainFirst / kChainNext (chain.h; small-M kernel only)
 };
 
 // gemm_w8a16_large.hip: the MFMA-tile kernel for M > 32, and the workspace it can use.  kTakesSlabs, with nothing
 // launched, for a call that 32-row slabs of the small-M kernel run faster.
 constexpr int kTakesSlabs = 1;
+// kEpiQkv only: nothing launched, a plain launch and a split kernel are faster.
+constexpr int kSplitApart = 2;
 int run_large_m(const GemmArgs &a);
 size_t large_m_workspace(int M, int N, int K, int epi);
 

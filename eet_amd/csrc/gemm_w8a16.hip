@@ -1066,6 +1066,37 @@ extern "C" int eet_gemm_w8a16_fused(const void *A, const void *Wpacked, const vo
                       workspace, workspace_bytes, eet::kChainOff, stream);
 }
 
+extern "C" int eet_gemm_w8a16_qkv(const void *A, const void *Wpacked, const void *scale, void *qkv, void *q_out,
+                                  void *k_cache, void *v_cache, const float *rope_cos_sin, int B, int S, int H, int dh,
+                                  int K, int T_cap, void *workspace, size_t workspace_bytes, void *stream)
+{
+    const char *fn = "eet_gemm_w8a16_qkv";
+    EET_REQUIRE(qkv && q_out && k_cache && v_cache, EET_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
+    EET_REQUIRE(B >= 0 && S >= 0 && H > 0 && dh > 0 && (long)B * S <= INT32_MAX && 3l * H * dh <= INT32_MAX,
+                EET_ERR_INVALID_ARGUMENT, "%s: bad sizes B=%d S=%d H=%d dh=%d", fn, B, S, H, dh);
+    EET_REQUIRE(dh % 32 == 0, EET_ERR_UNSUPPORTED_SHAPE, "%s: head size %d must be a multiple of 32", fn, dh);
+    EET_REQUIRE(S <= T_cap, EET_ERR_INVALID_ARGUMENT, "%s: rows [0, %d) exceed the cache capacity %d", fn, S, T_cap);
+    const int M = B * S, N = 3 * H * dh;
+    if (int rc = check_gemm_args(fn, A, Wpacked, scale, qkv, M, N, K))
+        return rc;
+    if (M == 0)
+        return EET_OK;
+    GemmArgs args{static_cast<const _Float16 *>(A), static_cast<const u32x4 *>(Wpacked),
+                  static_cast<const _Float16 *>(scale), static_cast<_Float16 *>(qkv), M, N, K, nullptr, kEpiQkv, nullptr,
+                  0.f, workspace, workspace_bytes, static_cast<hipStream_t>(stream)};
+    args.qkv = {static_cast<_Float16 *>(q_out), static_cast<_Float16 *>(k_cache), static_cast<_Float16 *>(v_cache),
+                rope_cos_sin, S, H, dh, T_cap};
+    const bool pieces = (reinterpret_cast<uintptr_t>(q_out) | reinterpret_cast<uintptr_t>(k_cache) |
+                         reinterpret_cast<uintptr_t>(v_cache) | reinterpret_cast<uintptr_t>(rope_cos_sin)) % 16 == 0;
+    if (M > 32 && pieces)   // the epilogue loads and stores 16 bytes at a time
+        if (const int rc = eet::run_large_m(args); rc != eet::kSplitApart)
+            return rc;
+    args.epi = kEpiNone;
+    if (int rc = run_gemm(args))
+        return rc;
+    return eet_qkv_split(qkv, q_out, k_cache, v_cache, B, S, H, dh, rope_cos_sin != nullptr, -1, 0, T_cap, stream);
+}
+
 extern "C" int eet_gemm_w8a16_chained(const void *A, const void *Wpacked, const void *scale, void *C, int M, int N,
                                       int K, int epilogue, const void *residual, const void *rms_gamma, float rms_eps,
                                       int chain, void *stream)

@@ -64,11 +64,11 @@ struct TileShape {
     static_assert((D - 1) * (kA + kW) <= 63, "the copies in flight must fit the wait counter");
 };
 
-template <int TM, int TN, int WM, int WN, int D>
+template <int TM, int TN, int WM, int WN, int D, bool QKV>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2))) void w8a16_large_m_kernel(
     const _Float16 *__restrict__ A, const u32x4 *__restrict__ Wp, const _Float16 *__restrict__ scale,
     _Float16 *__restrict__ C, int M, int N, int K, int m_blocks, int n_blocks,
-    const _Float16 *__restrict__ residual, int epi, int ksplit, float *__restrict__ partial)
+    const _Float16 *__restrict__ residual, int epi, int ksplit, float *__restrict__ partial, QkvOut out)
 {
 #if defined(__HIP_DEVICE_COMPILE__)  // buffer-resource builtins exist in the device pass only
     using S = TileShape<TM, TN, WM, WN, D>;
@@ -101,6 +101,16 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
     const int n_blk = band * kBand + r % bw, m_blk = r / bw;
     const int m0 = m_blk * S::kBM;
     const int ntb = n_blk * (WN * TN), nt0 = ntb + wn * TN;
+    // The n-tile of slot u of the block.  A block of fused Q | K | V channels is made of pairs of n-tiles half a head apart,
+    // which the rotation turns into one another, whatever its width: slots 2 p and 2 p + 1 hold pair n_blk * kPairs + p.
+    constexpr int kPairs = WN * TN / 2;
+    const int hh = QKV ? out.dh >> 5 : 1;   // pairs in a head
+    auto ntile = [&](int u) {
+        if constexpr (!QKV)
+            return ntb + u;
+        const int pair = n_blk * kPairs + (u >> 1), head = pair / hh;
+        return head * 2 * hh + (pair - head * hh) + (u & 1) * hh;
+    };
     const int rows = min(M - m0, S::kBM);
 
     // Both operands are addressed through buffer resources: a 32-bit lane offset plus a scalar offset per tile.
@@ -116,7 +126,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
     unsigned wtile[S::kW];  // byte offset of the n-tile's first k-tile
 #pragma unroll
     for (int i = 0; i < S::kW; ++i)
-        wtile[i] = (unsigned)min(ntb + wunit(i), ntiles - 1) * (unsigned)ktiles * 1024u;
+        wtile[i] = (unsigned)min(ntile(wunit(i)), ntiles - 1) * (unsigned)ktiles * 1024u;
     // Copy rg of the activations fills slots [64 rg, 64 rg + 64): block u = rg / 4, super-rows 4 (rg % 4) .. + 3.
     // Lane l writes slot s = l % 16 of super-row sj = 4 (rg % 4) + l / 16, which holds piece 2 pg + h of row sj of
     // m-tile 2u + e, where 4 (2e + h) + pg = s ^ sj.
@@ -260,6 +270,59 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
 
     // acc[t][mt][r] of lane (g, j): row mrow0 + 16*mt, channel 16*(nt0+t) + 4*g + r
     const int mrow0 = m0 + wm * TM * 16 + j;
+    if constexpr (QKV) {
+        // The block goes through LDS as fp16 -- the value that the plain epilogue stores -- and leaves in 16-byte pieces of
+        // rows: a lane takes 8 channels and their partners half a head on, turns them in fp32 and rounds again, as the split
+        // kernel does.  (Straight from the accumulators, 8 bytes a lane and their angles a row apart, it took 58 us instead
+        // of the plain 51 for 2000 rows, 6144 <- 2048.)  A row's 16-byte pieces are XORed by the row against bank conflicts.
+        constexpr int kPieces = S::kBN / 8;
+        static_assert(S::kBM * kPieces <= D * (S::kAVec + S::kWVec), "the block must fit the stage ring");
+        u32x4 *tile_lds = &lds[0][0];
+        auto piece_at = [&](int row, int piece) { return row * kPieces + (piece ^ (row & 7)); };
+        __syncthreads();   // every wavefront has read its last operands, every copy has landed
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+            const int u = wn * TN + t;
+            const half4 sc = *reinterpret_cast<const half4 *>(scale + min(ntile(u), ntiles - 1) * 16 + 4 * g);
+#pragma unroll
+            for (int mt = 0; mt < TM; ++mt) {
+                half4 o;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    o[r] = (_Float16)(acc[t][mt][r] * (float)sc[r]);
+                const int row = (wm * TM + mt) * 16 + j;
+                reinterpret_cast<u32x2 *>(tile_lds + piece_at(row, 2 * u + (g >> 1)))[g & 1] = __builtin_bit_cast(u32x2, o);
+            }
+        }
+        __syncthreads();
+        // piece q of a row: 8 channels of the first tile of pair q / 2
+        constexpr int kTasks = S::kBM * kPairs * 2, kThreads = 64 * S::kWaves;
+#pragma unroll 2
+        for (int task = tid; task < kTasks; task += kThreads) {
+            const int row = task / (kPairs * 2), q = task % (kPairs * 2), m = m0 + row;
+            const int pair = n_blk * kPairs + (q >> 1), head = pair / hh, part = head / out.H, h = head - part * out.H;
+            if (m >= M || part > 2)
+                continue;
+            const int b = m / out.S, pos = m - b * out.S, d = (pair - head * hh) * 16 + (q & 1) * 8, half = 16 * hh;
+            half8 x = __builtin_bit_cast(half8, tile_lds[piece_at(row, 4 * (q >> 1) + (q & 1))]);
+            half8 y = __builtin_bit_cast(half8, tile_lds[piece_at(row, 4 * (q >> 1) + 2 + (q & 1))]);
+            if (out.rope != nullptr && part < 2) {
+                const floatx4 *c = reinterpret_cast<const floatx4 *>(out.rope + (size_t)pos * out.dh + d);
+                const floatx4 *sn = reinterpret_cast<const floatx4 *>(out.rope + (size_t)pos * out.dh + d + half);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float a = (float)x[e], o = (float)y[e];
+                    x[e] = (_Float16)__builtin_fmaf(a, c[e / 4][e % 4], -(o * sn[e / 4][e % 4]));
+                    y[e] = (_Float16)__builtin_fmaf(o, c[e / 4][e % 4], a * sn[e / 4][e % 4]);
+                }
+            }
+            _Float16 *dst = (part == 0 ? out.q : part == 1 ? out.k : out.v) +
+                            (((size_t)b * out.H + h) * (part == 0 ? out.S : out.T) + pos) * out.dh + d;
+            *reinterpret_cast<half8 *>(dst) = x;
+            *reinterpret_cast<half8 *>(dst + half) = y;
+        }
+        return;
+    }
     if (ksplit > 1) {
 #pragma unroll
         for (int t = 0; t < TN; ++t) {
@@ -394,8 +457,9 @@ int launch_large_m(const GemmArgs &a, int ksplit)
     const int m_blocks = (a.M + S::kBM - 1) / S::kBM, n_blocks = (a.N + S::kBN - 1) / S::kBN;
     const int grid = ((m_blocks * n_blocks + 7) / 8) * 8;
     float *partial = ksplit > 1 ? static_cast<float *>(a.ws) : nullptr;
-    hipLaunchKernelGGL((w8a16_large_m_kernel<TM, TN, WM, WN, D>), dim3(grid, ksplit), dim3(64 * S::kWaves), 0, a.st, a.A,
-                       a.Wp, a.scale, a.C, a.M, a.N, a.K, m_blocks, n_blocks, a.residual, a.epi, ksplit, partial);
+    const auto kernel = a.epi == kEpiQkv ? w8a16_large_m_kernel<TM, TN, WM, WN, D, true> : w8a16_large_m_kernel<TM, TN, WM, WN, D, false>;
+    hipLaunchKernelGGL(kernel, dim3(grid, ksplit), dim3(64 * S::kWaves), 0, a.st, a.A, a.Wp, a.scale, a.C, a.M, a.N, a.K,
+                       m_blocks, n_blocks, a.residual, a.epi, ksplit, partial, a.qkv);
     EET_HIP_CHECK(hipGetLastError());
     if (ksplit > 1) {
         const int items = a.M * ((a.epi == kEpiSwiglu ? a.N / 2 : a.N) / 4);
@@ -514,6 +578,10 @@ bool slabs_win(int M, int N, int K, int epi)
     return K >= 3072 && N <= 4096 && (M <= 48 || (N <= 2048 && K >= 6144));
 }
 
+// What the split of the fused Q | K | V rows costs as a kernel of its own: 5.0 us at 45 rows of 12288 channels, 6.5 at 406,
+// 10.5 at 2000 rows of 6144, 69 at 8192 of 12288.
+float qkv_split_us(int M, int N) { return 4.f + (float)M * N * 4.f / 6e6f; }
+
 // What a call runs as (some block shape always does: the unsplit estimates are finite); tile < 0: 32-row slabs of the
 // small-M kernel.
 LargeMConfig plan_large_m(int M, int N, int K, int epi, size_t ws_bytes)
@@ -572,9 +640,16 @@ int eet::run_large_m(const GemmArgs &a)
         return eet::fail(EET_ERR_UNSUPPORTED_SHAPE, "eet_gemm_w8a16: K x N = %d x %d exceeds the 2 GiB weight limit",
                          a.K, a.N);
     const size_t ws_bytes = a.ws != nullptr && reinterpret_cast<uintptr_t>(a.ws) % 16 == 0 ? a.ws_bytes : 0;
-    const LargeMConfig c = plan_large_m(a.M, a.N, a.K, a.epi, ws_bytes);
+    LargeMConfig c = plan_large_m(a.M, a.N, a.K, a.epi, ws_bytes);
     if (c.tile < 0)
-        return kTakesSlabs;
+        return a.epi == kEpiQkv ? kSplitApart : kTakesSlabs;
+    if (a.epi == kEpiQkv && c.ksplit > 1) {
+        // the epilogue takes whole sums: a split of the k range has to save more than the split kernel costs
+        const LargeMConfig whole = plan_large_m(a.M, a.N, a.K, a.epi, 0);
+        if (whole.tile < 0 || whole.ksplit > 1 || c.us + qkv_split_us(a.M, a.N) < whole.us)
+            return kSplitApart;
+        c = whole;
+    }
     using Launcher = int (*)(const GemmArgs &, int);
     // in the order of kTiles; the last number is the depth of the stage ring, as deep as two workgroups of four
     // wavefronts (or one of eight) leave room for in the LDS

@@ -652,14 +652,24 @@ class _MmhaInt8:
             # RMSnorm folded into the GEMM's activation load
             _gemm(x, self.qkv_w, self.qkv_s, qkv, M, 3 * self.inner, hidden, EPI_NONE, None, self.gamma,
                   desc.layernorm_eps)
+        elif first_pass:
+            # the projection splits its rows (+ rotary at position s) into q and K, V rows [0, S) of the cache
+            _rmsnorm(x, self.gamma, xn, M, hidden, desc.layernorm_eps)
+            ws, ws_bytes = None, L.eet_gemm_w8a16_workspace(M, 3 * self.inner, hidden, EPI_NONE)
+            if ws_bytes:
+                ws = workspaces.get("gemm_split_k", ws_bytes // 4, torch.float32, dev).data_ptr()
+            check(L.eet_gemm_w8a16_qkv(xn.data_ptr(), self.qkv_w.data_ptr(), self.qkv_s.data_ptr(), qkv.data_ptr(),
+                                       qbuf.data_ptr(), self._k.data_ptr(), self._v.data_ptr(),
+                                       self.rope_table.data_ptr() if self._rope else None, B, S, H, dh, hidden,
+                                       self.t_cap, ws, ws_bytes, _stream()), "eet_gemm_w8a16_qkv")
         else:
             _rmsnorm(x, self.gamma, xn, M, hidden, desc.layernorm_eps)
             _gemm(xn, self.qkv_w, self.qkv_s, qkv, M, 3 * self.inner, hidden)
         if first_pass:
-            # split (+ rotary at position s) and write K, V rows [0, S) of the cache
-            check(L.eet_qkv_split(qkv.data_ptr(), qbuf.data_ptr(), self._k.data_ptr(),
-                                  self._v.data_ptr(), B, S, H, dh, 1 if self._rope else 0, -1, 0, self.t_cap,
-                                  _stream()), "eet_qkv_split")
+            if self.with_bias or M <= RMS_FUSE_MAX_M:
+                # split (+ rotary at position s) and write K, V rows [0, S) of the cache
+                check(L.eet_qkv_split(qkv.data_ptr(), qbuf.data_ptr(), self._k.data_ptr(), self._v.data_ptr(), B, S, H,
+                                      dh, 1 if self._rope else 0, -1, 0, self.t_cap, _stream()), "eet_qkv_split")
             alibi = None
             if bias is not None:
                 # [H, S, S] mask whose row i holds slope*j for j <= i: its last row is the whole table

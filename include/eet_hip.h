@@ -327,6 +327,17 @@ int eet_add_bias(void *out, const void *bias, int M, int N, void *stream);
 int eet_qkv_split(const void *qkv, void *q_out, void *k_cache, void *v_cache, int B, int S,
                   int H, int dh, int rope, int time_step, int t0, int T_cap, void *stream);
 
+/* A prompt's QKV projection and eet_qkv_split (time_step -1, t0 0) of its rows in one
+ * call: A[B*S][K], Wpacked / scale of [K][3*H*dh], rotary when rope_cos_sin (the table of
+ * eet_rope_table, at least S rows) is given.  More than 32 rows are split in the
+ * epilogue of the product where that is faster (and q, k, v and the table are 16-byte
+ * aligned); qkv is the [B*S][3*H*dh] buffer of the other calls, its contents undefined
+ * afterwards.  dh % 32 == 0; workspace as for eet_gemm_w8a16 with EET_EPILOGUE_NONE. */
+int eet_gemm_w8a16_qkv(const void *A, const void *Wpacked, const void *scale, void *qkv,
+                       void *q_out, void *k_cache, void *v_cache, const float *rope_cos_sin,
+                       int B, int S, int H, int dh, int K, int T_cap, void *workspace,
+                       size_t workspace_bytes, void *stream);
+
 /* gate[M][N] = up * gate / (1 + exp(-gate)).  Replaces gated_act_kernel, silu
  * (csrc/core/activation_kernel.cu:275-338). */
 int eet_swiglu(void *gate, const void *up, int M, int N, void *stream);

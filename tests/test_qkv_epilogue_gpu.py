@@ -1,0 +1,78 @@
+"""eet_gemm_w8a16_qkv: the split of a prompt's fused Q | K | V rows in the epilogue of the large-M product, for every block
+shape, against the product and eet_qkv_split as two calls on the same block shape.  The epilogue rounds to fp16 where the
+product stores and rotates that value in fp32 as the split kernel does.  A product or a rotation may be rounded to fp16
+directly or by way of fp32 (one instruction or two, as the compiler likes): the same but for one in some 2^12 values,
+and there both inputs of a rotation and its result are at most one unit of fp16 off, each 2^-10 of the pair's length at
+most and 2^-11 in the mean of the numbers between two powers of two: bound 2^-9."""
+import pytest
+import torch
+
+import eet_amd
+from eet_amd._lib import check, lib
+
+from gpu_util import gemm, stream
+from test_large_m_blocks_gpu import BLOCKS
+
+pytestmark = pytest.mark.gpu
+GUARD = 7.25
+
+
+def both(gpu, B, S, H, dh, K, T, rope, ws_bytes=0):
+    N, M = 3 * H * dh, B * S
+    g = torch.Generator().manual_seed(M + N)
+    w = (torch.randn(K, N, generator=g) * 0.02).half()
+    p, s = (t.to(gpu) for t in eet_amd.quant_weights(w, torch.int8))
+    x = torch.randn(M, K, generator=g).half().to(gpu)
+    table = eet_amd.ops._rope_table(T, dh, gpu) if rope else None
+    ws = torch.zeros(max(ws_bytes, 4) // 4, dtype=torch.float32, device=gpu)
+
+    def buffers():
+        return [torch.full(shape, GUARD, dtype=torch.float16, device=gpu) for shape in
+                ((B, H, S, dh), (B, H, T, dh), (B, H, T, dh))]
+    want, got, qkv = buffers(), buffers(), torch.empty(M, N, dtype=torch.float16, device=gpu)
+    rows = gemm(x, p, s, M, N, K)
+    check(lib().eet_qkv_split(rows.data_ptr(), *(t.data_ptr() for t in want), B, S, H, dh, int(rope), -1, 0, T, stream()))
+    check(lib().eet_gemm_w8a16_qkv(x.data_ptr(), p.data_ptr(), s.data_ptr(), qkv.data_ptr(), *(t.data_ptr() for t in got),
+                                   table.data_ptr() if rope else None, B, S, H, dh, K, T, ws.data_ptr() if ws_bytes else None,
+                                   ws_bytes, stream()))
+    return want, got
+
+
+@pytest.mark.parametrize("block", BLOCKS, ids=lambda b: "x".join(map(str, b)))
+def test_every_block(gpu, tuning, block):
+    """Heads that end inside a block and inside a wavefront's share, ragged rows over several sequences; cache rows
+    behind the prompt keep their value."""
+    tm, tn, wm, wn = block
+    tuning("EET_GEMM_LARGE_M_TILE", f"{tm},{tn},1,{wm},{wn}")
+    for B, S, H, dh in ((3, 37, 5, 128), (1, 16 * tm * wm + 1, 3, 64), (2, 100, 3, 96), (5, 9, 7, 32)):
+        for rope in (True, False):
+            want, got = both(gpu, B, S, H, dh, 320, S + 3, rope)
+            for name, a, b in zip("qkv", want, got):
+                what = f"{block} B {B} S {S} H {H} dh {dh} rope {rope}: {name}"
+                if rope and name != "v":
+                    d = (a.float() - b.float()).abs()
+                    pair = a.float().unflatten(-1, (2, dh // 2)).norm(dim=-2).repeat(1, 1, 1, 2)
+                    assert (d <= pair * 2 ** -9).all(), what
+                    assert int((d != 0).sum()) <= 4 + a.numel() // 1000, what
+                else:
+                    assert torch.equal(a, b), what
+
+
+@pytest.mark.parametrize("B,S,H,dh,K", [(1, 20, 4, 128, 512), (1, 45, 2, 128, 4096), (1, 64, 32, 128, 1024), (1, 33, 4, 32, 8192)])
+def test_as_the_library_chooses(gpu, B, S, H, dh, K):
+    """Few rows, and sizes at which a split of the k range or slabs of rows may be taken: within the rounding of fp32 sums
+    in another order (K * 2^-24 of the summed magnitudes, here below 2^-9) and two fp16 roundings of values below 8."""
+    N = 3 * H * dh
+    for ws in (0, lib().eet_gemm_w8a16_workspace(B * S, N, K, 0)):
+        want, got = both(gpu, B, S, H, dh, K, S, True, ws)
+        for a, b in zip(want, got):
+            assert float(a.float().abs().max()) < 8
+            assert float((a.float() - b.float()).abs().max()) <= 2 ** -9 + 3 * 2 ** -9
+
+
+def test_refused(gpu):
+    x = torch.zeros(1 << 16, dtype=torch.float16, device=gpu).data_ptr()
+    L = lib()
+    assert L.eet_gemm_w8a16_qkv(x, x, x, x, x, x, x, None, 1, 40, 1, 48, 64, 64, None, 0, None) != 0      # head size
+    assert L.eet_gemm_w8a16_qkv(x, x, x, x, x, x, x, None, 1, 40, 1, 32, 64, 39, None, 0, None) != 0      # cache rows
+    assert L.eet_gemm_w8a16_qkv(x, x, x, x, None, x, x, None, 1, 40, 1, 32, 64, 64, None, 0, None) != 0   # null
