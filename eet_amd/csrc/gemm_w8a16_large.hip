@@ -100,7 +100,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
     const int bw = min(kBand, n_blocks - band * kBand);   // column blocks of this band (the last one may be narrower)
     const int n_blk = band * kBand + r % bw, m_blk = r / bw;
     const int m0 = m_blk * S::kBM;
-    const int ntb = n_blk * (WN * TN), nt0 = ntb + wn * TN;
+    const int ntb = n_blk * (WN * TN);
     // The n-tile of slot u of the block.  A block of fused Q | K | V channels is made of pairs of n-tiles half a head apart,
     // which the rotation turns into one another, whatever its width: slots 2 p and 2 p + 1 hold pair n_blk * kPairs + p.
     constexpr int kPairs = WN * TN / 2;
@@ -268,35 +268,110 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
             tile_step(std::integral_constant<int, 3 % D>{}, std::false_type{}, 0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no copy may land in LDS after the workgroup has gone
 
-    // acc[t][mt][r] of lane (g, j): row mrow0 + 16*mt, channel 16*(nt0+t) + 4*g + r
-    const int mrow0 = m0 + wm * TM * 16 + j;
-    if constexpr (QKV) {
-        // The block goes through LDS as fp16 -- the value that the plain epilogue stores -- and leaves in 16-byte pieces of
-        // rows: a lane takes 8 channels and their partners half a head on, turns them in fp32 and rounds again, as the split
-        // kernel does.  (Straight from the accumulators, 8 bytes a lane and their angles a row apart, it took 58 us instead
-        // of the plain 51 for 2000 rows, 6144 <- 2048.)  A row's 16-byte pieces are XORed by the row against bank conflicts.
-        constexpr int kPieces = S::kBN / 8;
-        static_assert(S::kBM * kPieces <= D * (S::kAVec + S::kWVec), "the block must fit the stage ring");
-        u32x4 *tile_lds = &lds[0][0];
-        auto piece_at = [&](int row, int piece) { return row * kPieces + (piece ^ (row & 7)); };
-        __syncthreads();   // every wavefront has read its last operands, every copy has landed
+    // acc[t][mt][r] of lane (g, j): row 16 * (wm * TM + mt) + j of the block, channel 4 * g + r of the n-tile of slot wn * TN + t
+    if (!QKV && ksplit > 1) {
+        const int mrow0 = m0 + wm * TM * 16 + j, nt0 = ntb + wn * TN;
 #pragma unroll
         for (int t = 0; t < TN; ++t) {
-            const int u = wn * TN + t;
-            const half4 sc = *reinterpret_cast<const half4 *>(scale + min(ntile(u), ntiles - 1) * 16 + 4 * g);
+            if (nt0 + t >= ntiles)
+                continue;
 #pragma unroll
             for (int mt = 0; mt < TM; ++mt) {
-                half4 o;
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    o[r] = (_Float16)(acc[t][mt][r] * (float)sc[r]);
-                const int row = (wm * TM + mt) * 16 + j;
-                reinterpret_cast<u32x2 *>(tile_lds + piece_at(row, 2 * u + (g >> 1)))[g & 1] = __builtin_bit_cast(u32x2, o);
+                const int m = mrow0 + 16 * mt;
+                if (m < M)
+                    *reinterpret_cast<floatx4 *>(partial + ((size_t)split * M + m) * N + (nt0 + t) * 16 + 4 * g) =
+                        acc[t][mt];
             }
         }
-        __syncthreads();
+        return;
+    }
+    // Stores.  The block goes through LDS as fp16 and leaves in 16-byte pieces of rows.  Straight from the accumulators it
+    // left in 8 bytes a lane, 32 bytes of a row at a time, and the residual came in the same way (us, then / now: 2000 rows
+    // 2048 <- 2048 with residual 25.2 / 21.8, 5120 <- 5120 93.9 / 88.3; 406 rows 4096 <- 4096 25.1 / 22.9; plain 12288 <- 4096 at
+    // 406, 2048 and 8192 rows 50.2 / 47.7, 162 / 158, 617 / 604; SwiGLU, half the bytes and bound by its exponentials, equal;
+    // over 12 matrices 0.96 of the time from 400 rows on, 0.99 below).  A row's pieces are XORed with the row against
+    // bank conflicts.
+    constexpr int kPieces = S::kBN / 8, kThreads = 64 * S::kWaves;
+    static_assert(S::kBM * kPieces <= D * (S::kAVec + S::kWVec), "the block must fit the stage ring");
+    static_assert(kPieces % (TN % 2 == 0 ? 16 : 8) == 0, "the XOR stays in the row");
+    u32x4 *tile_lds = &lds[0][0];
+    auto piece_at = [&](int pieces, int row, int piece) { return row * pieces + (piece ^ (row & 7)); };
+    // this lane's 4 channels of row 16 * (wm * TM + mt) + j, in the block's n-tile u
+    auto stage = [&](int pieces, int mt, int u, half4 o) {
+        const int at = piece_at(pieces, (wm * TM + mt) * 16 + j, 2 * u + (g >> 1));
+        reinterpret_cast<u32x2 *>(tile_lds + at)[g & 1] = __builtin_bit_cast(u32x2, o);
+    };
+    half4 sc[TN];
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+        sc[t] = *reinterpret_cast<const half4 *>(scale + min(ntile(wn * TN + t), ntiles - 1) * 16 + 4 * g);
+    __syncthreads();   // every wavefront has read its last operands, every copy has landed
+    // pieces [0, n) of the block's rows: a thread takes n / kThreads of them, rows past M and columns past `cols` stay out
+    const int cols = epi == kEpiSwiglu ? N / 2 : N, col0 = epi == kEpiSwiglu ? ntb * 8 : ntb * 16;
+    auto leave = [&](auto pieces_c, auto &&piece) {
+        constexpr int kRow = decltype(pieces_c)::value, kMine = S::kBM * kRow / kThreads;
+        static_assert(S::kBM * kRow % kThreads == 0, "whole pieces");
+#pragma unroll
+        for (int i = 0; i < kMine; ++i) {
+            const int task = tid + i * kThreads, row = task / kRow, col = col0 + task % kRow * 8;
+            const half8 o = piece(i, __builtin_bit_cast(half8, tile_lds[piece_at(kRow, row, task % kRow)]));
+            if (row < rows && col < cols)
+                __builtin_memcpy(__builtin_assume_aligned(C + (size_t)(m0 + row) * cols + col, 8), &o, 16);
+        }
+    };
+    if constexpr (!QKV && TN % 2 == 0) {
+        if (epi == kEpiSwiglu) {
+#pragma unroll
+            for (int t = 0; t < TN; t += 2)
+#pragma unroll
+                for (int mt = 0; mt < TM; ++mt) {
+                    half4 o;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float gate = (float)(_Float16)(acc[t][mt][r] * (float)sc[t][r]);
+                        const float up = (float)(_Float16)(acc[t + 1][mt][r] * (float)sc[t + 1][r]);
+                        o[r] = (_Float16)(up * gate / (1.0f + __expf(-gate)));
+                    }
+                    stage(kPieces / 2, mt, (wn * TN + t) / 2, o);
+                }
+            __syncthreads();
+            leave(std::integral_constant<int, kPieces / 2>{}, [](int, half8 o) { return o; });
+            return;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int mt = 0; mt < TM; ++mt) {
+            half4 o;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                o[r] = (_Float16)(acc[t][mt][r] * (float)sc[t][r]);
+            stage(kPieces, mt, wn * TN + t, o);
+        }
+    if constexpr (!QKV) {
+        if (epi == kEpiResidual) {
+            // all of the thread's residual pieces are on their way before the first store (loads wait for stores before them);
+            // pieces outside read the nearest one inside
+            half8 res[TM * TN / 2];
+#pragma unroll
+            for (int i = 0; i < TM * TN / 2; ++i) {
+                const int task = tid + i * kThreads, row = task / kPieces, col = col0 + task % kPieces * 8;
+                __builtin_memcpy(&res[i], __builtin_assume_aligned(residual + (size_t)(m0 + min(row, rows - 1)) * N +
+                                                                       min(col, N - 8), 8), 16);
+            }
+            __syncthreads();
+            leave(std::integral_constant<int, kPieces>{}, [&](int i, half8 o) { return o + res[i]; });
+            return;
+        }
+    }
+    __syncthreads();
+    if constexpr (QKV) {
+        // A lane takes 8 channels and their partners half a head on, turns them in fp32 and rounds again, as the split kernel
+        // does.  (From the accumulators, with the angles of each lane's rows, this took 58 us instead of the plain 51 for
+        // 2000 rows, 6144 <- 2048.)
         // piece q of a row: 8 channels of the first tile of pair q / 2
-        constexpr int kTasks = S::kBM * kPairs * 2, kThreads = 64 * S::kWaves;
+        constexpr int kTasks = S::kBM * kPairs * 2;
 #pragma unroll 2
         for (int task = tid; task < kTasks; task += kThreads) {
             const int row = task / (kPairs * 2), q = task % (kPairs * 2), m = m0 + row;
@@ -304,8 +379,8 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
             if (m >= M || part > 2)
                 continue;
             const int b = m / out.S, pos = m - b * out.S, d = (pair - head * hh) * 16 + (q & 1) * 8, half = 16 * hh;
-            half8 x = __builtin_bit_cast(half8, tile_lds[piece_at(row, 4 * (q >> 1) + (q & 1))]);
-            half8 y = __builtin_bit_cast(half8, tile_lds[piece_at(row, 4 * (q >> 1) + 2 + (q & 1))]);
+            half8 x = __builtin_bit_cast(half8, tile_lds[piece_at(kPieces, row, 4 * (q >> 1) + (q & 1))]);
+            half8 y = __builtin_bit_cast(half8, tile_lds[piece_at(kPieces, row, 4 * (q >> 1) + 2 + (q & 1))]);
             if (out.rope != nullptr && part < 2) {
                 const floatx4 *c = reinterpret_cast<const floatx4 *>(out.rope + (size_t)pos * out.dh + d);
                 const floatx4 *sn = reinterpret_cast<const floatx4 *>(out.rope + (size_t)pos * out.dh + d + half);
@@ -321,87 +396,8 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
             *reinterpret_cast<half8 *>(dst) = x;
             *reinterpret_cast<half8 *>(dst + half) = y;
         }
-        return;
-    }
-    if (ksplit > 1) {
-#pragma unroll
-        for (int t = 0; t < TN; ++t) {
-            if (nt0 + t >= ntiles)
-                continue;
-#pragma unroll
-            for (int mt = 0; mt < TM; ++mt) {
-                const int m = mrow0 + 16 * mt;
-                if (m < M)
-                    *reinterpret_cast<floatx4 *>(partial + ((size_t)split * M + m) * N + (nt0 + t) * 16 + 4 * g) =
-                        acc[t][mt];
-            }
-        }
-        return;
-    }
-    // Stores.  Each goes through a buffer resource that ends with the block's last row (the lane's offset is past it
-    // exactly if the row is), so that no lane branches on its row.
-    const int cols = epi == kEpiSwiglu ? N / 2 : N;
-    auto rsrc_of = [&](const _Float16 *base, int mt) {
-        const int r0 = wm * TM * 16 + 16 * mt;
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(base + (size_t)(m0 + r0) * cols), 0,
-                                                 (unsigned)max(min(rows - r0, 16), 0) * (unsigned)cols * 2u,
-                                                 0x00020000);
-    };
-    half4 sc[TN];
-#pragma unroll
-    for (int t = 0; t < TN; ++t)
-        sc[t] = *reinterpret_cast<const half4 *>(scale + min(nt0 + t, ntiles - 1) * 16 + 4 * g);
-    if (epi == kEpiSwiglu) {
-        if constexpr (TN % 2 == 0) {
-            const int coff = j * cols * 2 + nt0 * 16 + g * 8;
-#pragma unroll
-            for (int mt = 0; mt < TM; ++mt) {
-                const __amdgpu_buffer_rsrc_t cr = rsrc_of(C, mt);
-#pragma unroll
-                for (int t = 0; t < TN; t += 2) {
-                    half4 o;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float gate = (float)(_Float16)(acc[t][mt][r] * (float)sc[t][r]);
-                        const float up = (float)(_Float16)(acc[t + 1][mt][r] * (float)sc[t + 1][r]);
-                        o[r] = (_Float16)(up * gate / (1.0f + __expf(-gate)));
-                    }
-                    if (nt0 + t + 1 < ntiles)
-                        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, o), cr, coff + t * 16, 0, 0);
-                }
-            }
-        }
-        return;
-    }
-    // The residual of an m-tile is fetched whole, one m-tile ahead (a load under a branch of its own would be waited
-    // for before the next is issued).
-    const int coff = j * N * 2 + nt0 * 32 + g * 8;
-    u32x2 res[2][TN];
-    auto fetch = [&](int mt) {
-        const __amdgpu_buffer_rsrc_t rr = rsrc_of(residual, mt);
-#pragma unroll
-        for (int t = 0; t < TN; ++t)
-            res[mt & 1][t] = __builtin_bit_cast(
-                u32x2, __builtin_amdgcn_raw_buffer_load_b64(rr, coff + t * 32, 0, 0));
-    };
-    if (epi == kEpiResidual)
-        fetch(0);
-#pragma unroll
-    for (int mt = 0; mt < TM; ++mt) {
-        if (epi == kEpiResidual && mt + 1 < TM)
-            fetch(mt + 1);
-        const __amdgpu_buffer_rsrc_t cr = rsrc_of(C, mt);
-#pragma unroll
-        for (int t = 0; t < TN; ++t) {
-            half4 o;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                o[r] = (_Float16)(acc[t][mt][r] * (float)sc[t][r]);
-            if (epi == kEpiResidual)
-                o = o + __builtin_bit_cast(half4, res[mt & 1][t]);
-            if (nt0 + t < ntiles)
-                __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, o), cr, coff + t * 32, 0, 0);
-        }
+    } else {
+        leave(std::integral_constant<int, kPieces>{}, [](int, half8 o) { return o; });
     }
 #endif
 }

@@ -49,13 +49,13 @@ def test_every_block(gpu, tuning, block):
             want, got = both(gpu, B, S, H, dh, 320, S + 3, rope)
             for name, a, b in zip("qkv", want, got):
                 what = f"{block} B {B} S {S} H {H} dh {dh} rope {rope}: {name}"
+                d = (a.float() - b.float()).abs()
+                assert int((d != 0).sum()) <= 4 + a.numel() // 1000, what
                 if rope and name != "v":
-                    d = (a.float() - b.float()).abs()
                     pair = a.float().unflatten(-1, (2, dh // 2)).norm(dim=-2).repeat(1, 1, 1, 2)
                     assert (d <= pair * 2 ** -9).all(), what
-                    assert int((d != 0).sum()) <= 4 + a.numel() // 1000, what
                 else:
-                    assert torch.equal(a, b), what
+                    assert (d <= a.float().abs() * 2 ** -10).all(), what
 
 
 @pytest.mark.parametrize("B,S,H,dh,K", [(1, 20, 4, 128, 512), (1, 45, 2, 128, 4096), (1, 64, 32, 128, 1024), (1, 33, 4, 32, 8192)])
