@@ -126,6 +126,30 @@ extern "C" int eet_gated_ffn_int8_decode(const void *x, const void *rms_gamma, f
                                 nullptr, 0.f, gemm_workspace, gemm_workspace_bytes, stream);
 }
 
+// The layers of a decoder one after another: what the two calls above launch for each, from one foreign-function call.
+extern "C" int eet_decoder_int8_decode(const eet_decoder_layer *layers, int num_layers, const void *x, const void *alibi,
+                                       const int64_t *pad, const float *rope_cos_sin, void *qkv_buf, void *ctx_buf,
+                                       void *attn_out, void *act_buf, void *out, int B, int H, int dh, int hidden, int d_ff,
+                                       float rms_eps, int step, int T_cap, void *workspace, size_t workspace_bytes,
+                                       void *o_workspace, size_t o_workspace_bytes, void *down_workspace,
+                                       size_t down_workspace_bytes, void *stream)
+{
+    EET_REQUIRE(layers && num_layers > 0, EET_ERR_INVALID_ARGUMENT, "eet_decoder_int8_decode: no layers");
+    for (int i = 0; i < num_layers; ++i) {
+        const eet_decoder_layer &l = layers[i];
+        if (int rc = mmha_int8_decode("eet_decoder_int8_decode", x, l.attn_gamma, rms_eps, l.qkv_w, l.qkv_scale, l.o_w,
+                                      l.o_scale, l.k_cache, l.v_cache, alibi, pad, rope_cos_sin, qkv_buf, ctx_buf, attn_out,
+                                      B, H, dh, hidden, step, T_cap, workspace, workspace_bytes, o_workspace,
+                                      o_workspace_bytes, nullptr, nullptr, nullptr, stream))
+            return rc;
+        if (int rc = eet_gated_ffn_int8_decode(attn_out, l.ffn_gamma, rms_eps, l.w01, l.scale01, l.w2, l.scale2, act_buf, out,
+                                               B, hidden, d_ff, 1, down_workspace, down_workspace_bytes, stream))
+            return rc;
+        x = out;
+    }
+    return EET_OK;
+}
+
 // The same incremental call in its replayable form (see eet_mmha_decode_replayable): recorded once
 // into a HIP graph, it serves every later token.
 extern "C" int eet_mmha_int8_decode_replayable(const void *x, const void *rms_gamma, float rms_eps, const void *qkv_w,

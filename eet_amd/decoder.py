@@ -164,9 +164,13 @@ class Int8Decoder:
         if cfg.alibi:
             self.past = S if first_pass else self.past + S
             bias = self._alibi(first_pass, x)
-        for attn, ffn in self.layers:
-            x = attn.forward(x, pad, self.reorder_state, True, True, first_pass, bias)
-            x = ffn.forward(x, True, True)
+        y = None if first_pass else ops.decode_layers(self.layers, x, pad, self.reorder_state, bias)
+        if y is None:
+            for attn, ffn in self.layers:
+                x = attn.forward(x, pad, self.reorder_state, True, True, first_pass, bias)
+                x = ffn.forward(x, True, True)
+        else:
+            x = y
         return ops._timed("final_rmsnorm", 2 * B * S * cfg.hidden * 2, lambda: self.final_norm.layer_norm(x))
 
     def logits(self, input_ids, first_pass=True, attention_mask=None):

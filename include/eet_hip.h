@@ -410,6 +410,24 @@ int eet_gated_ffn_int8_decode(const void *x, const void *rms_gamma, float rms_ep
                               int add_residual, void *gemm_workspace, size_t gemm_workspace_bytes,
                               void *stream);
 
+/* eet_mmha_int8_decode and eet_gated_ffn_int8_decode (with the residual add) of num_layers
+ * layers in turn, the output of one being the input of the next; x [B][hidden] is the input
+ * of the first, out the output of the last.  alibi, pad and the rotary table row are the
+ * same for all layers, and so are the sizes and rms_eps; the two GEMM workspaces are those
+ * of the output and the down projection.  `layers` is read before the call returns. */
+typedef struct {
+    const void *attn_gamma, *qkv_w, *qkv_scale, *o_w, *o_scale;
+    void *k_cache, *v_cache;
+    const void *ffn_gamma, *w01, *scale01, *w2, *scale2;
+} eet_decoder_layer;
+int eet_decoder_int8_decode(const eet_decoder_layer *layers, int num_layers, const void *x,
+                            const void *alibi, const int64_t *pad, const float *rope_cos_sin,
+                            void *qkv_buf, void *ctx_buf, void *attn_out, void *act_buf, void *out,
+                            int B, int H, int dh, int hidden, int d_ff, float rms_eps, int step,
+                            int T_cap, void *workspace, size_t workspace_bytes, void *o_workspace,
+                            size_t o_workspace_bytes, void *down_workspace,
+                            size_t down_workspace_bytes, void *stream);
+
 /* The output head of a decode step: out[M][N] = x[M][K] * w[N][K]^T, fp16 with fp32
  * sums.  Row m of x begins at x + m*x_stride halves (x_stride >= K, a multiple of 8);
  * w row-major, out contiguous.  M <= 16, K % 64 == 0, N % 16 == 0, N*K <= 2^28 (larger

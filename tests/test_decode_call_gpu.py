@@ -64,3 +64,50 @@ def test_feed_forward_refuses_a_host_input(monkeypatch, rows, pre_layernorm):
     with pytest.raises(RuntimeError, match="must be on the GPU"):
         op.forward(torch.zeros(rows, 1, 64, dtype=torch.float16), pre_layernorm, True)
     assert not any(key[1].type == "cpu" for key in ops.workspaces._bufs)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("alibi", [False, True])
+@pytest.mark.parametrize("rows", [1, 5, 32, 33])
+def test_all_layers_in_one_call(gpu, monkeypatch, alibi, rows):
+    """Int8Decoder's steps through one library call for all layers and op by op: the same bits, caches and steps; op by
+    op where a layer is not like the others, and from there on again in one call."""
+    cfg = D.DecoderConfig(num_layers=3, hidden=256, heads=2, d_ff=704, vocab=64, alibi=alibi, max_batch=rows, max_prompt=8,
+                          max_full_seq=16)
+    sd, _ = D.random_state_dict(cfg, seed=6)
+    one, each = (D.Int8Decoder(cfg, sd, device="cuda:0") for _ in range(2))
+    whole, taken = ops.decode_layers, []
+
+    def watched(*args):
+        y = whole(*args)
+        taken.append(y is not None)
+        return y
+    g = torch.Generator().manual_seed(rows)
+    prompt, mask = torch.randint(0, 64, (rows, 6), generator=g).to(gpu), torch.ones(rows, 6, dtype=torch.long, device=gpu)
+    mask[0, :2] = 0
+
+    def step(i, ids, mask, reorder=None):
+        out = []
+        for model, form in ((one, watched), (each, lambda *a: None)):
+            monkeypatch.setattr(ops, "decode_layers", form)
+            model.reorder_state = torch.empty(0, dtype=torch.long) if reorder is None else reorder
+            out.append(model.logits(ids, i < 0, mask).clone())
+        assert torch.equal(*out)
+        assert {a.step for m in (one, each) for a, _ in m.layers} == {6 + 1 + i if i >= 0 else 6}
+        for (a, _), (b, _) in zip(one.layers, each.layers):
+            if reorder is None:
+                assert torch.equal(a._k, b._k) and torch.equal(a._v, b._v)
+    step(-1, prompt, mask)
+    for i in range(3):
+        step(i, torch.randint(0, 64, (rows, 1), generator=g).to(gpu), mask if i < 2 else None)
+    assert taken == [rows <= 32] * 3
+    del taken[:]
+    calls, first = [], one.layers[1][0]
+    first.forward = lambda *a: calls.append(1) or type(first).forward(first, *a)       # a program's own
+    step(3, prompt[:, :1], None)
+    del first.forward
+    assert taken == [False] and calls == [1]
+    step(4, prompt[:, :1], None, torch.arange(rows, device=gpu).flip(0))               # a beam search's step
+    assert taken[1:] == [False]
+    first.step -= 1
+    assert whole(one.layers, one.embed[prompt[:, :1]], None, None, None) is None       # the layers disagree
