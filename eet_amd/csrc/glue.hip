@@ -20,6 +20,11 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 constexpr int kNormThreads = 256;
 constexpr int kNormMaxVec = 8;  // N <= 256 * 8 * 8 = 16384, the reference's limit (layer_norm.cu:588)
 
+// NV: vectors of 8 per thread.  The row and gamma are requested together and without a branch (past the end the last
+// vector again).  With gamma behind the sum and a branch a vector, us: 2000 x 2048 4.2 instead of 3.7, 2000 x 5120 8.1
+// instead of 7.1, 8192 x 8192 45 instead of 41; a prompt of 45 tokens through six layers 502 instead of 487 (with the
+// split-k reduce of the large-M product, changed alike).
+template <int NV>
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const _Float16 *__restrict__ x,
                                                                const _Float16 *__restrict__ gamma,
                                                                _Float16 *__restrict__ out, int N, float eps)
@@ -28,13 +33,18 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const _Float16 *_
     const int row = blockIdx.x, tid = threadIdx.x;
     const int nvec = N / 8;
     const uint4 *xr = reinterpret_cast<const uint4 *>(x + (size_t)row * N);
-    half8 v[kNormMaxVec];
+    const uint4 *gr = reinterpret_cast<const uint4 *>(gamma);
+    half8 v[NV], g[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        v[i] = __builtin_bit_cast(half8, xr[min(tid + i * kNormThreads, nvec - 1)]);
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        g[i] = __builtin_bit_cast(half8, gr[min(tid + i * kNormThreads, nvec - 1)]);
     float ss = 0.f;
 #pragma unroll
-    for (int i = 0; i < kNormMaxVec; ++i) {
-        const int c = tid + i * kNormThreads;
-        if (c < nvec) {
-            v[i] = __builtin_bit_cast(half8, xr[c]);
+    for (int i = 0; i < NV; ++i) {
+        if (tid + i * kNormThreads < nvec) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 float f = (float)v[i][e];
@@ -53,17 +63,15 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const _Float16 *_
     for (int w = 0; w < kNormThreads / 64; ++w)
         tot += red[w];
     const float inv = rsqrtf(tot / (float)N + eps);
-    const uint4 *gr = reinterpret_cast<const uint4 *>(gamma);
     uint4 *orow = reinterpret_cast<uint4 *>(out + (size_t)row * N);
 #pragma unroll
-    for (int i = 0; i < kNormMaxVec; ++i) {
+    for (int i = 0; i < NV; ++i) {
         const int c = tid + i * kNormThreads;
         if (c < nvec) {
-            half8 g = __builtin_bit_cast(half8, gr[c]);
             half8 o;
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                o[e] = (_Float16)((float)v[i][e] * inv * (float)g[e]);
+                o[e] = (_Float16)((float)v[i][e] * inv * (float)g[i][e]);
             orow[c] = __builtin_bit_cast(uint4, o);
         }
     }
@@ -333,7 +341,9 @@ extern "C" int eet_rmsnorm(const void *x, const void *gamma, void *out, int M, i
                 "eet_rmsnorm: need N %% 8 == 0 and N <= 16384, got %d", N);
     if (M == 0)
         return EET_OK;
-    hipLaunchKernelGGL(rmsnorm_kernel, dim3(M), dim3(kNormThreads), 0, static_cast<hipStream_t>(stream),
+    const int nv = (N / 8 + kNormThreads - 1) / kNormThreads;
+    const auto kernel = nv <= 1 ? rmsnorm_kernel<1> : nv <= 2 ? rmsnorm_kernel<2> : nv <= 4 ? rmsnorm_kernel<4> : rmsnorm_kernel<kNormMaxVec>;
+    hipLaunchKernelGGL(kernel, dim3(M), dim3(kNormThreads), 0, static_cast<hipStream_t>(stream),
                        static_cast<const _Float16 *>(x), static_cast<const _Float16 *>(gamma),
                        static_cast<_Float16 *>(out), N, eps);
     EET_HIP_CHECK(hipGetLastError());

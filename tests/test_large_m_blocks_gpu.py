@@ -130,3 +130,26 @@ def test_slabs_of_32_rows(gpu, M, K, N):
     want = up * gate / (1 + torch.exp(-gate))
     tol = 2.0 ** -10 * (1.1 * gate.abs() * up.abs() + 2 * want.abs()) + 2.0 ** -23
     assert ((got.float() - want).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("shares", [2, 3, 4, 5, 6, 7, 8])
+def test_shares_of_the_k_range(gpu, tuning, shares):
+    """The reduce kernel at every number of shares, those it is compiled for and the others, with each epilogue."""
+    M, K, F = 37, 64 * 17, 112
+    tuning("EET_GEMM_LARGE_M_TILE", f"4,2,{shares},1,4")
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(shares)).half()
+    u, p, s = quant(K, F, 11)
+    room = shares * M * 2 * F * 4
+    plain = gemm(x.to(gpu), p.to(gpu), s.to(gpu), M, F, K, ws_min_bytes=room).cpu()
+    check(plain, x, u, s, f"{shares} shares")
+    res = torch.randn(M, F, generator=torch.Generator().manual_seed(1)).half()
+    assert torch.equal(gemm_fused(x.to(gpu), p.to(gpu), s.to(gpu), M, F, K, 1, res.to(gpu), ws_min_bytes=room).cpu(), plain + res)
+    u2, p2, s2 = quant(K, F, 12)
+    w, sc = interleave_gate_up(p.to(gpu), s.to(gpu), p2.to(gpu), s2.to(gpu))
+    up = gemm(x.to(gpu), p2.to(gpu), s2.to(gpu), M, F, K, ws_min_bytes=room).cpu().float()
+    got = gemm_fused(x.to(gpu), w, sc, M, 2 * F, K, 2, None, ws_min_bytes=room).cpu().float()
+    want = up * plain.float() / (1 + torch.exp(-plain.float()))
+    # gate, up and the result are each rounded to fp16 once (2^-11), gate and up perhaps to the neighbouring value where
+    # one form rounds by way of fp32; gate enters with at most 1 + |gate| < 6 times its error
+    assert float(plain.abs().max()) < 5
+    assert ((got - want).abs() <= want.abs() * (2 ** -11 + 2 ** -10 + 6 * 2 ** -10) + 2 ** -24).all()
