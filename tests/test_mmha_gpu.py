@@ -162,3 +162,18 @@ def test_full_size_uniform_keys(gpu, B, H, step, cap, use_alibi):
     want = torch.einsum("bht,bhtd->bhd", torch.softmax(logits, -1), vv).reshape(B, H * dh)
     assert_close(ctx.cpu().numpy(), want.cpu().numpy(), what="ctx")
     assert torch.equal(kc[:, :, step - 1], k0) and torch.equal(vc[:, :, step - 1], v)
+
+
+@pytest.mark.parametrize("nsplit", [2, 7, 8, 9, 16])
+def test_merge_of_the_splits(gpu, tuning, nsplit):
+    """The merge kernel around the number of splits it requests at once, with splits that hold no row at all (padding, a
+    cache shorter than the splits)."""
+    tuning("EET_MMHA_NSPLIT", str(nsplit))
+    for (B, H, dh, step, use_pad, use_alibi) in [(2, 3, 128, 333, True, False), (1, 2, 96, 11, False, True), (2, 2, 64, 40, True, False)]:
+        q, k, v, kc, vc, pad, alibi = case(B, H, dh, step, step, step + nsplit, use_pad, use_alibi)
+        kcn, vcn = kc.numpy().copy(), vc.numpy().copy()
+        want = O.decode_attention(q.numpy(), k.numpy(), v.numpy(), kcn, vcn, step,
+                                  pad.numpy() if use_pad else None, alibi.numpy() if use_alibi else None)
+        ctx = mmha(q.to(gpu), k.to(gpu), v.to(gpu), kc.to(gpu), vc.to(gpu), step, pad.to(gpu) if use_pad else None,
+                   alibi.to(gpu) if use_alibi else None)
+        assert_close(ctx.cpu().numpy(), want, what=f"ctx B={B} H={H} dh={dh} step={step}")
