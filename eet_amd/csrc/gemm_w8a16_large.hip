@@ -288,7 +288,7 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
     // Stores.  The block goes through LDS as fp16 and leaves in 16-byte pieces of rows.  Straight from the accumulators it
     // left in 8 bytes a lane, 32 bytes of a row at a time, and the residual came in the same way (us, then / now: 2000 rows
     // 2048 <- 2048 with residual 25.2 / 21.8, 5120 <- 5120 93.9 / 88.3; 406 rows 4096 <- 4096 25.1 / 22.9; plain 12288 <- 4096 at
-    // 406, 2048 and 8192 rows 50.2 / 47.7, 162 / 158, 617 / 604; SwiGLU, half the bytes and bound by its exponentials, equal;
+    // 406, 2048 and 8192 rows 50.2 / 47.7, 162 / 158, 617 / 604; SwiGLU, half the bytes, equal;
     // over 12 matrices 0.96 of the time from 400 rows on, 0.99 below).  A row's pieces are XORed with the row against
     // bank conflicts.
     constexpr int kPieces = S::kBN / 8, kThreads = 64 * S::kWaves;
@@ -325,12 +325,14 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
             for (int t = 0; t < TN; t += 2)
 #pragma unroll
                 for (int mt = 0; mt < TM; ++mt) {
+                    // (a product with the reciprocal, 2^-22 off: the quotient to the last bit is ten instructions more and took
+                    // 81.0 us where this takes 77.4, 2000 rows, 11264 <- 2048, at the same error against 64 bits, 2.08e-4)
                     half4 o;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const float gate = (float)(_Float16)(acc[t][mt][r] * (float)sc[t][r]);
                         const float up = (float)(_Float16)(acc[t + 1][mt][r] * (float)sc[t + 1][r]);
-                        o[r] = (_Float16)(up * gate / (1.0f + __expf(-gate)));
+                        o[r] = (_Float16)(up * gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)));
                     }
                     stage(kPieces / 2, mt, (wn * TN + t) / 2, o);
                 }
@@ -449,7 +451,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
         for (int r = 0; r < 4; ++r) {
             const float gate = (float)(_Float16)(sg[r] * (float)cg[r]);
             const float up = (float)(_Float16)(su[r] * (float)cu[r]);
-            o[r] = (_Float16)(up * gate / (1.0f + __expf(-gate)));
+            o[r] = (_Float16)(up * gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)));
         }
     } else {
         floatx4 p[kHeld];
