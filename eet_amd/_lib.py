@@ -48,6 +48,7 @@ SIGNATURES = {
     "eet_gated_ffn_int8_decode": (_i, [_vp, _vp, _f] + [_vp] * 6 + [_i] * 4 + [_vp, _sz, _vp]),
     "eet_decoder_int8_decode": (_i, [_vp, _i] + [_vp] * 9 + [_i] * 5 + [_f, _i, _i] + [_vp, _sz] * 3 + [_vp]),
     "eet_rope_table": (_i, [_vp, _i, _i, _vp]),
+    "eet_embedding_f16": (_i, [_vp, _vp, _vp, _i, _c.c_int64, _i, _vp]),
     "eet_rmsnorm": (_i, [_vp, _vp, _vp, _i, _i, _f, _vp]),
     "eet_layernorm": (_i, [_vp, _vp, _vp, _vp, _i, _i, _f, _vp]),
     "eet_add_bias_residual_norm": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _f, _vp]),

@@ -78,6 +78,22 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const _Float16 *_
 }
 
 // ---------------------------------------------------------------------------
+// Token embedding of a decode step: out[r] = table[ids[r]], a workgroup per row.  torch's gather of up to 16 rows walks
+// the rows one after another in every thread (12 us for 16 rows of 8 KB, 2.3 for one); this is one memory latency behind
+// the index.  An index outside the table ends the program, as it does there.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(kNormThreads) void embedding_kernel(const int64_t *__restrict__ ids,
+                                                                 const uint4 *__restrict__ table,
+                                                                 uint4 *__restrict__ out, int64_t rows, int nvec)
+{
+    const int64_t id = ids[blockIdx.x];
+    if (id < 0 || id >= rows)
+        __builtin_trap();
+    for (int c = threadIdx.x; c < nvec; c += kNormThreads)
+        out[(size_t)blockIdx.x * nvec + c] = table[(size_t)id * nvec + c];
+}
+
+// ---------------------------------------------------------------------------
 // The bias / LayerNorm branch of the ops.  One kernel: y = x [+ residual] [+ bias] with the
 // reference's fp16 adds, then LayerNorm (gamma, beta: fp32 mean, then fp32 variance of the
 // centred values, (y - mean) * rsqrt(var + eps) * gamma + beta, one rounding) or, with beta
@@ -346,6 +362,21 @@ extern "C" int eet_rmsnorm(const void *x, const void *gamma, void *out, int M, i
     hipLaunchKernelGGL(kernel, dim3(M), dim3(kNormThreads), 0, static_cast<hipStream_t>(stream),
                        static_cast<const _Float16 *>(x), static_cast<const _Float16 *>(gamma),
                        static_cast<_Float16 *>(out), N, eps);
+    EET_HIP_CHECK(hipGetLastError());
+    return EET_OK;
+}
+
+extern "C" int eet_embedding_f16(const int64_t *ids, const void *table, void *out, int M, int64_t rows, int N, void *stream)
+{
+    EET_REQUIRE(ids && table && out, EET_ERR_INVALID_ARGUMENT, "eet_embedding_f16: null pointer");
+    EET_REQUIRE(M >= 0 && rows > 0 && N > 0, EET_ERR_INVALID_ARGUMENT, "eet_embedding_f16: bad sizes M=%d N=%d", M, N);
+    EET_REQUIRE(N % 8 == 0, EET_ERR_UNSUPPORTED_SHAPE, "eet_embedding_f16: need N %% 8 == 0, got %d", N);
+    EET_REQUIRE((reinterpret_cast<uintptr_t>(table) | reinterpret_cast<uintptr_t>(out)) % 16 == 0, EET_ERR_INVALID_ARGUMENT,
+                "eet_embedding_f16: table and out need 16-byte alignment");
+    if (M == 0)
+        return EET_OK;
+    hipLaunchKernelGGL(embedding_kernel, dim3(M), dim3(kNormThreads), 0, static_cast<hipStream_t>(stream), ids,
+                       static_cast<const uint4 *>(table), static_cast<uint4 *>(out), rows, N / 8);
     EET_HIP_CHECK(hipGetLastError());
     return EET_OK;
 }

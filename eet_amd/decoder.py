@@ -158,8 +158,7 @@ class Int8Decoder:
             pad = self.pre_padding_len
         else:
             pad = torch.sum(1 - attention_mask, 1, True).to(input_ids.device).long()
-        x = ops._timed("embedding (torch)", 2 * B * S * cfg.hidden * 2,
-                       lambda: torch.nn.functional.embedding(input_ids, self.embed))
+        x = ops._timed("embedding", 2 * B * S * cfg.hidden * 2, lambda: ops.embedding(input_ids, self.embed))
         bias = torch.empty(0)
         if cfg.alibi:
             self.past = S if first_pass else self.past + S

@@ -966,6 +966,24 @@ def _head_kernel_takes(h, weight):
             and device == _current_device() and weight.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0)
 
 
+def embedding(ids, weight):
+    """torch's embedding lookup.  Plain calls of up to 16 indices, which torch gathers slowly, run on eet_embedding_f16:
+    whole int64 indices and fp16 rows on the current device, and nothing that torch would do beyond the lookup."""
+    rows, device = ids.numel(), ids.get_device()
+    if (0 < rows <= 16 and device >= 0 and weight.get_device() == device and device == _current_device()
+            and ids.dtype is torch.int64 and weight.dtype is torch.float16 and weight.dim() == 2 and weight.shape[0] > 0
+            and weight.shape[1] > 0 and weight.shape[1] % 8 == 0 and weight.shape[1] < 2 ** 31
+            and ids.is_contiguous() and weight.is_contiguous() and type(ids) is torch.Tensor
+            and (type(weight) is torch.Tensor or type(weight) is torch.nn.Parameter)
+            and not (weight.requires_grad and torch.is_grad_enabled()) and not _transformed(weight) and not _transformed(ids)
+            and _dual_levels._current_level < 0 and weight.data_ptr() % 16 == 0):
+        out = weight.new_empty((*ids.shape, weight.shape[1]))
+        check(lib().eet_embedding_f16(ids.data_ptr(), weight.data_ptr(), out.data_ptr(), rows, weight.shape[0],
+                                      weight.shape[1], _current_stream()), "eet_embedding_f16")
+        return out
+    return torch.nn.functional.embedding(ids, weight)
+
+
 def head(h, weight):
     """Logits [B, 1, V] of the last position of h [B, S, K] under the fp16 output matrix [V, K].  Plain calls of up to
     16 sequences and 2^28 weights run on eet_head_f16 where it is the faster one, all others on torch's linear."""

@@ -428,6 +428,12 @@ int eet_decoder_int8_decode(const eet_decoder_layer *layers, int num_layers, con
                             size_t o_workspace_bytes, void *down_workspace,
                             size_t down_workspace_bytes, void *stream);
 
+/* The token embedding of a decode step: out[m][N] = table[ids[m]][N], fp16, for M rows of
+ * a table of `rows`; N % 8 == 0, table and out 16-byte aligned.  An index outside the
+ * table traps. */
+int eet_embedding_f16(const int64_t *ids, const void *table, void *out, int M, int64_t rows,
+                      int N, void *stream);
+
 /* The output head of a decode step: out[M][N] = x[M][K] * w[N][K]^T, fp16 with fp32
  * sums.  Row m of x begins at x + m*x_stride halves (x_stride >= K, a multiple of 8);
  * w row-major, out contiguous.  M <= 16, K % 64 == 0, N % 16 == 0, N*K <= 2^28 (larger

@@ -22,6 +22,26 @@ def test_rmsnorm(gpu, M, N):
     assert_close(out.cpu().numpy(), O.rmsnorm(x.numpy(), gamma.numpy(), 1e-6), rtol=2e-3, atol=1e-3)
 
 
+@pytest.mark.parametrize("B,S,V,N", [(1, 1, 7, 8), (16, 1, 1000, 4096), (2, 8, 33, 2056), (3, 5, 64, 5120), (17, 1, 64, 64)])
+def test_embedding(gpu, monkeypatch, B, S, V, N):
+    """ops.embedding gives torch's rows, first and last of the table among them, on the kernel up to 16 indices and on
+    torch beyond, and on torch for what is not a plain lookup."""
+    from eet_amd import ops
+    lookup, calls = torch.nn.functional.embedding, []
+    monkeypatch.setattr(ops.torch.nn.functional, "embedding", lambda *a: calls.append(1) or lookup(*a))
+    w = torch.randn(V, N, device=gpu).half()
+    ids = torch.randint(0, V, (B, S), device=gpu)
+    ids[0, 0], ids[-1, -1] = 0, V - 1
+    got = ops.embedding(ids, w)
+    assert got.shape == (B, S, N) and torch.equal(got, lookup(ids, w)) and len(calls) == (B * S > 16)
+    calls.clear()
+    for other_ids, other in ((ids.int(), w), (ids, w.float()), (ids, w[:, : N // 2]), (ids[:0], w),
+                             (ids, w.clone().requires_grad_()), (torch.stack([ids, ids], 2)[:, :, 0], w)):
+        y = ops.embedding(other_ids, other)
+        assert torch.equal(y, lookup(other_ids, other)) and y.requires_grad == other.requires_grad
+    assert len(calls) == (6 if B * S > 1 else 5)      # one index is whole under any stride
+
+
 @pytest.mark.parametrize("B,S,H,dh,rope,ts,t0", [(2, 5, 4, 128, 1, -1, 0), (3, 1, 4, 128, 1, 1030, 1030),
                                                    (2, 7, 5, 64, 0, -1, 0), (1, 1, 2, 32, 1, 17, 17),
                                                    (2, 1, 40, 128, 0, 9, 9), (2, 6, 3, 96, 1, -1, 0)])
