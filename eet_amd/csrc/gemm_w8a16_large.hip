@@ -31,7 +31,8 @@
 //     is interleaved with them one vector instruction per matrix instruction: neither the barrier nor the LDS
 //     latency is exposed even with one wavefront per SIMD;
 //   * the block shape follows the problem (kTiles below): 20 shapes from 32 x 64 to 256 x 256.
-// Measured against that earlier kernel (us, QKV / O / gate-up / down of a 4096-wide layer, weights from HBM):
+// Measured against that earlier kernel (us, QKV / O / gate-up / down of a 4096-wide layer, weights from HBM; both with
+// the stores straight from the accumulators that are described, with what replaced them, at the epilogue below):
 //   M = 64    12288 <- 4096  20.7 -> 17.8   4096 <- 4096  12.9 -> 10.8   22016 <- 4096  31.6 -> 25.7   4096 <- 11008  22.1 -> 17.7
 //   M = 406                  50.0 -> 54.2                 25.7 -> 24.7                  91.6 -> 80.8                  50.1 -> 50.9
 //   M = 1024                103.3 -> 88.3                 37.9 -> 40.2                   156 -> 155                   91.8 -> 88.7
