@@ -554,7 +554,7 @@ int launch_groups(const void *w, size_t K, size_t N, int parts, int ref128, int8
 bool one_pass_wins(size_t K, size_t N, size_t size)
 {
     const size_t n = K * N;
-    return size == 4 || n <= 36000000 || n >= 70000000;
+    return N < ((size_t)1 << 31) && (size == 4 || n <= 36000000 || n >= 70000000);   // its column indices are 32 bits wide
 }
 
 // How many workgroups share a column group: as many as its rows need, and as many as the chip still takes in one round.
@@ -594,8 +594,12 @@ int run(const void *w, size_t K, size_t N, int mode, int8_t *q, int8_t *packed, 
 
 }  // namespace
 
-// A count per group of columns and the column maxima of each part; the two passes use N words of it.
-extern "C" size_t eet_quantize_pack_device_workspace(size_t N) { return (N * kMaxParts + (N + 31) / 32 * (kCountStride + 32 * kMaxParts)) * sizeof(uint32_t); }
+// A count per group of columns (32 columns or more) and, in whole groups (64 columns or fewer), the column maxima of each
+// part; the two passes use N words of it.
+extern "C" size_t eet_quantize_pack_device_workspace(size_t N)
+{
+    return ((N + 31) / 32 * kCountStride + (N + 63) / 64 * 64 * kMaxParts) * sizeof(uint32_t);
+}
 
 extern "C" int eet_quantize_pack_device(const void *w, int w_dtype, size_t K, size_t N, int mode, int8_t *q,
                                         int8_t *packed, void *scale, void *workspace, size_t workspace_bytes,

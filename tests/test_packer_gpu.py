@@ -133,7 +133,7 @@ def test_converter_on_device(gpu):
 
 
 @pytest.mark.parametrize("K,N", [(64, 16), (128, 80), (2048, 16), (2112, 48), (1280, 1040), (8256, 112), (32832, 32),
-                                 (2624, 16400)])
+                                 (2624, 16400), (16384, 16), (32768, 16), (20480, 80)])
 @pytest.mark.parametrize("dtype", [np.float16, np.float32])
 def test_one_pass_matches_two_passes(gpu, K, N, dtype):
     """The one-pass kernel at the edges of its shares (rows a workgroup holds, one to sixteen workgroups per column
@@ -146,7 +146,7 @@ def test_one_pass_matches_two_passes(gpu, K, N, dtype):
     wd = torch.from_numpy(w).to(gpu)
     code = 0 if dtype == np.float32 else 1
     for nbytes in (lib().eet_quantize_pack_device_workspace(N), 4 * N):
-        ws = torch.full((nbytes // 4,), -1, dtype=torch.int32, device=gpu)
+        ws = torch.full((nbytes // 4 + 1024,), -1, dtype=torch.int32, device=gpu)
         for want_q in (True, False):
             q, p = (torch.zeros(K, N, dtype=torch.int8, device=gpu) for _ in range(2))
             s = torch.zeros(N, dtype=wd.dtype, device=gpu)
@@ -155,3 +155,4 @@ def test_one_pass_matches_two_passes(gpu, K, N, dtype):
             assert torch.equal(p.cpu(), ph)
             assert not want_q or torch.equal(q.cpu(), uh)
             assert torch.equal(s.cpu().view(torch.int16 if code else torch.int32), sh.view(torch.int16 if code else torch.int32))
+            assert (ws[nbytes // 4:] == -1).all()       # nothing behind the workspace
