@@ -326,14 +326,14 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
             for (int t = 0; t < TN; t += 2)
 #pragma unroll
                 for (int mt = 0; mt < TM; ++mt) {
-                    // (a product with the reciprocal, 2^-22 off: the quotient to the last bit is ten instructions more and took
-                    // 81.0 us where this takes 77.4, 2000 rows, 11264 <- 2048, at the same error against 64 bits, 2.08e-4)
+                    // (the rounded quotient, as 32 rows and fewer have it; a product with v_rcp_f32's reciprocal, 2^-22 off,
+                    // takes 77.4 us where this takes 81.0, 2000 rows, 11264 <- 2048)
                     half4 o;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const float gate = (float)(_Float16)(acc[t][mt][r] * (float)sc[t][r]);
                         const float up = (float)(_Float16)(acc[t + 1][mt][r] * (float)sc[t + 1][r]);
-                        o[r] = (_Float16)(up * gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)));
+                        o[r] = (_Float16)(up * gate / (1.0f + __expf(-gate)));
                     }
                     stage(kPieces / 2, mt, (wn * TN + t) / 2, o);
                 }
@@ -452,7 +452,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
         for (int r = 0; r < 4; ++r) {
             const float gate = (float)(_Float16)(sg[r] * (float)cg[r]);
             const float up = (float)(_Float16)(su[r] * (float)cu[r]);
-            o[r] = (_Float16)(up * gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)));
+            o[r] = (_Float16)(up * gate / (1.0f + __expf(-gate)));
         }
     } else {
         floatx4 p[kHeld];

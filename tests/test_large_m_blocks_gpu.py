@@ -153,3 +153,20 @@ def test_shares_of_the_k_range(gpu, tuning, shares):
     # one form rounds by way of fp32; gate enters with at most 1 + |gate| < 6 times its error
     assert float(plain.abs().max()) < 5
     assert ((got - want).abs() <= want.abs() * (2 ** -11 + 2 ** -10 + 6 * 2 ** -10) + 2 ** -24).all()
+
+
+@pytest.mark.parametrize("shares", [1, 3])
+def test_swiglu_does_not_depend_on_the_batch(gpu, tuning, shares):
+    """A row's SwiGLU is the same number, to the bit, in a batch of 32 rows (small-M kernel) and in a larger one: the
+    rounded fp32 quotient in both.  Products of small integers under powers of two, so that every sum is exact."""
+    M, K, F = 100, 64 * shares, 4096
+    g = torch.Generator().manual_seed(shares)
+    x = torch.randint(-4, 5, (M, K), generator=g).half().to(gpu)
+    (p, s), (pu, su) = ((eet_amd.pack_weights(torch.randint(-127, 128, (K, F), generator=g).to(torch.int8)).to(gpu),
+                         torch.full((F,), 2.0 ** -8, dtype=torch.float16, device=gpu)) for _ in range(2))
+    w, sc = interleave_gate_up(p, s, pu, su)
+    want = torch.cat([gemm_fused(rows.contiguous(), w, sc, len(rows), 2 * F, K, 2) for rows in x.split(32)])
+    for tm, tn, wm, wn in [b for b in BLOCKS if b[1] % 2 == 0]:
+        tuning("EET_GEMM_LARGE_M_TILE", f"{tm},{tn},{shares},{wm},{wn}")
+        got = gemm_fused(x, w, sc, M, 2 * F, K, 2, None, ws_min_bytes=shares * M * 2 * F * 4)
+        assert torch.equal(got, want), f"{tm}x{tn}x{wm}x{wn}: {int((got != want).sum())} of {got.numel()} differ"

@@ -76,3 +76,26 @@ def test_refused(gpu):
     assert L.eet_gemm_w8a16_qkv(x, x, x, x, x, x, x, None, 1, 40, 1, 48, 64, 64, None, 0, None) != 0      # head size
     assert L.eet_gemm_w8a16_qkv(x, x, x, x, x, x, x, None, 1, 40, 1, 32, 64, 39, None, 0, None) != 0      # cache rows
     assert L.eet_gemm_w8a16_qkv(x, x, x, x, None, x, x, None, 1, 40, 1, 32, 64, 64, None, 0, None) != 0   # null
+
+
+@pytest.mark.parametrize("block", BLOCKS, ids=lambda b: "x".join(map(str, b)))
+def test_same_rotation_as_the_split_kernel(gpu, tuning, block):
+    """Where the products are exact (small integers, scales that are powers of two) the rows, rotated or not, are those
+    of the split kernel to the bit: each value rounds to fp16 once, straight from the sum of its two products."""
+    tm, tn, wm, wn = block
+    tuning("EET_GEMM_LARGE_M_TILE", f"{tm},{tn},1,{wm},{wn}")
+    g = torch.Generator().manual_seed(tm * tn)
+    for B, S, H, dh, K in ((2, 200, 4, 128, 64), (1, 333, 6, 64, 128), (3, 45, 3, 96, 64), (1, 130, 5, 32, 64)):
+        N, M = 3 * H * dh, B * S
+        x = torch.randint(-4, 5, (M, K), generator=g).half().to(gpu)
+        p = eet_amd.pack_weights(torch.randint(-127, 128, (K, N), generator=g).to(torch.int8)).to(gpu)
+        s = torch.full((N,), 2.0 ** -8, dtype=torch.float16, device=gpu)
+        table = eet_amd.ops._rope_table(S, dh, gpu)
+        for rope in (True, False):
+            want, got = ([torch.full((B, H, S, dh), GUARD, dtype=torch.float16, device=gpu) for _ in "qkv"] for _ in range(2))
+            rows, qkv = gemm(x, p, s, M, N, K), torch.empty(M, N, dtype=torch.float16, device=gpu)
+            check(lib().eet_qkv_split(rows.data_ptr(), *(t.data_ptr() for t in want), B, S, H, dh, int(rope), -1, 0, S, stream()))
+            check(lib().eet_gemm_w8a16_qkv(x.data_ptr(), p.data_ptr(), s.data_ptr(), qkv.data_ptr(), *(t.data_ptr() for t in got),
+                                           table.data_ptr() if rope else None, B, S, H, dh, K, S, None, 0, stream()))
+            for name, a, b in zip("qkv", want, got):
+                assert torch.equal(a, b), f"{block} {B}x{S}x{H}x{dh} rope {rope}: {name}, {int((a != b).sum())} of {a.numel()} differ"
