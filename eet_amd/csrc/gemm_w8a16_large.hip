@@ -65,6 +65,16 @@ struct TileShape {
     static_assert((D - 1) * (kA + kW) <= 63, "the copies in flight must fit the wait counter");
 };
 
+// (a0 * b0 + c0, a1 * b1 + c1), each rounded once, to fp16.  Left to itself the compiler rounds some of a block's values by
+// way of fp32.
+__device__ __forceinline__ uint32_t fma_f16x2(float a0, float b0, float c0, float a1, float b1, float c1)
+{
+    uint32_t o;
+    asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(o) : "v"(a0), "v"(b0), "v"(c0));
+    asm("v_fma_mixhi_f16 %0, %1, %2, %3" : "+v"(o) : "v"(a1), "v"(b1), "v"(c1));
+    return o;
+}
+
 template <int TM, int TN, int WM, int WN, int D, bool QKV>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2))) void w8a16_large_m_kernel(
     const _Float16 *__restrict__ A, const u32x4 *__restrict__ Wp, const _Float16 *__restrict__ scale,
@@ -370,9 +380,9 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
     }
     __syncthreads();
     if constexpr (QKV) {
-        // A lane takes 8 channels and their partners half a head on, turns them in fp32 and rounds again, as the split kernel
-        // does.  (From the accumulators, with the angles of each lane's rows, this took 58 us instead of the plain 51 for
-        // 2000 rows, 6144 <- 2048.)
+        // A lane takes 8 channels and their partners half a head on, turns them in fp32 and rounds again, to the bit as the
+        // split kernel does.  (From the accumulators, with the angles of each lane's rows, this took 58 us instead of the
+        // plain 51 for 2000 rows, 6144 <- 2048.)
         // piece q of a row: 8 channels of the first tile of pair q / 2
         constexpr int kTasks = S::kBM * kPairs * 2;
 #pragma unroll 2
@@ -387,12 +397,16 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
             if (out.rope != nullptr && part < 2) {
                 const floatx4 *c = reinterpret_cast<const floatx4 *>(out.rope + (size_t)pos * out.dh + d);
                 const floatx4 *sn = reinterpret_cast<const floatx4 *>(out.rope + (size_t)pos * out.dh + d + half);
+                u32x4 px, py;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float a = (float)x[e], o = (float)y[e];
-                    x[e] = (_Float16)__builtin_fmaf(a, c[e / 4][e % 4], -(o * sn[e / 4][e % 4]));
-                    y[e] = (_Float16)__builtin_fmaf(o, c[e / 4][e % 4], a * sn[e / 4][e % 4]);
+                for (int e = 0; e < 8; e += 2) {
+                    const floatx4 ce = c[e / 4], se = sn[e / 4];
+                    const float a0 = (float)x[e], a1 = (float)x[e + 1], o0 = (float)y[e], o1 = (float)y[e + 1];
+                    px[e / 2] = fma_f16x2(a0, ce[e % 4], -(o0 * se[e % 4]), a1, ce[e % 4 + 1], -(o1 * se[e % 4 + 1]));
+                    py[e / 2] = fma_f16x2(o0, ce[e % 4], a0 * se[e % 4], o1, ce[e % 4 + 1], a1 * se[e % 4 + 1]);
                 }
+                x = __builtin_bit_cast(half8, px);
+                y = __builtin_bit_cast(half8, py);
             }
             _Float16 *dst = (part == 0 ? out.q : part == 1 ? out.k : out.v) +
                             (((size_t)b * out.H + h) * (part == 0 ? out.S : out.T) + pos) * out.dh + d;
