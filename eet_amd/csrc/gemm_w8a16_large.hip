@@ -341,8 +341,10 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
                     half4 o;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        const float gate = (float)(_Float16)(acc[t][mt][r] * (float)sc[t][r]);
-                        const float up = (float)(_Float16)(acc[t + 1][mt][r] * (float)sc[t + 1][r]);
+                        float ga = acc[t][mt][r], ua = acc[t + 1][mt][r];
+                        asm("" : "+v"(ga), "+v"(ua));   // (no product shared with the plain epilogue, which rounds it otherwise)
+                        const float gate = (float)(_Float16)(ga * (float)sc[t][r]);
+                        const float up = (float)(_Float16)(ua * (float)sc[t + 1][r]);
                         o[r] = (_Float16)(up * gate / (1.0f + __expf(-gate)));
                     }
                     stage(kPieces / 2, mt, (wn * TN + t) / 2, o);
@@ -358,8 +360,11 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
         for (int mt = 0; mt < TM; ++mt) {
             half4 o;
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                o[r] = (_Float16)(acc[t][mt][r] * (float)sc[t][r]);
+            for (int r = 0; r < 4; ++r) {
+                float f = acc[t][mt][r] * (float)sc[t][r];
+                asm("" : "+v"(f));   // rounded to fp32 first in every block (the compiler merged a lone pair of the two steps)
+                o[r] = (_Float16)f;
+            }
             stage(kPieces, mt, wn * TN + t, o);
         }
     if constexpr (!QKV) {

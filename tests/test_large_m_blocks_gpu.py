@@ -170,3 +170,26 @@ def test_swiglu_does_not_depend_on_the_batch(gpu, tuning, shares):
         tuning("EET_GEMM_LARGE_M_TILE", f"{tm},{tn},{shares},{wm},{wn}")
         got = gemm_fused(x, w, sc, M, 2 * F, K, 2, None, ws_min_bytes=shares * M * 2 * F * 4)
         assert torch.equal(got, want), f"{tm}x{tn}x{wm}x{wn}: {int((got != want).sum())} of {got.numel()} differ"
+
+
+def test_products_round_alike_in_every_block(gpu, tuning):
+    """A product is rounded to fp32 and then to fp16, whatever the block: with exact sums (integers below 2^24) the rows are
+    those of the formula to the bit, at any scale.  SwiGLU takes gate and up rounded at once: the same rows from every
+    block."""
+    M, K, N = 1000, 64, 8192
+    g = torch.Generator().manual_seed(1)
+    x = torch.randint(-2047, 2048, (M, K), generator=g).half()
+    q = torch.randint(-127, 128, (K, N), generator=g).to(torch.int8)
+    s = (torch.rand(N, generator=g) * 0.01 + 1e-3).half()
+    want = ((x.float() @ q.float()) * s.float()).half()
+    xd, pd, sd, small = x.to(gpu), eet_amd.pack_weights(q).to(gpu), s.to(gpu), (s / 1024).to(gpu)
+    wrong, first = {}, None
+    for block in BLOCKS:
+        tm, tn, wm, wn = block
+        tuning("EET_GEMM_LARGE_M_TILE", f"{tm},{tn},1,{wm},{wn}")
+        wrong[block] = int((gemm(xd, pd, sd, M, N, K).cpu() != want).sum())
+        if tn % 2 == 0:
+            got = gemm_fused(xd, pd, small, M, N, K, 2)      # neighbouring tiles of 16 channels as gate and up
+            first = got if first is None else first
+            wrong[block] += int((got != first).sum())
+    assert not any(wrong.values()), {block: n for block, n in wrong.items() if n}
