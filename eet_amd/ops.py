@@ -289,12 +289,17 @@ _rope_tables = {}
 
 
 def _rope_table(T, dh, device):
-    """fp32 [T, dh] table (cos | sin per position), built once per (T, dh, device)."""
+    """fp32 [T, dh] table (cos | sin per position), built once per (T, dh, device).  Shared by every op of the process, on
+    whatever stream and thread, so it is complete before anyone else can see it; one that is being recorded into a graph
+    is that caller's own."""
     key = (T, dh, str(device))
     t = _rope_tables.get(key)
     if t is None:
         t = torch.empty(T, dh, dtype=torch.float32, device=device)
         check(lib().eet_rope_table(t.data_ptr(), T, dh, _stream()), "eet_rope_table")
+        if torch.cuda.is_current_stream_capturing():
+            return t
+        torch.cuda.current_stream().synchronize()
         _rope_tables[key] = t
     return t
 
