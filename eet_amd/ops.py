@@ -1112,8 +1112,9 @@ def quant_weights_device(origin_weight, return_unprocessed_quantized_tensor=Fals
     scales = torch.empty(N, dtype=w.dtype, device=w.device)
     q = torch.empty(K, N, dtype=torch.int8, device=w.device) if return_unprocessed_quantized_tensor else None
     need = L.eet_quantize_pack_device_workspace(N)
-    ws = workspaces.get("quant_absmax", max(need // 4, 1), torch.int32, w.device)
     with torch.cuda.device(w.device):
+        # of this call alone: workgroups of one call meet in it, and calls on other streams may run beside them
+        ws = torch.empty(max(need // 4, 1), dtype=torch.int32, device=w.device)
         check(L.eet_quantize_pack_device(w.data_ptr(), 0 if w.dtype == torch.float32 else 1, K, N,
                                          {"ref128": 0, "sym127": 1}[mode], q.data_ptr() if q is not None else None,
                                          packed.data_ptr(), scales.data_ptr(), ws.data_ptr(), need, _stream()),

@@ -102,8 +102,10 @@ int eet_unprocess_ref_sm80(const int8_t *processed, size_t K, size_t N, int8_t *
  * gfx950 layout, scale[N] in w's dtype and, when q is not NULL, the
  * unprocessed q[K][N]; all device pointers.  Bit-identical to
  * eet_quantize_int8 followed by eet_pack_gfx950 in both modes.  workspace:
- * eet_quantize_pack_device_workspace(N) bytes of device memory (with as little
- * as 4 N bytes every matrix takes the slower of two ways).  The reference
+ * eet_quantize_pack_device_workspace(N) bytes of device memory, any contents;
+ * 4 N bytes are enough and make every call read the matrix twice.  Workgroups
+ * of a call meet in it: calls that can overlap in time must not share one.
+ * The reference
  * quantises on one host core only (cutlass_preprocessors.cc:581-678, reached
  * from fpA_intB_gemm_wrapper.cu:26-105, which rejects CUDA tensors at :33);
  * this entry point has no counterpart there. */

@@ -156,3 +156,31 @@ def test_one_pass_matches_two_passes(gpu, K, N, dtype):
             assert not want_q or torch.equal(q.cpu(), uh)
             assert torch.equal(s.cpu().view(torch.int16 if code else torch.int32), sh.view(torch.int16 if code else torch.int32))
             assert (ws[nbytes // 4:] == -1).all()       # nothing behind the workspace
+
+
+def test_overlapping_calls_do_not_share_a_workspace(gpu, monkeypatch):
+    """Calls on two streams may run side by side: each has maxima and arrival counts of its own."""
+    from eet_amd import ops
+    real, seen = ops.lib(), []
+
+    class Watched:
+        def __getattr__(self, name):
+            fn = getattr(real, name)
+            if name != "eet_quantize_pack_device":
+                return fn
+            return lambda *a: seen.append((a[8], a[9])) or fn(*a)
+    ws = [torch.from_numpy(tricky(512, 256, np.float16, i)).to(gpu) for i in range(2)]
+    want = [eet_amd.quant_weights_device(w) for w in ws]
+    torch.cuda.synchronize()
+    monkeypatch.setattr(ops, "lib", Watched)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for round in range(4):
+        got = []
+        for w, stream in zip(ws, streams):
+            with torch.cuda.stream(stream):
+                got.append(eet_amd.quant_weights_device(w))
+        (a, size), (b, _) = seen[-2:]
+        assert a + size <= b or b + size <= a, "one buffer for both streams"
+        torch.cuda.synchronize()
+        for pair, other in zip(got, want):
+            assert all(torch.equal(x, y) for x, y in zip(pair, other))
