@@ -925,11 +925,13 @@ def decode_layers(layers, x, pad, reorder, bias):
     o_ws = _k_split_ws(B, hidden, inner, EPI_RESIDUAL, dev)
     keep = (x, pad, bias, reorder)      # inputs of kernels still in flight
     for attn, _ in layers:
-        attn.step, attn._keep = step, keep
+        attn._keep = keep
     check(L.eet_decoder_int8_decode(b"".join(table), len(table), x.data_ptr(), alibi_ptr, pad_ptr, rope, qkv.data_ptr(),
                                     cbuf.data_ptr(), mid.data_ptr(), act.data_ptr(), out.data_ptr(), B, H, dh, hidden,
                                     d_ff, desc.layernorm_eps, step, t_cap, ws_ptr, need, *o_ws, *down_ws, st),
           "eet_decoder_int8_decode")
+    for attn, _ in layers:      # all of them or, where the call failed, none: no layer counts a row that it does not have
+        attn.step = step
     return out.as_strided((B, 1, hidden), (hidden, hidden, 1))
 
 

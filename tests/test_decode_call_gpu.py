@@ -111,3 +111,33 @@ def test_all_layers_in_one_call(gpu, monkeypatch, alibi, rows):
     assert taken[1:] == [False]
     first.step -= 1
     assert whole(one.layers, one.embed[prompt[:, :1]], None, None, None) is None       # the layers disagree
+
+
+def two_decoders(alibi, rows):
+    cfg = D.DecoderConfig(num_layers=3, hidden=256, heads=2, d_ff=704, vocab=64, alibi=alibi, max_batch=rows, max_prompt=8,
+                          max_full_seq=16)
+    sd, _ = D.random_state_dict(cfg, seed=7)
+    return [D.Int8Decoder(cfg, sd, device="cuda:0") for _ in range(2)]
+
+
+@pytest.mark.gpu
+def test_a_failed_call_leaves_every_layer_where_it_was(gpu, monkeypatch):
+    """No layer counts a token whose key and value it may not have; the call can be made again."""
+    model, other = two_decoders(False, 3)
+    g = torch.Generator().manual_seed(1)
+    prompt, token = (torch.randint(0, 64, (3, n), generator=g).to(gpu) for n in (6, 1))
+    for m in (model, other):
+        m.logits(prompt, True)
+    real = ops.check
+
+    def failing(status, what=""):
+        if what == "eet_decoder_int8_decode":
+            raise RuntimeError("launch failed")
+        real(status, what)
+    monkeypatch.setattr(ops, "check", failing)
+    with pytest.raises(RuntimeError, match="launch failed"):
+        model.logits(token, False)
+    assert [a.step for a, _ in model.layers] == [6, 6, 6]
+    monkeypatch.setattr(ops, "check", real)
+    got = model.logits(token, False).clone()
+    assert torch.equal(got, other.logits(token, False)) and [a.step for a, _ in model.layers] == [7, 7, 7]
