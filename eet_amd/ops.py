@@ -892,7 +892,8 @@ def decode_layers(layers, x, pad, reorder, bias):
         if (type(attn) is not kind or type(ffn) is not GatedFeedForwardNetworkInt8 or attn.desc is not desc
                 or ffn.desc is not desc or attn.step + 1 != step or attn._rows is not None or attn.biased
                 or ffn.beta is not None or ffn.o_bias is not None or ffn.cache_name != name or attn.t_cap != t_cap
-                or ffn.d_ff != d_ff or "forward" in attn.__dict__ or "forward" in ffn.__dict__):
+                or ffn.d_ff != d_ff or "forward" in attn.__dict__ or "forward" in ffn.__dict__
+                or attn.rope_table is not first.rope_table):
             return None
         table.append(_layer_pointers(
             attn.gamma.data_ptr(), attn.qkv_w.data_ptr(), attn.qkv_s.data_ptr(), attn.o_w.data_ptr(), attn.o_s.data_ptr(),

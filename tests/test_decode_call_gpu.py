@@ -141,3 +141,22 @@ def test_a_failed_call_leaves_every_layer_where_it_was(gpu, monkeypatch):
     monkeypatch.setattr(ops, "check", real)
     got = model.logits(token, False).clone()
     assert torch.equal(got, other.logits(token, False)) and [a.step for a, _ in model.layers] == [7, 7, 7]
+
+
+@pytest.mark.gpu
+def test_layers_with_rotary_tables_of_their_own(gpu, monkeypatch):
+    """A program may give an op another table (another base or scaling): each layer turns by its own."""
+    one, each = two_decoders(False, 3)
+    g = torch.Generator().manual_seed(2)
+    prompt, token = (torch.randint(0, 64, (3, n), generator=g).to(gpu) for n in (6, 1))
+    whole = ops.decode_layers
+    for m in (one, each):
+        m.logits(prompt, True)
+        table = m.layers[1][0].rope_table
+        m.layers[1][0].rope_table = table.flip(0).contiguous()
+    a = one.logits(token, False).clone()
+    monkeypatch.setattr(ops, "decode_layers", lambda *a: None)
+    assert torch.equal(a, each.logits(token, False))
+    each.layers[1][0].rope_table = table
+    each.layers[0][0].step, each.layers[1][0].step, each.layers[2][0].step = 6, 6, 6
+    assert not torch.equal(a, each.logits(token, False)) and whole is not ops.decode_layers
