@@ -21,6 +21,11 @@ inline int fail(int code, const char *fmt, ...)
     return code;
 }
 
+// glue.hip: eet_qkv_split, rotating by a caller's table (cos | sin of each position, [>= S][dh]) instead of its own
+// angles where one is given.
+int qkv_split(const void *qkv, void *q_out, void *k_cache, void *v_cache, int B, int S, int H, int dh, int rope,
+              int time_step, int t0, int T_cap, const float *rope_cos_sin, void *stream);
+
 }  // namespace eet
 
 #define EET_REQUIRE(cond, code, ...)              \

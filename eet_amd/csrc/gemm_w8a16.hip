@@ -1094,7 +1094,8 @@ extern "C" int eet_gemm_w8a16_qkv(const void *A, const void *Wpacked, const void
     args.epi = kEpiNone;
     if (int rc = run_gemm(args))
         return rc;
-    return eet_qkv_split(qkv, q_out, k_cache, v_cache, B, S, H, dh, rope_cos_sin != nullptr, -1, 0, T_cap, stream);
+    return eet::qkv_split(qkv, q_out, k_cache, v_cache, B, S, H, dh, rope_cos_sin != nullptr, -1, 0, T_cap, rope_cos_sin,
+                          stream);
 }
 
 extern "C" int eet_gemm_w8a16_chained(const void *A, const void *Wpacked, const void *scale, void *C, int M, int N,

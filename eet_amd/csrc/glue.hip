@@ -212,17 +212,24 @@ constexpr int kRopeMaxPairs = 128;  // head sizes up to 256 keep their angles in
 
 __global__ void qkv_split_kernel(const _Float16 *__restrict__ qkv, _Float16 *__restrict__ q_out,
                                  _Float16 *__restrict__ k_cache, _Float16 *__restrict__ v_cache, int S, int H,
-                                 int dh, int rope, int time_step, int t0, int T_cap)
+                                 int dh, int rope, int time_step, int t0, int T_cap, const float *__restrict__ cos_sin)
 {
     const int s = blockIdx.x, b = blockIdx.y;
     const int half_dh = dh / 2;
     const int per_head = half_dh / 4;  // threads per head
-    // All heads of a row turn by the same dh/2 angles: computed once per workgroup.
+    // All heads of a row turn by the same dh/2 angles: computed once per workgroup, or read from the caller's table.
     __shared__ float rot_cos[kRopeMaxPairs], rot_sin[kRopeMaxPairs];
     const bool table = rope && half_dh <= kRopeMaxPairs;
+    const int row = time_step >= 0 ? time_step : s;
+    const float *turns = cos_sin != nullptr ? cos_sin + (size_t)row * dh : nullptr;
     if (table) {
-        const float pos = (float)(time_step >= 0 ? time_step : s);
+        const float pos = (float)row;
         for (int i = threadIdx.x; i < half_dh; i += blockDim.x) {
+            if (turns != nullptr) {
+                rot_cos[i] = turns[i];
+                rot_sin[i] = turns[half_dh + i];
+                continue;
+            }
             const float ang = pos / powf(10000.0f, (float)(2 * i) / (float)dh);
             rot_cos[i] = cosf(ang);
             rot_sin[i] = sinf(ang);
@@ -239,13 +246,16 @@ __global__ void qkv_split_kernel(const _Float16 *__restrict__ qkv, _Float16 *__r
         half4 v1 = *reinterpret_cast<const half4 *>(qkv + src + 2 * (size_t)H * dh);
         half4 v2 = *reinterpret_cast<const half4 *>(qkv + src + 2 * (size_t)H * dh + half_dh);
         if (rope) {
-            const float pos = (float)(time_step >= 0 ? time_step : s);
+            const float pos = (float)row;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 float c, sn;
                 if (table) {
                     c = rot_cos[i0 + e];
                     sn = rot_sin[i0 + e];
+                } else if (turns != nullptr) {
+                    c = turns[i0 + e];
+                    sn = turns[half_dh + i0 + e];
                 } else {
                     const float ang = pos / powf(10000.0f, (float)(2 * (i0 + e)) / (float)dh);
                     c = cosf(ang);
@@ -430,8 +440,8 @@ extern "C" int eet_add_bias(void *out, const void *bias, int M, int N, void *str
     return EET_OK;
 }
 
-extern "C" int eet_qkv_split(const void *qkv, void *q_out, void *k_cache, void *v_cache, int B, int S, int H, int dh,
-                             int rope, int time_step, int t0, int T_cap, void *stream)
+int eet::qkv_split(const void *qkv, void *q_out, void *k_cache, void *v_cache, int B, int S, int H, int dh, int rope,
+                   int time_step, int t0, int T_cap, const float *rope_cos_sin, void *stream)
 {
     EET_REQUIRE(qkv && q_out && k_cache && v_cache, EET_ERR_INVALID_ARGUMENT, "eet_qkv_split: null pointer");
     EET_REQUIRE(B >= 0 && S >= 0 && H > 0 && dh > 0 && t0 >= 0, EET_ERR_INVALID_ARGUMENT,
@@ -447,9 +457,15 @@ extern "C" int eet_qkv_split(const void *qkv, void *q_out, void *k_cache, void *
     hipLaunchKernelGGL(qkv_split_kernel, dim3(S, B), dim3(threads), 0, static_cast<hipStream_t>(stream),
                        static_cast<const _Float16 *>(qkv), static_cast<_Float16 *>(q_out),
                        static_cast<_Float16 *>(k_cache), static_cast<_Float16 *>(v_cache), S, H, dh, rope, time_step,
-                       t0, T_cap);
+                       t0, T_cap, rope_cos_sin);
     EET_HIP_CHECK(hipGetLastError());
     return EET_OK;
+}
+
+extern "C" int eet_qkv_split(const void *qkv, void *q_out, void *k_cache, void *v_cache, int B, int S, int H, int dh,
+                             int rope, int time_step, int t0, int T_cap, void *stream)
+{
+    return eet::qkv_split(qkv, q_out, k_cache, v_cache, B, S, H, dh, rope, time_step, t0, T_cap, nullptr, stream);
 }
 
 static int elementwise_args(const char *fn, const void *a, const void *b, int M, int N)

@@ -100,3 +100,32 @@ def test_same_rotation_as_the_split_kernel(gpu, tuning, block):
                                            table.data_ptr() if rope else None, B, S, H, dh, K, S, None, 0, stream()))
             for name, a, b in zip("qkv", want, got):
                 assert torch.equal(a, b), f"{block} {B}x{S}x{H}x{dh} rope {rope}: {name}, {int((a != b).sum())} of {a.numel()} differ"
+
+
+@pytest.mark.parametrize("B,S,H,dh,K,off", [(1, 20, 4, 128, 512, 0), (2, 100, 3, 96, 256, 0), (2, 100, 3, 96, 256, 1),
+                                            (1, 33, 4, 32, 8192, 0), (1, 45, 2, 256, 4096, 0), (1, 9, 2, 320, 64, 0)])
+def test_every_route_turns_by_the_given_table(gpu, B, S, H, dh, K, off):
+    """Few rows, the epilogue, a table that is not 16-byte aligned, sizes that run as two launches, and a head too long for
+    the split kernel's LDS: rotated by the caller's cosines and sines.  Exact products, and in fp64 the two of a rotation:
+    one fp32 rounding of each factor's product and one to fp16 of a result no longer than the pair."""
+    N, M = 3 * H * dh, B * S
+    g = torch.Generator().manual_seed(S + dh)
+    x = torch.randint(-2, 3, (M, K), generator=g).half().to(gpu)
+    p = eet_amd.pack_weights(torch.randint(-127, 128, (K, N), generator=g).to(torch.int8)).to(gpu)
+    s = torch.full((N,), 2.0 ** -9, dtype=torch.float16, device=gpu)
+    angle = torch.arange(S)[:, None] / 500000.0 ** (torch.arange(dh // 2) / (dh // 2)) + 0.5
+    store = torch.empty(S * dh + 4, device=gpu)
+    table = store[off:off + S * dh].view(S, dh).copy_(torch.cat([angle.cos(), angle.sin()], 1))
+    rows = gemm(x, p, s, M, N, K).view(B, S, 3, H, dh).permute(2, 0, 3, 1, 4).double()
+    c, sn = (t.double().repeat(1, 2) for t in (table[:, :dh // 2], table[:, dh // 2:]))
+    turned = torch.cat([-rows[..., dh // 2:], rows[..., :dh // 2]], -1) * sn + rows * c
+    length = (rows ** 2 + torch.cat([rows[..., dh // 2:], rows[..., :dh // 2]], -1) ** 2).sqrt()
+    for ws_bytes in (0, lib().eet_gemm_w8a16_workspace(M, N, K, 0)):
+        ws = torch.zeros(max(ws_bytes, 4) // 4, dtype=torch.float32, device=gpu)
+        got, qkv = [torch.full((B, H, S, dh), GUARD, dtype=torch.float16, device=gpu) for _ in "qkv"], torch.empty(M, N).half().to(gpu)
+        check(lib().eet_gemm_w8a16_qkv(x.data_ptr(), p.data_ptr(), s.data_ptr(), qkv.data_ptr(), *(t.data_ptr() for t in got),
+                                       table.data_ptr(), B, S, H, dh, K, S, ws.data_ptr() if ws_bytes else None, ws_bytes,
+                                       stream()))
+        for a, want in zip(got[:2], turned[:2]):
+            assert ((a.double() - want).abs() <= length[0 if a is got[0] else 1] * (2 ** -11 + 2 ** -23) + 2 ** -25).all()
+        assert torch.equal(got[2].double(), rows[2])
