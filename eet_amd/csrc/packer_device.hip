@@ -273,7 +273,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
     using S = GroupShape<T>;
     __shared__ uint32_t part[WAVES][S::kGroup];
     __shared__ float s_all[S::kGroup], inv_all[S::kGroup];
-    __shared__ int flags[3];    // NaN among the weights; the exact path for all; the other parts did not arrive
+    __shared__ int flags[3];    // NaN among the weights; a column without a usable scale; the other parts did not arrive
     __shared__ uint32_t lq[WAVES][S::kGroup][9];   // [column][4-row word] of a unit, one word of padding per column
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int group = blockIdx.x / parts, mine = blockIdx.x % parts;
@@ -328,10 +328,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
         }
         return a;
     };
-    // the same from memory, without the weights that are NaN, for the units [from, to)
-    auto column_max_again = [&](int from, int to) {
+    // the same from memory, all units, without the weights that are NaN
+    auto column_max_again = [&]() {
         uint32_t m[4] = {0, 0, 0, 0};
-        for (int unit = from + wave; unit < to; unit += WAVES) {
+        for (int unit = wave; unit < 2 * ktiles; unit += WAVES) {
             const T *p = base + (size_t)(unit * kUnit + 4 * quad) * N;
 #pragma unroll
             for (int it = 0; it < 4; ++it) {
@@ -356,11 +356,25 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
         }
     constexpr uint32_t kInf = sizeof(T) == 2 ? 0x7c00u : 0x7f800000u;
     uint32_t a = column_max(m);
-    if (a > kInf)
-        flags[0] = flags[1] = 1;
+    const bool has_nan = a > kInf;
+    if (has_nan)
+        flags[0] = 1;
     __syncthreads();
-    if (flags[0])   // NaN weights are ignored, as on the host
-        a = column_max_again(unit0, unit1);
+    if (flags[0]) {   // NaN weights are ignored, as on the host
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+            m[d] = 0;
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u)
+            if (unit0 + wave + WAVES * u < unit1) {
+#pragma unroll
+                for (int it = 0; it < 4; ++it)
+#pragma unroll
+                    for (int d = 0; d < 4; ++d)
+                        m[d] = max_abs<T>(m[d], drop_nan<T>(v[u][it][d]));
+            }
+        a = column_max(m);
+    }
     if (parts > 1) {
         // the first wavefront holds every column's maximum: exchange, count up, wait for the other parts
         if (wave == 0) {
@@ -393,7 +407,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
         }
         __syncthreads();
         if (flags[2])   // a part is kept off the chip: its rows are read here
-            a = column_max_again(0, 2 * ktiles);
+            a = column_max_again();
     }
     if (threadIdx.x < S::kGroup) {
         float m;
@@ -403,19 +417,55 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
             m = __uint_as_float(a);
         const float s = ref128 ? m * (1.f / 128.f) : __fdiv_rn(m, 127.f);
         s_all[threadIdx.x] = s;
-        inv_all[threadIdx.x] = __fdiv_rn(1.f, s);
         if (mine == 0 && col0 + (int)threadIdx.x < N)
             scale[col0 + threadIdx.x] = static_cast<T>(s);
-        if (!(s > 0x1p-100f && s < 0x1p100f))
+        const bool usable = !has_nan && s > 0x1p-100f && s < 0x1p100f;
+        inv_all[threadIdx.x] = usable ? __fdiv_rn(1.f, s) : 0.f;
+        if (!usable)
             flags[1] = 1;
     }
     __syncthreads();
-    const bool odd = flags[1] != 0;
 
     float inv[S::kCols];
 #pragma unroll
     for (int i = 0; i < S::kCols; ++i)
         inv[i] = inv_all[c0 + i];
+    // The lane's columns without a usable scale (zero, tiny, huge, not finite, or with a NaN among these rows), and those
+    // that are such a column in any lane: their weights are divided one by one from the registers, and no others pay for
+    // that.  (us, two passes / the whole group read again and divided for one such column / now, a zero column in 32: 4096 x
+    // 4096 fp16 26.9 / 32.4 / 24.0, 5120 x 15360 82 / 114 / 81, 4096 x 11008 fp32 78 / 92 / 69.)
+    unsigned bare = 0, bare_any = 0;
+    if (flags[1] != 0) {
+#pragma unroll
+        for (int i = 0; i < S::kCols; ++i) {
+            bare |= (inv[i] == 0.f ? 1u : 0u) << i;
+            bare_any |= (__any(inv[i] == 0.f) ? 1u : 0u) << i;
+        }
+    }
+    auto divide_bare = [&](const u32x4 (&x)[4], uint32_t (&word)[S::kCols]) {
+        for (unsigned rest = bare_any; rest != 0; rest &= rest - 1) {
+            const int i = __builtin_ctz(rest), d = i * (int)sizeof(T) / 4;
+            const float s = s_all[c0 + i];
+            uint32_t o = 0;
+#pragma unroll
+            for (int it = 0; it < 4; ++it) {
+                uint32_t r = x[it][0];
+#pragma unroll
+                for (int k = 1; k < 4; ++k)
+                    r = d == k ? x[it][k] : r;
+                float xi;
+                if constexpr (sizeof(T) == 2)
+                    xi = (float)__builtin_bit_cast(_Float16, (uint16_t)(r >> (i % 2 * 16)));
+                else
+                    xi = __uint_as_float(r);
+                o |= (uint32_t)(quant_one(xi, s, nan_to, lo) + 128) << (8 * it);
+                __builtin_amdgcn_sched_barrier(0);   // one division at a time: four do not fit beside the matrix
+            }
+#pragma unroll
+            for (int k = 0; k < S::kCols; ++k)
+                word[k] = k == i && (bare >> k & 1) ? o : word[k];
+        }
+    };
 
     // the unit's words -- four rows of a column, q + 128 -- leave
     auto store = [&](const uint32_t (&word)[S::kCols], int unit) {
@@ -467,7 +517,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
     // 2^-17), and the correctly rounded quotient of the host is within 2^-17 of the exact one: unless v lies within
     // 2^-15 of a half, both round to the same integer.  The conversion rounds to nearest and clamps to 0 .. 255, i.e. +128
     // to 127.  Units with a weight near a half (one in eight of random weights) are left to the second loop, which reads
-    // them again and divides.
+    // them again and divides.  (A bare column's value is 128 or NaN here: not near, and the minimum skips a NaN.)
     constexpr float kNear = 0x1p-15f;
     unsigned again = 0;
 #pragma unroll
@@ -494,10 +544,16 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
                     : "v"(__builtin_amdgcn_fractf(f0) - 0.5f), "v"(__builtin_amdgcn_fractf(f1) - 0.5f));
             }
         }
-        if (odd || __any(near < kNear))
+#pragma unroll
+        for (int i = 0; i < S::kCols; ++i)
+            asm volatile("" : "+v"(word[i]));   // not after the branch, with all 32 quotients in registers
+        if (__any(near < kNear)) {
             again |= 1u << u;
-        else
-            store(word, unit);
+            continue;
+        }
+        if (bare_any != 0)
+            divide_bare(v[u], word);
+        store(word, unit);
     }
     while (again != 0) {
         const int u = __builtin_ctz(again), unit = unit0 + wave + WAVES * u;
@@ -517,12 +573,14 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
             for (int i = 0; i < S::kCols; ++i) {
                 const float xi = value_at<T>(x[it], i), f = __builtin_fmaf(xi, inv[i], 128.f);
                 word[i] = __builtin_amdgcn_cvt_pk_u8_f32(f, it, word[i]);
-                if (odd || __builtin_fabsf(__builtin_amdgcn_fractf(f) - 0.5f) < kNear) {
+                if (__builtin_fabsf(__builtin_amdgcn_fractf(f) - 0.5f) < kNear) {
                     const int t = quant_one(xi, s_all[c0 + i], nan_to, lo) + 128;
                     word[i] = (word[i] & ~(0xffu << (8 * it))) | (uint32_t)t << (8 * it);
                 }
             }
         }
+        if (bare_any != 0)
+            divide_bare(x, word);
         store(word, unit);
     }
 }

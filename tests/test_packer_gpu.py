@@ -184,3 +184,26 @@ def test_overlapping_calls_do_not_share_a_workspace(gpu, monkeypatch):
         torch.cuda.synchronize()
         for pair, other in zip(got, want):
             assert all(torch.equal(x, y) for x, y in zip(pair, other))
+
+
+@pytest.mark.parametrize("K,N", [(128, 80), (4096, 1040), (1280, 4096), (2048, 16400), (20480, 48)])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+def test_columns_without_a_scale(gpu, K, N, dtype):
+    """Zero, NaN, infinite, tiny and huge columns between ordinary ones, several of them and of the ordinary ones in every
+    lane's share, with a NaN in one part of the rows only: against the host packer, exact."""
+    rng = np.random.default_rng(K + N)
+    w = (rng.standard_normal((K, N)) * 0.02).astype(np.float32)
+    w[:, 1::7] = 0
+    w[:, 2::21] = np.nan
+    w[K - 3, 9::21] = np.nan
+    w[1, 16::21] = -np.nan
+    w[K // 2, 3::14] = np.inf
+    w[:, 10::14] *= 3e-6 if dtype == np.float16 else 1e-36
+    w[:, 4::14] *= 1e6 if dtype == np.float16 else 1e37
+    with np.errstate(over="ignore"):
+        w = torch.from_numpy(w.astype(dtype))
+    uh, ph, sh = eet_amd.quant_weights(w, torch.int8, True)
+    ud, pd, sd = eet_amd.quant_weights_device(w.to(gpu), True)
+    assert torch.equal(ud.cpu(), uh) and torch.equal(pd.cpu(), ph)
+    bits = torch.int16 if dtype == np.float16 else torch.int32
+    assert torch.equal(sd.cpu().view(bits), sh.view(bits))
