@@ -22,6 +22,7 @@
 #include <cstdint>
 
 #include "common.h"
+#include "tuning.h"
 
 namespace {
 
@@ -265,10 +266,9 @@ __device__ __forceinline__ float value_at(const u32x4 &v, int i)
 }
 
 template <typename T, int WAVES, int UNITS, bool QOUT>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4))) void quant_group_kernel(const T *__restrict__ w, int K, int N, int parts,
-                                                                 int ref128, uint32_t *maxima, uint32_t *arrived,
-                                                                 int8_t *__restrict__ q_out,
-                                                                 uint8_t *__restrict__ packed, T *__restrict__ scale)
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4))) void quant_group_kernel(
+    const T *__restrict__ w, int K, int N, int parts, int ref128, int max_polls, uint32_t *maxima, uint32_t *arrived,
+    int8_t *__restrict__ q_out, uint8_t *__restrict__ packed, T *__restrict__ scale)
 {
     using S = GroupShape<T>;
     __shared__ uint32_t part[WAVES][S::kGroup];
@@ -386,7 +386,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
             if (lane == 0)
                 __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             bool all = false;
-            for (int poll = 0; poll < kMaxPolls && !all; ++poll) {
+            for (int poll = 0; poll < max_polls && !all; ++poll) {
                 all = __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= (uint32_t)parts;
                 if (!all)
                     __builtin_amdgcn_s_sleep(8);
@@ -594,10 +594,11 @@ int launch_groups(const void *w, size_t K, size_t N, int parts, int ref128, int8
         hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, counts, n);
         EET_HIP_CHECK(hipGetLastError());
     }
+    const int limit = eet::tuning().pack_poll_limit;
     const auto kernel = q != nullptr ? quant_group_kernel<T, WAVES, UNITS, true> : quant_group_kernel<T, WAVES, UNITS, false>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)(groups * parts)), dim3(64 * WAVES), 0, st, static_cast<const T *>(w), (int)K,
-                       (int)N, parts, ref128, counts + n, counts, q, reinterpret_cast<uint8_t *>(packed),
-                       static_cast<T *>(scale));
+                       (int)N, parts, ref128, limit >= 0 ? limit : kMaxPolls, counts + n, counts, q,
+                       reinterpret_cast<uint8_t *>(packed), static_cast<T *>(scale));
     EET_HIP_CHECK(hipGetLastError());
     return EET_OK;
 }

@@ -57,6 +57,9 @@ int apply(const char *name, const char *value)
     else if (std::strcmp(name, "EET_CHAIN_SPIN_LIMIT") == 0) {
         t.chain_spin_limit = clear ? -1 : std::atoi(value);
         return EET_OK;
+    } else if (std::strcmp(name, "EET_PACK_POLL_LIMIT") == 0) {
+        t.pack_poll_limit = clear ? -1 : std::atoi(value);
+        return EET_OK;
     }
     if (slot == nullptr)
         return eet::fail(EET_ERR_INVALID_ARGUMENT, "eet_set_tuning: unknown key \"%s\"", name);
@@ -73,7 +76,7 @@ struct EnvInit {
             return;
         for (const char *name : {"EET_GEMM_SMALL_M_CONFIG", "EET_GEMM_LARGE_M_TILE", "EET_MMHA_NSPLIT",
                                  "EET_MMHA_THREADS", "EET_MMHA_UNROLL", "EET_PREFILL_LEGACY", "EET_PREFILL_SHAPE", "EET_PREFILL_GROUP",
-                                 "EET_CHAIN_SLEEP", "EET_CHAIN_SPIN_LIMIT"})
+                                 "EET_CHAIN_SLEEP", "EET_CHAIN_SPIN_LIMIT", "EET_PACK_POLL_LIMIT"})
             if (const char *v = std::getenv(name))
                 if (apply(name, v) != EET_OK)
                     std::fprintf(stderr, "[EET][WARN] %s\n", eet::last_error_slot().c_str());

@@ -25,6 +25,9 @@ struct Tuning {
     // EET_CHAIN_SPIN_LIMIT: polls before a chained wait gives up (-1: the default, 65536; 0 gives up at once);
     // EET_CHAIN_SLEEP: s_sleep(8) repetitions between two polls (0: the default, 1)
     int chain_spin_limit = -1, chain_sleep = 0;
+    // EET_PACK_POLL_LIMIT: polls before a workgroup of the one-pass packer stops waiting for the other parts of its
+    // columns and reads their rows itself (-1: the default, 16384; 0 at once)
+    int pack_poll_limit = -1;
 };
 
 const Tuning &tuning();

@@ -56,6 +56,7 @@ int eet_packed_layout_version(void);
  *   EET_PREFILL_GROUP "n" ((batch, head) pairs whose query blocks an XCD works on together in prefill
  *                         attention; "-1": every pair of a query block before the next block)
  *   EET_CHAIN_SPIN_LIMIT "n" / EET_CHAIN_SLEEP "n" (bounded wait of a chained launch)
+ *   EET_PACK_POLL_LIMIT "n" (bounded wait of the one-pass packer)
  * An override naming a kernel variant that does not exist is ignored.  The same
  * keys are read from the environment once, at load, when EET_HIP_TUNING=1; no
  * launch reads the environment (the reference queries occupancy and runs its

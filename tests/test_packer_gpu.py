@@ -207,3 +207,19 @@ def test_columns_without_a_scale(gpu, K, N, dtype):
     assert torch.equal(ud.cpu(), uh) and torch.equal(pd.cpu(), ph)
     bits = torch.int16 if dtype == np.float16 else torch.int32
     assert torch.equal(sd.cpu().view(bits), sh.view(bits))
+
+
+@pytest.mark.parametrize("K,N", [(128, 80), (2048, 96), (4096, 1040), (1280, 4096), (20480, 48), (2048, 16400)])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+def test_parts_that_do_not_wait(gpu, tuning, K, N, dtype):
+    """Every workgroup gives up its wait at once and reads the other parts' rows itself: the same bits, NaN and infinite
+    columns among them."""
+    w = tricky(K, N, dtype, K + N)
+    w[K // 2, 8::16], w[K - 1, 9], w[:, 10], w[5, 11], w[K - 2, 12] = np.nan, np.inf, np.nan, -np.nan, -np.inf
+    w = torch.from_numpy(w)
+    uh, ph, sh = eet_amd.quant_weights(w, torch.int8, True)
+    tuning("EET_PACK_POLL_LIMIT", 0)
+    ud, pd, sd = eet_amd.quant_weights_device(w.to(gpu), True)
+    assert torch.equal(ud.cpu(), uh) and torch.equal(pd.cpu(), ph)
+    bits = torch.int16 if dtype == np.float16 else torch.int32
+    assert torch.equal(sd.cpu().view(bits), sh.view(bits))
