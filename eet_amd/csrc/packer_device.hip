@@ -229,6 +229,7 @@ template <typename T>
 struct GroupShape {
     static constexpr int kCols = 16 / (int)sizeof(T);   // columns of a lane
     static constexpr int kGroup = 8 * kCols;            // columns of a group: 128 bytes of a row
+    static constexpr int kLine = 128 / kGroup;          // groups that share a cache line of int8
 };
 
 // largest of |x| over the register's values as unsigned integers, which order like them (NaN above everything)
@@ -276,7 +277,17 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
     __shared__ int flags[3];    // NaN among the weights; a column without a usable scale; the other parts did not arrive
     __shared__ uint32_t lq[WAVES][S::kGroup][9];   // [column][4-row word] of a unit, one word of padding per column
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int group = blockIdx.x / parts, mine = blockIdx.x % parts;
+    int group = blockIdx.x / parts, mine = blockIdx.x % parts;
+    if constexpr (QOUT && S::kLine > 2) {
+        // From fp32 a row of a group is a quarter of a cache line of q: the groups of a line follow one another on one XCD,
+        // whose L2 puts the line together.  (us, two passes / scattered over the XCDs / now: 14336 x 11008 297 / 333 / 296,
+        // 11008 x 4096 87 / 90 / 82, 14336 x 14336 380 / 352 / 323.  Halves of a line, from fp16, gain nothing.)
+        const int xcd = blockIdx.x % 8, turn = blockIdx.x / 8, id = turn / S::kLine * 8 + xcd;
+        group = id / parts * S::kLine + turn % S::kLine;
+        mine = id % parts;
+        if (group * S::kGroup >= N)
+            return;
+    }
     const int ktiles = K / 64, kt0 = (int)((long)mine * ktiles / parts), kt1 = (int)((long)(mine + 1) * ktiles / parts);
     const int col0 = group * S::kGroup, quad = lane >> 3, c0 = (lane & 7) * S::kCols;
     const bool cols_in = col0 + c0 < N;    // N % 16 == 0: a lane's columns are in range together
@@ -596,9 +607,11 @@ int launch_groups(const void *w, size_t K, size_t N, int parts, int ref128, int8
     }
     const int limit = eet::tuning().pack_poll_limit;
     const auto kernel = q != nullptr ? quant_group_kernel<T, WAVES, UNITS, true> : quant_group_kernel<T, WAVES, UNITS, false>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(groups * parts)), dim3(64 * WAVES), 0, st, static_cast<const T *>(w), (int)K,
-                       (int)N, parts, ref128, limit >= 0 ? limit : kMaxPolls, counts + n, counts, q,
-                       reinterpret_cast<uint8_t *>(packed), static_cast<T *>(scale));
+    constexpr size_t kLine = GroupShape<T>::kLine;
+    const size_t grid = q != nullptr && kLine > 2 ? ((groups + kLine - 1) / kLine * parts + 7) / 8 * 8 * kLine : groups * parts;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * WAVES), 0, st, static_cast<const T *>(w), (int)K, (int)N, parts,
+                       ref128, limit >= 0 ? limit : kMaxPolls, counts + n, counts, q, reinterpret_cast<uint8_t *>(packed),
+                       static_cast<T *>(scale));
     EET_HIP_CHECK(hipGetLastError());
     return EET_OK;
 }

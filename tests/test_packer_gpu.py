@@ -223,3 +223,14 @@ def test_parts_that_do_not_wait(gpu, tuning, K, N, dtype):
     assert torch.equal(ud.cpu(), uh) and torch.equal(pd.cpu(), ph)
     bits = torch.int16 if dtype == np.float16 else torch.int32
     assert torch.equal(sd.cpu().view(bits), sh.view(bits))
+
+
+@pytest.mark.parametrize("N", [16, 32, 48, 112, 128, 144, 1040, 2064, 4112, 16400])
+@pytest.mark.parametrize("K", [64, 320, 2624])
+def test_unprocessed_output_at_every_place_in_a_line(gpu, K, N):
+    """fp32 with the row-major output, whose workgroups are numbered by cache lines of that output: lines that N cuts off,
+    fewer lines than XCDs and more, one part and several."""
+    w = torch.from_numpy(tricky(K, max(N, 8), np.float32, K + N)[:, :N])
+    uh, ph, sh = eet_amd.quant_weights(w.contiguous(), torch.int8, True)
+    ud, pd, sd = eet_amd.quant_weights_device(w.contiguous().to(gpu), True)
+    assert torch.equal(ud.cpu(), uh) and torch.equal(pd.cpu(), ph) and torch.equal(sd.cpu().view(torch.int32), sh.view(torch.int32))
