@@ -626,7 +626,7 @@ int launch_groups(const void *w, size_t K, size_t N, int parts, int ref128, int8
 bool one_pass_wins(size_t K, size_t N, size_t size)
 {
     const size_t n = K * N;
-    return N < ((size_t)1 << 31) && (size == 4 || n <= 36000000 || n >= 70000000);   // its column indices are 32 bits wide
+    return size == 4 || n <= 36000000 || n >= 70000000;
 }
 
 // How many workgroups share a column group: as many as its rows need, and as many as the chip still takes in one round.
@@ -638,19 +638,37 @@ int parts_of(size_t units, size_t groups, int waves, int held, size_t slots)
     return (int)(parts > need ? parts : need);
 }
 
+// What a call runs as: wavefronts of a workgroup and workgroups of a column group, or no wavefronts for two passes.
+struct PackPlan {
+    int waves, parts;
+};
+
+template <typename T>
+PackPlan plan_pack(size_t K, size_t N, size_t ws_bytes)
+{
+    const PackPlan two_passes = {0, 0};
+    if (ws_bytes < eet_quantize_pack_device_workspace(N) || !one_pass_wins(K, N, sizeof(T)))
+        return two_passes;
+    const size_t units = K / kUnit, groups = (N + GroupShape<T>::kGroup - 1) / GroupShape<T>::kGroup;
+    const int wide = parts_of(units, groups, 16, 4, 256), narrow = parts_of(units, groups, 8, 5, 512);
+    if (wide <= kMaxParts && groups * wide <= 256)
+        return {16, wide};
+    // threads of a grid are counted in 32 bits (and the kernel's column indices are int); a row of workgroups to spare
+    if (narrow > kMaxParts || groups * narrow >= ((size_t)1 << 32) / (64 * 8) - 64)
+        return two_passes;
+    return {8, narrow};
+}
+
 template <typename T>
 int run(const void *w, size_t K, size_t N, int mode, int8_t *q, int8_t *packed, void *scale, uint32_t *ws, size_t ws_bytes,
         hipStream_t st)
 {
     const int ref128 = mode == EET_QUANT_REF128 ? 1 : 0;
-    if (ws_bytes >= eet_quantize_pack_device_workspace(N) && one_pass_wins(K, N, sizeof(T))) {
-        const size_t units = K / kUnit, groups = (N + GroupShape<T>::kGroup - 1) / GroupShape<T>::kGroup;
-        const int wide = parts_of(units, groups, 16, 4, 256), narrow = parts_of(units, groups, 8, 5, 512);
-        if (wide <= kMaxParts && groups * wide <= 256)
-            return launch_groups<T, 16, 4>(w, K, N, wide, ref128, q, packed, scale, ws, st);
-        if (narrow <= kMaxParts)
-            return launch_groups<T, 8, 5>(w, K, N, narrow, ref128, q, packed, scale, ws, st);
-    }
+    const PackPlan plan = plan_pack<T>(K, N, ws_bytes);
+    if (plan.waves == 16)
+        return launch_groups<T, 16, 4>(w, K, N, plan.parts, ref128, q, packed, scale, ws, st);
+    if (plan.waves == 8)
+        return launch_groups<T, 8, 5>(w, K, N, plan.parts, ref128, q, packed, scale, ws, st);
     hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, ws, N);
     EET_HIP_CHECK(hipGetLastError());
     const dim3 g1((unsigned)((N + 64 * kColsPerThread - 1) / (64 * kColsPerThread)),
@@ -673,19 +691,38 @@ extern "C" size_t eet_quantize_pack_device_workspace(size_t N)
     return ((N + 31) / 32 * kCountStride + (N + 63) / 64 * 64 * kMaxParts) * sizeof(uint32_t);
 }
 
+static int check_pack_args(const char *fn, int w_dtype, size_t K, size_t N)
+{
+    EET_REQUIRE(w_dtype == EET_DTYPE_F32 || w_dtype == EET_DTYPE_F16, EET_ERR_INVALID_ARGUMENT,
+                "%s: w_dtype must be EET_DTYPE_F32 or EET_DTYPE_F16, got %d", fn, w_dtype);
+    EET_REQUIRE(K > 0 && N > 0 && K % 64 == 0 && N % 16 == 0, EET_ERR_UNSUPPORTED_SHAPE,
+                "%s: need K %% 64 == 0 and N %% 16 == 0, got K=%zu N=%zu", fn, K, N);
+    EET_REQUIRE(K / 64 <= 65535 && (K + kMaxRows - 1) / kMaxRows <= 65535, EET_ERR_UNSUPPORTED_SHAPE,
+                "%s: K = %zu exceeds the grid limit", fn, K);
+    return EET_OK;
+}
+
+extern "C" int eet_quantize_pack_device_shape(int w_dtype, size_t K, size_t N, size_t workspace_bytes, int *waves, int *parts)
+{
+    const char *fn = "eet_quantize_pack_device_shape";
+    EET_REQUIRE(waves && parts, EET_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
+    if (int rc = check_pack_args(fn, w_dtype, K, N))
+        return rc;
+    const PackPlan plan = w_dtype == EET_DTYPE_F32 ? plan_pack<float>(K, N, workspace_bytes)
+                                                   : plan_pack<_Float16>(K, N, workspace_bytes);
+    *waves = plan.waves, *parts = plan.parts;
+    return EET_OK;
+}
+
 extern "C" int eet_quantize_pack_device(const void *w, int w_dtype, size_t K, size_t N, int mode, int8_t *q,
                                         int8_t *packed, void *scale, void *workspace, size_t workspace_bytes,
                                         void *stream)
 {
     EET_REQUIRE(w && packed && scale, EET_ERR_INVALID_ARGUMENT, "eet_quantize_pack_device: null pointer");
-    EET_REQUIRE(w_dtype == EET_DTYPE_F32 || w_dtype == EET_DTYPE_F16, EET_ERR_INVALID_ARGUMENT,
-                "eet_quantize_pack_device: w_dtype must be EET_DTYPE_F32 or EET_DTYPE_F16, got %d", w_dtype);
+    if (int rc = check_pack_args("eet_quantize_pack_device", w_dtype, K, N))
+        return rc;
     EET_REQUIRE(mode == EET_QUANT_REF128 || mode == EET_QUANT_SYM127, EET_ERR_INVALID_ARGUMENT,
                 "eet_quantize_pack_device: unknown mode %d", mode);
-    EET_REQUIRE(K > 0 && N > 0 && K % 64 == 0 && N % 16 == 0, EET_ERR_UNSUPPORTED_SHAPE,
-                "eet_quantize_pack_device: need K %% 64 == 0 and N %% 16 == 0, got K=%zu N=%zu", K, N);
-    EET_REQUIRE(K / 64 <= 65535 && (K + kMaxRows - 1) / kMaxRows <= 65535, EET_ERR_UNSUPPORTED_SHAPE,
-                "eet_quantize_pack_device: K = %zu exceeds the grid limit", K);
     EET_REQUIRE((reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(packed)) % 16 == 0 &&
                     (q == nullptr || reinterpret_cast<uintptr_t>(q) % 8 == 0),
                 EET_ERR_INVALID_ARGUMENT, "eet_quantize_pack_device: w and packed need 16-byte, q 8-byte alignment");

@@ -106,14 +106,18 @@ int eet_unprocess_ref_sm80(const int8_t *processed, size_t K, size_t N, int8_t *
  * eet_quantize_pack_device_workspace(N) bytes of device memory, any contents;
  * 4 N bytes are enough and make every call read the matrix twice.  Workgroups
  * of a call meet in it: calls that can overlap in time must not share one.
- * The reference
- * quantises on one host core only (cutlass_preprocessors.cc:581-678, reached
- * from fpA_intB_gemm_wrapper.cu:26-105, which rejects CUDA tensors at :33);
- * this entry point has no counterpart there. */
+ * The reference quantises on one host core only (cutlass_preprocessors.cc:581-678,
+ * reached from fpA_intB_gemm_wrapper.cu:26-105, which rejects CUDA tensors at
+ * :33); this entry point has no counterpart there. */
 size_t eet_quantize_pack_device_workspace(size_t N);
 int eet_quantize_pack_device(const void *w, int w_dtype, size_t K, size_t N, int mode,
                              int8_t *q, int8_t *packed, void *scale, void *workspace,
                              size_t workspace_bytes, void *stream);
+/* What such a call runs as: the wavefronts of a workgroup (16 or 8) and how many
+ * workgroups share a group of columns (128 bytes of a row) in the one-pass kernel, or
+ * waves = 0 for two passes.  Decided on the host; nothing is launched. */
+int eet_quantize_pack_device_shape(int w_dtype, size_t K, size_t N, size_t workspace_bytes,
+                                   int *waves, int *parts);
 
 /* C[M][N] (half) = A[M][K] (half) . (int8 W[K][N] * scale[N] (half)), fp32
  * accumulation, one rounding to half.  Wpacked comes from eet_pack_gfx950.

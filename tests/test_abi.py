@@ -227,3 +227,35 @@ def test_shares_are_counted_per_xcd(M, N, K):
     tm, tn, wm, wn, ks = large_m_shape(M, N, K, 1, ws)
     blocks = -(-M // (16 * tm * wm)) * -(-N // (16 * tn * wn))
     assert ks > 1 and blocks * ks <= 256 and -(-blocks // 8) * ks <= 32
+
+
+def pack_shape(w_dtype, K, N, ws=None):
+    L, v = _lib.lib(), [ctypes.c_int() for _ in range(2)]
+    ws = L.eet_quantize_pack_device_workspace(N) if ws is None else ws
+    assert L.eet_quantize_pack_device_shape(w_dtype, K, N, ws, *[ctypes.byref(x) for x in v]) == 0
+    return tuple(x.value for x in v)
+
+
+def test_packer_grids_and_workspace():
+    """Every launch the one-pass packer plans: at most 16 parts, rows that its wavefronts hold, fewer threads than the 32
+    bits they are counted in, and counts and maxima within the workspace.  fp32 N = 2^28 once had a grid of 2^32 threads."""
+    for K in (64, 128, 192, 320, 1024, 4096, 20480, 20544, 28672, 32768, 65536):
+        for N in (16, 48, 1040, 4096, 16400, 151936, 1 << 22, (1 << 22) + 16, 1 << 26, 1 << 27, 1 << 28, 1 << 29, 1 << 30,
+                  (1 << 31) - 16, 1 << 31, 1 << 33):
+            for w_dtype, columns in ((0, 32), (1, 64)):
+                waves, parts = pack_shape(w_dtype, K, N)
+                assert pack_shape(w_dtype, K, N, 4 * N) == (0, 0)
+                if not waves:
+                    continue
+                groups = -(-N // columns)
+                per_part = -(-(K // 64) // parts) * 2            # units of 32 rows, whole k-tiles
+                assert parts <= 16 and waves * {16: 4, 8: 5}[waves] >= per_part, (K, N, w_dtype)
+                lines = 128 // columns
+                grid = max(groups * parts, -(-(-(-groups // lines) * parts) // 8) * 8 * lines)
+                assert grid * waves * 64 < 1 << 32 and N < 1 << 31, (K, N, w_dtype)
+                words = groups * 32 + groups * parts * columns
+                assert words * 4 <= _lib.lib().eet_quantize_pack_device_workspace(N), (K, N, w_dtype)
+    L, v = _lib.lib(), [ctypes.byref(ctypes.c_int()) for _ in range(2)]
+    for bad in ((5, 64, 16, 64), (0, 96, 16, 64), (0, 64, 24, 64), (1, 0, 16, 64)):
+        assert L.eet_quantize_pack_device_shape(*bad, *v) < 0
+    assert L.eet_quantize_pack_device_shape(0, 64, 16, 64, None, v[1]) == -1
