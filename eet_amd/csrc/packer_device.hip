@@ -616,17 +616,34 @@ int launch_groups(const void *w, size_t K, size_t N, int parts, int ref128, int8
     return EET_OK;
 }
 
-// One pass or two.  fp32: always one (us, two passes / one: 4096 x 4096 31 / 23.5, 11008 x 4096 75 / 59, 5120 x 13696 120 /
-// 87, 16384 x 16384 472 / 286).  fp16 has twice the weights to a byte, so that the quantising of a workgroup's share, which
-// nothing overlaps where the grid fits the chip once, weighs more.  Up to 36 M weights one pass wins by its two launches
-// less (1024 x 1024 17.3 / 14.0, 4096 x 4096 24.3 / 20.1, 16384 x 1024 24.5 / 20.2, 6144 x 4096 30.1 / 27.7), from there the
-// registers of the chip no longer hold the matrix in one round, while the second pass of the other way is read from the
-// Infinity Cache (11008 x 4096 44.8 / 51.4, 4096 x 12288 47.1 / 52.4, 16384 x 4096 64.9 / 66.9); with more rounds, and
-// what does not fit that cache, one pass is ahead again (5120 x 13696 69.6 / 66.4, 16384 x 16384 268 / 219).
-bool one_pass_wins(size_t K, size_t N, size_t size)
+// One pass or two, measured at some 700 sizes (K 64 .. 32768, N 16 .. 262144, up to 450 M weights, from HBM); us, two
+// passes / one.
+// fp32: one (4096 x 4096 31 / 23.5, 5120 x 13696 120 / 87, 16384 x 16384 472 / 286).
+// fp16 has twice the weights to a byte, so that the quantising of a workgroup's share, which nothing overlaps where the grid
+// fits the chip once, weighs more.  Up to 36 M weights one pass wins by its two launches less (1024 x 1024 12.5 / 9.9, 4096
+// x 4096 25.7 / 22.1, 16384 x 1024 25.3 / 22.5, 0.92 of the time in the mean from 28 M on); from there the registers of the
+// chip no longer hold every matrix in one round, while the second pass of the other way is read from the Infinity Cache
+// (some forty sizes of 40-50 M 0.93 .. 1.10, 1.01 in the mean); with more rounds, and what does not fit that cache, one pass is ahead
+// again (0.94 at 70 M, 5120 x 15360 78.8 / 75.8, 8192 x 32000 261 / 198).  Behind by more than 4 % it is nowhere but at
+// 20480 x 4096 (81 / 87).
+// fp16 with the row-major output, whose stores are half lines of rows: only where the whole matrix is in the 16-wavefront
+// form (4096 x 4096 28.6 / 25.0) or small (512 x 22016 23.9 / 16.9); above, it is anything from 0.82 (8192 x 32000) to 1.22
+// (2560 x 12288 43 / 53; 20480 x 4096 100 / 122, 4096 x 32768 162 / 186).
+// Either type: rows for less than a unit per wavefront leave the workgroups nearly empty, which counts once there are many
+// of them (K = 64: N 50272 0.74-0.81, 98304 0.99-1.09, 262144 1.40; K = 128: 151936 0.86, 262144 1.05; K = 256 never).
+// fp16 with more than 20480 rows and few columns: the parts of a group end at 16 (28672 x 128 1.13, 32768 x 256 1.19, x 640
+// 0.95; 20480 x 256 1.00).
+template <typename T>
+bool one_pass_wins(size_t K, size_t N, bool unprocessed, bool wide)
 {
-    const size_t n = K * N;
-    return size == 4 || n <= 36000000 || n >= 70000000;
+    const size_t n = K * N, units = K / kUnit, groups = (N + GroupShape<T>::kGroup - 1) / GroupShape<T>::kGroup;
+    if (units < 8 && groups > 800 * units)
+        return false;
+    if (sizeof(T) == 4)
+        return true;
+    if (units > 640 && groups <= 8)
+        return false;
+    return unprocessed ? n <= (wide ? 24000000 : 15000000) : n <= 36000000 || n >= 70000000;
 }
 
 // How many workgroups share a column group: as many as its rows need, and as many as the chip still takes in one round.
@@ -644,19 +661,16 @@ struct PackPlan {
 };
 
 template <typename T>
-PackPlan plan_pack(size_t K, size_t N, size_t ws_bytes)
+PackPlan plan_pack(size_t K, size_t N, bool unprocessed, size_t ws_bytes)
 {
-    const PackPlan two_passes = {0, 0};
-    if (ws_bytes < eet_quantize_pack_device_workspace(N) || !one_pass_wins(K, N, sizeof(T)))
-        return two_passes;
     const size_t units = K / kUnit, groups = (N + GroupShape<T>::kGroup - 1) / GroupShape<T>::kGroup;
     const int wide = parts_of(units, groups, 16, 4, 256), narrow = parts_of(units, groups, 8, 5, 512);
-    if (wide <= kMaxParts && groups * wide <= 256)
-        return {16, wide};
-    // threads of a grid are counted in 32 bits (and the kernel's column indices are int); a row of workgroups to spare
-    if (narrow > kMaxParts || groups * narrow >= ((size_t)1 << 32) / (64 * 8) - 64)
-        return two_passes;
-    return {8, narrow};
+    const bool fits = wide <= kMaxParts && groups * wide <= 256;
+    // (threads of a grid are counted in 32 bits, and the kernel's column indices are int; a row of workgroups to spare)
+    if (ws_bytes < eet_quantize_pack_device_workspace(N) || !one_pass_wins<T>(K, N, unprocessed, fits) ||
+        (!fits && (narrow > kMaxParts || groups * narrow >= ((size_t)1 << 32) / (64 * 8) - 64)))
+        return {0, 0};
+    return fits ? PackPlan{16, wide} : PackPlan{8, narrow};
 }
 
 template <typename T>
@@ -664,7 +678,7 @@ int run(const void *w, size_t K, size_t N, int mode, int8_t *q, int8_t *packed, 
         hipStream_t st)
 {
     const int ref128 = mode == EET_QUANT_REF128 ? 1 : 0;
-    const PackPlan plan = plan_pack<T>(K, N, ws_bytes);
+    const PackPlan plan = plan_pack<T>(K, N, q != nullptr, ws_bytes);
     if (plan.waves == 16)
         return launch_groups<T, 16, 4>(w, K, N, plan.parts, ref128, q, packed, scale, ws, st);
     if (plan.waves == 8)
@@ -702,14 +716,15 @@ static int check_pack_args(const char *fn, int w_dtype, size_t K, size_t N)
     return EET_OK;
 }
 
-extern "C" int eet_quantize_pack_device_shape(int w_dtype, size_t K, size_t N, size_t workspace_bytes, int *waves, int *parts)
+extern "C" int eet_quantize_pack_device_shape(int w_dtype, size_t K, size_t N, int unprocessed, size_t workspace_bytes,
+                                              int *waves, int *parts)
 {
     const char *fn = "eet_quantize_pack_device_shape";
     EET_REQUIRE(waves && parts, EET_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
     if (int rc = check_pack_args(fn, w_dtype, K, N))
         return rc;
-    const PackPlan plan = w_dtype == EET_DTYPE_F32 ? plan_pack<float>(K, N, workspace_bytes)
-                                                   : plan_pack<_Float16>(K, N, workspace_bytes);
+    const PackPlan plan = w_dtype == EET_DTYPE_F32 ? plan_pack<float>(K, N, unprocessed != 0, workspace_bytes)
+                                                   : plan_pack<_Float16>(K, N, unprocessed != 0, workspace_bytes);
     *waves = plan.waves, *parts = plan.parts;
     return EET_OK;
 }

@@ -113,11 +113,12 @@ size_t eet_quantize_pack_device_workspace(size_t N);
 int eet_quantize_pack_device(const void *w, int w_dtype, size_t K, size_t N, int mode,
                              int8_t *q, int8_t *packed, void *scale, void *workspace,
                              size_t workspace_bytes, void *stream);
-/* What such a call runs as: the wavefronts of a workgroup (16 or 8) and how many
- * workgroups share a group of columns (128 bytes of a row) in the one-pass kernel, or
- * waves = 0 for two passes.  Decided on the host; nothing is launched. */
-int eet_quantize_pack_device_shape(int w_dtype, size_t K, size_t N, size_t workspace_bytes,
-                                   int *waves, int *parts);
+/* What such a call, with q or without (unprocessed), runs as: the wavefronts of a
+ * workgroup (16 or 8) and how many workgroups share a group of columns (128 bytes of a
+ * row) in the one-pass kernel, or waves = 0 for two passes.  Decided on the host;
+ * nothing is launched. */
+int eet_quantize_pack_device_shape(int w_dtype, size_t K, size_t N, int unprocessed,
+                                   size_t workspace_bytes, int *waves, int *parts);
 
 /* C[M][N] (half) = A[M][K] (half) . (int8 W[K][N] * scale[N] (half)), fp32
  * accumulation, one rounding to half.  Wpacked comes from eet_pack_gfx950.

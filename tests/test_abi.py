@@ -229,10 +229,10 @@ def test_shares_are_counted_per_xcd(M, N, K):
     assert ks > 1 and blocks * ks <= 256 and -(-blocks // 8) * ks <= 32
 
 
-def pack_shape(w_dtype, K, N, ws=None):
+def pack_shape(w_dtype, K, N, ws=None, unprocessed=0):
     L, v = _lib.lib(), [ctypes.c_int() for _ in range(2)]
     ws = L.eet_quantize_pack_device_workspace(N) if ws is None else ws
-    assert L.eet_quantize_pack_device_shape(w_dtype, K, N, ws, *[ctypes.byref(x) for x in v]) == 0
+    assert L.eet_quantize_pack_device_shape(w_dtype, K, N, unprocessed, ws, *[ctypes.byref(x) for x in v]) == 0
     return tuple(x.value for x in v)
 
 
@@ -242,8 +242,8 @@ def test_packer_grids_and_workspace():
     for K in (64, 128, 192, 320, 1024, 4096, 20480, 20544, 28672, 32768, 65536):
         for N in (16, 48, 1040, 4096, 16400, 151936, 1 << 22, (1 << 22) + 16, 1 << 26, 1 << 27, 1 << 28, 1 << 29, 1 << 30,
                   (1 << 31) - 16, 1 << 31, 1 << 33):
-            for w_dtype, columns in ((0, 32), (1, 64)):
-                waves, parts = pack_shape(w_dtype, K, N)
+            for w_dtype, columns, unprocessed in ((0, 32, 0), (0, 32, 1), (1, 64, 0), (1, 64, 1)):
+                waves, parts = pack_shape(w_dtype, K, N, None, unprocessed)
                 assert pack_shape(w_dtype, K, N, 4 * N) == (0, 0)
                 if not waves:
                     continue
@@ -256,6 +256,16 @@ def test_packer_grids_and_workspace():
                 words = groups * 32 + groups * parts * columns
                 assert words * 4 <= _lib.lib().eet_quantize_pack_device_workspace(N), (K, N, w_dtype)
     L, v = _lib.lib(), [ctypes.byref(ctypes.c_int()) for _ in range(2)]
-    for bad in ((5, 64, 16, 64), (0, 96, 16, 64), (0, 64, 24, 64), (1, 0, 16, 64)):
+    for bad in ((5, 64, 16, 0, 64), (0, 96, 16, 0, 64), (0, 64, 24, 1, 64), (1, 0, 16, 1, 64)):
         assert L.eet_quantize_pack_device_shape(*bad, *v) < 0
-    assert L.eet_quantize_pack_device_shape(0, 64, 16, 64, None, v[1]) == -1
+    assert L.eet_quantize_pack_device_shape(0, 64, 16, 0, 64, None, v[1]) == -1
+
+
+@pytest.mark.parametrize("w_dtype,K,N,unprocessed,waves", [
+    (1, 4096, 4096, 0, 16), (1, 1024, 32000, 0, 8), (1, 11008, 4096, 0, 0), (1, 5120, 15360, 0, 8), (1, 28672, 256, 0, 0),
+    (1, 28672, 1024, 0, 16), (1, 4096, 4096, 1, 16), (1, 2560, 12288, 1, 0), (1, 512, 22016, 1, 8), (1, 5120, 15360, 1, 0),
+    (1, 64, 64000, 0, 8), (1, 64, 128256, 0, 0), (0, 64, 128256, 0, 0), (0, 256, 128256, 0, 8), (0, 28672, 256, 0, 16),
+    (0, 14336, 11008, 1, 8), (0, 28672, 4096, 0, 0)])
+def test_packer_takes_the_faster_way(w_dtype, K, N, unprocessed, waves):
+    """Either side of every line of the rule."""
+    assert pack_shape(w_dtype, K, N, None, unprocessed)[0] == waves

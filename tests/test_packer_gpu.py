@@ -234,3 +234,32 @@ def test_unprocessed_output_at_every_place_in_a_line(gpu, K, N):
     uh, ph, sh = eet_amd.quant_weights(w.contiguous(), torch.int8, True)
     ud, pd, sd = eet_amd.quant_weights_device(w.contiguous().to(gpu), True)
     assert torch.equal(ud.cpu(), uh) and torch.equal(pd.cpu(), ph) and torch.equal(sd.cpu().view(torch.int32), sh.view(torch.int32))
+
+
+@pytest.mark.parametrize("K,N,parts", [(64, 16400, 1), (512, 22016, 1), (1088, 16464, 1), (2048, 16400, 2), (1024, 32000, 1),
+                                       (3072, 9232, 3), (5120, 6144, 5), (5120, 13696, 4), (13696, 5120, 11)])
+def test_eight_wavefronts_fp16(gpu, K, N, parts):
+    """fp16 in the 8-wavefront form, with one part and several, one round of workgroups and more, groups cut off by N and by
+    the rows a wavefront holds: the result of the two passes, which a call with 4 N bytes of workspace takes and which the
+    other tests hold to the host packer.  With the row-major output too where that takes the form."""
+    import ctypes
+    from eet_amd._lib import check, lib
+    g = torch.Generator(device=gpu).manual_seed(K + N)
+    w = torch.randn(K, N, generator=g, device=gpu, dtype=torch.float16) * 0.02
+    w[:, 1::67] = 0
+    w[K // 2, 8::131], w[K - 1, 9] = float("nan"), float("inf")
+    need, form = lib().eet_quantize_pack_device_workspace(N), [ctypes.c_int() for _ in range(2)]
+
+    def run(nbytes, want_q):
+        ws = torch.full((nbytes // 4 + 256,), -1, dtype=torch.int32, device=gpu)
+        q, p, s = (torch.zeros(*shape, dtype=t, device=gpu) for shape, t in (((K, N), torch.int8), ((K, N), torch.int8),
+                                                                             ((N,), torch.float16)))
+        check(lib().eet_quantize_pack_device(w.data_ptr(), 1, K, N, 0, q.data_ptr() if want_q else None, p.data_ptr(),
+                                             s.data_ptr(), ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream))
+        assert (ws[nbytes // 4:] == -1).all()
+        return q, p, s.view(torch.int16)
+    for want_q in (0, 1):
+        check(lib().eet_quantize_pack_device_shape(1, K, N, want_q, need, *[ctypes.byref(x) for x in form]))
+        assert [x.value for x in form] == [8, parts] or (want_q and form[0].value == 0)
+        for one, two in zip(run(need, want_q), run(4 * N, want_q)):
+            assert torch.equal(one, two)
