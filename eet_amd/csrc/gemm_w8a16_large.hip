@@ -526,9 +526,10 @@ int launch_large_m(const GemmArgs &a, int ksplit)
 // against 34.7 for what is taken now).  Fitted, shape by shape, to 14300 launches on MI355X: 20 weight matrices of
 // decoders 1024 .. 5120 wide, 40 .. 8192 rows, one to eight shares of the k range; a fit is a fit: some of its
 // constants (a store or residual of nothing, two workgroups cheaper than one and a bit) mean nothing by themselves.
-// Checked against launches that are not in it (649 problems: those matrices at 25 row counts 33 .. 8192 and six
-// matrices 1536 and 8192 wide): on average 1.5 % behind the fastest of the 20 shapes and their shares, at most 25 %;
-// the same on the widths outside the fit.
+// Fitted and checked with stores straight from the accumulators, before blocks left through LDS (649 problems outside the
+// fit: those matrices at 25 row counts 33 .. 8192 and six matrices 1536 and 8192 wide: on average 1.5 % behind the fastest
+// of the 20 shapes and their shares, at most 25 %, the same on the widths outside the fit).  With the epilogue as it is
+// (229 problems, 17 matrices, 48 .. 8192 rows): 1.9 % and 16 %; other store terms gain 0.1 %.
 struct TileCost {
     int tm, tn, wm, wn;
     float base, store, res, per_tile[11];

@@ -80,7 +80,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const _Float16 *_
 // ---------------------------------------------------------------------------
 // Token embedding of a decode step: out[r] = table[ids[r]], a workgroup per row.  torch's gather of up to 16 rows walks
 // the rows one after another in every thread (12 us for 16 rows of 8 KB, 2.3 for one); this is one memory latency behind
-// the index.  An index outside the table ends the program, as it does there.
+// the index.  An index outside the table ends the program rather than reading there.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kNormThreads) void embedding_kernel(const int64_t *__restrict__ ids,
                                                                  const uint4 *__restrict__ table,

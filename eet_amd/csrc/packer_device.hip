@@ -1,14 +1,15 @@
 // The offline packer on the GPU: fp16 / fp32 [K][N] weights already resident in
-// HBM -> per-output-channel int8 + scales -> gfx950 tile layout, in two passes.
+// HBM -> per-output-channel int8 + scales -> gfx950 tile layout.
 //
 // Same results, bit for bit, as eet_quantize_int8 followed by eet_pack_gfx950
 // (packer.cc), i.e. as the reference's symmetric_quantize
 // (3rdparty/cutlass_kernels/cutlass_preprocessors.cc:581-678) in
 // EET_QUANT_REF128 mode: every step is a single correctly rounded IEEE fp32
-// operation (|x| and max, one multiply or divide for the scale, one divide per
-// weight, an exact round-half-away), so host and device cannot differ.  The
-// reference has no device quantiser; converting a checkpoint on the host costs
-// seconds per billion weights, here the time of reading it twice from HBM.
+// operation (|x| and max, one multiply or divide for the scale, the quotient, an
+// exact round-half-away), so host and device cannot differ; a product with the
+// reciprocal stands for the quotient only where both provably round to the same
+// integer.  The reference has no device quantiser; converting a checkpoint on the
+// host costs seconds per billion weights, here the time of reading it from HBM.
 //
 // HBM-bound.  Most matrices go in one pass that holds them in the registers of
 // the chip (quant_group_kernel; one_pass_wins has the rule and the times).  The

@@ -1102,8 +1102,8 @@ def quant_weights_torch(w, mode="ref128"):
 
 def quant_weights_device(origin_weight, return_unprocessed_quantized_tensor=False, mode="ref128"):
     """quant_weights for a weight that already lives on the GPU (fp16 / fp32
-    [K, N], K % 64 == 0, N % 16 == 0): two HIP kernels instead of the host
-    threads, same bits.  Returns [processed, scales] or [unprocessed,
+    [K, N], K % 64 == 0, N % 16 == 0): HIP kernels, one pass over the matrix
+    or two, instead of the host threads, same bits.  Returns [processed, scales] or [unprocessed,
     processed, scales] like quant_weights, as GPU tensors.  The reference
     only quantises CPU tensors (fpA_intB_gemm_wrapper.cu:33)."""
     w = origin_weight
