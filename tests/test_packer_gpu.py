@@ -138,7 +138,8 @@ def test_converter_on_device(gpu):
 def test_one_pass_matches_two_passes(gpu, K, N, dtype):
     """The one-pass kernel at the edges of its shares (rows a workgroup holds, one to sixteen workgroups per column
     group, groups cut off by N) and with NaN and infinite weights, against the two-pass kernels, which a call with no
-    more than 4 N bytes of workspace takes, and the host packer.  Exact: every step is one correctly rounded operation."""
+    more than 4 N bytes of workspace takes, and the host packer.  (fp16 2624 x 16400 takes two passes either way; fp16 in the
+    8-wavefront form is test_eight_wavefronts_fp16.)  Exact: every step is one correctly rounded operation."""
     from eet_amd._lib import check, lib
     w = tricky(K, N, dtype, K * 3 + N)
     w[K // 2, 8], w[K - 1, 9], w[:, 10], w[5, 11] = np.nan, np.inf, np.nan, np.nan

@@ -1,7 +1,7 @@
 """eet_gemm_w8a16_qkv: the split of a prompt's fused Q | K | V rows in the epilogue of the large-M product, for every block
 shape, against the product and eet_qkv_split as two calls on the same block shape.  The epilogue rounds to fp16 where the
 product stores and rotates that value in fp32 as the split kernel does, each result rounded once; to the bit where the
-products are exact (the last test).  On random weights the bound leaves room for a product that one form rounds by way of
+products are exact (test_same_rotation_as_the_split_kernel).  On random weights the bound leaves room for a product that one form rounds by way of
 fp32 and the other directly, as the compiler likes: the same but for one in some 2^12 values, and there both inputs of a
 rotation and its result are at most one unit of fp16 off, each 2^-10 of the pair's length at most and 2^-11 in the mean of
 the numbers between two powers of two: bound 2^-9."""
