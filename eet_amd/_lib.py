@@ -27,6 +27,7 @@ SIGNATURES = {
     "eet_quantize_pack_device_shape": (_i, [_i, _sz, _sz, _i, _sz, _vp, _vp]),
     "eet_gemm_w8a16": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _vp, _sz, _vp]),
     "eet_gemm_w8a16_workspace": (_sz, [_i, _i, _i, _i]),
+    "eet_gemm_w8a16_zeroed_workspace": (_sz, [_i, _i, _i, _i]),
     "eet_gemm_w8a16_fused": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _f, _vp, _sz, _vp]),
     "eet_gemm_w8a16_residual_norm": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp, _f, _vp, _vp, _sz, _vp]),
     "eet_gemm_w8a16_large_m_shape": (_i, [_i, _i, _i, _i, _sz, _vp, _vp, _vp, _vp, _vp]),
@@ -64,6 +65,8 @@ SIGNATURES = {
     "eet_head_f16": (_i, [_vp, _l, _vp, _vp, _i, _i, _i, _vp]),
     "eet_prefill_attention": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
 }
+
+ZEROED_WORKSPACE = 1 << 63     # EET_ZEROED_WORKSPACE
 
 _lib = None
 

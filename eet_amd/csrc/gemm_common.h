@@ -65,6 +65,7 @@ struct GemmArgs {
     size_t ws_bytes;
     hipStream_t st;
     QkvOut qkv = {};  // kEpiQkv
+    bool ws_zeroed = false;  // the caller vouches for the small-M kernel's counters in ws (EET_ZEROED_WORKSPACE)
     int chain = 0;  // kChainOff / kChainFirst / kChainNext (chain.h; small-M kernel only)
     // RMSnorm of the finished rows, beside them (large-M kernel only): norm_out = RMSnorm(C) * norm_gamma, or null
     const _Float16 *norm_gamma = nullptr;

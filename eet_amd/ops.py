@@ -22,7 +22,7 @@ import threading
 
 import torch
 
-from ._lib import check, lib
+from ._lib import ZEROED_WORKSPACE, check, lib
 
 _EMPTY = torch.empty(0)
 
@@ -238,16 +238,16 @@ RMS_FUSE_MAX_M = 32     # the RMSnorm prologue exists in the small-M kernel only
 
 
 def _k_split_ws(M, N, K, epilogue, device):
-    """(pointer, bytes) of the small-M kernel's k-split workspace for this call, or (None, 0).  A buffer of its
-    own, zero when created (the arrival counters at its start must start at zero; every call leaves them so).
+    """(pointer, bytes | ZEROED_WORKSPACE) of the small-M kernel's k-split workspace for this call, or (None, 0).  A buffer
+    of its own, zero when created (the arrival counters at its start must start at zero; every call leaves them so).
     One buffer per device, like every named workspace here (and like the reference's MManager buffers,
     csrc/op/mmanager.hpp:141-205): the ops of a process are meant to run on one stream; launches on two
     streams that can overlap in time must not share it."""
-    need = lib().eet_gemm_w8a16_workspace(M, N, K, epilogue) if M <= RMS_FUSE_MAX_M else 0
+    need = lib().eet_gemm_w8a16_zeroed_workspace(M, N, K, epilogue) if M <= RMS_FUSE_MAX_M else 0
     if not need:
         return None, 0
     buf = workspaces.get("gemm_small_m_k_split", (need + 3) // 4, torch.float32, device, zero=True)
-    return buf.data_ptr(), buf.numel() * 4
+    return buf.data_ptr(), buf.numel() * 4 | ZEROED_WORKSPACE
 
 
 def _gemm(a, w, scale, out, M, N, K, epilogue=EPI_NONE, residual=None, rms_gamma=None, rms_eps=0.0):

@@ -130,8 +130,7 @@ int eet_quantize_pack_device_shape(int w_dtype, size_t K, size_t N, int unproces
  * (fpA_intB_gemm_template.h:443-495, cutlass_heuristic.cc:80-84):
  *   M > 32   a launch that has too few tiles to fill the chip (M in the tens to
  *            hundreds): raw fp32 sums, added in a second small kernel;
- *   M <= 32  a launch without the RMSnorm prologue whose N leaves about one 16-channel
- *            tile per CU (the O and down projections at N = 4096 / 5120): 2 or 4
+ *   M <= 32  a launch without the RMSnorm prologue and SwiGLU: 2 or 4
  *            workgroups share a group of tiles, exchange their fp32 sums through the
  *            workspace and the last one to arrive finishes them -- one launch.
  *            For this use the first 32 KiB of the workspace (its arrival counters)
@@ -139,7 +138,15 @@ int eet_quantize_pack_device_shape(int w_dtype, size_t K, size_t N, int unproces
  *            call leaves them zero.  Keep such a workspace for
  *            M <= 32 calls only (an M > 32 call writes partial sums over the
  *            counters), and never hand one workspace to two calls that can overlap
- *            in time.
+ *            in time.  A workspace is looked at by the calls with N = 4096 / 5120 (the
+ *            O and down projections with about one 16-channel tile per CU), of which
+ *            eet_gemm_w8a16_workspace tells; at every other N what M <= 32 calls are
+ *            handed is not touched, whatever it holds, unless the caller vouches for it:
+ * workspace_bytes | EET_ZEROED_WORKSPACE says that the rules above hold for this
+ * workspace.  An M <= 32 call may then split at any N, for which it can use
+ * eet_gemm_w8a16_zeroed_workspace bytes (at least those of eet_gemm_w8a16_workspace;
+ * 0: no split; fewer are accepted).  Every call that takes such a workspace takes the
+ * flag, the operator-level ones included; with M > 32 it is EET_ERR_INVALID_ARGUMENT.
  * Replaces fastertransformer::gemm_fp16_int_bias_act<uint8_t>
  * (3rdparty/cutlass_kernels/fpA_intB_gemm.cu:35-62) as called with
  * bias = nullptr and no activation from csrc/op/llama_mmha.cpp:313-337,
@@ -148,6 +155,8 @@ int eet_gemm_w8a16(const void *A, const void *Wpacked, const void *scale, void *
                    int M, int N, int K, void *workspace, size_t workspace_bytes,
                    void *stream);
 size_t eet_gemm_w8a16_workspace(int M, int N, int K, int epilogue);
+#define EET_ZEROED_WORKSPACE ((size_t)1 << 63)
+size_t eet_gemm_w8a16_zeroed_workspace(int M, int N, int K, int epilogue);
 
 /* The same GEMM with a fused epilogue.
  *   EET_EPILOGUE_NONE      C[M][N] as above.
@@ -188,12 +197,12 @@ int eet_gemm_w8a16_residual_norm(const void *A, const void *Wpacked, const void 
 /* The launch shape the small-M kernel (1 <= M <= 32) runs a call with: n-tiles per
  * workgroup, wavefronts per workgroup, k-tiles per register batch, and how many
  * workgroups share a tile's k range (1, 2 or 4; what a call runs with when it hands
- * over the workspace eet_gemm_w8a16_workspace asks for -- without it, 1) -- the tuning
- * override EET_GEMM_SMALL_M_CONFIG when a kernel of that shape exists for the
+ * over the workspace eet_gemm_w8a16_zeroed_workspace asks for, with the flag -- without
+ * a workspace, 1) -- the tuning override EET_GEMM_SMALL_M_CONFIG when a kernel of that shape exists for the
  * call, otherwise the table's choice.  For sweeps and for tests that must know
  * which variant ran.  It also checks, on the host, that the library holds a kernel
- * for what the table answers in every form of the call (with the workspace,
- * without it, chained) and fails with EET_ERR_INVALID_ARGUMENT if not.  The
+ * for what the table answers in every form of the call (with the workspace and the
+ * flag, with the workspace, without it, chained) and fails with EET_ERR_INVALID_ARGUMENT if not.  The
  * reference's counterpart is the CutlassGemmConfig its
  * heuristic returns (cutlass_heuristic.cc:106-207). */
 int eet_gemm_w8a16_small_m_shape(int M, int N, int K, int epilogue, int rms_prologue, int *nt,
@@ -394,7 +403,8 @@ int eet_kv_cache_gather_rows(const void *k_src, const void *v_src, void *k_dst, 
  * their fp16 scales; the other arguments are those of eet_mmha_decode.
  * gemm_workspace: optional (NULL / 0), the eet_gemm_w8a16 workspace of the output
  * projection, eet_gemm_w8a16_workspace(B, hidden, H*dh, EET_EPILOGUE_RESIDUAL) bytes
- * under that function's rules (counters zero before first use).
+ * under that function's rules (counters zero before first use), or
+ * eet_gemm_w8a16_zeroed_workspace bytes | EET_ZEROED_WORKSPACE.
  * Replaces LlamaMmha::forward_inc (csrc/op/llama_mmha.cpp:202-266) and
  * BaichuanMmha::forward_inc (csrc/op/baichuan_mmha.cpp:166-216) without the
  * beam reorder, which stays a separate call (eet_kv_cache_reorder). */
@@ -423,7 +433,7 @@ int eet_mmha_int8_decode_beams(const void *x, const void *rms_gamma, float rms_e
  * (+ x when add_residual).  act_buf [B][d_ff] is scratch; out [B][hidden] must
  * not alias x.  gemm_workspace: optional (NULL / 0), the eet_gemm_w8a16 workspace of
  * the down projection, eet_gemm_w8a16_workspace(B, hidden, d_ff, epilogue) bytes under
- * that function's rules.  Replaces GatedFeedForwardNetworkInt8::forward
+ * that function's rules, or those of eet_gemm_w8a16_zeroed_workspace with its flag.  Replaces GatedFeedForwardNetworkInt8::forward
  * (csrc/op/gated_ffn_int8.cpp:98-132) at decode sizes. */
 int eet_gated_ffn_int8_decode(const void *x, const void *rms_gamma, float rms_eps, const void *w01,
                               const void *scale01, const void *w2, const void *scale2,

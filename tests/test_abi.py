@@ -66,6 +66,16 @@ def test_device_entry_points_validate_before_launch():
     assert L.eet_gemm_w8a16_workspace(16, 4096, 11008, 1) == 32768 + 64 * 4 * 4 * 1 * 1024      # NT 4, 4 shares
     assert L.eet_gemm_w8a16_workspace(8, 5120, 13696, 1) == 32768 + 64 * 4 * 5 * 1 * 1024       # NT 5, 4 shares
     assert L.eet_gemm_w8a16_workspace(32, 4096, 4096, 2) == 0                                     # not with SwiGLU
+    for M, N, K in ((1, 1024, 8192), (16, 3072, 8192), (32, 2048, 5632)):   # other channel counts: where the caller vouches for it
+        assert L.eet_gemm_w8a16_workspace(M, N, K, 1) == 0 and L.eet_gemm_w8a16_zeroed_workspace(M, N, K, 1) > 32768
+        assert L.eet_gemm_w8a16_zeroed_workspace(M, N, K, 2) == 0
+    assert L.eet_gemm_w8a16_zeroed_workspace(32, 4096, 4096, 1) == L.eet_gemm_w8a16_workspace(32, 4096, 4096, 1)
+    assert L.eet_gemm_w8a16_zeroed_workspace(40, 2048, 5632, 1) == 0 and L.eet_gemm_w8a16_zeroed_workspace(8, 2048, 5600, 1) == 0
+    zeroed = 1 << 20 | _lib.ZEROED_WORKSPACE
+    assert L.eet_gemm_w8a16(p, p, p, p, 33, 16, 64, p, zeroed, None) == -1    # more rows would write over its counters
+    assert L.eet_gemm_w8a16_fused(p, p, p, p, 33, 16, 64, 0, None, None, 0.0, p, zeroed, None) == -1
+    assert L.eet_gemm_w8a16_residual_norm(p, p, p, p, 33, 16, 64, p, p, 1e-6, p, p, zeroed, None) == -1
+    assert L.eet_gemm_w8a16_qkv(p, p, p, p, p, p, p, None, 1, 33, 1, 32, 64, 40, p, zeroed, None) == -1
     assert L.eet_gemm_w8a16_workspace(2048, 4096, 4096, 0) == 0
     need = L.eet_gemm_w8a16_workspace(64, 4096, 11008, 0)
     assert need >= 2 * 64 * 4096 * 4 and need % (64 * 4096 * 4) == 0

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import eet_amd
-from eet_amd._lib import check, lib
+from eet_amd._lib import ZEROED_WORKSPACE, check, lib
 from oracle import ops as O
 
 from gpu_util import assert_close, stream
@@ -34,7 +34,7 @@ def test_picked_shape(gpu, M, N, K, want):
     u, p, s = eet_amd.quant_weights(w, torch.int8, True)
     x, res = torch.randn(M, K, generator=g).half(), torch.randn(M, N, generator=g).half()
     ref = O.dequant_matmul(x.numpy(), u.numpy(), s.numpy())
-    need = lib().eet_gemm_w8a16_workspace(M, N, K, 1)
+    need = lib().eet_gemm_w8a16_zeroed_workspace(M, N, K, 1)
     assert (need > 0) == (got[3] > 1)
     ws = torch.zeros(need + 16, dtype=torch.uint8, device=gpu)
     xd, pd, sd, rd = x.to(gpu), p.to(gpu), s.to(gpu), res.to(gpu)
@@ -42,8 +42,52 @@ def test_picked_shape(gpu, M, N, K, want):
         for _ in range(2):                                     # the arrival counters are zero again
             out = torch.full((M + 1, N), 7.25, dtype=torch.float16, device=gpu)
             check(lib().eet_gemm_w8a16_fused(xd.data_ptr(), pd.data_ptr(), sd.data_ptr(), out.data_ptr(), M, N, K, 1,
-                                             rd.data_ptr(), None, 0.0, ws.data_ptr() if given else None, given, stream()))
+                                             rd.data_ptr(), None, 0.0, ws.data_ptr() if given else None, given | (ZEROED_WORKSPACE if given else 0),
+                                             stream()))
             c = out.cpu()
             assert (c[M] == 7.25).all() and not ws[:32768].any()
             # the product is within 1e-2 / 1e-3 of the oracle; the fp16 sum with the residual adds half an ulp of at most 8
             assert_close(c[:M].numpy(), ref + res.numpy().astype(np.float32), atol=5e-3, what=f"{M} {N} {K} {given}")
+
+
+# 4 shares, or 2, where the caller vouches for its counters; nothing to be asked for, and nothing touched, where it does not
+@pytest.mark.parametrize("M,N,K", [(1, 1024, 8192), (16, 3072, 8192), (32, 2048, 5632), (32, 1040, 2112)])
+def test_a_workspace_nobody_vouches_for_is_left_alone(gpu, M, N, K):
+    """The caller's buffer for calls of more than 32 rows, say, whose sums lie where the arrival counters would."""
+    assert lib().eet_gemm_w8a16_workspace(M, N, K, 1) == 0 and shape(M, N, K, 1, 0)[3] > 1
+    g = torch.Generator().manual_seed(M + N + K)
+    w = (torch.randn(K, N, generator=g) * 0.02).half()
+    u, p, s = eet_amd.quant_weights(w, torch.int8, True)
+    x, res = torch.randn(M, K, generator=g).half(), torch.randn(M, N, generator=g).half()
+    want = O.dequant_matmul(x.numpy(), u.numpy(), s.numpy()) + res.numpy().astype(np.float32)
+    xd, pd, sd, rd = x.to(gpu), p.to(gpu), s.to(gpu), res.to(gpu)
+    ws = torch.full((1 << 23,), 1, dtype=torch.uint8, device=gpu)
+    for bytes_ in (ws.numel(), (1 << 63) - 1, (1 << 64) - 1):          # a large enough size, however it is put, says nothing
+        out = torch.full((M, N), float("nan"), dtype=torch.float16, device=gpu)
+        check(lib().eet_gemm_w8a16_fused(xd.data_ptr(), pd.data_ptr(), sd.data_ptr(), out.data_ptr(), M, N, K, 1, rd.data_ptr(),
+                                         None, 0.0, ws.data_ptr(), bytes_, stream()))
+        assert_close(out.cpu().numpy(), want, atol=5e-3, what=f"{M} {N} {K}")
+        assert (ws == 1).all()
+
+
+def test_an_operator_call_leaves_it_alone_too(gpu):
+    M, hidden, d_ff = 32, 2048, 5632
+    g = torch.Generator().manual_seed(7)
+    w01, w2 = (torch.randint(0, 256, (n,), dtype=torch.uint8, generator=g).to(gpu) for n in (hidden * 2 * d_ff, d_ff * hidden))
+    s01, s2 = ((torch.rand(n, generator=g) * 1e-4).half().to(gpu) for n in (2 * d_ff, hidden))
+    x, gamma = torch.randn(M, hidden, generator=g).half().to(gpu), torch.ones(hidden, dtype=torch.float16, device=gpu)
+    act = torch.empty(M, d_ff, dtype=torch.float16, device=gpu)
+
+    def ffn(ws, nbytes):
+        out = torch.full((M, hidden), float("nan"), dtype=torch.float16, device=gpu)
+        check(lib().eet_gated_ffn_int8_decode(x.data_ptr(), gamma.data_ptr(), 1e-6, w01.data_ptr(), s01.data_ptr(), w2.data_ptr(),
+                                              s2.data_ptr(), act.data_ptr(), out.data_ptr(), M, hidden, d_ff, 1,
+                                              ws.data_ptr() if ws is not None else None, nbytes, stream()))
+        return out
+    dirty = torch.full((1 << 23,), 1, dtype=torch.uint8, device=gpu)
+    assert torch.equal(ffn(dirty, dirty.numel()), ffn(None, 0)) and (dirty == 1).all()
+    need = lib().eet_gemm_w8a16_zeroed_workspace(M, hidden, d_ff, 1)
+    ws = torch.zeros(need, dtype=torch.uint8, device=gpu)
+    split = ffn(ws, need | ZEROED_WORKSPACE)
+    assert ws[32768:].any() and not ws[:32768].any()                   # it was used, and can be used again
+    assert_close(split.cpu().numpy(), ffn(None, 0).float().cpu().numpy(), what="4 shares and one")
