@@ -809,8 +809,11 @@ namespace {
 
 // Largest split launch the static entry point takes: B*H*nsplit <= 512 partial
 // records of (max, sum, acc[dh <= 128]) floats.  plan_by_pairs splits only when
-// B*H < 256 and never into more than ceil(256 / (B*H)) parts, which fits
-// (B*H*nsplit < 256 + B*H); other cuts are considered only where they fit.
+// B*H < 256 and step >= 512 and never into more than ceil(256 / (B*H)) parts, which
+// fits (B*H*nsplit < 256 + B*H).  These calls, and no others, use the array, with
+// choose_plan's cut where it fits: callers on two streams rely on their other
+// launches (32 heads at 200 rows, 288 .. 384 pairs of head size 64 / 96, which are
+// faster with a split and a workspace of their own) not meeting in it.
 constexpr size_t kScratchRecords = 512;
 constexpr size_t kScratchFloats = kScratchRecords * (128 + 2);
 
@@ -848,8 +851,10 @@ extern "C" int eet_mmha_decode_static(const void *q, const void *k, const void *
 {
     Plan plan;
     if (int rc = check_mmha_args("eet_mmha_decode_static", q, k, v, qkv_stride, k_cache, v_cache, ctx, B, H, dh, step,
-                                 T_cap, rope_cos_sin, kScratchFloats * sizeof(float), &plan))
+                                 T_cap, rope_cos_sin, 0, &plan))
         return rc;
+    if (plan_by_pairs(B * H, dh, step).nsplit > 1)   // cannot do without the array
+        plan = pick_plan(B * H, dh, step, kScratchFloats * sizeof(float));
     const size_t need = partial_bytes(B * H, dh, plan);
     EET_REQUIRE(need <= kScratchFloats * sizeof(float), EET_ERR_WORKSPACE,
                 "eet_mmha_decode_static: B*H*nsplit = %d*%d*%d partial records (%zu bytes) exceed the static scratch of "

@@ -265,7 +265,10 @@ int eet_chain_status(int *gave_up, int clear, void *stream);
  *             at decode time.  Needs k, v != NULL.
  *   workspace eet_mmha_decode_workspace(B, H, dh, step) bytes of device memory, any
  *             contents; less, or none, is accepted and the launch cut accordingly
- *             unless B*H < 256 and step >= 512 (about B*H * 256 / (B*H) records then)
+ *             unless B*H < 256 and step >= 512, where a call needs at least
+ *             B*H * min(ceil(256 / (B*H)), step / 256) * (dh + 2) * 4 bytes.  Calls with
+ *             B*H < 512 may write to what they are handed, also where that much is
+ *             not needed: two calls that can overlap in time must not share it.
  * softmax denominator carries the reference's + 1e-6.
  * Replaces masked_attention_dispatch (csrc/core/attention_dispatch.cu:888-928)
  * and fused_masked_attention_dispatch with q_bias == nullptr (:1338-1426). */
@@ -299,13 +302,14 @@ int eet_mmha_decode_beams(const void *q, const void *k, const void *v, long qkv_
 /* eet_mmha_decode for callers that cannot allocate device memory or carry a
  * workspace around: code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc.  It has no counterpart in the reference.  Same
- * arguments and results as eet_mmha_decode, without the workspace: the partial
- * results of a split launch (B*H < 256) live in a static device array of
+ * arguments and results as eet_mmha_decode, without the workspace: calls that need
+ * one there (B*H < 256 and step >= 512) are cut to fit a static device array of
  * eet_mmha_decode_static_capacity() bytes (260 KiB) that every GPU the library
- * runs on holds until the process ends.  Calls no hipMalloc / hipFree.  A call
- * whose B*H*nsplit*(dh+2)*4 bytes exceed the capacity (only reachable through a
- * tuning override) fails with EET_ERR_WORKSPACE.  All calls on one GPU share the
- * array: calls that overlap in time on different streams of one GPU race;
+ * runs on holds until the process ends, for their partial results; no other call
+ * uses it, these are run as eet_mmha_decode runs them without a workspace.  Calls
+ * no hipMalloc / hipFree.  A call whose B*H*nsplit*(dh+2)*4 bytes exceed the capacity (only reachable through a
+ * tuning override) fails with EET_ERR_WORKSPACE.  The calls that use it share the
+ * array of a GPU: two of them that overlap in time on different streams race;
  * nothing needs clearing between calls.  The first call on each GPU looks the
  * array's device address up (hipGetSymbolAddress, a runtime query that may load
  * the code object): make that first call OUTSIDE a stream capture (one warm call

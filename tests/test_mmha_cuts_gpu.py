@@ -54,3 +54,24 @@ def test_cut_by_estimate(gpu, B, H, dh, step, usual, best, padded):
         assert (ws[given:] == 255).all()
     if least:
         assert run(least - 4)[0] == -4                             # what the usual cut needs is asked for as ever
+
+
+# the three that a workspace of their own splits although they can do without one
+@pytest.mark.parametrize("B,H,dh,step", [(1, 32, 128, 200), (18, 16, 64, 1300), (9, 32, 96, 1000)])
+def test_static_array_is_for_calls_that_need_a_workspace(gpu, B, H, dh, step):
+    """Two streams may run such calls side by side: a launch that shares the array has the sums of other cuts."""
+    L, cap = lib(), step + 2
+    assert records(B, H, dh, L.eet_mmha_decode_workspace(B, H, dh, step)) > 1
+    g = torch.Generator().manual_seed(step)
+    kc, vc = (torch.randn(B, H, cap, dh, generator=g).half().to(gpu) for _ in range(2))
+    q, k, v = (torch.randn(B, H, dh, generator=g).half().to(gpu) for _ in range(3))
+
+    def run(fn, *ws):
+        ctx = torch.empty(B, H * dh, dtype=torch.float16, device=gpu)
+        assert fn(q.data_ptr(), k.data_ptr(), v.data_ptr(), 0, kc.data_ptr(), vc.data_ptr(), ctx.data_ptr(), None, None, B, H, dh,
+                  step, cap, None, *ws, stream()) == 0
+        return ctx
+    own = torch.empty(L.eet_mmha_decode_workspace(B, H, dh, step), dtype=torch.uint8, device=gpu)
+    got, alone = run(L.eet_mmha_decode_static), run(L.eet_mmha_decode, None, 0)
+    split = run(L.eet_mmha_decode, own.data_ptr(), own.numel())
+    assert torch.equal(got, alone) and not torch.equal(got, split)
