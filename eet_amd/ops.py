@@ -67,7 +67,11 @@ class _Workspaces:
         key = (name, device, dtype)
         buf = self._bufs.get(key)
         if buf is None or buf.numel() < numel:
-            alloc = torch.zeros if zero else torch.empty      # zero: a buffer whose first use needs zeros
+            # zero: a buffer whose first use needs zeros.  None while a graph is being recorded, which would write them
+            # when it is replayed: an eager call ahead of that would find none.
+            if zero and torch.cuda.is_current_stream_capturing():
+                return None
+            alloc = torch.zeros if zero else torch.empty
             buf = alloc(max(int(numel), 1), dtype=dtype, device=device)
             self._bufs[key] = buf
         for handed in self._recorders:
@@ -247,6 +251,8 @@ def _k_split_ws(M, N, K, epilogue, device):
     if not need:
         return None, 0
     buf = workspaces.get("gemm_small_m_k_split", (need + 3) // 4, torch.float32, device, zero=True)
+    if buf is None:
+        return None, 0
     return buf.data_ptr(), buf.numel() * 4 | ZEROED_WORKSPACE
 
 

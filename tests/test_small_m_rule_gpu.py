@@ -91,3 +91,40 @@ def test_an_operator_call_leaves_it_alone_too(gpu):
     split = ffn(ws, need | ZEROED_WORKSPACE)
     assert ws[32768:].any() and not ws[:32768].any()                   # it was used, and can be used again
     assert_close(split.cpu().numpy(), ffn(None, 0).float().cpu().numpy(), what="4 shares and one")
+
+
+@pytest.mark.parametrize("hidden,d_ff", [(2048, 5632), (4096, 11008)])
+def test_recorded_first_then_called(gpu, hidden, d_ff):
+    """An op whose first call is recorded into a graph, with no eager call ahead, and is called before the first replay: the
+    counters of a buffer that the graph alone would zero are not used.  (Split and unsplit products round to neighbouring fp16
+    values, 2^-8 apart below 8.)"""
+    from eet_amd import ops
+    M, g, e = 32, torch.Generator(device=gpu).manual_seed(11), torch.empty(0)
+    desc = ops.MetaDesc(dtype=torch.float16, batch_size=M, head_num=hidden // 128, hidden_units=hidden, layer_num=1, max_seq_len=1,
+                        max_full_seq_len=8, activation_fn="silu", d_ff=d_ff, cuda_device="cuda:0", is_int8=True)
+    mats = [ops.quant_weights_device(torch.randn(k, n, generator=g, device=gpu).half() * 0.02)
+            for k, n in ((hidden, d_ff), (hidden, d_ff), (d_ff, hidden))]
+    ffn = ops.GatedFeedForwardNetworkInt8(desc, *mats[0], e, *mats[1], e, *mats[2], e,
+                                          torch.ones(hidden, dtype=torch.float16, device=gpu), e)
+    x = torch.randn(M, 1, hidden, generator=g, device=gpu).half()
+    want = ffn.forward(x, True, True).clone()
+    other = ffn.forward(x * 2, True, True).clone()
+    torch.cuda.synchronize()
+    ops.workspaces.clear()
+    pool, filler, graph = torch.cuda.graph_pool_handle(), torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(filler, pool=pool):      # memory that another graph of the program has used before
+        junk = torch.full((1 << 25,), 77, dtype=torch.int32, device=gpu)
+    filler.replay()
+    torch.cuda.synchronize()
+    del junk
+    with torch.cuda.graph(graph, pool=pool):
+        recorded = ffn.forward(x, True, True)
+    got = ffn.forward(x * 2, True, True)
+    assert_close(got.float().cpu().numpy(), other.float().cpu().numpy(), atol=5e-3, what="before the first replay")
+    for _ in range(3):
+        recorded.fill_(float("nan"))
+        graph.replay()
+        assert_close(recorded.float().cpu().numpy(), want.float().cpu().numpy(), atol=5e-3, what="replay")
+        assert_close(ffn.forward(x * 2, True, True).float().cpu().numpy(), other.float().cpu().numpy(), atol=5e-3, what="eager, between")
+    del recorded, got
+    ops.workspaces.clear()        # the graph's own memory goes with it
