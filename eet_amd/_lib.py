@@ -63,6 +63,7 @@ SIGNATURES = {
     "eet_kv_cache_reorder": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "eet_kv_cache_gather_rows": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "eet_head_f16": (_i, [_vp, _l, _vp, _vp, _i, _i, _i, _vp]),
+    "eet_head_f16_shape": (_i, [_i, _i, _i, _vp]),
     "eet_prefill_attention": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
 }
 

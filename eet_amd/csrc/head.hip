@@ -241,13 +241,29 @@ int head_tiles(int tiles, int M, int K)
 
 }  // namespace
 
+static int check_head_sizes(const char *fn, int M, int N, int K)
+{
+    EET_REQUIRE(M > 0 && M <= 16 && N > 0 && K > 0 && K % 64 == 0 && N % 16 == 0, EET_ERR_UNSUPPORTED_SHAPE,
+                "%s: need 1 <= M <= 16, K %% 64 == 0 and N %% 16 == 0, got M=%d N=%d K=%d", fn, M, N, K);
+    EET_REQUIRE((size_t)N * K <= ((size_t)1 << 28), EET_ERR_UNSUPPORTED_SHAPE,
+                "%s: a matrix of %d x %d is larger than 2^28 elements", fn, N, K);
+    return EET_OK;
+}
+
+extern "C" int eet_head_f16_shape(int M, int N, int K, int *tiles)
+{
+    EET_REQUIRE(tiles, EET_ERR_INVALID_ARGUMENT, "eet_head_f16_shape: null pointer");
+    if (int rc = check_head_sizes("eet_head_f16_shape", M, N, K))
+        return rc;
+    *tiles = head_tiles(N / 16, M, K);
+    return EET_OK;
+}
+
 extern "C" int eet_head_f16(const void *x, long x_stride, const void *w, void *out, int M, int N, int K, void *stream)
 {
     EET_REQUIRE(x && w && out, EET_ERR_INVALID_ARGUMENT, "eet_head_f16: null pointer");
-    EET_REQUIRE(M > 0 && M <= 16 && N > 0 && K > 0 && K % 64 == 0 && N % 16 == 0, EET_ERR_UNSUPPORTED_SHAPE,
-                "eet_head_f16: need 1 <= M <= 16, K %% 64 == 0 and N %% 16 == 0, got M=%d N=%d K=%d", M, N, K);
-    EET_REQUIRE((size_t)N * K <= ((size_t)1 << 28), EET_ERR_UNSUPPORTED_SHAPE,
-                "eet_head_f16: a matrix of %d x %d is larger than 2^28 elements", N, K);
+    if (int rc = check_head_sizes("eet_head_f16", M, N, K))
+        return rc;
     EET_REQUIRE(x_stride >= K && x_stride % 8 == 0 && ((size_t)(M - 1) * x_stride + K) * 2 <= ((size_t)1 << 31),
                 EET_ERR_INVALID_ARGUMENT, "eet_head_f16: x_stride %ld must be a multiple of 8, at least K", x_stride);
     EET_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) % 16 == 0, EET_ERR_INVALID_ARGUMENT,

@@ -477,6 +477,11 @@ int eet_embedding_f16(const int64_t *ids, const void *table, void *out, int M, i
 int eet_head_f16(const void *x, long x_stride, const void *w, void *out, int M, int N, int K,
                  void *stream);
 
+/* What eet_head_f16 runs a call of these sizes as (host only, for sweeps and for tests that
+ * must know which kernel ran): *tiles = 1, 2 or 4 tiles of 16 columns per workgroup, or 0,
+ * one workgroup per CU that walks over the tiles with the activations in LDS. */
+int eet_head_f16_shape(int M, int N, int K, int *tiles);
+
 /* Causal prefill attention over the prompt, reading K and V from the caches
  * filled by eet_qkv_split.  q [B][H][S][dh]; ctx [B][S][H*dh]; alibi NULL or
  * [H][S] half (slope * j, the diagonal row of the reference's mask); pad as in

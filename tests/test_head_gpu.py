@@ -1,10 +1,12 @@
 """The fp16 output head (eet_head_f16, ops.head) against an fp32 product."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from eet_amd import ops
-from eet_amd._lib import lib
+from eet_amd._lib import check, lib
 
 
 def test_argument_errors():
@@ -119,6 +121,34 @@ def test_one_workgroup_per_cu(gpu, M, S, N, K):
     w = (torch.randn(N, K, device=gpu) * 0.02).half()
     first = ops.head(h, w)
     assert all(torch.equal(first, ops.head(h, w)) for _ in range(3))
+
+
+def tiles(M, N, K):
+    v = ctypes.c_int(-1)
+    check(lib().eet_head_f16_shape(M, N, K, ctypes.byref(v)))
+    return v.value
+
+
+def test_which_kernel():
+    """What the sizes of the two tests above run as."""
+    assert [tiles(*s) for s in ((1, 8016, 448), (16, 6144, 1088), (5, 10256, 2048))] == [2, 2, 4]
+    assert all(tiles(*s) == 0 for s in ((16, 20480, 3072), (2, 18432, 4096), (16, 40960, 1024), (9, 24624, 3136), (1, 20480, 1536),
+                                        (12, 40976, 2560), (16, 24576, 4096)))
+    assert tiles(5, 20496, 1088) == 2
+    v, L = ctypes.c_int(), lib()
+    assert [L.eet_head_f16_shape(M, N, K, ctypes.byref(v)) for M, N, K in ((0, 16, 64), (17, 16, 64), (1, 24, 64), (1, 16, 96),
+                                                                           (1, 1 << 20, 512))] == [-2] * 5
+    assert L.eet_head_f16_shape(1, 16, 64, None) == -1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,S,N,K,form", [(2, 1, 17632, 6144, 1), (1, 1, 20752, 2048, 2), (16, 2, 20480, 5120, 2),
+                                          (16, 1, 17632, 512, 4),          # several rounds of workgroups
+                                          (9, 1, 16400, 1088, 0),          # one or two k blocks per wavefront and tile, and
+                                          (16, 2, 20496, 1088, 0)])        # the last turn with one tile
+def test_kernel_by_size(gpu, M, S, N, K, form):
+    assert tiles(M, N, K) == form
+    test_one_workgroup_per_cu(gpu, M, S, N, K)
 
 
 @pytest.mark.gpu
