@@ -538,9 +538,20 @@ float plan_us(int BH, int dh, int step, const Plan &p)
 // plan_by_pairs.  Over those problems this takes 0.94 of the time of plan_by_pairs (0.92 under 128 pairs, 0.94 under 256,
 // 0.98 above; 0.82 at best, 1.03 at worst), without the margin 0.94 as well, but 1.12 at worst.  us, plan_by_pairs / here,
 // heads of 128: 1 x 32, 200 rows 7.7 / 5.9, 513 9.4 / 7.2; 4 x 40, 1024 22.0 / 18.7, 3001 49.7 / 40.9; 8 x 40, 2048 69 / 56.
-Plan choose_plan(int BH, int dh, int step, size_t bytes)
+//
+// A launch that is replayed has one cut for every step up to `step` (step_max): one that is not ahead of plan_by_pairs at
+// step, step / 2, step / 4, ... 16 alike is not taken.  (A second kernel for a split costs 2 us whatever the step: 8 x 40
+// pairs in a cache of 4096 rows, no split / four, 32 rows 8.8 / 11.5, 256 14.5 / 15.8, 1024 35 / 34, 4096 129 / 110;
+// 1 x 16 of 64, 2048, eight splits / sixteen, 64 rows 5.9 / 7.1, 1024 7.1 / 7.7.)
+Plan choose_plan(int BH, int dh, int step, size_t bytes, bool replayed)
 {
     const Plan usual = plan_by_pairs(BH, dh, step);
+    auto never_behind = [&](const Plan &p) {
+        for (int s = step; s >= 16; s /= 2)
+            if (plan_us(BH, dh, s, p) > plan_us(BH, dh, s, usual))
+                return false;
+        return true;
+    };
     if (BH >= 512 || partial_bytes(BH, dh, usual) > bytes)   // (a call that lacks that workspace is refused)
         return usual;
     Plan best = usual;
@@ -551,7 +562,7 @@ Plan choose_plan(int BH, int dh, int step, size_t bytes)
         for (int threads : {256, 512})
             for (int ring : {2, 4}) {
                 const Plan p{threads, nsplit, ring};
-                if (partial_bytes(BH, dh, p) > bytes)
+                if (partial_bytes(BH, dh, p) > bytes || (replayed && !never_behind(p)))
                     continue;
                 if (const float us = plan_us(BH, dh, step, p); us < best_us)
                     best = p, best_us = us;
@@ -560,13 +571,13 @@ Plan choose_plan(int BH, int dh, int step, size_t bytes)
     return best;
 }
 
-Plan pick_plan(int BH, int dh, int step, size_t bytes)
+Plan pick_plan(int BH, int dh, int step, size_t bytes, bool replayed)
 {
     static thread_local eet::RecentAnswers<Plan, 8> recent;   // a decoder's layers ask for the same one
     const eet::Tuning &tune = eet::tuning();
-    Plan p = recent.get(BH, dh, step, 0, [&] { return choose_plan(BH, dh, step, ~(size_t)0); });
+    Plan p = recent.get(BH, dh, step, replayed, [&] { return choose_plan(BH, dh, step, ~(size_t)0, replayed); });
     if (partial_bytes(BH, dh, p) > bytes)
-        p = choose_plan(BH, dh, step, bytes);
+        p = choose_plan(BH, dh, step, bytes, replayed);
     if (tune.mmha_nsplit > 0 || tune.mmha_threads > 0 || tune.mmha_ring > 0) {
         const int forced_threads = tune.mmha_threads, forced_ring = tune.mmha_ring;
         p = plan_by_pairs(BH, dh, step);
@@ -664,19 +675,21 @@ extern "C" int eet_rope_table(float *table, int T, int dh, void *stream)
     return EET_OK;
 }
 
-extern "C" size_t eet_mmha_decode_workspace(int B, int H, int dh, int step)
+static size_t mmha_workspace(int B, int H, int dh, int step, bool replayed)
 {
     if (B <= 0 || H <= 0 || dh <= 0 || step <= 0)
         return 0;
     const size_t usual = partial_bytes(B * H, dh, plan_by_pairs(B * H, dh, step));   // what a call cannot do without
-    const size_t need = partial_bytes(B * H, dh, pick_plan(B * H, dh, step, ~(size_t)0));
+    const size_t need = partial_bytes(B * H, dh, pick_plan(B * H, dh, step, ~(size_t)0, replayed));
     return need > usual ? need : usual;
 }
+
+extern "C" size_t eet_mmha_decode_workspace(int B, int H, int dh, int step) { return mmha_workspace(B, H, dh, step, false); }
 
 // Argument checks shared by the entry points; fills `plan`.
 static int check_mmha_args(const char *fn, const void *q, const void *k, const void *v, long qkv_stride,
                            const void *k_cache, const void *v_cache, const void *ctx, int B, int H, int dh, int step,
-                           int T_cap, const float *rope_cos_sin, size_t workspace_bytes, Plan *plan)
+                           int T_cap, const float *rope_cos_sin, size_t workspace_bytes, Plan *plan, bool replayed = false)
 {
     EET_REQUIRE(q && k_cache && v_cache && ctx, EET_ERR_INVALID_ARGUMENT, "%s: null pointer", fn);
     EET_REQUIRE((k == nullptr) == (v == nullptr), EET_ERR_INVALID_ARGUMENT,
@@ -690,7 +703,7 @@ static int check_mmha_args(const char *fn, const void *q, const void *k, const v
                 "%s: qkv_stride must be a non-negative multiple of 8", fn);
     EET_REQUIRE(rope_cos_sin == nullptr || k != nullptr, EET_ERR_INVALID_ARGUMENT,
                 "%s: a rotary row needs the new k, v (it rotates q and the appended k)", fn);
-    *plan = pick_plan(B * H, dh, step, workspace_bytes);
+    *plan = pick_plan(B * H, dh, step, workspace_bytes, replayed);
     return EET_OK;
 }
 
@@ -776,7 +789,7 @@ extern "C" int eet_step_advance(int *step_dev, int by, void *stream)
 
 extern "C" size_t eet_mmha_decode_replayable_workspace(int B, int H, int dh, int step_max)
 {
-    return eet_mmha_decode_workspace(B, H, dh, step_max);
+    return mmha_workspace(B, H, dh, step_max, true);
 }
 
 extern "C" int eet_mmha_decode_replayable(const void *q, const void *k, const void *v, long qkv_stride, void *k_cache,
@@ -791,7 +804,7 @@ extern "C" int eet_mmha_decode_replayable(const void *q, const void *k, const vo
                 step_max, alibi_ld);
     Plan plan;
     if (int rc = check_mmha_args("eet_mmha_decode_replayable", q, k, v, qkv_stride, k_cache, v_cache, ctx, B, H, dh,
-                                 step_max, T_cap, rope_table, workspace ? workspace_bytes : 0, &plan))
+                                 step_max, T_cap, rope_table, workspace ? workspace_bytes : 0, &plan, true))
         return rc;
     const size_t need = partial_bytes(B * H, dh, plan);
     EET_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), EET_ERR_WORKSPACE,
@@ -854,7 +867,7 @@ extern "C" int eet_mmha_decode_static(const void *q, const void *k, const void *
                                  T_cap, rope_cos_sin, 0, &plan))
         return rc;
     if (plan_by_pairs(B * H, dh, step).nsplit > 1)   // cannot do without the array
-        plan = pick_plan(B * H, dh, step, kScratchFloats * sizeof(float));
+        plan = pick_plan(B * H, dh, step, kScratchFloats * sizeof(float), false);
     const size_t need = partial_bytes(B * H, dh, plan);
     EET_REQUIRE(need <= kScratchFloats * sizeof(float), EET_ERR_WORKSPACE,
                 "eet_mmha_decode_static: B*H*nsplit = %d*%d*%d partial records (%zu bytes) exceed the static scratch of "

@@ -279,3 +279,18 @@ def test_packer_grids_and_workspace():
 def test_packer_takes_the_faster_way(w_dtype, K, N, unprocessed, waves):
     """Either side of every line of the rule."""
     assert pack_shape(w_dtype, K, N, None, unprocessed)[0] == waves
+
+
+def test_cuts_of_replayed_attention():
+    """A launch that is replayed keeps its cut at every step up to step_max: a split that long caches gain by and short ones
+    lose by is for the calls that are cut anew at each step."""
+    L = _lib.lib()
+
+    def records(fn, B, H, dh, step):
+        return fn(B, H, dh, step) // (B * H * (dh + 2) * 4)
+    for size, once, replayed in (((8, 40, 128, 1024), 4, 0), ((8, 40, 128, 4096), 4, 0), ((12, 32, 96, 2048), 4, 0),
+                                 ((1, 32, 128, 256), 8, 0), ((1, 16, 64, 2048), 16, 8),
+                                 ((4, 40, 128, 2048), 8, 6), ((1, 32, 128, 1024), 8, 8), ((4, 40, 128, 1024), 3, 3),
+                                 ((8, 32, 128, 4096), 0, 0), ((1, 32, 128, 1), 0, 0)):
+        assert records(L.eet_mmha_decode_workspace, *size) == once, size
+        assert records(L.eet_mmha_decode_replayable_workspace, *size) == replayed, size
