@@ -66,7 +66,7 @@ def test_device_entry_points_validate_before_launch():
     assert L.eet_gemm_w8a16_workspace(16, 4096, 11008, 1) == 32768 + 64 * 4 * 4 * 1 * 1024      # NT 4, 4 shares
     assert L.eet_gemm_w8a16_workspace(8, 5120, 13696, 1) == 32768 + 64 * 4 * 5 * 1 * 1024       # NT 5, 4 shares
     assert L.eet_gemm_w8a16_workspace(32, 4096, 4096, 2) == 0                                     # not with SwiGLU
-    for M, N, K in ((1, 1024, 8192), (16, 3072, 8192), (32, 2048, 5632)):   # other channel counts: where the caller vouches for it
+    for M, N, K in ((8, 1024, 8192), (16, 3072, 8192), (32, 2048, 5632)):   # other channel counts: where the caller vouches for it
         assert L.eet_gemm_w8a16_workspace(M, N, K, 1) == 0 and L.eet_gemm_w8a16_zeroed_workspace(M, N, K, 1) > 32768
         assert L.eet_gemm_w8a16_zeroed_workspace(M, N, K, 2) == 0
     assert L.eet_gemm_w8a16_zeroed_workspace(32, 4096, 4096, 1) == L.eet_gemm_w8a16_workspace(32, 4096, 4096, 1)
@@ -294,3 +294,16 @@ def test_cuts_of_replayed_attention():
                                  ((8, 32, 128, 4096), 0, 0), ((1, 32, 128, 1), 0, 0)):
         assert records(L.eet_mmha_decode_workspace, *size) == once, size
         assert records(L.eet_mmha_decode_replayable_workspace, *size) == replayed, size
+
+
+def test_small_m_shapes_of_a_few_rows():
+    """A launch of one to seven rows is not shaped as one of eight: with few activations a split costs more than it saves."""
+    v = [ctypes.c_int() for _ in range(4)]
+
+    def shape(M, N, K):
+        assert _lib.lib().eet_gemm_w8a16_small_m_shape(M, N, K, 1, 0, *[ctypes.byref(x) for x in v]) == 0
+        return tuple(x.value for x in v)
+    for M, N, K, want in ((1, 3072, 8192, (1, 8, 2, 1)), (2, 3072, 8192, (1, 8, 2, 1)), (1, 4080, 11008, (1, 16, 1, 1)),
+                          (2, 2560, 6912, (1, 16, 1, 1)), (17, 1024, 2816, (1, 16, 1, 1)), (32, 3072, 8192, (3, 8, 1, 4)),
+                          (16, 3072, 8192, (3, 8, 1, 4)), (8, 4096, 16384, (1, 8, 2, 1)), (1, 4096, 11008, (1, 16, 1, 1))):
+        assert shape(M, N, K) == want, (M, N, K, shape(M, N, K))

@@ -51,7 +51,7 @@ def test_picked_shape(gpu, M, N, K, want):
 
 
 # 4 shares, or 2, where the caller vouches for its counters; nothing to be asked for, and nothing touched, where it does not
-@pytest.mark.parametrize("M,N,K", [(1, 1024, 8192), (16, 3072, 8192), (32, 2048, 5632), (32, 1040, 2112)])
+@pytest.mark.parametrize("M,N,K", [(8, 1024, 8192), (16, 3072, 8192), (32, 2048, 5632), (32, 1040, 2112)])
 def test_a_workspace_nobody_vouches_for_is_left_alone(gpu, M, N, K):
     """The caller's buffer for calls of more than 32 rows, say, whose sums lie where the arrival counters would."""
     assert lib().eet_gemm_w8a16_workspace(M, N, K, 1) == 0 and shape(M, N, K, 1, 0)[3] > 1
