@@ -447,6 +447,8 @@ __global__ __launch_bounds__(THREADS) void mmha_decode_split_kernel(
 #endif
 }
 
+constexpr int kHeld = 8;   // splits that the merge requests at once
+
 template <int DH>
 __global__ __launch_bounds__(DH) void mmha_decode_merge_kernel(const float *__restrict__ partial,
                                                                _Float16 *__restrict__ ctx, int nsplit)
@@ -456,7 +458,6 @@ __global__ __launch_bounds__(DH) void mmha_decode_merge_kernel(const float *__re
     // Two loops over the splits -- the maximum, then the sums -- are two memory latencies after another, and more where
     // a load waits for the one before.  Up to kHeld splits are requested at once instead (past the last that one again):
     // six 4096-wide layers at batch 1 and 3001 rows, four steps, 1512 -> 1481 us.
-    constexpr int kHeld = 8;
     float ms[kHeld], part_sum[kHeld], part_acc[kHeld];
 #pragma unroll
     for (int s = 0; s < kHeld; ++s) {
@@ -523,7 +524,8 @@ Plan plan_by_pairs(int BH, int dh, int step)
 // What a launch takes, about, us: launch and merge in LDS by the width of a workgroup and by the wavefronts of the busiest
 // CU, a second kernel for a split, and the streaming, where a stream's chain of rows (two or four in flight), the busiest
 // CU's bytes and HBM each hold the others up in part.  Fitted to 813 problems of up to 511 pairs (16 .. 40 heads, batch
-// 1 .. 32, 16 .. 4096 rows, head sizes 64 / 96 / 128, all cuts of up to 16 splits), where it is 4 % off.
+// 1 .. 32, 16 .. 4096 rows, head sizes 64 / 96 / 128, all cuts of up to 16 splits), where it is 4 % off.  More than kHeld
+// splits are merged one latency after another (1 x 12 of 128, 2393 rows, 8 / 9 / 16 splits 10.1 / 10.6 / 12.4 us).
 float plan_us(int BH, int dh, int step, const Plan &p)
 {
     const int streams = p.threads / lanes_per_row(dh), per = (step + p.nsplit - 1) / p.nsplit;
@@ -531,18 +533,20 @@ float plan_us(int BH, int dh, int step, const Plan &p)
     const float lat = (float)((per + streams - 1) / streams) * (p.ring == 2 ? 0.287f : 0.193f);
     const float cu = 0.0167f * rounds * per * dh / 256.f, hbm = 0.117f * (float)BH * step * dh * 4e-6f;
     return 2.7f + (p.ring == 2 ? 0.37f : 0.57f) * rounds * p.threads / 256.f + 0.31f * p.threads / 256.f +
-           __builtin_sqrtf(lat * lat + cu * cu + hbm * hbm) + (p.nsplit > 1 ? 1.96f + 0.068f * p.nsplit : 0.f);
+           __builtin_sqrtf(lat * lat + cu * cu + hbm * hbm) + (p.nsplit > 1 ? 1.96f + 0.068f * p.nsplit : 0.f) +
+           (p.nsplit > kHeld ? 1.2f : 0.f);
 }
 
 // Up to 511 pairs: the cut with the least plan_us that `bytes` of workspace allow, where it is at least 4 % under that of
 // plan_by_pairs.  Over those problems this takes 0.94 of the time of plan_by_pairs (0.92 under 128 pairs, 0.94 under 256,
-// 0.98 above; 0.82 at best, 1.03 at worst), without the margin 0.94 as well, but 1.12 at worst.  us, plan_by_pairs / here,
+// 0.98 above; 0.82 at best), without the margin 0.94 as well, but 1.12 at worst; over 170 others (8 .. 40 heads) 0.93, 1.04 at
+// worst, and 1.17 where 16 splits counted as if merged at once.  us, plan_by_pairs / here,
 // heads of 128: 1 x 32, 200 rows 7.7 / 5.9, 513 9.4 / 7.2; 4 x 40, 1024 22.0 / 18.7, 3001 49.7 / 40.9; 8 x 40, 2048 69 / 56.
 //
 // A launch that is replayed has one cut for every step up to `step` (step_max): one that is not ahead of plan_by_pairs at
 // step, step / 2, step / 4, ... 16 alike is not taken.  (A second kernel for a split costs 2 us whatever the step: 8 x 40
 // pairs in a cache of 4096 rows, no split / four, 32 rows 8.8 / 11.5, 256 14.5 / 15.8, 1024 35 / 34, 4096 129 / 110;
-// 1 x 16 of 64, 2048, eight splits / sixteen, 64 rows 5.9 / 7.1, 1024 7.1 / 7.7.)
+// 12 x 32 of 96, 2048, none / four, 64 rows 8.4 / 10.4, 1536 46.2 / 43.5.)
 Plan choose_plan(int BH, int dh, int step, size_t bytes, bool replayed)
 {
     const Plan usual = plan_by_pairs(BH, dh, step);

@@ -289,7 +289,9 @@ def test_cuts_of_replayed_attention():
     def records(fn, B, H, dh, step):
         return fn(B, H, dh, step) // (B * H * (dh + 2) * 4)
     for size, once, replayed in (((8, 40, 128, 1024), 4, 0), ((8, 40, 128, 4096), 4, 0), ((12, 32, 96, 2048), 4, 0),
-                                 ((1, 32, 128, 256), 8, 0), ((1, 16, 64, 2048), 16, 8),
+                                 ((1, 32, 128, 256), 8, 0),
+                                 # more than eight splits are merged one after another: no more than the usual nine, or eight
+                                 ((1, 12, 128, 2393), 9, 9), ((1, 16, 64, 2048), 8, 8),
                                  ((4, 40, 128, 2048), 8, 6), ((1, 32, 128, 1024), 8, 8), ((4, 40, 128, 1024), 3, 3),
                                  ((8, 32, 128, 4096), 0, 0), ((1, 32, 128, 1), 0, 0)):
         assert records(L.eet_mmha_decode_workspace, *size) == once, size
