@@ -693,16 +693,18 @@ PackPlan plan_pack(size_t K, size_t N, bool unprocessed, size_t ws_bytes)
     const size_t units = K / kUnit, groups = (N + GroupShape<T>::kGroup - 1) / GroupShape<T>::kGroup;
     const int wide = parts_of(units, groups, 16, 4, 256), narrow = parts_of(units, groups, 8, 5, 512);
     const bool fits = wide <= kMaxParts && groups * wide <= 256;
-    // Groups of fp16 columns shared by workgroups that leave more than a sixth of the slots empty, or that are three
-    // and more to a group and a few too many for one round: the two passes, which have neither, are ahead from 11 M weights
-    // on (us, two passes / one, by the share of the slots: 0.67 2560 x 11008 28.0 / 33.2; 0.69 2048 x 5632 16.2 / 17.0,
-    // 4096 x 5632 25.1 / 30.0; 0.77 6144 x 4224 25.8 / 28.0; 0.81 5120 x 6656 33.3 / 37.3; 0.82 2560 x 8960 23.7 / 23.3; 1.01
-    // 3072 x 11008 33.2 / 38.2; 1.03 4096 x 8448 33.1 / 40.0.  From 0.85 to 1 one pass takes 0.87 .. 1.06 of the two; with the
-    // row-major output 2048 x 5632 17.5 / 18.2, 4096 x 5632 28.3 / 31.4).  Groups with a workgroup each
-    // need no exchange and stay (1216 x 12288, 0.75: 17.9 / 15.4).
-    const size_t slots = fits ? 256 : 512, total = groups * (fits ? wide : narrow);
-    const bool idle = sizeof(T) == 2 && total > groups && K * N > 11000000 &&
-                      (total * 100 < slots * 84 || (total > slots && total * 10 <= slots * 11 && total >= 3 * groups));
+    // Groups of fp16 columns shared by workgroups that leave more than 18 % of the slots empty, or that are three and more
+    // to a group and a few too many for one round: the two passes, which have neither, are ahead where a workgroup's
+    // wavefronts hold two units and more (2048 rows) and the matrix has 11 M weights, 16 M with three workgroups to a group.  Measured
+    // at 158 sizes of 11-36 M weights, two passes / one, by the share of the slots: up to 0.75 0.84 .. 1.04 (0.95 in the mean:
+    // 2560 x 11008 32.6 / 36.8 us, 4096 x 5632 28.5 / 32.9), to 0.82 0.81 .. 1.04 (0.95: 2432 x 12800 35.2 / 43.8, 5120 x
+    // 6656 38.3 / 42.9), to 0.84 0.98 .. 1.05, above 0.93 .. 1.12 (1.03), 1.01 .. 1.1 0.78 .. 0.89 (3072 x 11008 38.3 / 42.9).
+    // Left with one pass by the other lines: 1856 x 6208 (0.76) 20.9 / 18.9, 1728 x 6400 (0.78) 19.6 / 18.1, 2752 x 4224
+    // (0.77, three) 19.8 / 19.2.  Groups with a workgroup each need no exchange and stay (1216 x 12288, 0.75: 17.9 / 15.4).
+    const size_t slots = fits ? 256 : 512, parts = fits ? wide : narrow, total = groups * parts;
+    const bool idle = sizeof(T) == 2 && parts > 1 && units >= 64 && K * N > (parts > 2 ? 16000000 : 11000000) &&
+                      (total * 100 < slots * 82 || (total > slots && total * 10 <= slots * 11 && parts > 2));
+    // (threads of a grid are counted in 32 bits, and the kernel's column indices are int; a row of workgroups to spare)
     if (ws_bytes < eet_quantize_pack_device_workspace(N) || idle || !one_pass_wins<T>(K, N, unprocessed, fits) ||
         (!fits && (narrow > kMaxParts || groups * narrow >= ((size_t)1 << 32) / (64 * 8) - 64)))
         return {0, 0};

@@ -308,3 +308,18 @@ def test_idle_cus_take_two_passes():
     assert waves(2560, 10240) == 8 and waves(5120, 13696) == 8           # 480 of 512; several rounds
     assert waves(1024, 11008) == 16                                      # no group is shared
     assert waves(2048, 5632, 0) == 16                                    # fp32
+
+
+def test_idle_cus_that_do_not_matter():
+    """Sizes inside the range of the two-pass rule that measure faster, or no slower, in one: fewer than two units to a wavefront, three
+    workgroups to a group and under 16 M weights, 82 % of the slots taken.  And the other side of each line."""
+    import ctypes
+    from eet_amd._lib import check, lib
+
+    def waves(K, N):
+        w, p = ctypes.c_int(), ctypes.c_int()
+        check(lib().eet_quantize_pack_device_shape(1, K, N, 0, lib().eet_quantize_pack_device_workspace(N), ctypes.byref(w), ctypes.byref(p)))
+        return w.value
+    assert waves(1856, 6208) == 16 and waves(1984, 6144) == 16 and waves(2048, 6144) == 0
+    assert waves(2752, 4224) == 16 and waves(3712, 4160) == 16 and waves(4032, 4160) == 0
+    assert waves(2560, 8960) == 8 and waves(3136, 6784) == 16 and waves(2944, 6656) == 0 and waves(5120, 6656) == 0
