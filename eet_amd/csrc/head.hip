@@ -216,10 +216,12 @@ __global__ __launch_bounds__(64 * kResidentWaves) void head_resident_kernel(cons
 }
 
 // Tiles per workgroup, see above; 0: head_resident_kernel.  That one costs a tile and 210 k of start per turn, the
-// activations once, and its own start, more where its wavefronts have unequal parts; rows 8 KiB apart take head_kernel a
-// quarter longer than the sum says, rows an odd number of 4 KiB apart take this one 15 % longer.  Fewer than five turns
-// are left to head_kernel (4096 <- 1024 3.3 / 4.8 us).  Over 656 sizes (K 1024 .. 5120, N 4096 .. 128256, M 1 .. 16; weights
-// from HBM) the two take 0.956 of head_kernel's time, 0.71 at best, 1.03 at worst.
+// activations once, and its own start, more where its wavefronts have unequal parts; rows a multiple of 8 KiB apart take
+// head_kernel a quarter longer than the sum says (K = 8192, outside the fit, alike: 24576 rows M = 8 83.1 / 77.5 us, 32000 107.1
+// / 98.6, and this one ahead at all of ten sizes), rows 4 KiB apart take this one 15 % longer (12 KiB apart, outside the
+// fit, it would be ahead by 1 to 12 %).  Fewer than five turns are left to head_kernel (4096 <- 1024 3.3 / 4.8 us).  Over
+// 656 sizes (K 1024 .. 5120, N 4096 .. 128256, M 1 .. 16; weights from HBM) the two take 0.956 of head_kernel's time, 0.71 at
+// best, 1.03 at worst.
 int head_tiles(int tiles, int M, int K)
 {
     int best = 1;

@@ -1015,8 +1015,9 @@ def _head_kernel_wins(B, V, K):
     Measured over graph replays at K 512 .. 8192, V 1024 .. 256000, B 1 / 4 / 8 / 16, weights from HBM (832 sizes): 0.80
     of the library's time on the whole, behind it by more than 3 % at 27 sizes and at most 14 %; with the kernel
     everywhere and thresholds from four matrices it was 0.84, 177 sizes and 51 %.  K = 4096, us, kernel / library, B = 1
-    and 16: V 4096 8.3 / 12.8 and 10.2 / 13.0, 10240 19.5 / 19.5 and 22.6 / 20.1, 20480 31.2 / 54.5 and 41.4 / 55.2, 32000
-    48.4 / 56.4 and 51.3 / 57.6, 50272 78.0 / 85.2 and 89.7 / 86.7."""
+    and 16: V 4096 8.3 / 12.8 and 10.2 / 13.0, 10240 19.5 / 19.5 and 22.6 / 20.1; with the kernel of one workgroup per CU,
+    which came after that fit, 20480 31.2 / 56.0 and 34.5 / 56.1, 32000 47.4 / 58.3 and 51.3 / 59.3, 50272 75.1 / 90.1 and
+    81.8 / 90.6 (K = 3072 .. 5120 that are no multiple of 2048, where the library stays: 0.95 .. 1.10 of its time)."""
     if K > 6144:                    # its workgroups each read every activation
         return False
     if 8192 < V < 16000:            # one to four tiles per CU, in broken rounds: the library splits K
